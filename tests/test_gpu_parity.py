@@ -486,6 +486,42 @@ def test_find_leaf_rejects_foreign_child_index(dev, reps):
     assert list(want["status"]) == [2, 0, 0] * reps
 
 
+@pytest.mark.parametrize("dim,nodes", [(3, 40000), (2, 70000), (3, 200), (2, (1 << 23) + 3)])
+def test_find_leaf_table_of_any_octree(dev, dim, nodes):
+    """Tables over octrees no build writes: leaves whose data is not -1,
+    child indexes outside the octree, descents that end within the table,
+    one level below it and deeper; past 2^23 nodes the table's entries are
+    the wide ones.  Every field equals the oracle's."""
+    rng = np.random.default_rng(nodes)
+    nc, used = 1 << dim, min(nodes, 70000)
+    children = np.full((nodes, nc), -1, np.int32)
+    leaf = np.full(nodes, (1 << nc) - 1, np.int32)
+    # a tree over the last `used` nodes, breadth first, all of the root and 60% of the others inner
+    ids = np.concatenate([[0], rng.permutation(np.arange(nodes - used + 1, nodes))])
+    nxt = 1
+    for i in ids[: used // 2]:
+        for o in np.nonzero((rng.random(nc) < 0.6) | (i == 0))[0]:
+            if nxt < used:
+                children[i, o] = ids[nxt]
+                leaf[i] &= ~(1 << int(o))
+                nxt += 1
+    pick = ids[rng.integers(0, used, used // 4)]
+    o = rng.integers(0, nc, pick.size)
+    is_leaf = (leaf[pick] >> o) & 1 == 1
+    children[pick[is_leaf], o[is_leaf]] = rng.integers(0, 99, int(is_leaf.sum()))   # data
+    bad = ids[rng.integers(1, max(used // 100, 8), max(used // 1000, 3))]
+    children[bad, 0] = rng.choice([nodes, nodes + 7, -3], bad.size)
+    leaf[bad] &= ~1                                                                # foreign
+    bits = 12
+    q = rng.integers(0, 1 << bits, (300000, dim)).astype(np.int32)
+    got = dev.find_leaf(q, bits, children, leaf)
+    want = oracle.find_leaf(q, bits, children, leaf)
+    for k in ("parent", "octant", "data", "level", "status"):
+        assert np.array_equal(got[k].astype(np.int64), want[k].astype(np.int64)), k
+    assert set(np.unique(want["status"])) >= {0, 2}
+    assert (want["data"][want["status"] == 0] >= 0).any()
+
+
 # ----------------------------------------------------- reference data ----
 def _data_points():
     path = os.path.join(os.path.dirname(__file__), "golden", "data_points.npz")
