@@ -30,7 +30,6 @@ struct pgvd_batch {
   std::vector<int64_t> h_m, h_O, h_koff, h_ooff;
   // device
   SegInfo *seg = nullptr;
-  uint32_t *kofs = nullptr;
   SegState *ss = nullptr;
   SegState *ss_host = nullptr;      // pinned
   RunState *st = nullptr;
@@ -38,10 +37,11 @@ struct pgvd_batch {
   uint32_t *tables = nullptr;
   BatchDev dev;
   void *keys_a = nullptr, *keys_b = nullptr, *brt = nullptr;
-  uint32_t *ps = nullptr, *defer = nullptr;
+  uint32_t *ps = nullptr, *row_tot = nullptr;
+  uint64_t *miss_words = nullptr;
   int32_t *parent = nullptr;
   char *zero = nullptr;
-  size_t zero_bytes = 0, off_hist = 0, off_sort = 0, off_lbu = 0, off_lbl = 0;
+  size_t zero_bytes = 0, off_hist = 0, off_sort = 0, off_lbu = 0;
   int32_t *octree = nullptr;
   int64_t oct_cap = 0;
   hipGraph_t graph = nullptr;
@@ -101,7 +101,7 @@ void release_graph(pgvd_batch *b) {
   b->graph_pts = nullptr;
 }
 
-// (Re)builds the five tile tables for the plan's sort_ipt / brt_rows, and the
+// (Re)builds the tile tables for the plan's sort_ipt / brt_rows, and the
 // look-back workspace they size.
 int build_tables(pgvd_batch *b) {
   const std::vector<SegInfo> &si = b->h_seg;
@@ -109,7 +109,8 @@ int build_tables(pgvd_batch *b) {
   const HostTable sort = make_table(si, (int64_t)b->sort_ipt * kBlock, [](const SegInfo &x) { return (int64_t)x.n; });
   const HostTable scan = make_table(si, kScanTile, [](const SegInfo &x) { return (int64_t)x.n + 1; });
   const HostTable brt = make_table(si, (int64_t)b->brt_rows * kBlock, [](const SegInfo &x) { return (int64_t)x.n + 1; });
-  const HostTable node = make_table(si, kBlock, [](const SegInfo &x) { return (int64_t)x.n + 1; });
+  const HostTable node = make_table(si, kGatherTile, [](const SegInfo &x) { return (int64_t)x.n + 1; });
+  const HostTable row = make_table(si, kBlock, [](const SegInfo &x) { return (int64_t)x.n + 1; });
   std::vector<uint32_t> all;
   size_t off[10];
   const HostTable *ts[5] = {&chunk, &sort, &scan, &brt, &node};
@@ -119,6 +120,8 @@ int build_tables(pgvd_batch *b) {
     off[2 * i + 1] = all.size();
     all.insert(all.end(), ts[i]->first.begin(), ts[i]->first.end());
   }
+  const size_t off_row = all.size();
+  all.insert(all.end(), row.first.begin(), row.first.end());
   dfree(b->tables);
   CHK(dalloc(&b->tables, all.size() * 4));
   HIPCHK(hipMemcpy(b->tables, all.data(), all.size() * 4, hipMemcpyHostToDevice));
@@ -130,21 +133,21 @@ int build_tables(pgvd_batch *b) {
     tt[i]->first = b->tables + off[2 * i + 1];
     *cnt[i] = (int64_t)ts[i]->seg.size();
   }
+  d.row_first = b->tables + off_row;
+  d.row_tot = b->row_tot;
   d.sort_ipt = b->sort_ipt;
   d.brt_rows = b->brt_rows;
   d.digit_bits = b->digit_bits;
   d.sort_waves = b->sort_waves;
   b->passes = (b->mbits + b->digit_bits - 1) / b->digit_bits;
   // zero-initialised workspace: digit histograms, sort look-back (all
-  // passes), unique and local-split scan look-back
+  // passes), unique look-back
   size_t o = 0;
   b->off_hist = o;
   o += align256((size_t)b->B * b->passes * 256 * 4);
   b->off_sort = o;
   o += align256((size_t)b->passes * (size_t)d.n_sort * 256 * 4);
   b->off_lbu = o;
-  o += align256((size_t)d.n_scan * 8);
-  b->off_lbl = o;
   o += align256((size_t)d.n_scan * 8);
   if (o > b->zero_bytes) {
     dfree(b->zero);
@@ -186,11 +189,11 @@ void enqueue_typed(pgvd_batch *b, const void *pts) {
                        s);
   uint32_t *lsx = reinterpret_cast<uint32_t *>(sorted);   // free after unique
   launch_brt_seg<K>(uniq, b->mbits, b->dim, d, static_cast<BrtNodeT<K> *>(b->brt), b->parent,
-                    lsx, b->defer, b->st, s);
-  launch_ls_scan_seg(lsx, b->ps, d, reinterpret_cast<uint64_t *>(b->zero + b->off_lbl), b->st, s);
+                    lsx, b->miss_words, b->st, s);
+  launch_chunk_scan_seg(d, s);
   launch_oct_offsets(d, b->st, s);
   launch_gather_seg<K>(static_cast<const BrtNodeT<K> *>(b->brt), b->ps, lsx, b->dim, d,
-                       b->octree, b->oct_cap, b->defer, b->st, s);
+                       b->octree, b->oct_cap, b->miss_words, b->st, s);
 }
 
 void enqueue(pgvd_batch *b, const void *pts) {
@@ -238,7 +241,7 @@ void regather_typed(pgvd_batch *b) {
   K *sorted = static_cast<K *>(b->parity ? b->keys_b : b->keys_a);
   launch_gather_seg<K>(static_cast<const BrtNodeT<K> *>(b->brt), b->ps,
                        reinterpret_cast<const uint32_t *>(sorted), b->dim, b->dev, b->octree,
-                       b->oct_cap, b->defer, b->st, b->s);
+                       b->oct_cap, b->miss_words, b->st, b->s);
 }
 
 int finish_impl(pgvd_batch *b) {
@@ -248,7 +251,7 @@ int finish_impl(pgvd_batch *b) {
   uint32_t stt = b->st_host->status;
   if (stt & ST_CAPACITY) {
     // grow to the reported total and fill again from the kept BRT / prefix
-    // sums; the gather appended nothing to its overflow list when it failed
+    // sums
     const int64_t need = (int64_t)b->st_host->octree_size;
     CHK(ensure_octree(b, need + need / 8 + 1024));
     b->st_host->status &= ~(uint32_t)ST_CAPACITY;
@@ -336,7 +339,6 @@ int pgvd_batch_create(pgvd_ctx *ctx, const int64_t *sizes, int64_t count, int di
   b->h_m.assign(count, 0);
   b->h_O.assign(count, 0);
   b->h_ooff.assign(count, 0);
-  std::vector<uint32_t> kofs(count + 1);
   int64_t p = 0, k = 0;
   for (int64_t i = 0; i < count; ++i) {
     SegInfo si{};
@@ -346,25 +348,21 @@ int pgvd_batch_create(pgvd_ctx *ctx, const int64_t *sizes, int64_t count, int di
     si.prepend = ref_next_pow2((int)sizes[i]) != sizes[i] ? 1u : 0u;   // padding (Q1)
     b->h_seg[i] = si;
     b->h_koff[i] = k;
-    kofs[i] = (uint32_t)k;
     p += sizes[i];
     k += sizes[i] + 1;
   }
-  kofs[count] = (uint32_t)k;
   auto bail = [&](int rc) {
     pgvd_batch_destroy(b);
     return rc;
   };
   int rc;
   if ((rc = dalloc(&b->seg, count * sizeof(SegInfo)))) return bail(rc);
-  if ((rc = dalloc(&b->kofs, (count + 1) * 4))) return bail(rc);
   if ((rc = dalloc(&b->ss, count * sizeof(SegState)))) return bail(rc);
   if ((rc = dalloc(&b->st, sizeof(RunState)))) return bail(rc);
   if (hipHostMalloc((void **)&b->ss_host, count * sizeof(SegState)) != hipSuccess ||
       hipHostMalloc((void **)&b->st_host, sizeof(RunState)) != hipSuccess)
     return bail(fail(PGVD_ERR_ALLOC, "hipHostMalloc failed"));
-  if (hipMemcpy(b->seg, b->h_seg.data(), count * sizeof(SegInfo), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(b->kofs, kofs.data(), (count + 1) * 4, hipMemcpyHostToDevice) != hipSuccess)
+  if (hipMemcpy(b->seg, b->h_seg.data(), count * sizeof(SegInfo), hipMemcpyHostToDevice) != hipSuccess)
     return bail(fail(PGVD_ERR_HIP, "batch table upload failed"));
   const size_t kbytes = (size_t)slots * b->kb;
   if ((rc = dalloc(&b->keys_a, kbytes))) return bail(rc);
@@ -373,9 +371,11 @@ int pgvd_batch_create(pgvd_ctx *ctx, const int64_t *sizes, int64_t count, int di
   if ((rc = dalloc(&b->brt, (size_t)slots * nb))) return bail(rc);
   if ((rc = dalloc(&b->ps, (size_t)slots * 4))) return bail(rc);
   if ((rc = dalloc(&b->parent, (size_t)slots * 4))) return bail(rc);
-  if ((rc = dalloc(&b->defer, (size_t)slots * 4))) return bail(rc);
+  // a sum per row of 256 key slots; a miss word per 64 key slots of a tile of
+  // at most 1024 (the BRT's and the gather's in turn)
+  if ((rc = dalloc(&b->row_tot, (size_t)(slots / kBlock + count) * 4))) return bail(rc);
+  if ((rc = dalloc(&b->miss_words, (size_t)(slots / 64 + 16 * count) * 8))) return bail(rc);
   b->dev.seg = b->seg;
-  b->dev.kofs = b->kofs;
   b->dev.ss = b->ss;
   b->dev.B = count;
   if ((rc = build_tables(b))) return bail(rc);
@@ -392,7 +392,6 @@ int pgvd_batch_destroy(pgvd_batch *b) {
   (void)hipStreamSynchronize(b->s);
   release_graph(b);
   dfree(b->seg);
-  dfree(b->kofs);
   dfree(b->ss);
   dfree(b->st);
   if (b->ss_host) (void)hipHostFree(b->ss_host);
@@ -403,7 +402,8 @@ int pgvd_batch_destroy(pgvd_batch *b) {
   dfree(b->brt);
   dfree(b->ps);
   dfree(b->parent);
-  dfree(b->defer);
+  dfree(b->row_tot);
+  dfree(b->miss_words);
   dfree(b->zero);
   dfree(b->octree);
   if (b->ev0) (void)hipEventDestroy(b->ev0);

@@ -116,8 +116,8 @@ template <typename K> struct BrtWin { static constexpr int R = 4, H = 256; };
 // key probes.  A node whose range or split leaves the window is handed to
 // defer(true, c) and left to the global-memory pass.  lsx[m-1] = 0;
 // m == 1 gives lsx[0] = 1.  Every lane calls defer once per row, converged.
-// With chunk_tot, each row of 256 nodes (a chunk) also stores the sum of
-// its local splits, deferred nodes left out (their pass adds them).
+// Each row of 256 nodes (a chunk) also stores the sum of its local splits in
+// chunk_tot, deferred nodes left out (their pass adds them).
 template <typename K, int DIM, int R, typename Defer>
 __device__ inline void brt_window(const K *__restrict__ keys, int m, int b0, int mbits,
                                   BrtNodeT<K> *__restrict__ brt, int32_t *__restrict__ parent,
@@ -202,18 +202,14 @@ __device__ inline void brt_window(const K *__restrict__ keys, int m, int b0, int
       lsx[c] = ls;
     }
     defer(miss, c);
-    if (chunk_tot) {
-      const uint32_t sum = wave_reduce_add(ls);
-      if ((t & 63) == 0) s_rowsum[r * (kBlock / 64) + (t >> 6)] = sum;
-    }
+    const uint32_t sum = wave_reduce_add(ls);
+    if ((t & 63) == 0) s_rowsum[r * (kBlock / 64) + (t >> 6)] = sum;
   }
-  if (chunk_tot) {
-    __syncthreads();
-    if (threadIdx.x < R && b0 + (int)threadIdx.x * kBlock < m) {
-      uint32_t tot = 0;
-      for (int w = 0; w < kBlock / 64; ++w) tot += s_rowsum[threadIdx.x * (kBlock / 64) + w];
-      chunk_tot[(b0 >> 8) + threadIdx.x] = tot;
-    }
+  __syncthreads();
+  if (threadIdx.x < R && b0 + (int)threadIdx.x * kBlock < m) {
+    uint32_t tot = 0;
+    for (int w = 0; w < kBlock / 64; ++w) tot += s_rowsum[threadIdx.x * (kBlock / 64) + w];
+    chunk_tot[(b0 >> 8) + threadIdx.x] = tot;
   }
 }
 
@@ -265,56 +261,57 @@ __global__ __launch_bounds__(kBlock) void brt_ls_defer_kernel(const K *__restric
 }
 
 // Batched form: BRT tiles of R*256 key slots per instance (n+1 slots each);
-// instance s's arrays start at key slot kofs, m = ss[s].m.  Deferred nodes
-// are recorded by key slot.
+// instance s's arrays start at key slot kofs, its chunk sums at row_first[s],
+// m = ss[s].m.  Tile b's deferred nodes are marked in its own R * 4 words
+// (word R * 4 b + ..., one per 64 slots of the tile), as in the single-tree
+// form; one queue counter that every wave appends to took the pass of 384
+// instances (55 M points) from 0.5 to 1.1 ms.
 template <typename K, int DIM, int R>
-__global__ __launch_bounds__(kBlock) void brt_seg_kernel(const K *__restrict__ keys, int mbits,
-                                                         const SegInfo *__restrict__ seg,
-                                                         TileTable tt,
-                                                         const SegState *__restrict__ ss,
-                                                         BrtNodeT<K> *__restrict__ brt,
-                                                         int32_t *__restrict__ parent,
-                                                         uint32_t *__restrict__ lsx,
-                                                         uint32_t *__restrict__ defer,
-                                                         RunState *st) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PGVD_BRT_WPE))) void
+brt_seg_kernel(const K *__restrict__ keys, int mbits, const SegInfo *__restrict__ seg,
+               TileTable tt, const uint32_t *__restrict__ row_first,
+               const SegState *__restrict__ ss, BrtNodeT<K> *__restrict__ brt,
+               int32_t *__restrict__ parent, uint32_t *__restrict__ lsx,
+               uint32_t *__restrict__ chunk_tot, uint64_t *__restrict__ miss_words,
+               RunState *st) {
   constexpr int SEG = R * kBlock;
   const uint32_t tile = xcd_segment(blockIdx.x, gridDim.x);
   const uint32_t s = tt.seg[tile];
   const int m = (int)ss[s].m;
   const int b0 = (int)(tile - tt.first[s]) * SEG;
-  if (b0 >= m) return;
+  uint64_t *words = miss_words + (size_t)tile * (SEG / 64);
+  if (b0 >= m) {
+    if (threadIdx.x < SEG / 64) words[threadIdx.x] = 0;
+    return;
+  }
   const uint32_t kofs = seg[s].kofs;
-  brt_window<K, DIM, R>(keys + kofs, m, b0, mbits, brt + kofs, parent + kofs, lsx + kofs, nullptr, st,
-                        [&](bool miss, int c) {
-                          wave_append(miss, kofs + (uint32_t)c, &st->counters[CTR_BRT_DEFER],
-                                      defer);
+  brt_window<K, DIM, R>(keys + kofs, m, b0, mbits, brt + kofs, parent + kofs, lsx + kofs,
+                        chunk_tot + row_first[s], st, [&](bool miss, int c) {
+                          wave_mask(miss, words, (uint32_t)(c - b0) >> 6);
                         });
 }
 
-template <typename K, int DIM>
-__global__ __launch_bounds__(kBlock) void brt_seg_defer_kernel(const K *__restrict__ keys,
-                                                               int mbits,
-                                                               const uint32_t *__restrict__ kofs_all,
-                                                               uint32_t B,
-                                                               const SegState *__restrict__ ss,
-                                                               BrtNodeT<K> *__restrict__ brt,
-                                                               int32_t *__restrict__ parent,
-                                                               uint32_t *__restrict__ lsx,
-                                                               const uint32_t *__restrict__ defer,
-                                                               RunState *st) {
-  const uint32_t cnt = st->counters[CTR_BRT_DEFER];
-  for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < cnt; k += gridDim.x * kBlock) {
-    const uint32_t slot = defer[k];
-    const uint32_t s = find_seg(kofs_all, B, slot);
-    const uint32_t kofs = kofs_all[s];
-    const int c = (int)(slot - kofs);
+template <typename K, int DIM, int R>
+__global__ __launch_bounds__(kBlock) void brt_seg_defer_kernel(
+    const K *__restrict__ keys, int mbits, const SegInfo *__restrict__ seg, TileTable tt,
+    uint32_t ntiles, const uint32_t *__restrict__ row_first, const SegState *__restrict__ ss,
+    BrtNodeT<K> *__restrict__ brt, int32_t *__restrict__ parent, uint32_t *__restrict__ lsx,
+    uint32_t *__restrict__ chunk_tot, const uint64_t *__restrict__ miss_words, RunState *st) {
+  constexpr uint32_t SEG = R * kBlock;
+  for_each_masked(miss_words, ntiles * (SEG / 64), [&](uint32_t q) {
+    const uint32_t tile = q / SEG;
+    const uint32_t s = tt.seg[tile];
+    const uint32_t kofs = seg[s].kofs;
+    const int c = (int)((tile - tt.first[s]) * SEG + q % SEG);
     const int m = (int)ss[s].m;
     const K *kk = keys + kofs;
     const K cur = kk[c];
     const BrtOut<K> o = brt_eval_wide(cur, [&](int x) { return kk[x]; }, mbits, m, c);
     brt_flags(o, st);
-    (void)brt_store<K, DIM>(c, cur, o, mbits, brt + kofs, parent + kofs, lsx + kofs);
-  }
+    const uint32_t ls =
+        brt_store<K, DIM>(c, cur, o, mbits, brt + kofs, parent + kofs, lsx + kofs);
+    if (ls) atomicAdd(&chunk_tot[row_first[s] + ((uint32_t)c >> 8)], ls);
+  });
 }
 
 // Order-exact recomputation of the parent claims when some split was an
@@ -397,25 +394,28 @@ bool brt_seg_rows_ok(int key_bytes, int rows) {
 
 template <typename K, int DIM, int R>
 void brt_seg_dim(const K *keys, int mbits, const BatchDev &b, BrtNodeT<K> *brt, int32_t *parent,
-                 uint32_t *lsx, uint32_t *defer, RunState *st, hipStream_t s) {
-  brt_seg_kernel<K, DIM, R><<<(unsigned)b.n_brt, kBlock, 0, s>>>(keys, mbits, b.seg, b.brt, b.ss,
-                                                                 brt, parent, lsx, defer, st);
-  brt_seg_defer_kernel<K, DIM><<<2048, kBlock, 0, s>>>(keys, mbits, b.kofs, (uint32_t)b.B, b.ss,
-                                                       brt, parent, lsx, defer, st);
+                 uint32_t *lsx, uint64_t *miss_words, RunState *st, hipStream_t s) {
+  brt_seg_kernel<K, DIM, R><<<(unsigned)b.n_brt, kBlock, 0, s>>>(
+      keys, mbits, b.seg, b.brt, b.row_first, b.ss, brt, parent, lsx, b.row_tot, miss_words, st);
+  const int64_t g2 = (b.n_brt * R * (kBlock / 64) + kBlock - 1) / kBlock;
+  const unsigned grid2 = (unsigned)(g2 < 4096 ? g2 : 4096);
+  brt_seg_defer_kernel<K, DIM, R><<<grid2, kBlock, 0, s>>>(
+      keys, mbits, b.seg, b.brt, (uint32_t)b.n_brt, b.row_first, b.ss, brt, parent, lsx, b.row_tot,
+      miss_words, st);
 }
 
 template <typename K>
 void launch_brt_seg(const K *keys, int mbits, int dim, const BatchDev &b, BrtNodeT<K> *brt,
-                    int32_t *parent, uint32_t *lsx, uint32_t *defer, RunState *st,
+                    int32_t *parent, uint32_t *lsx, uint64_t *miss_words, RunState *st,
                     hipStream_t s) {
   if (b.n_brt <= 0) return;
   const bool small = b.brt_rows == 2;
   if (dim == 2) {
-    if (small) brt_seg_dim<K, 2, 2>(keys, mbits, b, brt, parent, lsx, defer, st, s);
-    else brt_seg_dim<K, 2, 4>(keys, mbits, b, brt, parent, lsx, defer, st, s);
+    if (small) brt_seg_dim<K, 2, 2>(keys, mbits, b, brt, parent, lsx, miss_words, st, s);
+    else brt_seg_dim<K, 2, 4>(keys, mbits, b, brt, parent, lsx, miss_words, st, s);
   } else {
-    if (small) brt_seg_dim<K, 3, 2>(keys, mbits, b, brt, parent, lsx, defer, st, s);
-    else brt_seg_dim<K, 3, 4>(keys, mbits, b, brt, parent, lsx, defer, st, s);
+    if (small) brt_seg_dim<K, 3, 2>(keys, mbits, b, brt, parent, lsx, miss_words, st, s);
+    else brt_seg_dim<K, 3, 4>(keys, mbits, b, brt, parent, lsx, miss_words, st, s);
   }
 }
 
@@ -437,7 +437,7 @@ void launch_claims_if_malformed(const BrtNodeT<K> *brt, int32_t *parent, int64_t
   template void launch_brt_ls<K>(const K *, int64_t, int, int, BrtNodeT<K> *, int32_t *,       \
                                  uint32_t *, uint32_t *, uint32_t *, RunState *, hipStream_t); \
   template void launch_brt_seg<K>(const K *, int, int, const BatchDev &, BrtNodeT<K> *,        \
-                                  int32_t *, uint32_t *, uint32_t *, RunState *, hipStream_t);
+                                  int32_t *, uint32_t *, uint64_t *, RunState *, hipStream_t);
 PGVD_INST(uint32_t)
 PGVD_INST(uint64_t)
 PGVD_INST(Key128)

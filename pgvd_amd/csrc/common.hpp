@@ -226,19 +226,6 @@ __device__ inline uint32_t wave_reduce_add(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan_add(v), 63);
 }
 
-// Appends `idx` to list[] for every lane with `take` set, one atomic per wave
-// on *count.  Call with the whole wave converged.
-template <typename T>
-__device__ inline void wave_append(bool take, T idx, uint32_t *count, T *list) {
-  const uint64_t mb = __ballot(take);
-  if (!mb) return;
-  const int leader = __ffsll((unsigned long long)mb) - 1;
-  uint32_t base = 0;
-  if ((int)__lane_id() == leader) base = atomicAdd(count, (uint32_t)__popcll(mb));
-  base = __shfl(base, leader, 64);
-  if (take) list[base + (uint32_t)__popcll(mb & lanemask_lt())] = idx;
-}
-
 // Miss masks: a converged wave records which of its 64 lanes take a node as
 // one word, words[word] = ballot(take), stored by lane 0.  No atomics, so
 // the word must belong to this wave alone (word = first index >> 6 for 64
@@ -246,17 +233,6 @@ __device__ inline void wave_append(bool take, T idx, uint32_t *count, T *list) {
 __device__ inline void wave_mask(bool take, uint64_t *words, uint32_t word) {
   const uint64_t b = __ballot(take);
   if (__lane_id() == 0) words[word] = b;
-}
-
-// Instance owning key slot `slot`: the largest s with kofs[s] <= slot
-// (kofs strictly increasing, kofs[B] = total slots).
-__device__ inline uint32_t find_seg(const uint32_t *kofs, uint32_t B, uint32_t slot) {
-  uint32_t lo = 0, hi = B;
-  while (hi - lo > 1) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (kofs[mid] <= slot) lo = mid; else hi = mid;
-  }
-  return lo;
 }
 
 // Workgroup b of a grid of nb runs on XCD b % 8 (round-robin dispatch).  This

@@ -27,8 +27,6 @@ enum {
   CTR_SPLITS = kMaxPasses + 1,
   CTR_SCAN = kMaxPasses + 2,
   CTR_LS = kMaxPasses + 3,
-  CTR_BRT_DEFER = kMaxPasses + 4,   // BRT nodes left to the global-memory pass
-  CTR_OCT_DEFER = kMaxPasses + 5,   // octree gathers left to the global pass
 };
 
 // Per-run scalars that kernels read and write on the device.  Cleared by the
@@ -319,6 +317,8 @@ int onesweep_tile_size(int key_bytes, bool payload);
 
 // ---- scan.hip ----
 constexpr int kScanTile = 4096;
+// BRT nodes per workgroup of the octree gather (octree.hip).
+constexpr int kGatherTile = 512;
 inline int64_t scan_tiles(int64_t n) { return (n + kScanTile - 1) / kScanTile; }
 // Unique over [zero?] + keys[0..n): writes out[0..m) and st->m.  With labels,
 // sets bit r of conflict_bits for every run r whose labels are not all equal.
@@ -402,11 +402,15 @@ void launch_local_splits(const BrtNodeT<K> *brt, int64_t m, int dim, uint32_t *l
 // Device-side description of a batch plan.  Tile tables:
 //   chunk: kEncodeChunk points      sort: sort_ipt*256 keys
 //   scan:  kScanTile key slots      brt:  brt_rows*256 key slots
-//   node:  256 key slots
-// (key-slot tables cover n+1 slots per instance).
+//   node:  kGatherTile key slots
+// (key-slot tables cover n+1 slots per instance); instance s's rows of 256
+// key slots start at row row_first[s], and row_tot holds a local-split sum
+// per row (exclusive prefix sums within the instance after
+// launch_chunk_scan_seg).
 struct BatchDev {
   const SegInfo *seg = nullptr;
-  const uint32_t *kofs = nullptr;   // B+1 entries: first key slot per instance, then the total
+  const uint32_t *row_first = nullptr;
+  uint32_t *row_tot = nullptr;
   SegState *ss = nullptr;
   int64_t B = 0;
   int sort_ipt = 16, brt_rows = 4;
@@ -440,22 +444,22 @@ int launch_onesweep_seg(K *keys, K *keys_alt, const BatchDev &b, int passes,
 template <typename K>
 void launch_unique_seg(const K *keys, K *out, const BatchDev &b, uint64_t *lookback,
                        RunState *st, hipStream_t s);
-// Per-instance BRT + packed local splits (as launch_brt_ls); defer holds
-// up to one key-slot index per key slot.
+// Per-instance BRT + packed local splits and row sums (as launch_brt_ls);
+// miss_words: brt_rows * 4 words per brt tile.
 template <typename K>
 void launch_brt_seg(const K *keys, int mbits, int dim, const BatchDev &b, BrtNodeT<K> *brt,
-                    int32_t *parent, uint32_t *lsx, uint32_t *defer, RunState *st,
+                    int32_t *parent, uint32_t *lsx, uint64_t *miss_words, RunState *st,
                     hipStream_t s);
-// Per-instance inclusive scan of the local splits; ss[s].octree_size.
-void launch_ls_scan_seg(const uint32_t *lsx, uint32_t *ps, const BatchDev &b,
-                        uint64_t *lookback, RunState *st, hipStream_t s);
+// Per-instance exclusive scan of row_tot, in place; ss[s].octree_size.
+void launch_chunk_scan_seg(const BatchDev &b, hipStream_t s);
 // ss[s].oct_off = exclusive scan of the octree sizes; st->octree_size = total.
 void launch_oct_offsets(const BatchDev &b, RunState *st, hipStream_t s);
 // Per-instance octree gather into octree[oct_off[s]..) (instance-local child
-// indices); flags ST_CAPACITY if the total exceeds capacity.
+// indices), and the inclusive prefix sums ps; flags ST_CAPACITY if the total
+// exceeds capacity.  miss_words: kGatherTile / 64 words per node tile.
 template <typename K>
-void launch_gather_seg(const BrtNodeT<K> *brt, const uint32_t *ps, const uint32_t *lsx, int dim,
-                       const BatchDev &b, int32_t *octree, int64_t capacity, uint32_t *defer,
+void launch_gather_seg(const BrtNodeT<K> *brt, uint32_t *ps, const uint32_t *lsx, int dim,
+                       const BatchDev &b, int32_t *octree, int64_t capacity, uint64_t *miss_words,
                        RunState *st, hipStream_t s);
 
 }  // namespace pgvd

@@ -448,11 +448,8 @@ __device__ inline void gather_owners_queued(uint32_t nact, uint32_t q0, int w0, 
 
 // BRT entries (links, ps, lsx) staged either side of a workgroup's nodes.
 constexpr int kGatherHalo = 256;
-// BRT nodes per workgroup of the single-tree gather: kGatherRows rows of 256.
-#ifndef PGVD_GATHER_ROWS
-#define PGVD_GATHER_ROWS 2
-#endif
-constexpr int kGatherRows = PGVD_GATHER_ROWS;
+// BRT nodes per workgroup: kGatherRows rows of 256.
+constexpr int kGatherRows = kGatherTile / kBlock;
 // Staged octree nodes per workgroup, in percent of its BRT nodes: 58% of
 // 512 (296 nodes, a uniform window owns ~240) keeps the LDS at 20.0 KB, so
 // that eight workgroups fit a CU (62% gave 20.8 KB and seven).
@@ -470,13 +467,12 @@ constexpr int kGatherStagePct = PGVD_GATHER_STAGE_PCT;
 // octree nodes the workgroup's BRT nodes own are the contiguous range
 // [ps[q0-1], ps[q_last]); when it holds at most R*256 nodes it is built in
 // LDS and written out in coalesced runs.
-// With chunk_excl (exclusive prefix sums of the local splits per chunk of
-// 256 nodes), the window's prefix sums are computed here from lsx instead
-// of read from ps, and the workgroup writes them to ps_out for its own
-// nodes (and for node m-1 when that starts the next chunk).
+// The window's prefix sums come from chunk_excl (exclusive prefix sums of
+// the local splits per chunk of 256 nodes) and lsx, and the workgroup writes
+// them to ps_out for its own nodes (and for node m-1 when that starts the
+// next chunk).
 template <typename K, int DIM, int R, bool CONF, typename Defer>
 __device__ inline void gather_window(const BrtNodeT<K> *__restrict__ brt,
-                                     const uint32_t *__restrict__ ps,
                                      const uint32_t *__restrict__ lsx,
                                      const uint32_t *__restrict__ chunk_excl,
                                      uint32_t *__restrict__ ps_out,
@@ -510,14 +506,13 @@ __device__ inline void gather_window(const BrtNodeT<K> *__restrict__ brt,
     const bool in = g >= 0 && g < (int)m;
     lx[r] = lsx[in ? g : 0];
     lk[r] = load_links(brt + (in && g < (int)m - 1 ? g : 0));
-    if (!chunk_excl) pv[r] = ps[in ? g : 0];
   }
-  uint32_t base;   // the prefix sum before the window
-  if (chunk_excl) {
-    // The window is whole chunks (q0 is a multiple of 256), so the base of
-    // the first one plus a running scan gives every prefix sum.
-    __shared__ uint32_t s_w[WR * 4];
-    base = q0 ? chunk_excl[(q0 >> 8) - 1] : 0u;
+  // The window is whole chunks (q0 is a multiple of 256), so the base of
+  // the first one (the prefix sum before the window) plus a running scan
+  // gives every prefix sum.
+  __shared__ uint32_t s_w[WR * 4];
+  const uint32_t base = q0 ? chunk_excl[(q0 >> 8) - 1] : 0u;
+  {
     uint32_t v[WR], ex[WR];
 #pragma unroll
     for (int r = 0; r < WR; ++r) {
@@ -534,8 +529,6 @@ __device__ inline void gather_window(const BrtNodeT<K> *__restrict__ brt,
       if (q < m) ps_out[q] = pv[1 + j];
     }
     if (t == 0 && q0 + STAGE == m - 1) ps_out[m - 1] = pv[R + 1];
-  } else {
-    base = w0 > 0 ? ps[w0 - 1] : 0u;
   }
 #pragma unroll
   for (int r = 0; r < WR; ++r) {
@@ -550,7 +543,9 @@ __device__ inline void gather_window(const BrtNodeT<K> *__restrict__ brt,
   const uint32_t lo = q0 ? s_pl[q0 - 1 - w0] >> kPlShift : 0u;
   const uint32_t span = (s_pl[qlast - w0] >> kPlShift) - lo;
   const bool staged = span <= (uint32_t)SN;   // uniform over the workgroup
-  const uint32_t a0 = (uint32_t)(((uint64_t)(base + lo) * STRIDE) & 3u);
+  // (an instance of a batch starts at any word of the octree)
+  const uint32_t a0 =
+      (uint32_t)(reinterpret_cast<uintptr_t>(octree + (size_t)(base + lo) * STRIDE) >> 2) & 3u;
   // The nodes that own octree nodes (about half), compacted so that each
   // lane takes one: entry e = j * 256 + t of the rows.
   __shared__ uint16_t s_aidx[STAGE];
@@ -659,9 +654,8 @@ __device__ inline void single_node(int32_t *octree, uint32_t *node_conflict) {
 }
 
 // Nodes the window cannot resolve are marked in miss_words (one word per 64
-// BRT nodes) for the global-memory pass.
-// With chunk_excl the prefix sums ps[0..m) are written here (see
-// gather_window); without it they are read.
+// BRT nodes) for the global-memory pass.  The prefix sums ps[0..m) are
+// written here (see gather_window).
 // Waves per SIMD the window pass is compiled for (its register budget):
 // eight, with the LDS of eight workgroups per CU, ran it 5% faster than
 // seven although some SGPRs then spill to VGPR lanes.
@@ -686,26 +680,27 @@ gather_kernel(
   if (m == 1) {             // single unique key: one node, no children
     if (q0 == 0 && threadIdx.x == 0) {
       single_node<DIM>(octree, node_conflict);
-      if (chunk_excl) ps[0] = 1;
+      ps[0] = 1;
     }
     return;
   }
   if (q0 >= m - 1) return;
-  gather_window<K, DIM, kGatherRows, CONF>(brt, ps, lsx, chunk_excl, ps, keys, conflict_bits,
-                                           mbits, m,
-                                     q0, octree,
-                        node_conflict, st,
-                        [&](bool miss, uint32_t q) { wave_mask(miss, miss_words, q >> 6); });
+  gather_window<K, DIM, kGatherRows, CONF>(
+      brt, lsx, chunk_excl, ps, keys, conflict_bits, mbits, m, q0, octree, node_conflict, st,
+      [&](bool miss, uint32_t q) { wave_mask(miss, miss_words, q >> 6); });
 }
 
-// Batched form: gather tiles of 256 key slots per instance; instance s writes
-// its nodes at octree[oct_off[s]..) with instance-local child indices.
+// Batched form: gather tiles of kGatherTile key slots per instance; instance
+// s writes its nodes at octree[oct_off[s]..) with instance-local child
+// indices.  Tile b's missed nodes are marked in its own kGatherTile / 64
+// words.
 template <typename K, int DIM>
-__global__ __launch_bounds__(kBlock) void gather_seg_kernel(
-    const BrtNodeT<K> *__restrict__ brt, const uint32_t *__restrict__ ps,
-    const uint32_t *__restrict__ lsx, const SegInfo *__restrict__ seg, TileTable tt,
-    const SegState *__restrict__ ss, int32_t *__restrict__ octree, int64_t capacity,
-    uint32_t *__restrict__ defer, RunState *st) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PGVD_GATHER_WPE))) void
+gather_seg_kernel(const BrtNodeT<K> *__restrict__ brt, uint32_t *__restrict__ ps,
+                  const uint32_t *__restrict__ lsx, const SegInfo *__restrict__ seg, TileTable tt,
+                  const uint32_t *__restrict__ row_first, const uint32_t *__restrict__ chunk_excl,
+                  const SegState *__restrict__ ss, int32_t *__restrict__ octree, int64_t capacity,
+                  uint64_t *__restrict__ miss_words, RunState *st) {
   constexpr int STRIDE = (1 << DIM) + 1;
   if ((int64_t)st->octree_size > capacity) {
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&st->status, (uint32_t)ST_CAPACITY);
@@ -715,19 +710,22 @@ __global__ __launch_bounds__(kBlock) void gather_seg_kernel(
   const uint32_t s = tt.seg[tile];
   const SegState sst = ss[s];
   const uint32_t m = sst.m;
-  const uint32_t q0 = (tile - tt.first[s]) * kBlock;
+  const uint32_t q0 = (tile - tt.first[s]) * kGatherTile;
   int32_t *oct = octree + (size_t)sst.oct_off * STRIDE;
-  if (m == 1) {
-    if (q0 == 0 && threadIdx.x == 0) single_node<DIM>(oct, nullptr);
+  uint64_t *words = miss_words + (size_t)tile * (kGatherTile / 64);
+  const uint32_t kofs = seg[s].kofs;
+  if (m == 1 || q0 >= m - 1) {
+    if (threadIdx.x < kGatherTile / 64) words[threadIdx.x] = 0;
+    if (m == 1 && q0 == 0 && threadIdx.x == 0) {
+      single_node<DIM>(oct, nullptr);
+      ps[kofs] = 1;
+    }
     return;
   }
-  if (q0 >= m - 1) return;
-  const uint32_t kofs = seg[s].kofs;
-  gather_window<K, DIM, 1, false>(brt + kofs, ps + kofs, lsx + kofs, nullptr, nullptr,
-                        (const K *)nullptr, nullptr, 0, m, q0,
-                        oct, nullptr, st, [&](bool miss, uint32_t q) {
-                          wave_append(miss, kofs + q, &st->counters[CTR_OCT_DEFER], defer);
-                        });
+  gather_window<K, DIM, kGatherRows, false>(
+      brt + kofs, lsx + kofs, chunk_excl + row_first[s], ps + kofs, (const K *)nullptr, nullptr, 0,
+      m, q0, oct, nullptr, st,
+      [&](bool miss, uint32_t q) { wave_mask(miss, words, (q - q0) >> 6); });
 }
 
 // Gather, second pass: the BRT nodes marked in miss_words, reading global
@@ -767,17 +765,16 @@ __global__ __launch_bounds__(kBlock) void gather_defer_kernel(
 template <typename K, int DIM>
 __global__ __launch_bounds__(kBlock) void gather_seg_defer_kernel(
     const BrtNodeT<K> *__restrict__ brt, const uint32_t *__restrict__ ps,
-    const uint32_t *__restrict__ lsx, const uint32_t *__restrict__ kofs_all, uint32_t B,
-    const SegState *__restrict__ ss, int32_t *__restrict__ octree, int64_t capacity,
-    const uint32_t *__restrict__ defer, RunState *st) {
+    const uint32_t *__restrict__ lsx, const SegInfo *__restrict__ seg, TileTable tt,
+    uint32_t ntiles, const SegState *__restrict__ ss, int32_t *__restrict__ octree,
+    int64_t capacity, const uint64_t *__restrict__ miss_words, RunState *st) {
   constexpr int STRIDE = (1 << DIM) + 1;
   if ((int64_t)st->octree_size > capacity) return;
-  const uint32_t cnt = st->counters[CTR_OCT_DEFER];
-  for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < cnt; k += gridDim.x * kBlock) {
-    const uint32_t slot = defer[k];
-    const uint32_t s = find_seg(kofs_all, B, slot);
-    const uint32_t kofs = kofs_all[s];
-    const uint32_t q = slot - kofs;
+  for_each_masked(miss_words, ntiles * (uint32_t)(kGatherTile / 64), [&](uint32_t w) {
+    const uint32_t tile = w / kGatherTile;
+    const uint32_t s = tt.seg[tile];
+    const uint32_t kofs = seg[s].kofs;
+    const uint32_t q = (tile - tt.first[s]) * kGatherTile + w % kGatherTile;
     const BrtNodeT<K> *b = brt + kofs;
     const uint32_t *p = ps + kofs;
     const uint32_t *lx = lsx + kofs;
@@ -797,7 +794,7 @@ __global__ __launch_bounds__(kBlock) void gather_seg_defer_kernel(
     (void)gather_one_bfs<K, DIM, false>(q, load_links(b + q), b, excl, p[q] - excl, fetch,
                                  (const K *)nullptr, nullptr, 0, oct + (size_t)excl * STRIDE,
                                  nullptr, st);
-  }
+  });
 }
 
 template <int DIM>
@@ -1001,22 +998,25 @@ void launch_octree(const BrtNodeT<K> *brt, const int32_t *parent, uint32_t *ps,
 }
 
 template <typename K, int DIM>
-void gather_seg_dim(const BrtNodeT<K> *brt, const uint32_t *ps, const uint32_t *lsx,
-                    const BatchDev &b, int32_t *octree, int64_t capacity, uint32_t *defer,
-                    RunState *st, hipStream_t s) {
-  gather_seg_kernel<K, DIM><<<(unsigned)b.n_node, kBlock, 0, s>>>(brt, ps, lsx, b.seg, b.node, b.ss,
-                                                                  octree, capacity, defer, st);
-  gather_seg_defer_kernel<K, DIM><<<2048, kBlock, 0, s>>>(brt, ps, lsx, b.kofs, (uint32_t)b.B,
-                                                          b.ss, octree, capacity, defer, st);
+void gather_seg_dim(const BrtNodeT<K> *brt, uint32_t *ps, const uint32_t *lsx, const BatchDev &b,
+                    int32_t *octree, int64_t capacity, uint64_t *miss_words, RunState *st,
+                    hipStream_t s) {
+  gather_seg_kernel<K, DIM><<<(unsigned)b.n_node, kBlock, 0, s>>>(
+      brt, ps, lsx, b.seg, b.node, b.row_first, b.row_tot, b.ss, octree, capacity, miss_words, st);
+  const int64_t g2 = (b.n_node * (kGatherTile / 64) + kBlock - 1) / kBlock;
+  const unsigned grid2 = (unsigned)(g2 < 4096 ? g2 : 4096);
+  gather_seg_defer_kernel<K, DIM><<<grid2, kBlock, 0, s>>>(brt, ps, lsx, b.seg, b.node,
+                                                           (uint32_t)b.n_node, b.ss, octree,
+                                                           capacity, miss_words, st);
 }
 
 template <typename K>
-void launch_gather_seg(const BrtNodeT<K> *brt, const uint32_t *ps, const uint32_t *lsx, int dim,
-                       const BatchDev &b, int32_t *octree, int64_t capacity, uint32_t *defer,
+void launch_gather_seg(const BrtNodeT<K> *brt, uint32_t *ps, const uint32_t *lsx, int dim,
+                       const BatchDev &b, int32_t *octree, int64_t capacity, uint64_t *miss_words,
                        RunState *st, hipStream_t s) {
   if (b.n_node <= 0) return;
-  if (dim == 2) gather_seg_dim<K, 2>(brt, ps, lsx, b, octree, capacity, defer, st, s);
-  else gather_seg_dim<K, 3>(brt, ps, lsx, b, octree, capacity, defer, st, s);
+  if (dim == 2) gather_seg_dim<K, 2>(brt, ps, lsx, b, octree, capacity, miss_words, st, s);
+  else gather_seg_dim<K, 3>(brt, ps, lsx, b, octree, capacity, miss_words, st, s);
 }
 
 #define PGVD_INST(K)                                                                          \
@@ -1025,8 +1025,8 @@ void launch_gather_seg(const BrtNodeT<K> *brt, const uint32_t *ps, const uint32_
                                  const uint32_t *, int64_t, int, int, int32_t *, uint32_t *,   \
                                  int64_t, int, uint32_t *, RunState *, hipStream_t,            \
                                  hipEvent_t *);                                                \
-  template void launch_gather_seg<K>(const BrtNodeT<K> *, const uint32_t *, const uint32_t *,  \
-                                     int, const BatchDev &, int32_t *, int64_t, uint32_t *,    \
+  template void launch_gather_seg<K>(const BrtNodeT<K> *, uint32_t *, const uint32_t *, int,   \
+                                     const BatchDev &, int32_t *, int64_t, uint64_t *,         \
                                      RunState *, hipStream_t);                                 \
   template void launch_local_splits<K>(const BrtNodeT<K> *, int64_t, int, uint32_t *,          \
                                        uint64_t *, hipStream_t);
