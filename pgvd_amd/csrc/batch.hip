@@ -26,6 +26,10 @@ struct pgvd_batch {
   int64_t B = 0, total_pts = 0, total_slots = 0;
   int sort_ipt = 16, brt_rows = 4;
   int digit_bits = 8, sort_waves = 3;
+  bool sample_ok = false;           // every instance fits the sample sort
+  bool use_sample = false;          // it sorts (else the radix passes)
+  SsPlan ss_plan;
+  char *ss_ws = nullptr;
   std::vector<SegInfo> h_seg;
   std::vector<int64_t> h_m, h_O, h_koff, h_ooff;
   // device
@@ -41,7 +45,7 @@ struct pgvd_batch {
   uint64_t *miss_words = nullptr;
   int32_t *parent = nullptr;
   char *zero = nullptr;
-  size_t zero_bytes = 0, off_hist = 0, off_sort = 0, off_lbu = 0;
+  size_t zero_bytes = 0, zero_cap = 0, off_hist = 0, off_sort = 0, off_lbu = 0;
   int32_t *octree = nullptr;
   int64_t oct_cap = 0;
   hipGraph_t graph = nullptr;
@@ -93,6 +97,25 @@ HostTable make_table(const std::vector<SegInfo> &si, int64_t tile, F units) {
   return t;
 }
 
+int ss_buckets_for(int kb, int64_t n) {
+  return kb == 4 ? ss_buckets<uint32_t>(n) : (kb == 8 ? ss_buckets<uint64_t>(n) : ss_buckets<Key128>(n));
+}
+int ss_tile_for(int kb) {
+  return kb == 4 ? ss_tile<uint32_t>() : (kb == 8 ? ss_tile<uint64_t>() : ss_tile<Key128>());
+}
+
+// The sample sort's workspace (its size does not depend on the settings).
+int ss_alloc(pgvd_batch *b, int64_t buckets) {
+  const size_t bytes = b->kb == 4   ? ss_ws_bytes<uint32_t>(buckets, b->B, b->total_slots)
+                       : b->kb == 8 ? ss_ws_bytes<uint64_t>(buckets, b->B, b->total_slots)
+                                    : ss_ws_bytes<Key128>(buckets, b->B, b->total_slots);
+  CHK(dalloc(&b->ss_ws, bytes));
+  if (b->kb == 4) ss_carve<uint32_t>(b->ss_ws, buckets, b->B, b->total_slots, b->ss_plan);
+  else if (b->kb == 8) ss_carve<uint64_t>(b->ss_ws, buckets, b->B, b->total_slots, b->ss_plan);
+  else ss_carve<Key128>(b->ss_ws, buckets, b->B, b->total_slots, b->ss_plan);
+  return PGVD_OK;
+}
+
 void release_graph(pgvd_batch *b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -120,6 +143,22 @@ int build_tables(pgvd_batch *b) {
     off[2 * i + 1] = all.size();
     all.insert(all.end(), ts[i]->first.begin(), ts[i]->first.end());
   }
+  // the sample sort's tiles and buckets
+  HostTable sst;
+  std::vector<uint32_t> bucket_first(si.size() + 1, 0);
+  if (b->sample_ok) {
+    sst = make_table(si, ss_tile_for(b->kb), [](const SegInfo &x) { return (int64_t)x.n; });
+    for (size_t i = 0; i < si.size(); ++i) {
+      const uint32_t nb = (uint32_t)ss_buckets_for(b->kb, si[i].n);
+      bucket_first[i + 1] = bucket_first[i] + nb;
+      b->ss_plan.max_nb = std::max(b->ss_plan.max_nb, nb);
+    }
+  }
+  const size_t off_sst = all.size();
+  all.insert(all.end(), sst.seg.begin(), sst.seg.end());
+  all.insert(all.end(), sst.first.begin(), sst.first.end());
+  const size_t off_bf = all.size();
+  all.insert(all.end(), bucket_first.begin(), bucket_first.end());
   const size_t off_row = all.size();
   all.insert(all.end(), row.first.begin(), row.first.end());
   dfree(b->tables);
@@ -140,20 +179,30 @@ int build_tables(pgvd_batch *b) {
   d.digit_bits = b->digit_bits;
   d.sort_waves = b->sort_waves;
   b->passes = (b->mbits + b->digit_bits - 1) / b->digit_bits;
-  // zero-initialised workspace: digit histograms, sort look-back (all
-  // passes), unique look-back
+  if (b->sample_ok) {
+    b->ss_plan.seg = b->seg;
+    b->ss_plan.ss = b->ss;
+    b->ss_plan.tiles.seg = b->tables + off_sst;
+    b->ss_plan.tiles.first = b->tables + off_sst + sst.seg.size();
+    b->ss_plan.bucket_first = b->tables + off_bf;
+    b->ss_plan.n_tiles = (int64_t)sst.seg.size();
+    if (!b->ss_ws) CHK(ss_alloc(b, bucket_first.back()));
+  }
+  // zero-initialised workspace: unique look-back and, for the radix passes,
+  // digit histograms and their look-back (all passes)
   size_t o = 0;
   b->off_hist = o;
-  o += align256((size_t)b->B * b->passes * 256 * 4);
+  if (!b->use_sample) o += align256((size_t)b->B * b->passes * 256 * 4);
   b->off_sort = o;
-  o += align256((size_t)b->passes * (size_t)d.n_sort * 256 * 4);
+  if (!b->use_sample) o += align256((size_t)b->passes * (size_t)d.n_sort * 256 * 4);
   b->off_lbu = o;
   o += align256((size_t)d.n_scan * 8);
-  if (o > b->zero_bytes) {
+  if (o > b->zero_cap) {
     dfree(b->zero);
     CHK(dalloc(&b->zero, o));
-    b->zero_bytes = o;
+    b->zero_cap = o;
   }
+  b->zero_bytes = o;
   release_graph(b);
   return PGVD_OK;
 }
@@ -179,14 +228,21 @@ void enqueue_typed(pgvd_batch *b, const void *pts) {
   const float effw = (float)(b->clamped ? width : width - 1);
   if (!b->quantized) launch_bbox_seg(static_cast<const float *>(pts), b->dim, d, s);
   uint32_t *bhist = reinterpret_cast<uint32_t *>(b->zero + b->off_hist);
-  launch_encode_seg<K>(pts, b->quantized ? 1 : 0, b->dim, b->bits, effw, d, kA, bhist, b->passes,
-                       b->st, s);
-  b->parity = launch_onesweep_seg<K>(kA, kB, d, b->passes, bhist,
-                                     reinterpret_cast<uint32_t *>(b->zero + b->off_sort), b->st, s);
+  launch_encode_seg<K>(pts, b->quantized ? 1 : 0, b->dim, b->bits, effw, d, kA, bhist,
+                       b->use_sample ? 0 : b->passes, b->st, s);
+  if (b->use_sample) {
+    // (sorted in place for unique: keys in A, B free)
+    launch_sample_sort<K>(kA, nullptr, kB, nullptr, nullptr, b->ss_plan, b->mbits, 0, b->st, s);
+    b->parity = 1;
+  } else {
+    b->parity = launch_onesweep_seg<K>(kA, kB, d, b->passes, bhist,
+                                       reinterpret_cast<uint32_t *>(b->zero + b->off_sort), b->st,
+                                       s);
+  }
   K *sorted = b->parity ? kB : kA;
   K *uniq = b->parity ? kA : kB;
-  launch_unique_seg<K>(sorted, uniq, d, reinterpret_cast<uint64_t *>(b->zero + b->off_lbu), b->st,
-                       s);
+  launch_unique_seg<K>(b->use_sample ? uniq : sorted, uniq, d, b->use_sample,
+                       reinterpret_cast<uint64_t *>(b->zero + b->off_lbu), b->st, s);
   uint32_t *lsx = reinterpret_cast<uint32_t *>(sorted);   // free after unique
   launch_brt_seg<K>(uniq, b->mbits, b->dim, d, static_cast<BrtNodeT<K> *>(b->brt), b->parent,
                     lsx, b->miss_words, b->st, s);
@@ -364,6 +420,11 @@ int pgvd_batch_create(pgvd_ctx *ctx, const int64_t *sizes, int64_t count, int di
     return bail(fail(PGVD_ERR_ALLOC, "hipHostMalloc failed"));
   if (hipMemcpy(b->seg, b->h_seg.data(), count * sizeof(SegInfo), hipMemcpyHostToDevice) != hipSuccess)
     return bail(fail(PGVD_ERR_HIP, "batch table upload failed"));
+  // the sample sort unless an instance is too large for it or the caller
+  // chose how the radix passes run
+  b->sample_ok = true;
+  for (int64_t i = 0; i < count; ++i) b->sample_ok &= ss_buckets_for(b->kb, sizes[i]) > 0;
+  b->use_sample = b->sample_ok && !(opts && (opts->sort_ipt || opts->digit_bits || opts->sort_waves));
   const size_t kbytes = (size_t)slots * b->kb;
   if ((rc = dalloc(&b->keys_a, kbytes))) return bail(rc);
   if ((rc = dalloc(&b->keys_b, kbytes))) return bail(rc);
@@ -404,6 +465,7 @@ int pgvd_batch_destroy(pgvd_batch *b) {
   dfree(b->parent);
   dfree(b->row_tot);
   dfree(b->miss_words);
+  dfree(b->ss_ws);
   dfree(b->zero);
   dfree(b->octree);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
@@ -475,7 +537,20 @@ int pgvd_batch_tune(pgvd_batch *b, const void *pts, int *sort_ipt, int *brt_rows
   float best = 1e30f, t = 0;
   int bi = b->sort_ipt, br = b->brt_rows, bd = b->digit_bits, bw = b->sort_waves;
   int rc = PGVD_OK;
+  // the sample sort first, where every instance fits it
+  float sbest = 1e30f;
+  int sr = br;
+  if (b->sample_ok) {
+    b->use_sample = true;
+    for (int r : rows) {
+      b->brt_rows = r;
+      if ((rc = time_it(&t))) break;
+      if (t < sbest) { sbest = t; sr = r; }
+    }
+    b->use_sample = false;
+  }
   for (int ipt : ipts) {
+    if (rc) break;
     for (int r : rows) {
       b->sort_ipt = ipt;
       b->brt_rows = r;
@@ -498,6 +573,10 @@ int pgvd_batch_tune(pgvd_batch *b, const void *pts, int *sort_ipt, int *brt_rows
     b->sort_waves = waves[k];
     if ((rc = time_it(&t))) break;
     if (t < best) { best = t; bw = waves[k]; }
+  }
+  if (b->sample_ok && sbest <= best) {
+    b->use_sample = true;
+    br = sr;
   }
   b->use_graph = graph;
   b->sort_ipt = bi;

@@ -21,56 +21,18 @@
 // (OR == AND) is copied, not split.  The host reads the segment count after
 // the level-0 plan and after each level's scan while the device keeps
 // working, and stops launching levels when none is left.
-#include "kernels.hpp"
-#include "tilescan.hpp"
+#include "bucket_dev.hpp"
 
 namespace pgvd {
 
 namespace {
 
-// ---- per key width ---------------------------------------------------------
-// CAP keys (and labels) of one LDS sort item; BS threads of IPT keys each;
-// scatter tiles of kBlock threads x TIPT keys.
-template <typename K> struct Bk;
-template <> struct Bk<uint32_t> { static constexpr int CAP = 8192, BS = 1024, IPT = 8, TIPT = 16; };
-template <> struct Bk<uint64_t> { static constexpr int CAP = 5120, BS = 1024, IPT = 5, TIPT = 16; };
-template <> struct Bk<Key128> { static constexpr int CAP = 2560, BS = 512, IPT = 5, TIPT = 8; };
 // Waves per SIMD the LDS sort is compiled for: 8 (two 1024-thread
 // workgroups per CU, 64 VGPRs) for level-0 buckets of 64-bit keys without
 // labels, where the kernel fits them without spilling; 4 (one workgroup, or
 // two of 512) where it needs more registers.
 template <typename K, bool LAB, bool MATCH> constexpr int sort_wpe() {
   return (sizeof(K) == 8 && !LAB && !MATCH) ? 8 : 4;
-}
-
-// 64-bit halves of a key (OR / AND accumulation)
-__device__ inline uint64_t klo(uint32_t a) { return a; }
-__device__ inline uint64_t klo(uint64_t a) { return a; }
-__device__ inline uint64_t klo(Key128 a) { return a.lo; }
-__device__ inline uint64_t khi(uint32_t) { return 0; }
-__device__ inline uint64_t khi(uint64_t) { return 0; }
-__device__ inline uint64_t khi(Key128 a) { return a.hi; }
-
-__device__ inline bool kless(uint32_t a, uint32_t b) { return a < b; }
-__device__ inline bool kless(uint64_t a, uint64_t b) { return a < b; }
-__device__ inline bool kless(Key128 a, Key128 b) { return a.hi < b.hi || (a.hi == b.hi && a.lo < b.lo); }
-
-// nbits (<= 14) bits of a key from bit `shift` up
-template <typename K>
-__device__ inline uint32_t kbits(K a, int shift, uint32_t mask) {
-  return klow32(kshr(a, shift)) & mask;
-}
-
-// all-ones key
-template <typename K> __device__ inline K kones();
-template <> __device__ inline uint32_t kones<uint32_t>() { return ~0u; }
-template <> __device__ inline uint64_t kones<uint64_t>() { return ~0ull; }
-template <> __device__ inline Key128 kones<Key128>() { return {~0ull, ~0ull}; }
-
-// number of low bits that vary: bitlen(or ^ and)
-__device__ inline int varying_bits(uint64_t olo, uint64_t ohi, uint64_t alo, uint64_t ahi) {
-  const uint64_t xh = ohi ^ ahi, xl = olo ^ alo;
-  return xh ? 128 - __builtin_clzll(xh) : (xl ? 64 - __builtin_clzll(xl) : 0);
 }
 
 // A new segment's accumulators: OR 0, AND all ones -- in the high half only
@@ -348,80 +310,6 @@ __global__ __launch_bounds__(kBlock) void bk_split2_kernel(TileIO<K, LAB> io, ui
   const uint32_t hi = min(lo + (uint32_t)TILE, ghi);
   scatter_tile<K, LAB, Bk<K>::TIPT, false>(io, n, lo, hi, shift, nb2, cursor + g * nb2, 1,
                                            sm.keys, sm.vals);
-}
-
-// ---- LDS sort of one item ---------------------------------------------------------
-// Stable LSD passes in LDS over the BS IPT keys k[] (and labels v[]) of a
-// workgroup; key index le = 64 IPT w + 64 j + lane lives in wave w,
-// register j; ranks by ballot matching.  On return s_keys / s_vals hold the
-// pairs in order of bits [0, 8 (passes - 1) + last_bits).  Slots past the
-// item hold all-ones keys at the highest indices, which stay behind every
-// real key.  s_cnt: NW 256 words, s_dig 256, s_w NW.
-template <typename K, bool LAB, int BS, int IPT>
-__device__ inline void lds_radix(K (&k)[IPT], uint32_t (&v)[IPT], int passes, int last_bits,
-                                 K *s_keys, uint32_t *s_vals, uint32_t *s_cnt, uint32_t *s_dig,
-                                 uint32_t *s_w) {
-  constexpr int NW = BS / 64;
-  static_assert(64 * IPT < (1 << 16), "a rank fits 16 bits");
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const uint32_t wofs = (uint32_t)w * 64u * IPT;
-  for (int p = 0; p < passes; ++p) {
-    const int sh = 8 * p;
-    const int nbits = p == passes - 1 ? last_bits : 8;   // uniform
-    const uint32_t dmask = (1u << nbits) - 1;
-    for (int i = t; i < NW * 256; i += BS) s_cnt[i] = 0;
-    __syncthreads();
-    uint32_t rk[IPT];   // rank within (wave, digit) | digit << 16
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      const uint32_t d = kdigit(k[j], sh) & dmask;
-      uint32_t plo = ~0u, phi = ~0u;
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        if (b < nbits) {
-          const int32_t sb = __builtin_amdgcn_sbfe((int32_t)d, b, 1);
-          const uint64_t bb = __ballot(sb < 0);
-          plo = __builtin_amdgcn_bitop3_b32(plo, (uint32_t)bb, (uint32_t)sb, 0x90);
-          phi = __builtin_amdgcn_bitop3_b32(phi, (uint32_t)(bb >> 32), (uint32_t)sb, 0x90);
-        }
-      }
-      const uint32_t c = s_cnt[w * 256 + d];
-      const uint32_t below = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0u));
-      rk[j] = (c + below) | (d << 16);
-      // every lane of the group stores the same new count
-      s_cnt[w * 256 + d] = c + (uint32_t)(__popc(plo) + __popc(phi));
-    }
-    __syncthreads();
-    uint32_t tot = 0;
-    if (t < 256) {
-#pragma unroll
-      for (int ww = 0; ww < NW; ++ww) {
-        const uint32_t c = s_cnt[ww * 256 + t];
-        s_cnt[ww * 256 + t] = tot;
-        tot += c;
-      }
-    }
-    uint32_t all;
-    const uint32_t dex = block_excl_sum<uint32_t, NW>(tot, s_w, &all);
-    if (t < 256) s_dig[t] = dex;
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      const uint32_t d = rk[j] >> 16;
-      const uint32_t q = (rk[j] & 0xffffu) + s_dig[d] + s_cnt[w * 256 + d];
-      s_keys[q] = k[j];
-      if (LAB) s_vals[q] = v[j];
-    }
-    __syncthreads();
-    if (p + 1 < passes) {
-#pragma unroll
-      for (int j = 0; j < IPT; ++j) {
-        k[j] = s_keys[wofs + j * 64 + lane];
-        if (LAB) v[j] = s_vals[wofs + j * 64 + lane];
-      }
-      __syncthreads();   // s_keys and s_cnt are rewritten by the next pass
-    }
-  }
 }
 
 // ---- merge sort of one item in LDS -----------------------------------------------

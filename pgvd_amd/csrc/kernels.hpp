@@ -79,7 +79,8 @@ struct SegState {
   uint32_t m;          // unique keys (incl. the padding zero)
   uint32_t octree_size;
   uint32_t oct_off;    // first octree node of the instance in the batch output
-  uint32_t pad_[3];
+  uint32_t dups;       // 1: the sample sort saw equal keys (or a zero key to merge)
+  uint32_t pad_[2];
 };
 // Tiles of one stage over the instances: tile t belongs to instance seg[t];
 // instance s owns tiles [first[s], first[s+1]).
@@ -428,6 +429,39 @@ bool onesweep_seg_waves_ok(int waves);
 // BRT window configurations (nodes per thread).
 bool brt_seg_rows_ok(int key_bytes, int rows);
 
+// ---- sample.hip: the sample sort of one or many segments ----
+constexpr int kSsMaxBuckets = 512;    // per segment
+constexpr int kSsLutWords = 2049;     // a segment's splitter table
+// A plan: the segments (tables as a batch's, or seg null and one segment of n
+// keys in nb buckets) and the workspace ss_carve lays out.
+struct SsPlan {
+  const SegInfo *seg = nullptr;
+  SegState *ss = nullptr;                  // with seg: where duplicates are reported
+  TileTable tiles{};                       // of ss_tile<K>() keys
+  const uint32_t *bucket_first = nullptr;  // B + 1 entries
+  uint32_t n = 0, nb = 0;
+  uint32_t max_nb = 0;                     // buckets of the largest segment
+  int64_t n_segs = 0, n_tiles = 0, n_buckets = 0;
+  void *splitters = nullptr;
+  uint32_t *lut = nullptr, *counts = nullptr, *cursors = nullptr, *n_big = nullptr;
+  BkItem *items = nullptr, *big = nullptr;
+  uint16_t *ids = nullptr;                 // every key's bucket
+};
+// Buckets of a segment of n keys; 0: too many keys for this sort.
+template <typename K> int ss_buckets(int64_t n);
+template <typename K> int ss_tile();
+template <typename K> size_t ss_ws_bytes(int64_t buckets, int64_t segs, int64_t slots);
+template <typename K>
+void ss_carve(void *ws, int64_t buckets, int64_t segs, int64_t slots, SsPlan &p);
+// Sorts every segment of kA (keys and, with labels, labels in input order)
+// into (kA, vA) through (kB, vB).  A segment of a table lands one slot to the
+// right where a zero key is prepended, which leaves the slot to that key.
+// Equal neighbours (and a zero key to merge) set ss[s].dups, or st->msd_dups
+// for the single segment.
+template <typename K>
+void launch_sample_sort(K *kA, uint32_t *vA, K *kB, uint32_t *vB, const uint32_t *labels,
+                        const SsPlan &p, int mbits, int prepend, RunState *st, hipStream_t s);
+
 void launch_seg_init(SegState *ss, int64_t B, hipStream_t s);                   // morton.hip
 void launch_bbox_seg(const float *pts, int dim, const BatchDev &b, hipStream_t s);
 // Quantize (float points, per-instance bbox) or take int32 grid points, Morton
@@ -441,9 +475,11 @@ template <typename K>
 int launch_onesweep_seg(K *keys, K *keys_alt, const BatchDev &b, int passes,
                         const uint32_t *bhist, uint32_t *lookback, RunState *st, hipStream_t s);
 // Per-instance unique (with its zero-key padding) into out[kofs..); ss[s].m.
+// in_place: out is keys, where the sample sort left instance s's keys from
+// slot kofs + prepend on; only instances with ss[s].dups are compacted.
 template <typename K>
-void launch_unique_seg(const K *keys, K *out, const BatchDev &b, uint64_t *lookback,
-                       RunState *st, hipStream_t s);
+void launch_unique_seg(const K *keys, K *out, const BatchDev &b, bool in_place,
+                       uint64_t *lookback, RunState *st, hipStream_t s);
 // Per-instance BRT + packed local splits and row sums (as launch_brt_ls);
 // miss_words: brt_rows * 4 words per brt tile.
 template <typename K>

@@ -308,6 +308,38 @@ __device__ inline void store4(K *__restrict__ keys, int64_t ch, const K (&k)[4])
   for (int v = 0; v < (int)(4 * sizeof(K) / 16); ++v) dst[v] = src[v];
 }
 
+// 3D keys of at most 64 bits: Morton spread by table, byte by byte
+// (s_spread3[v] = bit i of v at bit 3i), instead of 64-bit mask steps.
+template <typename K, int DIM>
+constexpr bool kSpreadTable = DIM == 3 && sizeof(K) == 8;
+template <typename K, int DIM>
+__device__ inline void fill_spread3(uint32_t *s_spread3) {
+  static_assert(kBlock == 256, "one table entry per thread");
+  if (kSpreadTable<K, DIM>) s_spread3[threadIdx.x] = (uint32_t)spread3(threadIdx.x);
+}
+// The Morton key of one point's coordinates (the table's barrier passed).
+template <typename K, int DIM>
+__device__ inline K encode_coords(const int64_t *c, int bits, const uint32_t *s_spread3) {
+  uint64_t lo, hi = 0;
+  if constexpr (kSpreadTable<K, DIM>) {
+    // bits <= 21: the three coordinates' bytes j give key bits 24j ..
+    const uint32_t cmask = (1u << bits) - 1u;
+    const uint32_t x = (uint32_t)c[0] & cmask, y = (uint32_t)c[1] & cmask,
+                   z = (uint32_t)c[2] & cmask;
+    uint64_t w[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int sh = 8 * j;
+      w[j] = s_spread3[(x >> sh) & 255u] | s_spread3[(y >> sh) & 255u] << 1 |
+             s_spread3[(z >> sh) & 255u] << 2;
+    }
+    lo = w[0] | w[1] << 24 | w[2] << 48;
+  } else {
+    morton128<DIM, (sizeof(K) > 8)>(c, bits, lo, hi);
+  }
+  return from128<K>(lo, hi);
+}
+
 template <typename K, int DIM, int HBINS>
 __global__ __launch_bounds__(kBlock) void encode_vec_kernel(
     const float *__restrict__ pts, int64_t n, int bits, float effw, int custom, float bmin0,
@@ -325,13 +357,8 @@ __global__ __launch_bounds__(kBlock) void encode_vec_kernel(
   uint32_t *s_msd = sh;
   if (msd_hist) passes = 0;
   for (int i = threadIdx.x; i < passes * 256; i += kBlock) sh[i] = 0;
-  // 3D keys of at most 64 bits: Morton spread by table, byte by byte
-  // (s_spread3[v] = bit i of v at bit 3i), instead of 64-bit mask steps.
-  constexpr bool kTable = DIM == 3 && sizeof(K) == 8;
-  __shared__ uint32_t s_spread3[kTable ? 256 : 1];
-  if (kTable) s_spread3[threadIdx.x] = (uint32_t)spread3(threadIdx.x);
-  static_assert(!kTable || kBlock == 256, "one table entry per thread");
-  const uint32_t cmask32 = bits >= 32 ? ~0u : (1u << bits) - 1u;
+  __shared__ uint32_t s_spread3[kSpreadTable<K, DIM> ? 256 : 1];
+  fill_spread3<K, DIM>(s_spread3);
   if (msd_hist)
     for (int i = threadIdx.x; i < msd_nb; i += kBlock) s_msd[i] = 0;
   const uint32_t msd_mask = (uint32_t)msd_nb - 1;
@@ -357,23 +384,7 @@ __global__ __launch_bounds__(kBlock) void encode_vec_kernel(
   auto encode_one = [&](const float *p) -> K {
     int64_t c[DIM];
     neg |= quantize_point<DIM>(p, mn, dwidth, effw, c);
-    uint64_t lo, hi = 0;
-    if constexpr (kTable) {
-      // bits <= 21: the three coordinates' bytes j give key bits 24j ..
-      const uint32_t x = (uint32_t)c[0] & cmask32, y = (uint32_t)c[1] & cmask32,
-                     z = (uint32_t)c[2] & cmask32;
-      uint64_t w[3];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const int sh = 8 * j;
-        w[j] = s_spread3[(x >> sh) & 255u] | s_spread3[(y >> sh) & 255u] << 1 |
-               s_spread3[(z >> sh) & 255u] << 2;
-      }
-      lo = w[0] | w[1] << 24 | w[2] << 48;
-    } else {
-      morton128<DIM, (sizeof(K) > 8)>(c, bits, lo, hi);
-    }
-    const K key = from128<K>(lo, hi);
+    const K key = encode_coords<K, DIM>(c, bits, s_spread3);
     for (int r = 0; r < passes; ++r) atomicAdd(&sh[r * 256 + kdigit(key, 8 * r)], 1u);
     if (msd_hist) atomicAdd(&s_msd[klow32(kshr(key, msd_shift)) & msd_mask], 1u);
     return key;
@@ -471,8 +482,8 @@ __global__ __launch_bounds__(kBlock) void seg_init_kernel(SegState *ss, int64_t 
   if (i >= B) return;
   SegState z;
   for (int k = 0; k < 3; ++k) { z.bb_min[k] = 0xFFFFFFFFu; z.bb_max[k] = 0u; }
-  z.m = 0; z.octree_size = 0; z.oct_off = 0;
-  for (int k = 0; k < 3; ++k) z.pad_[k] = 0;
+  z.m = 0; z.octree_size = 0; z.oct_off = 0; z.dups = 0;
+  for (int k = 0; k < 2; ++k) z.pad_[k] = 0;
   ss[i] = z;
 }
 
@@ -489,13 +500,45 @@ __global__ __launch_bounds__(kBlock) void bbox_seg_kernel(const float *__restric
   float mn[DIM], mx[DIM];
 #pragma unroll
   for (int k = 0; k < DIM; ++k) { mn[k] = __int_as_float(0x7f800000); mx[k] = -mn[k]; }
-  for (uint32_t i = threadIdx.x; i < cnt; i += kBlock) {
+  // The chunk's floats from the first 16-byte boundary on, three float4s a
+  // lane: float j of them is component (pre + j) % DIM (12 is a multiple of
+  // both 2 and 3); the floats before the boundary and after the last whole
+  // group one by one.  Bound by the read: 384 instances (0.66 GB) took 190 us
+  // point by point, three loads of a 12-byte stride in flight per lane.
+  const uint32_t total = cnt * DIM;
+  const uint32_t pre = min((uint32_t)((16u - ((uintptr_t)p & 15u)) & 15u) / 4u, total);
+  const uint32_t groups = (total - pre) / 12u;
+  const float4 *p4 = reinterpret_cast<const float4 *>(p + pre);
+  float amn[12], amx[12];
 #pragma unroll
-    for (int k = 0; k < DIM; ++k) {
-      const float v = p[(size_t)i * DIM + k];
-      mn[k] = fminf(mn[k], v);
-      mx[k] = fmaxf(mx[k], v);
+  for (int j = 0; j < 12; ++j) { amn[j] = __int_as_float(0x7f800000); amx[j] = -amn[j]; }
+  for (uint32_t g = threadIdx.x; g < groups; g += 2 * kBlock) {
+    const uint32_t h = g + kBlock < groups ? g + kBlock : g;
+    float4 v[6];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) { v[u] = p4[3 * g + u]; v[3 + u] = p4[3 * h + u]; }
+#pragma unroll
+    for (int u = 0; u < 6; ++u) {
+      const float f[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int a = 4 * (u % 3) + j;
+        amn[a] = fminf(amn[a], f[j]);
+        amx[a] = fmaxf(amx[a], f[j]);
+      }
     }
+  }
+  const uint32_t rot = pre % DIM;   // uniform
+#pragma unroll
+  for (int j = 0; j < 12; ++j)
+#pragma unroll
+    for (int k = 0; k < DIM; ++k)
+      if ((rot + j) % DIM == (uint32_t)k) { mn[k] = fminf(mn[k], amn[j]); mx[k] = fmaxf(mx[k], amx[j]); }
+  for (uint32_t e = threadIdx.x; e < total - 12u * groups; e += kBlock) {
+    const uint32_t f = e < pre ? e : e + 12u * groups;
+#pragma unroll
+    for (int k = 0; k < DIM; ++k)
+      if (f % DIM == (uint32_t)k) { mn[k] = fminf(mn[k], p[f]); mx[k] = fmaxf(mx[k], p[f]); }
   }
   __shared__ float smn[4][DIM], smx[4][DIM];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -523,6 +566,8 @@ __global__ __launch_bounds__(kBlock) void encode_seg_kernel(
     const SegState *__restrict__ ss, int bits, float effw, K *__restrict__ keys,
     uint32_t *__restrict__ bhist, int passes, int dbits, RunState *st) {
   __shared__ uint32_t sh[kMaxPasses * 256];
+  __shared__ uint32_t s_spread3[kSpreadTable<K, DIM> ? 256 : 1];
+  fill_spread3<K, DIM>(s_spread3);
   const uint32_t dmask = (1u << dbits) - 1u;
   for (int i = threadIdx.x; i < passes * 256; i += kBlock) sh[i] = 0;
   const uint32_t chunk = blockIdx.x;
@@ -547,25 +592,31 @@ __global__ __launch_bounds__(kBlock) void encode_seg_kernel(
   __syncthreads();
   bool neg = false;
   K *out = keys + si.kofs + start;
-  for (uint32_t i = threadIdx.x; i < cnt; i += kBlock) {
-    const size_t pi = (size_t)(si.pofs + start + i) * DIM;
-    int64_t c[DIM];
-    if (INT) {
-      const int32_t *q = static_cast<const int32_t *>(pts) + pi;
+  // four points a lane at a time, their loads issued together
+  constexpr int U = 4;
+  const size_t p0 = (size_t)(si.pofs + start) * DIM;
+  for (uint32_t i0 = threadIdx.x; i0 < cnt; i0 += U * kBlock) {
+    float f[U][DIM];
+    int64_t c[U][DIM];
 #pragma unroll
-      for (int k = 0; k < DIM; ++k) c[k] = q[k];
-    } else {
-      const float *q = static_cast<const float *>(pts) + pi;
-      float f[DIM];
+    for (int u = 0; u < U; ++u) {
+      const size_t pi = p0 + (size_t)(i0 + u * kBlock < cnt ? i0 + u * kBlock : i0) * DIM;
 #pragma unroll
-      for (int k = 0; k < DIM; ++k) f[k] = q[k];
-      neg |= quantize_point<DIM>(f, mn, dwidth, effw, c);
+      for (int k = 0; k < DIM; ++k) {
+        if (INT) c[u][k] = static_cast<const int32_t *>(pts)[pi + k];
+        else f[u][k] = static_cast<const float *>(pts)[pi + k];
+      }
     }
-    uint64_t lo, hi;
-    morton128<DIM, (sizeof(K) > 8)>(c, bits, lo, hi);
-    const K key = from128<K>(lo, hi);
-    out[i] = key;
-    for (int r = 0; r < passes; ++r) atomicAdd(&sh[r * 256 + kdigit_w(key, dbits * r, dmask)], 1u);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (!INT) neg |= quantize_point<DIM>(f[u], mn, dwidth, effw, c[u]);
+      const K key = encode_coords<K, DIM>(c[u], bits, s_spread3);
+      if (i0 + u * kBlock < cnt) {
+        out[i0 + u * kBlock] = key;
+        for (int r = 0; r < passes; ++r)
+          atomicAdd(&sh[r * 256 + kdigit_w(key, dbits * r, dmask)], 1u);
+      }
+    }
   }
   if (neg) atomicOr(&st->status, (uint32_t)ST_NEG_COORD);
   __syncthreads();

@@ -714,7 +714,7 @@ gather_seg_kernel(const BrtNodeT<K> *__restrict__ brt, uint32_t *__restrict__ ps
   int32_t *oct = octree + (size_t)sst.oct_off * STRIDE;
   uint64_t *words = miss_words + (size_t)tile * (kGatherTile / 64);
   const uint32_t kofs = seg[s].kofs;
-  if (m == 1 || q0 >= m - 1) {
+  if (m < 2 || q0 >= m - 1) {
     if (threadIdx.x < kGatherTile / 64) words[threadIdx.x] = 0;
     if (m == 1 && q0 == 0 && threadIdx.x == 0) {
       single_node<DIM>(oct, nullptr);

@@ -267,10 +267,11 @@ __global__ __launch_bounds__(kBlock) void chunk_scan_kernel(uint32_t *__restrict
 // ---- batched form ----
 // Per-instance unique: instance s reads keys[kofs .. kofs+n) (sorted) and
 // writes [zero?] + its distinct keys to out[kofs..); scan tiles cover n+1
-// slots per instance, the last one writes ss[s].m.
+// slots per instance, the last one writes ss[s].m.  in_place (out == keys,
+// sorted from slot kofs + prepend on): an instance without duplicates only
+// gets its m and its zero key.
 template <typename K>
-__global__ __launch_bounds__(kBlock) void unique_seg_kernel(const K *__restrict__ keys,
-                                                            K *__restrict__ out,
+__global__ __launch_bounds__(kBlock) void unique_seg_kernel(const K *keys, K *out, int in_place,
                                                             const SegInfo *__restrict__ seg,
                                                             TileTable tt, SegState *ss,
                                                             uint64_t *lookback, RunState *st) {
@@ -281,9 +282,17 @@ __global__ __launch_bounds__(kBlock) void unique_seg_kernel(const K *__restrict_
   const uint32_t s = tt.seg[tile];
   const int lo = (int)tt.first[s];
   const SegInfo si = seg[s];
-  unique_tile<K, false>(keys + si.kofs, nullptr, si.n, si.prepend, out + si.kofs, nullptr,
-                        lookback, tile, lo, (uint32_t)(tile - lo) * kScanTile,
-                        tile == (int)tt.first[s + 1] - 1 ? &ss[s].m : nullptr);
+  uint32_t *m_out = tile == (int)tt.first[s + 1] - 1 ? &ss[s].m : nullptr;
+  if (in_place && !ss[s].dups) {
+    if (threadIdx.x == 0) {
+      if (tile == lo && si.prepend) out[si.kofs] = kzero_value<K>();
+      if (m_out) *m_out = si.n + si.prepend;
+    }
+    return;
+  }
+  unique_tile<K, false>(keys + si.kofs + (in_place ? si.prepend : 0u), nullptr, si.n, si.prepend,
+                        out + si.kofs, nullptr, lookback, tile, lo,
+                        (uint32_t)(tile - lo) * kScanTile, m_out);
 }
 
 // chunk_scan_kernel per instance: one workgroup scans, in place, instance s's
@@ -386,11 +395,11 @@ void launch_scan_u32(const uint32_t *in, uint32_t *out, int64_t n, uint64_t *loo
 }
 
 template <typename K>
-void launch_unique_seg(const K *keys, K *out, const BatchDev &b, uint64_t *lookback,
-                       RunState *st, hipStream_t s) {
+void launch_unique_seg(const K *keys, K *out, const BatchDev &b, bool in_place,
+                       uint64_t *lookback, RunState *st, hipStream_t s) {
   if (b.n_scan <= 0) return;
-  unique_seg_kernel<K><<<(unsigned)b.n_scan, kBlock, 0, s>>>(keys, out, b.seg, b.scan, b.ss,
-                                                            lookback, st);
+  unique_seg_kernel<K><<<(unsigned)b.n_scan, kBlock, 0, s>>>(keys, out, in_place ? 1 : 0, b.seg,
+                                                            b.scan, b.ss, lookback, st);
 }
 
 void launch_chunk_scan_seg(const BatchDev &b, hipStream_t s) {
@@ -407,8 +416,8 @@ void launch_oct_offsets(const BatchDev &b, RunState *st, hipStream_t s) {
                                  uint64_t *, RunState *, hipStream_t, const RunState *);       \
   template void launch_splits_scan<K>(const BrtNodeT<K> *, int32_t *, uint32_t *, uint32_t *,  \
                                       int64_t, int, int, uint64_t *, RunState *, hipStream_t);  \
-  template void launch_unique_seg<K>(const K *, K *, const BatchDev &, uint64_t *, RunState *, \
-                                     hipStream_t);
+  template void launch_unique_seg<K>(const K *, K *, const BatchDev &, bool, uint64_t *,       \
+                                     RunState *, hipStream_t);
 PGVD_INST(uint32_t)
 PGVD_INST(uint64_t)
 PGVD_INST(Key128)
