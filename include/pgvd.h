@@ -372,8 +372,8 @@ typedef struct pgvd_octree_result {
   int64_t octree_size;      /* octree nodes                                      */
   int dim, bits, mbits, key_bytes;
   int malformed;            /* 1 if some BRT split took the FP32-quirk value     */
-  int bucket_sort;          /* 1 if the bucket sort ordered the keys, 0 the
-                               LSD radix passes                               */
+  int bucket_sort;          /* 1 if the bucket sort ordered the keys, 0 if the
+                               sample sort or the LSD radix passes did        */
   /* device pointers owned by the context, valid until its next build:       */
   const void *keys;         /* m sorted unique keys                              */
   const void *brt;          /* m-1 pgvd_brt_node{32,64,128}                      */

@@ -233,11 +233,11 @@ int carve_build(Get &&get, const void *pts, int64_t n, int dim, int bits, bool l
   b.chunks = static_cast<uint32_t *>(p);
   const bool quantized = opts && opts->quantized_input;
   const bool custom = opts && opts->use_custom_bb;
-  // float points (vectorised encode, which builds the bucket histogram) on
+  // aligned points (vectorised encode, which builds the bucket histogram) on
   // a context (the sort's levels are decided on the host): bucket sort;
   // otherwise the LSD passes
   b.bk_b = -1;
-  if (bucket_ok && !quantized && encode_vectorised(static_cast<const float *>(pts), b.kA))
+  if (bucket_ok && encode_vectorised(pts, b.kA))
     b.bk_b = std::min(bucket_bits_for<K>(n), std::min(mbits, kBkMaxBits));
   // the LSD passes' look-back words stay for keys of at most 64 bits (the
   // bucket sort hands clustered keys to the passes)
@@ -299,12 +299,17 @@ int build_launch(pgvd_ctx *ctx, const BuildBufs<K> &b, RunState *st, int32_t *oc
   const bool bbox_pass = !quantized && !custom;
   if (!bbox_pass) {
     Stage t(ctx, "prep", s);
-    launch_prep(st, reinterpret_cast<uint32_t *>(zb), z.total / 4, s);
+    launch_prep(st, reinterpret_cast<uint32_t *>(zb), (bucket ? z.sort_lb : z.total) / 4, s);
   }
   CHK(launch_status("prep"));
   if (quantized) {
     Stage t(ctx, "encode", s);
-    launch_encode_int<K>(static_cast<const int32_t *>(pts), n, dim, bits, kA, hist, passes, s);
+    if (bucket)
+      launch_encode_int<K>(static_cast<const int32_t *>(pts), n, dim, bits, kA, hist, 0, st, s,
+                           msd_hist, mbits - bk_b, 1 << bk_b);
+    else
+      launch_encode_int<K>(static_cast<const int32_t *>(pts), n, dim, bits, kA, hist, passes, st,
+                           s);
   } else {
     if (bbox_pass) {
       Stage t(ctx, "bbox", s);
@@ -1415,7 +1420,7 @@ int pgvd_build_octree_finish(pgvd_ctx *ctx, pgvd_octree_result *out) {
   out->mbits = L.mbits;
   out->key_bytes = L.kb;
   out->malformed = R.malformed ? 1 : 0;
-  out->bucket_sort = R.msd_ok ? 1 : 0;
+  out->bucket_sort = R.msd_ok && !R.ss_ok ? 1 : 0;
   out->keys = L.keys_u;
   out->brt = L.brt;
   out->parent = L.parent;

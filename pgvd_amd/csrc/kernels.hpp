@@ -39,6 +39,7 @@ struct RunState {
   uint32_t m;                // unique key count (incl. the padding zero)
   uint32_t octree_size;      // O = ps[m-1]
   uint32_t msd_ok;           // 1: the bucket sort (bucket.hip) sorted the keys
+  uint32_t ss_ok;            // 1: the sample sort (sample.hip) did (msd_ok is then set too)
   uint32_t msd_dups;         // 1: the bucket sort saw equal keys (or a zero key to merge)
   uint32_t counters[kNumCounters];
   // bucket sort (bucket.hip): the current level's segments and their keys,
@@ -117,7 +118,7 @@ void launch_encode(const float *pts, int64_t n, int dim, int bits, float effw,
                    hipStream_t s, uint32_t *msd_hist = nullptr, int msd_shift = 0,
                    int msd_nb = 0);
 // true when launch_encode takes the vectorised form (and so fills msd_hist)
-bool encode_vectorised(const float *pts, const void *keys);
+bool encode_vectorised(const void *pts, const void *keys);
 // Morton encode from integer points (int32 or int64 coordinates).
 template <typename K>
 void launch_points_to_morton(const void *pts, int coord_bytes, int64_t n, int64_t padded_n,
@@ -133,7 +134,8 @@ void launch_histogram(const K *keys, int64_t n, uint32_t *hist, int passes, hipS
 // Morton encode + digit histograms from int32 grid points (no padding).
 template <typename K>
 void launch_encode_int(const int32_t *pts, int64_t n, int dim, int bits, K *keys,
-                       uint32_t *hist, int passes, hipStream_t s);
+                       uint32_t *hist, int passes, RunState *st, hipStream_t s,
+                       uint32_t *msd_hist = nullptr, int msd_shift = 0, int msd_nb = 0);
 
 // ---- stages.hip (the reference's elementary stage kernels) ----
 template <typename K>

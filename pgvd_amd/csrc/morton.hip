@@ -27,6 +27,7 @@ __device__ inline void prep_run(RunState *st, uint4 *zero, size_t nzero16) {
   if (tid == 0) {
     for (int k = 0; k < 3; ++k) { st->bb_min[k] = 0xFFFFFFFFu; st->bb_max[k] = 0u; }
     st->status = 0; st->malformed = 0; st->m = 0; st->octree_size = 0; st->msd_ok = 0;
+    st->ss_ok = 0;
     for (int k = 0; k < kNumCounters; ++k) st->counters[k] = 0;
     st->msd_dups = 0;
     st->bk_segs = 0; st->bk_keys = 0; st->bk_next_segs = 0; st->bk_next_keys = 0;
@@ -340,9 +341,10 @@ __device__ inline K encode_coords(const int64_t *c, int bits, const uint32_t *s_
   return from128<K>(lo, hi);
 }
 
-template <typename K, int DIM, int HBINS>
+// INT: the points are int32 grid coordinates (no box, no quantization).
+template <typename K, int DIM, int HBINS, bool INT>
 __global__ __launch_bounds__(kBlock) void encode_vec_kernel(
-    const float *__restrict__ pts, int64_t n, int bits, float effw, int custom, float bmin0,
+    const void *__restrict__ points, int64_t n, int bits, float effw, int custom, float bmin0,
     float bmin1, float bmin2, float bmax0, float bmax1, float bmax2, K *__restrict__ keys,
     uint32_t *__restrict__ hist, int passes, RunState *st, uint32_t *__restrict__ msd_hist,
     int msd_shift, int msd_nb) {
@@ -362,8 +364,11 @@ __global__ __launch_bounds__(kBlock) void encode_vec_kernel(
   if (msd_hist)
     for (int i = threadIdx.x; i < msd_nb; i += kBlock) s_msd[i] = 0;
   const uint32_t msd_mask = (uint32_t)msd_nb - 1;
-  float mn[3], mx[3];
-  if (custom) {
+  // (an int32 chunk is moved as the floats of its bits)
+  const float *pts = static_cast<const float *>(points);
+  float mn[3] = {0, 0, 0}, mx[3] = {0, 0, 0};
+  if (INT) {
+  } else if (custom) {
     mn[0] = bmin0; mn[1] = bmin1; mn[2] = bmin2;
     mx[0] = bmax0; mx[1] = bmax1; mx[2] = bmax2;
   } else {
@@ -383,7 +388,12 @@ __global__ __launch_bounds__(kBlock) void encode_vec_kernel(
   const int64_t stride = (int64_t)gridDim.x * kBlock;
   auto encode_one = [&](const float *p) -> K {
     int64_t c[DIM];
-    neg |= quantize_point<DIM>(p, mn, dwidth, effw, c);
+    if constexpr (INT) {
+#pragma unroll
+      for (int k = 0; k < DIM; ++k) c[k] = __float_as_int(p[k]);
+    } else {
+      neg |= quantize_point<DIM>(p, mn, dwidth, effw, c);
+    }
     const K key = encode_coords<K, DIM>(c, bits, s_spread3);
     for (int r = 0; r < passes; ++r) atomicAdd(&sh[r * 256 + kdigit(key, 8 * r)], 1u);
     if (msd_hist) atomicAdd(&s_msd[klow32(kshr(key, msd_shift)) & msd_mask], 1u);
@@ -660,7 +670,7 @@ void launch_bbox(const float *pts, int64_t n, int dim, float *partials, RunState
   else bbox_kernel<3><<<grid, kBlock, 0, s>>>(pts, n, st);
 }
 
-bool encode_vectorised(const float *pts, const void *keys) {
+bool encode_vectorised(const void *pts, const void *keys) {
   return aligned16(pts) && aligned16(keys);
 }
 
@@ -670,6 +680,24 @@ bool encode_vectorised(const float *pts, const void *keys) {
 #ifndef PGVD_ENCODE_GRID
 #define PGVD_ENCODE_GRID 1024
 #endif
+template <typename K, bool INT>
+void launch_encode_vec(const void *pts, int64_t n, int dim, int bits, float effw, int custom_bb,
+                       const float *a, const float *b, K *keys, uint32_t *hist, int passes,
+                       RunState *st, hipStream_t s, uint32_t *msd_hist, int msd_shift,
+                       int msd_nb) {
+  const int vgrid = std::min(grid_for(n / 4 + 1, kBlock), PGVD_ENCODE_GRID);
+  if (msd_nb > kBkMaxBuckets) msd_hist = nullptr;
+  const bool big = msd_hist && msd_nb > (1 << kEncodeMaxBucketBits);
+  auto go = [&](auto kernel) {
+    kernel<<<vgrid, kBlock, 0, s>>>(pts, n, bits, effw, custom_bb, a[0], a[1], a[2], b[0], b[1],
+                                    b[2], keys, hist, passes, st, msd_hist, msd_shift, msd_nb);
+  };
+  if (dim == 2 && !big) go(encode_vec_kernel<K, 2, 4096, INT>);
+  else if (dim == 2) go(encode_vec_kernel<K, 2, kBkMaxBuckets, INT>);
+  else if (!big) go(encode_vec_kernel<K, 3, 4096, INT>);
+  else go(encode_vec_kernel<K, 3, kBkMaxBuckets, INT>);
+}
+
 template <typename K>
 void launch_encode(const float *pts, int64_t n, int dim, int bits, float effw, int custom_bb,
                    const float *bbmin, const float *bbmax, K *keys, int64_t *qout,
@@ -680,27 +708,8 @@ void launch_encode(const float *pts, int64_t n, int dim, int bits, float effw, i
   if (custom_bb)
     for (int k = 0; k < dim; ++k) { a[k] = bbmin[k]; b[k] = bbmax[k]; }
   if (keys && hist && !qout && encode_vectorised(pts, keys)) {
-    const int vgrid = std::min(grid_for(n / 4 + 1, kBlock), PGVD_ENCODE_GRID);
-    if (msd_nb > kBkMaxBuckets) msd_hist = nullptr;
-    const bool big = msd_hist && msd_nb > (1 << kEncodeMaxBucketBits);
-    if (dim == 2 && !big)
-      encode_vec_kernel<K, 2, 4096><<<vgrid, kBlock, 0, s>>>(pts, n, bits, effw, custom_bb, a[0],
-                                                             a[1], a[2], b[0], b[1], b[2], keys,
-                                                             hist, passes, st, msd_hist,
-                                                             msd_shift, msd_nb);
-    else if (dim == 2)
-      encode_vec_kernel<K, 2, kBkMaxBuckets><<<vgrid, kBlock, 0, s>>>(
-          pts, n, bits, effw, custom_bb, a[0], a[1], a[2], b[0], b[1], b[2], keys, hist, passes,
-          st, msd_hist, msd_shift, msd_nb);
-    else if (!big)
-      encode_vec_kernel<K, 3, 4096><<<vgrid, kBlock, 0, s>>>(pts, n, bits, effw, custom_bb, a[0],
-                                                             a[1], a[2], b[0], b[1], b[2], keys,
-                                                             hist, passes, st, msd_hist,
-                                                             msd_shift, msd_nb);
-    else
-      encode_vec_kernel<K, 3, kBkMaxBuckets><<<vgrid, kBlock, 0, s>>>(
-          pts, n, bits, effw, custom_bb, a[0], a[1], a[2], b[0], b[1], b[2], keys, hist, passes,
-          st, msd_hist, msd_shift, msd_nb);
+    launch_encode_vec<K, false>(pts, n, dim, bits, effw, custom_bb, a, b, keys, hist, passes, st, s,
+                                msd_hist, msd_shift, msd_nb);
     return;
   }
   if (dim == 2)
@@ -736,7 +745,14 @@ void launch_histogram(const K *keys, int64_t n, uint32_t *hist, int passes, hipS
 
 template <typename K>
 void launch_encode_int(const int32_t *pts, int64_t n, int dim, int bits, K *keys, uint32_t *hist,
-                       int passes, hipStream_t s) {
+                       int passes, RunState *st, hipStream_t s, uint32_t *msd_hist, int msd_shift,
+                       int msd_nb) {
+  if (encode_vectorised(pts, keys)) {
+    const float none[3] = {0, 0, 0};
+    launch_encode_vec<K, true>(pts, n, dim, bits, 0.0f, 0, none, none, keys, hist, passes, st, s,
+                               msd_hist, msd_shift, msd_nb);
+    return;
+  }
   const int grid = grid_for(n, kBlock * 4);
   if (dim == 2) encode_int_kernel<K, 2><<<grid, kBlock, 0, s>>>(pts, n, bits, keys, hist, passes);
   else encode_int_kernel<K, 3><<<grid, kBlock, 0, s>>>(pts, n, bits, keys, hist, passes);
@@ -778,7 +794,7 @@ void launch_encode_seg(const void *pts, int quantized, int dim, int bits, float 
   template void launch_histogram<K>(const K *, int64_t, uint32_t *, int, hipStream_t,          \
                                     const RunState *, uint32_t *, size_t);                     \
   template void launch_encode_int<K>(const int32_t *, int64_t, int, int, K *, uint32_t *, int,  \
-                                     hipStream_t);                                             \
+                                     RunState *, hipStream_t, uint32_t *, int, int);           \
   template void launch_encode_seg<K>(const void *, int, int, int, float, const BatchDev &, K *, \
                                      uint32_t *, int, RunState *, hipStream_t);
 PGVD_INST(uint32_t)

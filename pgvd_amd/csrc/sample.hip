@@ -199,7 +199,10 @@ __global__ __launch_bounds__(kSsMaxBuckets) void ss_plan_kernel(SsPlan p, uint32
     }
     p.items[sg.bucket + b] = it;
   }
-  if (!p.seg && b == 0) st->msd_ok = 1u;   // the whole path's keys are sorted from here on
+  if (!p.seg && b == 0) {   // the whole path's keys are sorted from here on
+    st->msd_ok = 1u;
+    st->ss_ok = 1u;
+  }
 }
 
 // Scatters each tile's keys (and labels) to their buckets: the tile's keys

@@ -113,3 +113,22 @@ def test_bucket_13_bit_level0(dev):
     """20 M uniform points: 2^13 top-level buckets (the encode kernel's larger
     bucket histogram), against the oracle."""
     _check(dev, _uniform(20_000_000, 3, seed=25), 21, where="2^13 buckets")
+
+
+@pytest.mark.parametrize("dim,bits,n,spread", [
+    (2, 16, 4099, 1 << 16), (2, 20, 1 << 20, 1 << 20), (3, 21, 600001, 1 << 21),
+    (3, 10, 200003, 1 << 10), (2, 30, 70001, 300), (3, 21, 50000, 1)])
+def test_int32_grid_points_match_radix(dev, dim, bits, n, spread):
+    """int32 grid points take the bucket sort as float points do (the sample
+    sort where they crowd): the same tree as with the radix passes that
+    no_host_wait asks for.  Coordinates past the grid and below zero keep
+    their low bits."""
+    rng = np.random.default_rng(n)
+    q = rng.integers(0, spread, (n, dim)).astype(np.int32)
+    q[::1000] -= 1 << min(bits + 1, 30)
+    q[7::1000] += 1 << min(bits, 29)
+    got = dev.build_octree(q, bits)
+    want = dev.build_octree(q, bits, no_host_wait=True)
+    assert want["bucket_sort"] == 0
+    assert got["bucket_sort"] == (spread == 1 << bits)      # else crowded
+    assert_tree_equal(got, want)
