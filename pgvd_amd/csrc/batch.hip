@@ -232,7 +232,8 @@ void enqueue_typed(pgvd_batch *b, const void *pts) {
                        b->use_sample ? 0 : b->passes, b->st, s);
   if (b->use_sample) {
     // (sorted in place for unique: keys in A, B free)
-    launch_sample_sort<K>(kA, nullptr, kB, nullptr, nullptr, b->ss_plan, b->mbits, 0, b->st, s);
+    launch_sample_sort<K>(kA, nullptr, kA, nullptr, kB, nullptr, b->ss_plan, b->mbits, 0, b->st,
+                          s);
     b->parity = 1;
   } else {
     b->parity = launch_onesweep_seg<K>(kA, kB, d, b->passes, bhist,

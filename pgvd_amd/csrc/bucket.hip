@@ -54,21 +54,23 @@ __device__ inline void init_seg(BkSeg *sg, uint32_t start, uint32_t count, bool 
 // and the second scatter's tile starts, and the level-1 segments (buckets
 // above CAP) with their accumulators.
 constexpr int kPlanBlock = 1024;
-// The LSD passes take over when more than 1 / PGVD_BK_LSD_SHARE of the keys
-// are left to the levels (0: never).
+// Another sort takes the whole array when more than 1 / PGVD_BK_LSD_SHARE of
+// the keys are crowded (0: never).
 #ifndef PGVD_BK_LSD_SHARE
 #define PGVD_BK_LSD_SHARE 4
 #endif
 __global__ __launch_bounds__(kPlanBlock) void bk_plan_kernel(
     const uint32_t *__restrict__ hist, uint32_t n, int nb, int nb2, int tile2, uint32_t cap,
-    int wide, int lsd_ok, uint32_t *__restrict__ start, uint32_t *__restrict__ cursor,
+    int wide, int lsd_ok, uint32_t seg_max, uint32_t *__restrict__ start,
+    uint32_t *__restrict__ cursor,
     BkSeg *__restrict__ segs, uint32_t *__restrict__ hrows, RunState *st, RunState *host) {
   __shared__ uint32_t s_w[kPlanBlock / 64];
-  __shared__ uint32_t s_nseg, s_bigkeys;
+  __shared__ uint32_t s_nseg, s_bigkeys, s_max;
   const int t = threadIdx.x;
   if (t == 0) {
     s_nseg = 0;
     s_bigkeys = 0;
+    s_max = 0;
   }
   const int per = (nb + kPlanBlock - 1) / kPlanBlock;   // <= 16 consecutive buckets per thread
   uint32_t v[16];
@@ -91,6 +93,7 @@ __global__ __launch_bounds__(kPlanBlock) void bk_plan_kernel(
         const uint32_t sid = atomicAdd(&s_nseg, 1u);
         init_seg(&segs[sid], ex, v[i], wide != 0);
         atomicAdd(&s_bigkeys, v[i]);
+        atomicMax(&s_max, v[i]);
       }
       ex += v[i];
     }
@@ -101,12 +104,15 @@ __global__ __launch_bounds__(kPlanBlock) void bk_plan_kernel(
   // the level-1 segments' histogram rows start at zero
   for (uint32_t i = t; i < nseg * 256u; i += kPlanBlock) hrows[i] = 0u;
   if (t == 0) {
-    // Keys that clustered so much that a quarter of them are left to the
-    // levels sort faster by the LSD passes where those are few (keys of at
-    // most 64 bits): then the scatters and bucket sorts do nothing, and the
-    // host launches the passes over the keys as encoded.
-    const bool lsd = lsd_ok && PGVD_BK_LSD_SHARE > 0 &&
-                     (uint64_t)s_bigkeys * PGVD_BK_LSD_SHARE > (uint64_t)n;
+    // Crowded buckets go to the sample sort.  Where they hold more than a
+    // quarter of the keys (of at most 64 bits), an array small enough for it
+    // is left to it whole (no scatter first), and past a bucket too large for
+    // it the LSD passes take the array.  Either way the scatters and bucket
+    // sorts then do nothing and the host launches the other sort over the
+    // keys as encoded.
+    const bool crowded = PGVD_BK_LSD_SHARE > 0 &&
+                         (uint64_t)s_bigkeys * PGVD_BK_LSD_SHARE > (uint64_t)n;
+    const bool lsd = crowded && lsd_ok && (n <= seg_max || s_max > seg_max);
     st->bk_lsd = lsd ? 1u : 0u;
     st->bk_segs = lsd ? 0u : nseg;
     st->bk_keys = lsd ? 0u : s_bigkeys;
@@ -116,6 +122,7 @@ __global__ __launch_bounds__(kPlanBlock) void bk_plan_kernel(
     host->bk_lsd = lsd ? 1u : 0u;
     host->bk_segs = lsd ? 0u : nseg;
     host->bk_keys = lsd ? 0u : s_bigkeys;
+    host->bk_max = s_max;
     __threadfence_system();
     // (a histogram that does not count every key leaves the keys unsorted:
     // then the status says so and nothing downstream trusts the order)
@@ -992,7 +999,8 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host,
   constexpr int TILE = kBlock * C::TIPT;
   constexpr int wide = sizeof(K) > 8 ? 1 : 0;
   bk_plan_kernel<<<1, kPlanBlock, 0, s>>>(a.hist, (uint32_t)n, nb, nb2, TILE, (uint32_t)C::CAP,
-                                          wide, sizeof(K) <= 8 ? 1 : 0, m.start, m.cursor,
+                                          wide, sizeof(K) <= 8 ? 1 : 0,
+                                          (uint32_t)ss_max_keys<K>(), m.start, m.cursor,
                                           m.segs[0], m.hrows[0], st, st_host);
   if (hipGetLastError() != hipSuccess) return 1;
   // the host learns the level-1 segment count (written by the plan into its
@@ -1044,9 +1052,19 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host,
         <<<(unsigned)nb, C::BS, 0, s>>>(san, 0, a.mbits - b, st);
   if (hipGetLastError() != hipSuccess) return 1;
   if (!spin_wait(ev)) return 1;
-  if (st_host->bk_lsd) return 3;   // the LSD passes sort instead
+  if (st_host->bk_lsd) {
+    if (n > ss_max_keys<K>()) return 3;   // the LSD passes sort instead
+    launch_sample_sort<K>(kA, a.labels, kA, vA, kB, vB, m.ss.whole, a.mbits, a.prepend, st, s);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+  }
   uint32_t nseg = st_host->bk_segs;
   uint64_t nkeys = st_host->bk_keys;
+  if (nseg > 0 && st_host->bk_max <= ss_max_keys<K>()) {
+    // (the segments' keys are where the level-0 scatters left them)
+    launch_sample_sort_buckets<K>(p0 ? kB : kA, lab ? v0 : nullptr, kA, vA, kB, vB, m.ss, m.segs[0],
+                                  nseg, nkeys, st_host->bk_max, n, a.mbits, a.prepend, st, s);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+  }
   int levels = 0;
   int parity = p0;
   int cur = 0;

@@ -125,6 +125,18 @@ __device__ inline uint64_t ksub(uint64_t a, uint64_t b) { return a - b; }
 __device__ inline Key128 ksub(Key128 a, Key128 b) {
   return {a.lo - b.lo, a.hi - b.hi - (a.lo < b.lo ? 1ull : 0ull)};
 }
+// The smaller and the larger key (by value: a conditional on two structs picks
+// an address and sends both to scratch memory).
+template <typename K> __device__ inline K kmin(K a, K b) { return kless(a, b) ? a : b; }
+template <typename K> __device__ inline K kmax(K a, K b) { return kless(a, b) ? b : a; }
+template <> __device__ inline Key128 kmin<Key128>(Key128 a, Key128 b) {
+  const bool l = kless(a, b);
+  return {l ? a.lo : b.lo, l ? a.hi : b.hi};
+}
+template <> __device__ inline Key128 kmax<Key128>(Key128 a, Key128 b) {
+  const bool l = kless(a, b);
+  return {l ? b.lo : a.lo, l ? b.hi : a.hi};
+}
 __device__ inline uint32_t kshfl_xor(uint32_t a, int d) { return (uint32_t)__shfl_xor((int)a, d, 64); }
 __device__ inline uint64_t kshfl_xor(uint64_t a, int d) {
   return (uint64_t)__shfl_xor((unsigned long long)a, d, 64);
@@ -141,9 +153,8 @@ __device__ inline void block_minmax(K &mn, K &mx, K *s_mm) {
   constexpr int NW = BS / 64;
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) {
-    const K a = kshfl_xor(mn, d), b = kshfl_xor(mx, d);
-    mn = kless(a, mn) ? a : mn;
-    mx = kless(mx, b) ? b : mx;
+    mn = kmin(mn, kshfl_xor(mn, d));
+    mx = kmax(mx, kshfl_xor(mx, d));
   }
   if ((threadIdx.x & 63) == 0) {
     s_mm[threadIdx.x >> 6] = mn;
@@ -151,8 +162,8 @@ __device__ inline void block_minmax(K &mn, K &mx, K *s_mm) {
   }
   __syncthreads();
   for (int w = 0; w < NW; ++w) {
-    mn = kless(s_mm[w], mn) ? s_mm[w] : mn;
-    mx = kless(mx, s_mm[NW + w]) ? s_mm[NW + w] : mx;
+    mn = kmin(mn, s_mm[w]);
+    mx = kmax(mx, s_mm[NW + w]);
   }
 }
 
@@ -318,8 +329,8 @@ __device__ inline void lds_bin_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cn
 #pragma unroll
   for (int j = 0; j < IPT; ++j)
     if ((uint32_t)j * BS + t < cnt) {
-      mn = kless(k[j], mn) ? k[j] : mn;
-      mx = kless(mx, k[j]) ? k[j] : mx;
+      mn = kmin(mn, k[j]);
+      mx = kmax(mx, k[j]);
     }
   for (uint32_t i = t; i < (uint32_t)kBins; i += BS) s_bin[i] = 0;
   block_minmax<K, BS>(mn, mx, s_mm);

@@ -108,10 +108,9 @@ size_t pgvd_capi::plain_footprint_bytes(int64_t n, int dim, int bits, bool label
   b += kBboxPartBytes;                                   // bbox_part
   b += kb == 4 ? bucket_ws_bytes<uint32_t>(n)            // the bucket sort's workspace
                 : (kb == 8 ? bucket_ws_bytes<uint64_t>(n) : bucket_ws_bytes<Key128>(n));
-  if (kb <= 8) {                                         // and the sample sort's
-    const int nb = kb == 4 ? ss_buckets<uint32_t>(n) : ss_buckets<uint64_t>(n);
-    if (nb > 1) b += kb == 4 ? ss_ws_bytes<uint32_t>(nb, 1, n) : ss_ws_bytes<uint64_t>(nb, 1, n);
-  }
+  if (kb == 4 && n > bucket_cap<uint32_t>()) b += ss_tree_bytes<uint32_t>(n);   // and the
+  if (kb == 8 && n > bucket_cap<uint64_t>()) b += ss_tree_bytes<uint64_t>(n);   // sample sort's
+  if (kb == 16 && n > bucket_cap<Key128>()) b += ss_tree_bytes<Key128>(n);
   b += (size_t)((nk + kBlock - 1) / kBlock) * 4;         // chunks
   b += zero_layout(n, kb, (mbits + 7) / 8, labels).total;
   b += (size_t)oct_nodes * ((1u << dim) + 1) * 4;        // octree
@@ -185,7 +184,6 @@ struct BuildBufs {
   float *bbox_part = nullptr;
   int bk_b = -1;                           // bucket sort's level-0 bits (-1: LSD passes)
   BucketMem bk;                            // the bucket sort's workspace
-  SsPlan ss;                               // the sample sort's plan (n_segs 0: none)
 };
 
 // What a build leaves for the caller (the unique keys, the packed local
@@ -251,15 +249,9 @@ int carve_build(Get &&get, const void *pts, int64_t n, int dim, int bits, bool l
   if (b.bk_b >= 0) {
     CHK(get("bucket_ws", bucket_ws_bytes<K>(n), &p));
     bucket_carve<K>(p, n, b.bk);
-    // keys too clustered for the bucket sort: the sample sort, where the
-    // array is small enough for it (128-bit keys go through the levels)
-    const int nb = kb <= 8 ? ss_buckets<K>(n) : 0;
-    if (nb > 1) {
-      CHK(get("sample_ws", ss_ws_bytes<K>(nb, 1, n), &p));
-      ss_carve<K>(p, nb, 1, n, b.ss);
-      b.ss.n = (uint32_t)n;
-      b.ss.nb = b.ss.max_nb = (uint32_t)nb;
-      b.ss.n_tiles = (n + ss_tile<K>() - 1) / ss_tile<K>();
+    if (n > bucket_cap<K>()) {   // else no bucket can be crowded
+      CHK(get("sample_ws", ss_tree_bytes<K>(n), &p));
+      ss_tree_carve<K>(p, n, b.bk.ss);
     }
   }
   return PGVD_OK;
@@ -342,11 +334,6 @@ int build_launch(pgvd_ctx *ctx, const BuildBufs<K> &b, RunState *st, int32_t *oc
                                                                   : fail(PGVD_ERR_HIP, "bucket sort");
     bucket_sorted = rc == 0;
     // rc 3: clustered keys of at most 64 bits; the encoded keys are untouched
-    if (!bucket_sorted && b.ss.n_segs > 0) {
-      launch_sample_sort<K>(kA, b.vA, kB, b.vB, labels, b.ss, mbits, prepend, st, s);
-      CHK(launch_status("sample sort"));
-      bucket_sorted = true;
-    }
     if (!bucket_sorted)
       launch_histogram<K>(kA, n, hist, passes, s, nullptr, sort_lb, (z.total - z.sort_lb) / 4);
   }

@@ -45,7 +45,8 @@ struct RunState {
   // bucket sort (bucket.hip): the current level's segments and their keys,
   // the next level's, the LDS sort items so far, the current level's tiles
   uint32_t bk_segs, bk_keys, bk_next_segs, bk_next_keys, bk_items, bk_tiles;
-  uint32_t bk_lsd;           // 1: too clustered, the LSD passes sort instead
+  uint32_t bk_lsd;           // 1: too clustered, another sort takes the encoded keys
+  uint32_t bk_max;           // keys of the largest crowded bucket
 };
 
 // Fixed-layout BRT node in device memory (the reference's BrtNode,
@@ -276,6 +277,59 @@ struct BkSeg {
 struct BkItem {
   uint32_t start, count, parity, sbits;
 };
+// ---- sample.hip: the sample sort of one or many segments ----
+constexpr int kSsMaxBuckets = 512;    // per segment
+constexpr int kSsLutWords = 2049;     // a segment's splitter table
+// A plan: the segments (tables as a batch's, or seg null and one segment of n
+// keys in nb buckets) and the workspace ss_carve lays out.
+struct SsPlan {
+  const SegInfo *seg = nullptr;
+  SegState *ss = nullptr;                  // with seg: where duplicates are reported
+  TileTable tiles{};                       // of ss_tile<K>() keys
+  const uint32_t *bucket_first = nullptr;  // B + 1 entries
+  // for segments the device listed (ss_segments_from_buckets): the tiles and
+  // buckets in use, at most n_tiles and n_buckets; null: all of them
+  const uint32_t *limits = nullptr;
+  uint32_t n = 0, nb = 0;
+  uint32_t max_nb = 0;                     // buckets of the largest segment
+  int64_t n_segs = 0, n_tiles = 0, n_buckets = 0;
+  void *splitters = nullptr;
+  uint32_t *lut = nullptr, *counts = nullptr, *cursors = nullptr, *n_big = nullptr;
+  BkItem *items = nullptr, *big = nullptr;
+  uint16_t *ids = nullptr;                 // every key's bucket
+};
+// Buckets of a segment of n keys; 0: too many keys for this sort.
+template <typename K> int ss_buckets(int64_t n);
+template <typename K> int64_t ss_max_keys();   // the most that gives buckets
+template <typename K> int ss_tile();
+template <typename K> size_t ss_ws_bytes(int64_t buckets, int64_t segs, int64_t slots);
+template <typename K>
+void ss_carve(void *ws, int64_t buckets, int64_t segs, int64_t slots, SsPlan &p);
+// The single tree's workspace: for the whole array of n keys as one segment
+// (where it is small enough), or for the crowded buckets of the bucket sort.
+struct SsTree {
+  SsPlan whole, crowded;
+  void *tables = nullptr;   // of the crowded buckets
+};
+template <typename K> size_t ss_tree_bytes(int64_t n);
+template <typename K> void ss_tree_carve(void *ws, int64_t n, SsTree &t);
+// Sorts every segment of kin (keys and, with vin, labels) into (kA, vA): kin is
+// kA or kB, and each key passes through the other one.  A segment of a table lands one slot to the
+// right where a zero key is prepended, which leaves the slot to that key.
+// Equal neighbours (and a zero key to merge) set ss[s].dups, or st->msd_dups
+// for the single segment.
+template <typename K>
+void launch_sample_sort(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, K *kB,
+                        uint32_t *vB, const SsPlan &p, int mbits, int prepend, RunState *st,
+                        hipStream_t s);
+// The same for the first nseg crowded buckets (nkeys keys, at most
+// ss_max_keys in each) that the bucket sort's plan listed in segs.
+template <typename K>
+void launch_sample_sort_buckets(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, K *kB,
+                                uint32_t *vB, const SsTree &t, const BkSeg *segs, uint32_t nseg,
+                                uint64_t nkeys, uint32_t max_keys, int64_t n, int mbits,
+                                int prepend, RunState *st, hipStream_t s);
+
 struct BucketMem {
   uint32_t *start = nullptr, *cursor = nullptr;
   BkSeg *segs[2] = {nullptr, nullptr};
@@ -283,6 +337,7 @@ struct BucketMem {
   uint32_t *lcursor = nullptr;
   BkItem *items = nullptr;
   uint32_t max_segs = 0, max_items = 0;
+  SsTree ss;               // the sample sort's workspace
 };
 template <typename K>
 struct BucketArgs {
@@ -430,39 +485,6 @@ bool onesweep_seg_digit_ok(int key_bytes, int digit_bits);
 bool onesweep_seg_waves_ok(int waves);
 // BRT window configurations (nodes per thread).
 bool brt_seg_rows_ok(int key_bytes, int rows);
-
-// ---- sample.hip: the sample sort of one or many segments ----
-constexpr int kSsMaxBuckets = 512;    // per segment
-constexpr int kSsLutWords = 2049;     // a segment's splitter table
-// A plan: the segments (tables as a batch's, or seg null and one segment of n
-// keys in nb buckets) and the workspace ss_carve lays out.
-struct SsPlan {
-  const SegInfo *seg = nullptr;
-  SegState *ss = nullptr;                  // with seg: where duplicates are reported
-  TileTable tiles{};                       // of ss_tile<K>() keys
-  const uint32_t *bucket_first = nullptr;  // B + 1 entries
-  uint32_t n = 0, nb = 0;
-  uint32_t max_nb = 0;                     // buckets of the largest segment
-  int64_t n_segs = 0, n_tiles = 0, n_buckets = 0;
-  void *splitters = nullptr;
-  uint32_t *lut = nullptr, *counts = nullptr, *cursors = nullptr, *n_big = nullptr;
-  BkItem *items = nullptr, *big = nullptr;
-  uint16_t *ids = nullptr;                 // every key's bucket
-};
-// Buckets of a segment of n keys; 0: too many keys for this sort.
-template <typename K> int ss_buckets(int64_t n);
-template <typename K> int ss_tile();
-template <typename K> size_t ss_ws_bytes(int64_t buckets, int64_t segs, int64_t slots);
-template <typename K>
-void ss_carve(void *ws, int64_t buckets, int64_t segs, int64_t slots, SsPlan &p);
-// Sorts every segment of kA (keys and, with labels, labels in input order)
-// into (kA, vA) through (kB, vB).  A segment of a table lands one slot to the
-// right where a zero key is prepended, which leaves the slot to that key.
-// Equal neighbours (and a zero key to merge) set ss[s].dups, or st->msd_dups
-// for the single segment.
-template <typename K>
-void launch_sample_sort(K *kA, uint32_t *vA, K *kB, uint32_t *vB, const uint32_t *labels,
-                        const SsPlan &p, int mbits, int prepend, RunState *st, hipStream_t s);
 
 void launch_seg_init(SegState *ss, int64_t B, hipStream_t s);                   // morton.hip
 void launch_bbox_seg(const float *pts, int dim, const BatchDev &b, hipStream_t s);

@@ -59,7 +59,7 @@ struct SsOut {
   uint32_t *dups;
 };
 __device__ inline SsOut ss_out(const SsPlan &p, uint32_t s, uint32_t prepend, RunState *st) {
-  if (!p.seg) return {0u, prepend, 0u, &st->msd_dups};
+  if (!p.ss) return {0u, prepend, 0u, &st->msd_dups};
   const uint32_t pre = p.seg[s].prepend;
   return {p.seg[s].kofs, pre, pre, &p.ss[s].dups};
 }
@@ -137,6 +137,7 @@ __global__ __launch_bounds__(kBlock) void ss_count_kernel(const K *__restrict__ 
   __shared__ K s_sp[kSsMaxBuckets];
   __shared__ uint32_t s_lut[kSsLutWords];
   const uint32_t tile = blockIdx.x;
+  if (p.limits && tile >= p.limits[0]) return;
   const uint32_t s = p.seg ? p.tiles.seg[tile] : 0u;
   const SsSeg sg = ss_segment(p, s);
   if (sg.nb < 2) return;
@@ -222,6 +223,7 @@ __global__ __launch_bounds__(kBlock) void ss_scatter_kernel(const K *__restrict_
   __shared__ uint32_t s_cnt[kSsMaxBuckets], s_lstart[kSsMaxBuckets], s_gstart[kSsMaxBuckets];
   __shared__ uint32_t s_w4[4];
   const uint32_t tile = blockIdx.x;
+  if (p.limits && tile >= p.limits[0]) return;
   const uint32_t s = p.seg ? p.tiles.seg[tile] : 0u;
   const SsSeg sg = ss_segment(p, s);
   if (sg.nb < 2) return;
@@ -281,22 +283,25 @@ __global__ __launch_bounds__(kBlock) void ss_scatter_kernel(const K *__restrict_
 }
 
 // Sorts each bucket (at most CAP keys) in LDS, from the buffer that holds it
-// into kA (and vA) at its own positions, shifted by the segment's prepended
+// (kmid, or kin for a segment of one bucket; either may be kA) into kA (and
+// vA) at its own positions, shifted by the segment's prepended
 // key.  Reports equal neighbours, and a zero key at the front where one is
 // prepended.
 template <typename K, bool LAB, int BS, int IPT>
-__global__ __launch_bounds__(BS) void ss_sort_kernel(K *kA, uint32_t *vA, const K *kB,
-                                                     const uint32_t *vB, SsPlan p,
-                                                     uint32_t prepend, RunState *st) {
+__global__ __launch_bounds__(BS) void ss_sort_kernel(const K *kin, const uint32_t *vin,
+                                                     const K *kmid, const uint32_t *vmid, K *kA,
+                                                     uint32_t *vA, SsPlan p, uint32_t prepend,
+                                                     RunState *st) {
   constexpr int CAP = BS * IPT;
   __shared__ K s_keys[CAP];
   __shared__ uint32_t s_vals[LAB ? CAP : 1];
   __shared__ __align__(16) uint32_t s_tmp[bin_words<K, BS>()];
+  if (p.limits && blockIdx.x >= p.limits[1]) return;
   const BkItem it = p.items[blockIdx.x];
   const uint32_t s0 = it.start, cnt = min(it.count, (uint32_t)CAP);
   if (cnt == 0) return;
-  const K *in = it.parity ? kB : kA;
-  const uint32_t *vin = it.parity ? vB : vA;
+  const K *in = it.parity ? kmid : kin;
+  const uint32_t *lin = it.parity ? vmid : vin;
   const SsOut o = ss_out(p, it.sbits, prepend, st);
   const uint32_t t = threadIdx.x;
   K k[IPT];
@@ -305,7 +310,7 @@ __global__ __launch_bounds__(BS) void ss_sort_kernel(K *kA, uint32_t *vA, const 
   for (int j = 0; j < IPT; ++j) {
     const uint32_t i = (uint32_t)j * BS + t;
     k[j] = i < cnt ? in[s0 + i] : kzero_value<K>();
-    v[j] = (LAB && i < cnt) ? vin[s0 + i] : 0u;
+    v[j] = (LAB && i < cnt) ? lin[s0 + i] : 0u;
   }
   lds_bin_sort<K, LAB, BS, IPT>(k, v, cnt, [&](uint32_t i) { return in[s0 + i]; }, s_keys,
                                   s_vals, s_tmp);
@@ -330,8 +335,8 @@ __global__ __launch_bounds__(BS) void ss_sort_kernel(K *kA, uint32_t *vA, const 
 // 1024 keys).  Always reports duplicates: telling equal neighbours apart is
 // left to unique.
 template <typename K, bool LAB>
-__global__ __launch_bounds__(kSsBlock) void ss_big_kernel(K *__restrict__ kA, uint32_t *__restrict__ vA,
-                                                          K *__restrict__ kB, uint32_t *__restrict__ vB,
+__global__ __launch_bounds__(kSsBlock) void ss_big_kernel(K *kmid, uint32_t *vmid, K *kA,
+                                                          uint32_t *vA, K *kB, uint32_t *vB,
                                                           SsPlan p, RunState *st) {
   constexpr int NW = kSsBlock / 64;
   __shared__ uint32_t s_base[256], s_wc[NW * 256];
@@ -342,11 +347,12 @@ __global__ __launch_bounds__(kSsBlock) void ss_big_kernel(K *__restrict__ kA, ui
     const BkItem it = p.big[e];
     const SsOut o = ss_out(p, it.sbits, 0u, st);
     if (t == 0) raise_flag(o.dups);
-    // from buffer B (a big bucket was scattered: a segment of one bucket fits)
+    // from kmid (a big bucket was scattered: a segment of one bucket fits)
+    // and the other buffer in turn, to end in A (shifted only where kmid is B)
     K *const outk = kA + o.shift;
     uint32_t *const outv = LAB ? vA + o.shift : nullptr;
-    K *src = kB, *dst = outk;
-    uint32_t *vsrc = vB, *vdst = outv;
+    K *src = kmid, *dst = kmid == kA ? kB : outk;
+    uint32_t *vsrc = vmid, *vdst = kmid == kA ? vB : outv;
     uint64_t olo = 0, ohi = 0, alo = ~0ull, ahi = ~0ull;
     for (uint32_t i = t; i < it.count; i += kSsBlock) {
       const K x = src[it.start + i];
@@ -439,11 +445,13 @@ template <typename K>
 int64_t ss_bucket_keys() { return (int64_t)SsItem<K>::CAP * 40 / 100; }
 
 template <typename K>
+int64_t ss_max_keys() { return ss_bucket_keys<K>() * kSsMaxBuckets; }
+
+template <typename K>
 int ss_buckets(int64_t n) {
   if (n <= SsItem<K>::CAP) return 1;
   const int64_t T = ss_bucket_keys<K>();
-  const int64_t nb = (n + T - 1) / T;
-  return nb <= kSsMaxBuckets ? (int)nb : 0;
+  return n <= ss_max_keys<K>() ? (int)((n + T - 1) / T) : 0;
 }
 
 template <typename K>
@@ -473,56 +481,181 @@ void ss_carve(void *ws, int64_t buckets, int64_t segs, int64_t slots, SsPlan &p)
   p.n_segs = segs;
 }
 
-template <typename K, int CAP, int BS>
-void ss_sort(K *kA, uint32_t *vA, K *kB, uint32_t *vB, bool lab, const SsPlan &p, int prepend,
-             RunState *st, hipStream_t s) {
-  const unsigned items = (unsigned)p.n_buckets;
-  if (lab)
-    ss_sort_kernel<K, true, BS, CAP / BS><<<items, BS, 0, s>>>(kA, vA, kB, vB, p,
-                                                               (uint32_t)prepend, st);
-  else
-    ss_sort_kernel<K, false, BS, CAP / BS><<<items, BS, 0, s>>>(kA, nullptr, kB, nullptr, p,
-                                                                (uint32_t)prepend, st);
+// The crowded buckets' tables, at most S segments: SegInfo[S], first tiles
+// and first buckets (S + 1 each), the two limits, tile -> segment.
+struct SsTables {
+  SegInfo *seg;
+  uint32_t *tile_first, *bucket_first, *limits, *tile_seg;
+};
+inline SsTables ss_tables(void *ws, int64_t S) {
+  char *q = static_cast<char *>(ws);
+  auto take = [&](size_t bytes) { char *r = q; q += align256_dev(bytes); return r; };
+  SsTables t;
+  t.seg = reinterpret_cast<SegInfo *>(take((size_t)S * sizeof(SegInfo)));
+  t.tile_first = reinterpret_cast<uint32_t *>(take((size_t)(S + 1) * 4));
+  t.bucket_first = reinterpret_cast<uint32_t *>(take((size_t)(S + 1) * 4));
+  t.limits = reinterpret_cast<uint32_t *>(take(8));
+  t.tile_seg = reinterpret_cast<uint32_t *>(q);
+  return t;
+}
+// (a crowded bucket holds more than the bucket sort's CAP keys)
+template <typename K>
+int64_t ss_crowded_segs(int64_t n) { return n / Bk<K>::CAP + 2; }
+template <typename K>
+int64_t ss_crowded_buckets(int64_t n) { return n / ss_bucket_keys<K>() + ss_crowded_segs<K>(n); }
+template <typename K>
+int64_t ss_crowded_tiles(int64_t n) { return n / ss_tile<K>() + ss_crowded_segs<K>(n); }
+
+template <typename K>
+size_t ss_tree_bytes(int64_t n) {
+  const int64_t S = ss_crowded_segs<K>(n);
+  const size_t tables = align256_dev((size_t)S * sizeof(SegInfo)) +
+                        2 * align256_dev((size_t)(S + 1) * 4) + align256_dev(8) +
+                        align256_dev((size_t)ss_crowded_tiles<K>(n) * 4);
+  return tables + ss_ws_bytes<K>(ss_crowded_buckets<K>(n), S, n);
 }
 
 template <typename K>
-void launch_sample_sort(K *kA, uint32_t *vA, K *kB, uint32_t *vB, const uint32_t *labels,
-                        const SsPlan &p, int mbits, int prepend, RunState *st, hipStream_t s) {
-  const bool lab = labels != nullptr;
+void ss_tree_carve(void *ws, int64_t n, SsTree &t) {
+  const int64_t S = ss_crowded_segs<K>(n);
+  const size_t tables = ss_tree_bytes<K>(n) - ss_ws_bytes<K>(ss_crowded_buckets<K>(n), S, n);
+  char *rest = static_cast<char *>(ws) + tables;
+  t.tables = ws;
+  ss_carve<K>(rest, ss_crowded_buckets<K>(n), S, n, t.crowded);
+  const int nb = ss_buckets<K>(n);
+  if (nb > 1) {
+    ss_carve<K>(rest, nb, 1, n, t.whole);
+    t.whole.n = (uint32_t)n;
+    t.whole.nb = t.whole.max_nb = (uint32_t)nb;
+    t.whole.n_tiles = (n + ss_tile<K>() - 1) / ss_tile<K>();
+  }
+}
+
+// One workgroup: the tables of the nseg crowded buckets segs[].  mostly: where
+// they hold more than a quarter of the n keys, the sample sort, not the bucket
+// sort, is reported to have sorted them.
+__global__ __launch_bounds__(kSsBlock) void ss_tables_kernel(const BkSeg *__restrict__ segs,
+                                                             uint32_t nseg, uint32_t T,
+                                                             uint32_t tile, uint32_t n,
+                                                             int mostly, SsTables o,
+                                                             RunState *st) {
+  __shared__ uint32_t s_w[kSsBlock / 64];
+  uint32_t tiles = 0, buckets = 0;   // before this round's segments (uniform)
+  for (uint32_t base = 0; base < nseg; base += kSsBlock) {
+    const uint32_t i = base + threadIdx.x;
+    const uint32_t cnt = i < nseg ? segs[i].count : 0u;
+    const uint32_t nt = (cnt + tile - 1) / tile, nb = (cnt + T - 1) / T;
+    uint32_t all_t, all_b;
+    const uint32_t ft = tiles + block_excl_sum<uint32_t, kSsBlock / 64>(nt, s_w, &all_t);
+    __syncthreads();   // s_w is reused
+    const uint32_t fb = buckets + block_excl_sum<uint32_t, kSsBlock / 64>(nb, s_w, &all_b);
+    __syncthreads();
+    if (i < nseg) {
+      SegInfo x{};
+      x.n = cnt;
+      x.kofs = segs[i].start;
+      o.seg[i] = x;
+      o.tile_first[i] = ft;
+      o.bucket_first[i] = fb;
+      for (uint32_t k = 0; k < nt; ++k) o.tile_seg[ft + k] = i;
+    }
+    tiles += all_t;
+    buckets += all_b;
+  }
+  if (threadIdx.x == 0) {
+    o.tile_first[nseg] = tiles;
+    o.bucket_first[nseg] = buckets;
+    o.limits[0] = tiles;
+    o.limits[1] = buckets;
+    if (mostly && (uint64_t)st->bk_keys * 4 > n) st->ss_ok = 1u;
+  }
+}
+
+template <typename K, int CAP, int BS>
+void ss_sort(const K *kin, const uint32_t *vin, const K *kmid, const uint32_t *vmid, K *kA,
+             uint32_t *vA, const SsPlan &p, int prepend, RunState *st, hipStream_t s) {
+  const unsigned items = (unsigned)p.n_buckets;
+  if (vin)
+    ss_sort_kernel<K, true, BS, CAP / BS><<<items, BS, 0, s>>>(kin, vin, kmid, vmid, kA, vA, p,
+                                                               (uint32_t)prepend, st);
+  else
+    ss_sort_kernel<K, false, BS, CAP / BS><<<items, BS, 0, s>>>(kin, nullptr, kmid, nullptr, kA,
+                                                                nullptr, p, (uint32_t)prepend, st);
+}
+
+template <typename K>
+void launch_sample_sort(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, K *kB,
+                        uint32_t *vB, const SsPlan &p, int mbits, int prepend, RunState *st,
+                        hipStream_t s) {
+  K *kmid = kin == kA ? kB : kA;
+  uint32_t *vmid = kin == kA ? vB : vA;
   const unsigned segs = (unsigned)p.n_segs, tiles = (unsigned)p.n_tiles;
   const unsigned zgrid = (unsigned)std::min<int64_t>((p.n_buckets + kBlock - 1) / kBlock, 1024);
   ss_zero_kernel<<<zgrid, kBlock, 0, s>>>(p.counts, (uint32_t)p.n_buckets, p.n_big);
   if (p.max_nb <= kSsMaxBuckets / 4)
-    ss_splitters_kernel<K, kSsIpt / 4><<<segs, kSsBlock, 0, s>>>(kA, p, mbits);
+    ss_splitters_kernel<K, kSsIpt / 4><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
   else if (p.max_nb <= kSsMaxBuckets / 2)
-    ss_splitters_kernel<K, kSsIpt / 2><<<segs, kSsBlock, 0, s>>>(kA, p, mbits);
+    ss_splitters_kernel<K, kSsIpt / 2><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
   else
-    ss_splitters_kernel<K, kSsIpt><<<segs, kSsBlock, 0, s>>>(kA, p, mbits);
-  ss_count_kernel<K><<<tiles, kBlock, 0, s>>>(kA, p, mbits);
+    ss_splitters_kernel<K, kSsIpt><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
+  ss_count_kernel<K><<<tiles, kBlock, 0, s>>>(kin, p, mbits);
   ss_plan_kernel<<<segs, kSsMaxBuckets, 0, s>>>(p, (uint32_t)SsItem<K>::CAP, st);
-  if (lab)
-    ss_scatter_kernel<K, true><<<tiles, kBlock, 0, s>>>(kA, labels, kB, vB, p);
+  if (vin)
+    ss_scatter_kernel<K, true><<<tiles, kBlock, 0, s>>>(kin, vin, kmid, vmid, p);
   else
-    ss_scatter_kernel<K, false><<<tiles, kBlock, 0, s>>>(kA, nullptr, kB, nullptr, p);
+    ss_scatter_kernel<K, false><<<tiles, kBlock, 0, s>>>(kin, nullptr, kmid, nullptr, p);
   // Few buckets leave the chip to one workgroup per CU or less: then twice
   // the threads on each (300,000 keys: 170 against 181 us a build); with many,
   // two workgroups of half of them on each CU (55 M keys: 3.03 against 3.35 ms
   // a batch).
-  using C = SsItem<K>;
-  const unsigned items = (unsigned)p.n_buckets;
-  if (items <= 512) ss_sort<K, C::CAP, 1024>(kA, vA, kB, vB, lab, p, prepend, st, s);
-  else ss_sort<K, C::CAP, 512>(kA, vA, kB, vB, lab, p, prepend, st, s);
-  if (lab) ss_big_kernel<K, true><<<64, kSsBlock, 0, s>>>(kA, vA, kB, vB, p, st);
-  else ss_big_kernel<K, false><<<64, kSsBlock, 0, s>>>(kA, nullptr, kB, nullptr, p, st);
+  constexpr int CAP = SsItem<K>::CAP;
+  if (p.n_buckets <= 512)
+    ss_sort<K, CAP, 1024>(kin, vin, kmid, vmid, kA, vA, p, prepend, st, s);
+  else
+    ss_sort<K, CAP, 512>(kin, vin, kmid, vmid, kA, vA, p, prepend, st, s);
+  if (vin)
+    ss_big_kernel<K, true><<<64, kSsBlock, 0, s>>>(kmid, vmid, kA, vA, kB, vB, p, st);
+  else
+    ss_big_kernel<K, false><<<64, kSsBlock, 0, s>>>(kmid, nullptr, kA, nullptr, kB, nullptr, p, st);
+}
+
+template <typename K>
+void launch_sample_sort_buckets(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, K *kB,
+                                uint32_t *vB, const SsTree &t, const BkSeg *segs, uint32_t nseg,
+                                uint64_t nkeys, uint32_t max_keys, int64_t n, int mbits,
+                                int prepend, RunState *st, hipStream_t s) {
+  const SsTables o = ss_tables(t.tables, ss_crowded_segs<K>(n));
+  const uint32_t T = (uint32_t)ss_bucket_keys<K>();
+  ss_tables_kernel<<<1, kSsBlock, 0, s>>>(segs, nseg, T, (uint32_t)ss_tile<K>(), (uint32_t)n,
+                                          sizeof(K) <= 8 ? 1 : 0, o, st);
+  SsPlan p = t.crowded;
+  p.seg = o.seg;
+  p.tiles.seg = o.tile_seg;
+  p.tiles.first = o.tile_first;
+  p.bucket_first = o.bucket_first;
+  p.limits = o.limits;
+  p.n_segs = nseg;
+  p.n_tiles = (int64_t)(nkeys / ss_tile<K>()) + nseg;
+  p.n_buckets = (int64_t)(nkeys / T) + nseg;
+  p.max_nb = (max_keys + T - 1) / T;
+  launch_sample_sort<K>(kin, vin, kA, vA, kB, vB, p, mbits, prepend, st, s);
 }
 
 #define PGVD_SS_INST(K)                                                                       \
   template int ss_buckets<K>(int64_t);                                                        \
+  template int64_t ss_max_keys<K>();                                                          \
   template int ss_tile<K>();                                                                  \
   template size_t ss_ws_bytes<K>(int64_t, int64_t, int64_t);                                  \
   template void ss_carve<K>(void *, int64_t, int64_t, int64_t, SsPlan &);                     \
-  template void launch_sample_sort<K>(K *, uint32_t *, K *, uint32_t *, const uint32_t *,     \
-                                      const SsPlan &, int, int, RunState *, hipStream_t);
+  template size_t ss_tree_bytes<K>(int64_t);                                                  \
+  template void ss_tree_carve<K>(void *, int64_t, SsTree &);                                  \
+  template void launch_sample_sort<K>(const K *, const uint32_t *, K *, uint32_t *, K *,      \
+                                      uint32_t *, const SsPlan &, int, int, RunState *,       \
+                                      hipStream_t);                                           \
+  template void launch_sample_sort_buckets<K>(const K *, const uint32_t *, K *, uint32_t *,   \
+                                              K *, uint32_t *, const SsTree &, const BkSeg *, \
+                                              uint32_t, uint64_t, uint32_t, int64_t, int,     \
+                                              int, RunState *, hipStream_t);
 PGVD_SS_INST(uint32_t)
 PGVD_SS_INST(uint64_t)
 PGVD_SS_INST(Key128)

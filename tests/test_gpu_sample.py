@@ -98,3 +98,22 @@ def test_batch_matches_radix_passes(dev, dim, bits, cap, tile):
             assert_tree_equal(got, want, FIELDS, where=f"instance {i} (n={sizes[i]})")
     finally:
         d.free()
+
+
+@pytest.mark.parametrize("dim,bits,n,labels", [(3, 21, 1 << 21, False), (3, 21, 1500001, True),
+                                               (3, 42, 700001, True), (2, 16, 1800001, False)])
+@pytest.mark.parametrize("share,sigma", [(0.1, 1e-3), (0.9, 1e-3), (0.9, 2e-5)])
+def test_crowded_buckets_match_radix(dev, dim, bits, n, labels, share, sigma):
+    """Arrays too large to be one segment: the bucket sort's crowded buckets,
+    some of them of repeated keys, beside its ordinary ones."""
+    pts = np.random.default_rng(3).random((n, dim), dtype=np.float32) * 2 - 1
+    k = int(share * n)
+    pts[:k] = clustered(k, dim, 9, sigma, (0.1, 0.02))
+    lab = np.random.default_rng(5).integers(0, 3, n).astype(np.uint32) if labels else None
+    got = dev.build_octree(pts, bits, labels=lab)
+    want = dev.build_octree(pts, bits, labels=lab, no_host_wait=True)
+    assert want["bucket_sort"] == 0
+    assert_tree_equal(got, want, FIELDS)
+    if labels:
+        for f in ("key_conflict", "node_conflict"):
+            assert np.array_equal(got[f], want[f]), f
