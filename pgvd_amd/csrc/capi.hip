@@ -966,12 +966,12 @@ int pgvd_cell_walk(pgvd_ctx *ctx, const float *segs, int64_t n, int bits, const 
   void *counts = nullptr, *ws = nullptr, *scratch = nullptr;
   CHK(pool_get(ctx, "walk_counts", 4 * static_cast<size_t>(n), &counts));
   CHK(pool_get(ctx, "walk_ws", 8 * static_cast<size_t>(walk_scan_ws_words(n)), &ws));
-  // With a cell buffer, the first walk keeps each segment's first 32 cells
-  // (up to 2 GB of scratch, or PGVD_WALK_SCRATCH_BYTES from the
+  // With a cell buffer, the first walk keeps each segment's first cells (32,
+  // or more for few segments; up to 2 GB of scratch, or PGVD_WALK_SCRATCH_BYTES from the
   // environment), so that only longer walks run twice; past that, a count
   // walk and a write walk.
-  constexpr int kLog2K = 5;
-  const size_t spec_bytes = (static_cast<size_t>(n) << kLog2K) * 20;
+  const int log2k = walk_log2_kept(n);
+  const size_t spec_bytes = (static_cast<size_t>(n) << log2k) * 16;
   size_t spec_limit = size_t(2) << 30;
   if (const char *e = std::getenv("PGVD_WALK_SCRATCH_BYTES")) spec_limit = std::strtoull(e, nullptr, 10);
   if (cells && spec_bytes <= spec_limit)
@@ -981,7 +981,7 @@ int pgvd_cell_walk(pgvd_ctx *ctx, const float *segs, int64_t n, int bits, const 
     Stage t(ctx, "cell_walk_count", st);
     launch_cell_walk_count(segs, n, bits, octree, octree_size, static_cast<uint32_t *>(counts),
                            status, offsets, static_cast<uint64_t *>(ws),
-                           static_cast<int32_t *>(scratch), kLog2K, st);
+                           scratch, log2k, st);
     CHK(launch_status("cell_walk_count"));
   }
   HIPCHK(hipMemcpyAsync(&total, offsets + n, 8, hipMemcpyDeviceToHost, st));
@@ -991,8 +991,7 @@ int pgvd_cell_walk(pgvd_ctx *ctx, const float *segs, int64_t n, int bits, const 
   if (total > capacity) return fail(PGVD_ERR_CAPACITY, "cell buffer too small (*total_out cells needed)");
   Stage t(ctx, "cell_walk", st);
   launch_cell_walk_write(segs, n, bits, octree, octree_size, offsets, cells,
-                         static_cast<const int32_t *>(scratch), static_cast<uint32_t *>(counts),
-                         kLog2K, st);
+                         scratch, static_cast<uint32_t *>(counts), log2k, st);
   return launch_status("cell_walk");
 }
 

@@ -502,7 +502,9 @@ __global__ __launch_bounds__(kBlock) void mc_visit_kernel(
       const int32_t *c = cells + 5 * g;
       const int32_t ox = c[0], oy = c[1], w = c[2];
       float ts[4], px[4], py[4];
-      const uint32_t keep = walk_isects(ax, ay, bx, by, ox, oy, w, ts, px, py);
+      float vx, vy, len;
+      walk_dir(ax, ay, bx, by, vx, vy, len);
+      const uint32_t keep = walk_isects(ax, ay, vx, vy, len, ox, oy, w, ts, px, py);
       const int nk = __popc(keep);
       float4 part = make_float4(0, 0, 0, 0);
       int32_t l = -1;

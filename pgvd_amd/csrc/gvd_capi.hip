@@ -39,14 +39,14 @@ int walk_pooled(pgvd_ctx *ctx, const float *segs, int64_t n, int bits, const int
   CHK(pool_get(ctx, "mc_offsets", 8 * static_cast<size_t>(n + 1), &offsets));
   CHK(pool_get(ctx, "walk_counts", 4 * static_cast<size_t>(n), &counts));
   CHK(pool_get(ctx, "walk_ws", 8 * static_cast<size_t>(walk_scan_ws_words(n)), &ws));
-  constexpr int kLog2K = 5;
-  const size_t spec_bytes = (static_cast<size_t>(n) << kLog2K) * 20;
+  const int log2k = walk_log2_kept(n);
+  const size_t spec_bytes = (static_cast<size_t>(n) << log2k) * 16;
   if (spec_bytes <= (size_t(2) << 30)) CHK(pool_get(ctx, "walk_scratch", spec_bytes, &scratch));
   {
     Stage t(ctx, "gvd_walk", st);
     launch_cell_walk_count(segs, n, bits, octree, O, static_cast<uint32_t *>(counts), status,
                            static_cast<int64_t *>(offsets), static_cast<uint64_t *>(ws),
-                           static_cast<int32_t *>(scratch), kLog2K, st);
+                           scratch, log2k, st);
   }
   HIPCHK(hipGetLastError());
   int64_t total = 0;
@@ -57,8 +57,8 @@ int walk_pooled(pgvd_ctx *ctx, const float *segs, int64_t n, int bits, const int
   {
     Stage t(ctx, "gvd_walk_write", st);
     launch_cell_walk_write(segs, n, bits, octree, O, static_cast<const int64_t *>(offsets),
-                           static_cast<int32_t *>(cells), static_cast<const int32_t *>(scratch),
-                           static_cast<uint32_t *>(counts), kLog2K, st);
+                           static_cast<int32_t *>(cells), scratch,
+                           static_cast<uint32_t *>(counts), log2k, st);
   }
   HIPCHK(hipGetLastError());
   *offsets_out = static_cast<int64_t *>(offsets);

@@ -195,16 +195,18 @@ void launch_find_leaf(const int32_t *pts, int64_t q, int dim, int bits, const in
 // writes counts (n), status (nullable) and offsets (n + 1, exclusive scan);
 // ws holds walk_scan_ws_words(n) words.  The write pass puts each segment's
 // cells (5 int32 each) at cells + 5 * offsets[i].  With scratch (n << log2k
-// cells), the count pass also keeps each segment's first 2^log2k cells
-// there, and the write pass moves them and walks again only the segments
-// that had more.
+// 16-byte records), the count pass also keeps each segment's first 2^log2k
+// cells there, and the write pass moves them and walks again only the
+// segments that had more.  walk_log2_kept: 32 cells for many segments, more
+// while the records stay within 64 MB (few long walks then run once).
 int64_t walk_scan_ws_words(int64_t n);
+int walk_log2_kept(int64_t n);
 void launch_cell_walk_count(const float *segs, int64_t n, int bits, const int32_t *octree,
                             int64_t size, uint32_t *counts, int32_t *status, int64_t *offsets,
-                            uint64_t *ws, int32_t *scratch, int log2k, hipStream_t s);
+                            uint64_t *ws, void *scratch, int log2k, hipStream_t s);
 void launch_cell_walk_write(const float *segs, int64_t n, int bits, const int32_t *octree,
                             int64_t size, const int64_t *offsets, int32_t *cells,
-                            const int32_t *scratch, uint32_t *counts, int log2k, hipStream_t s);
+                            const void *scratch, uint32_t *counts, int log2k, hipStream_t s);
 // offsets[0] = 0, offsets[i + 1] = counts[0] + ... + counts[i] (n + 1
 // entries); ws holds walk_scan_ws_words(n) words.
 void launch_offsets_scan(const uint32_t *counts, int64_t n, int64_t *offsets, uint64_t *ws,

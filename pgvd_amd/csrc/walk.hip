@@ -97,68 +97,113 @@ __device__ inline void walk_leaf_path(float px, float py, int bits,
 
 // One pass over the segments.  MODE kWalkCount: counts and status;
 // kWalkWrite: the cells at offsets[i]; kWalkSpec: counts and status, and
-// the first K cells of segment i at scratch + 5 * K * i; kWalkRest: for the
-// segments with more than K cells, cells K.. at offsets[i] + K.
+// the first K cells of segment i as records at scratch + K i; kWalkRest: for
+// the segments with more than K cells, cells K.. at offsets[i] + K.
+//
+// A wave takes the segments [w per, (w + 1) per) in turn: a lane whose segment
+// has ended takes the next one once kWalkRefill lanes stand idle (segments
+// differ in length, and 64 of them take as long as their longest: 2^20
+// segments of up to 1/256 of the grid visit 11 cells on average and 30 at
+// most).  What bounds it then is the requests: each lane's node words and
+// records lie on lines of their own.  A kept cell is one 16-byte record
+// (origin x, origin y, parent, octant | level << 2), one store in place of five.
 enum { kWalkCount = 0, kWalkWrite = 1, kWalkSpec = 2, kWalkRest = 3 };
+#ifndef PGVD_WALK_REFILL
+#define PGVD_WALK_REFILL 16
+#endif
+constexpr uint32_t kWalkRefill = PGVD_WALK_REFILL;
 
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void cell_walk_kernel(
-    const float *__restrict__ segs, int64_t n, int bits, const int32_t *__restrict__ octree,
-    int64_t size, uint32_t *__restrict__ counts, int32_t *__restrict__ status,
-    const int64_t *__restrict__ offsets, int32_t *__restrict__ cells, int K) {
+    const float *__restrict__ segs, int64_t n, int64_t per, int bits,
+    const int32_t *__restrict__ octree, int64_t size, uint32_t *__restrict__ counts,
+    int32_t *__restrict__ status, const int64_t *__restrict__ offsets,
+    int32_t *__restrict__ cells, int4 *__restrict__ scratch, int K) {
   // each lane's last descent, node per depth (depth 0 is the root)
   __shared__ int32_t s_path[(kMaxBits + 1) * kBlock];
   int32_t *path = s_path + threadIdx.x;
   path[0] = 0;
-  for (int64_t s = (int64_t)blockIdx.x * kBlock + threadIdx.x; s < n;
-       s += (int64_t)gridDim.x * kBlock) {
-    if (MODE == kWalkRest && counts[s] <= (uint32_t)K) continue;
-    const float ax = segs[4 * s], ay = segs[4 * s + 1], bx = segs[4 * s + 2], by = segs[4 * s + 3];
-    const int dx = bx > ax ? 1 : (bx < ax ? -1 : 0);
-    const int dy = by > ay ? 1 : (by < ay ? -1 : 0);
-    float ct = 0.0f, cx = ax, cy = ay;
-    int32_t bcell[5], cell[5], ncell[5];
-    uint64_t pkey = 0;
-    int plev = 0;
-    walk_leaf(bx, by, bits, octree, size, bcell);
-    walk_leaf_path(cx, cy, bits, octree, size, path, pkey, plev, cell);
-    int32_t *out = MODE == kWalkWrite || MODE == kWalkRest ? cells + 5 * offsets[s]
-                   : MODE == kWalkSpec                     ? cells + 5 * (int64_t)K * s
-                                                           : nullptr;
-    int count = 0, st = 0;
-    bool done = false;
-    do {
+  const uint32_t wave = blockIdx.x * (kBlock / 64) +
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  int64_t next = wave * per;                       // uniform over the wave
+  const int64_t end = next + per < n ? next + per : n;
+  bool active = false;
+  int64_t s = 0;
+  float ax = 0, ay = 0, vx = 0, vy = 0, len = 0, ct = 0, cx = 0, cy = 0;
+  int dx = 0, dy = 0, count = 0;
+  int32_t bcell[5], cell[5] = {0, 0, 1, 0, 0}, ncell[5];
+  uint64_t pkey = 0;
+  int plev = 0;
+  bcell[0] = bcell[1] = 0;
+  // The whole wave takes every round, idle lanes included (the ballot counts
+  // them): one way back to the loop's head, and scalar conditions for the
+  // refill and the end.  A `continue` for the idle lanes would let them turn in
+  // a loop of their own, apart from the lanes that still walk.
+  for (;;) {
+    const uint64_t idle = __ballot(!active);
+    const uint32_t nidle = (uint32_t)__popcll(idle);
+    if (next >= end && nidle == 64) break;
+    if (next < end && nidle >= kWalkRefill) {
+      const int64_t mine = next + __popcll(idle & lanemask_lt());
+      next += nidle;
+      if (!active && mine < end && !(MODE == kWalkRest && counts[mine] <= (uint32_t)K)) {
+        s = mine;
+        ax = segs[4 * s];
+        ay = segs[4 * s + 1];
+        const float bx = segs[4 * s + 2], by = segs[4 * s + 3];
+        dx = bx > ax ? 1 : (bx < ax ? -1 : 0);
+        dy = by > ay ? 1 : (by < ay ? -1 : 0);
+        walk_dir(ax, ay, bx, by, vx, vy, len);
+        ct = 0.0f;
+        cx = ax;
+        cy = ay;
+        count = 0;
+        plev = 0;
+        walk_leaf(bx, by, bits, octree, size, bcell);
+        walk_leaf_path(cx, cy, bits, octree, size, path, pkey, plev, cell);
+        active = true;
+      }
+    } else if (active) {
+      int st = 0;
+      bool done = false;
       if (++count > kWalkMax) {
         st = 1;
         --count;
-        break;
-      }
-      const bool put = MODE == kWalkWrite || (MODE == kWalkSpec && count <= K) ||
-                       (MODE == kWalkRest && count > K);
-      if (put) {
+        done = true;
+      } else {
+        if (MODE == kWalkSpec) {
+          if (count <= K)
+            scratch[(int64_t)K * s + count - 1] =
+                make_int4(cell[0], cell[1], cell[3], cell[4] | plev << 2);
+        } else if (MODE == kWalkWrite || (MODE == kWalkRest && count > K)) {
+          int32_t *out = cells + 5 * (offsets[s] + count - 1);
 #pragma unroll
-        for (int k = 0; k < 5; ++k) out[5 * (count - 1) + k] = cell[k];
-      }
-      float ts[4], px[4], py[4];
-      const uint32_t keep = walk_isects(ax, ay, bx, by, cell[0], cell[1], cell[2], ts, px, py);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (((keep >> i) & 1) && ts[i] > ct) {
-          ct = ts[i];
-          cx = px[i];
-          cy = py[i];
+          for (int k = 0; k < 5; ++k) out[k] = cell[k];
         }
-      if (cx == (float)cell[0] && cx != 0.0f && dx == -1) cx -= 1.0f;
-      if (cy == (float)cell[1] && cy != 0.0f && dy == -1) cy -= 1.0f;
-      walk_leaf_path(cx, cy, bits, octree, size, path, pkey, plev, ncell);
-      done = keep == 0 || (cell[0] == bcell[0] && cell[1] == bcell[1]) ||
-             (ncell[0] == cell[0] && ncell[1] == cell[1]);
+        float ts[4], px[4], py[4];
+        const uint32_t keep = walk_isects(ax, ay, vx, vy, len, cell[0], cell[1], cell[2], ts, px, py);
 #pragma unroll
-      for (int k = 0; k < 5; ++k) cell[k] = ncell[k];
-    } while (!done);
-    if (MODE == kWalkCount || MODE == kWalkSpec) {
-      counts[s] = (uint32_t)count;
-      if (status) status[s] = st;
+        for (int i = 0; i < 4; ++i)
+          if (((keep >> i) & 1) && ts[i] > ct) {
+            ct = ts[i];
+            cx = px[i];
+            cy = py[i];
+          }
+        if (cx == (float)cell[0] && cx != 0.0f && dx == -1) cx -= 1.0f;
+        if (cy == (float)cell[1] && cy != 0.0f && dy == -1) cy -= 1.0f;
+        walk_leaf_path(cx, cy, bits, octree, size, path, pkey, plev, ncell);
+        done = keep == 0 || (cell[0] == bcell[0] && cell[1] == bcell[1]) ||
+               (ncell[0] == cell[0] && ncell[1] == cell[1]);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) cell[k] = ncell[k];
+      }
+      if (done) {
+        if (MODE == kWalkCount || MODE == kWalkSpec) {
+          counts[s] = (uint32_t)count;
+          if (status) status[s] = st;
+        }
+        active = false;
+      }
     }
   }
 }
@@ -166,18 +211,22 @@ __global__ __launch_bounds__(kBlock) void cell_walk_kernel(
 // Moves the speculative pass's first min(count, K) cells of every segment
 // to their offsets; one thread per (segment, slot), K a power of two.
 __global__ __launch_bounds__(kBlock) void walk_compact_kernel(
-    const int32_t *__restrict__ scratch, const uint32_t *__restrict__ counts,
-    const int64_t *__restrict__ offsets, int64_t n, int log2k, int32_t *__restrict__ cells) {
+    const int4 *__restrict__ scratch, const uint32_t *__restrict__ counts,
+    const int64_t *__restrict__ offsets, int64_t n, int log2k, int bits,
+    int32_t *__restrict__ cells) {
   const int64_t slots = n << log2k;
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < slots;
        i += (int64_t)gridDim.x * kBlock) {
     const int64_t s = i >> log2k;
     const uint32_t k = (uint32_t)(i & ((int64_t(1) << log2k) - 1));
     if (k < counts[s]) {
-      const int32_t *src = scratch + 5 * i;
+      const int4 r = scratch[i];
       int32_t *dst = cells + 5 * (offsets[s] + k);
-#pragma unroll
-      for (int j = 0; j < 5; ++j) dst[j] = src[j];
+      dst[0] = r.x;
+      dst[1] = r.y;
+      dst[2] = (int32_t)(1u << (bits - (r.w >> 2)));
+      dst[3] = r.z;
+      dst[4] = r.w & 3;
     }
   }
 }
@@ -222,22 +271,34 @@ __global__ void walk_ws_zero_kernel(uint64_t *ws, int64_t words) {
 
 int64_t walk_scan_ws_words(int64_t n) { return 4 + (n + 4 * kBlock - 1) / (4 * kBlock); }
 
+int walk_log2_kept(int64_t n) {
+  int k = 5;
+  while (k < 10 && (n << (k + 1)) * 16 <= (int64_t(64) << 20)) ++k;
+  return k;
+}
+
+// The walk's grid and segments per wave: about 20 waves per CU (what the
+// descents' LDS allows), each with its own run of segments; fewer segments
+// than that take one wave per 64.
+static unsigned walk_grid(int64_t n, int64_t *per) {
+  const int64_t waves = std::min<int64_t>((n + 63) / 64, 256 * 20);
+  *per = (n + waves - 1) / waves;
+  return (unsigned)((waves + kBlock / 64 - 1) / (kBlock / 64));
+}
+
 void launch_cell_walk_count(const float *segs, int64_t n, int bits, const int32_t *octree,
                             int64_t size, uint32_t *counts, int32_t *status, int64_t *offsets,
-                            uint64_t *ws, int32_t *scratch, int log2k, hipStream_t s) {
-  int64_t grid = (n + kBlock - 1) / kBlock;
-  if (grid > 8192) grid = 8192;
+                            uint64_t *ws, void *scratch, int log2k, hipStream_t s) {
+  int64_t per;
+  const unsigned grid = walk_grid(n, &per);
   if (scratch)
-    cell_walk_kernel<kWalkSpec><<<(unsigned)grid, kBlock, 0, s>>>(
-        segs, n, bits, octree, size, counts, status, nullptr, scratch, 1 << log2k);
+    cell_walk_kernel<kWalkSpec><<<grid, kBlock, 0, s>>>(segs, n, per, bits, octree, size, counts,
+                                                        status, nullptr, nullptr,
+                                                        static_cast<int4 *>(scratch), 1 << log2k);
   else
-    cell_walk_kernel<kWalkCount><<<(unsigned)grid, kBlock, 0, s>>>(
-        segs, n, bits, octree, size, counts, status, nullptr, nullptr, 0);
-  const int64_t words = walk_scan_ws_words(n);
-  walk_ws_zero_kernel<<<(unsigned)std::min<int64_t>((words + kBlock - 1) / kBlock, 1024), kBlock,
-                        0, s>>>(ws, words);
-  const int64_t tiles = (n + 4 * kBlock - 1) / (4 * kBlock);
-  walk_scan_kernel<<<(unsigned)tiles, kBlock, 0, s>>>(counts, n, offsets, ws);
+    cell_walk_kernel<kWalkCount><<<grid, kBlock, 0, s>>>(segs, n, per, bits, octree, size, counts,
+                                                         status, nullptr, nullptr, nullptr, 0);
+  launch_offsets_scan(counts, n, offsets, ws, s);
 }
 
 void launch_offsets_scan(const uint32_t *counts, int64_t n, int64_t *offsets, uint64_t *ws,
@@ -251,20 +312,21 @@ void launch_offsets_scan(const uint32_t *counts, int64_t n, int64_t *offsets, ui
 
 void launch_cell_walk_write(const float *segs, int64_t n, int bits, const int32_t *octree,
                             int64_t size, const int64_t *offsets, int32_t *cells,
-                            const int32_t *scratch, uint32_t *counts, int log2k, hipStream_t s) {
-  int64_t grid = (n + kBlock - 1) / kBlock;
-  if (grid > 8192) grid = 8192;
+                            const void *scratch, uint32_t *counts, int log2k, hipStream_t s) {
+  int64_t per;
+  const unsigned grid = walk_grid(n, &per);
   if (!scratch) {
-    cell_walk_kernel<kWalkWrite><<<(unsigned)grid, kBlock, 0, s>>>(
-        segs, n, bits, octree, size, nullptr, nullptr, offsets, cells, 0);
+    cell_walk_kernel<kWalkWrite><<<grid, kBlock, 0, s>>>(segs, n, per, bits, octree, size, nullptr,
+                                                         nullptr, offsets, cells, nullptr, 0);
     return;
   }
   int64_t cgrid = ((n << log2k) + kBlock - 1) / kBlock;
   if (cgrid > 16384) cgrid = 16384;
-  walk_compact_kernel<<<(unsigned)cgrid, kBlock, 0, s>>>(scratch, counts, offsets, n, log2k,
-                                                          cells);
-  cell_walk_kernel<kWalkRest><<<(unsigned)grid, kBlock, 0, s>>>(
-      segs, n, bits, octree, size, counts, nullptr, offsets, cells, 1 << log2k);
+  walk_compact_kernel<<<(unsigned)cgrid, kBlock, 0, s>>>(static_cast<const int4 *>(scratch), counts,
+                                                         offsets, n, log2k, bits, cells);
+  cell_walk_kernel<kWalkRest><<<grid, kBlock, 0, s>>>(segs, n, per, bits, octree, size, counts,
+                                                      nullptr, offsets, cells, nullptr,
+                                                      1 << log2k);
 }
 
 }  // namespace pgvd

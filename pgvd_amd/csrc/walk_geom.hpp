@@ -18,17 +18,23 @@ __device__ inline float dot2(float ux, float uy, float vx, float vy) {
   return r;
 }
 
+// The segment's direction, normalised, and its length.
+__device__ inline void walk_dir(float ax, float ay, float bx, float by, float &vx, float &vy,
+                                float &len) {
+  vx = bx - ax;
+  vy = by - ay;
+  len = sqrtf(dot2(vx, vy, vx, vy));
+  vx = vx / len;
+  vy = vy / len;
+}
+
 // OctreeUtils.cpp:80-172 for the cell at (ox, oy) of width w: candidates
 // in the reference's order (bottom, right, top, left) in fixed slots t, x,
 // y; returns the mask of those kept (the reference's list is the kept slots
-// in order).
-__device__ inline uint32_t walk_isects(float ax, float ay, float bx, float by, int32_t ox,
-                                       int32_t oy, int32_t w, float (&ts)[4], float (&px)[4],
-                                       float (&py)[4]) {
-  float vx = bx - ax, vy = by - ay;
-  const float len = sqrtf(dot2(vx, vy, vx, vy));
-  vx = vx / len;
-  vy = vy / len;
+// in order).  (vx, vy), len: walk_dir of the segment.
+__device__ inline uint32_t walk_isects(float ax, float ay, float vx, float vy, float len,
+                                       int32_t ox, int32_t oy, int32_t w, float (&ts)[4],
+                                       float (&px)[4], float (&py)[4]) {
   const float mnx = (float)ox, mny = (float)oy;
   const float mxx = (float)ox + (float)w, mxy = (float)oy + (float)w;
   ts[0] = ((float)oy - ay) / vy;          // bottom
