@@ -10,8 +10,8 @@
 //           LDS and copies the run out at its offset in turn;
 //   parse:  a workgroup takes 4 x 8192 bytes, marks where tokens start
 //           (a non-space after a space), scans the counts to token numbers,
-//           parses every token from LDS and writes the tile's records
-//           k - 1 as one run (token 0 is N, read by the host).
+//           lists the starts, and parses the tokens from LDS one to a lane,
+//           token k into value k - 1 (token 0 is N, read by the host).
 #include "kernels.hpp"
 #include "tilescan.hpp"
 
@@ -52,16 +52,21 @@ __device__ inline int dec_len(int32_t v) {
   return n + (v < 0);
 }
 
-// Prints v and one space at s[at..]; returns the position after the space.
-__device__ inline int put_dec(uint8_t *s, int at, int32_t v) {
-  const int n = dec_len(v);
+// Prints v, n = dec_len(v) characters, and one space at s[at..]; returns the
+// position after the space.  Two digits a step: their values come from one
+// multiplication and a table of the 100 pairs.
+__device__ inline int put_dec(uint8_t *s, int at, int32_t v, int n, const uint16_t *pairs) {
   uint32_t u = v < 0 ? 0u - (uint32_t)v : (uint32_t)v;
   int e = at + n;
   s[e] = ' ';
-  do {
-    s[--e] = (uint8_t)('0' + u % 10u);
-    u /= 10u;
-  } while (u);
+  while (u >= 10u) {
+    const uint32_t q = u / 100u, two = pairs[u - q * 100u];
+    s[--e] = (uint8_t)(two >> 8);
+    s[--e] = (uint8_t)two;
+    u = q;
+  }
+  // a digit is left, or none (an even number of them is out, unless v is 0)
+  if (e > at + (v < 0)) s[--e] = (uint8_t)('0' + u);
   if (v < 0) s[at] = '-';
   return at + n + 1;
 }
@@ -81,31 +86,41 @@ static_assert(kFmtRounds >= 1 && kFmtRounds <= 4, "round lengths are packed in 1
 // A tile is kFmtRounds rounds of 256 nodes with one look-back: the rounds'
 // text lengths are scanned together as 16-bit fields of one word (a round
 // holds at most 256 * 108 bytes, below 2^16), then each round is printed
-// into LDS and copied out in turn.
+// into LDS, from the byte that its run begins at in a 16-byte line of the
+// text, and the lines are copied out whole (the first and last by bytes).
+// What bounds it is the byte stores into LDS and the digits' arithmetic; an
+// octree of 2^22 uniform 3D points takes 91 us (106 with a division for each
+// digit, the lengths found twice and words put together from bytes).
 template <int DIM>
 __global__ __launch_bounds__(kFmtBlock) void format_text_kernel(
     const int32_t *__restrict__ octree, int64_t O, int64_t N_hdr, int hdr_len,
     uint8_t *__restrict__ text, int64_t capacity, uint64_t *__restrict__ ws, int ntiles) {
   constexpr int STRIDE = (1 << DIM) + 1;
-  __shared__ uint8_t s_txt[kFmtBlock * kMaxNodeText];
+  __shared__ __align__(16) uint8_t s_txt[kFmtBlock * kMaxNodeText + 16];
+  __shared__ uint16_t s_pairs[100];
   __shared__ uint64_t s_w[kFmtBlock / 64];
   __shared__ int s_tile;
   const int t = threadIdx.x;
   if (t == 0) s_tile = (int)atomicAdd(reinterpret_cast<unsigned int *>(ws + kWsCounter), 1u);
+  if (t < 100) s_pairs[t] = (uint16_t)((uint32_t)('0' + t / 10) | (uint32_t)('0' + t % 10) << 8);
   __syncthreads();
   const int tile = s_tile;
   const int64_t first = (int64_t)tile * kFmtBlock * kFmtRounds;
   uint64_t packed = 0;
+  uint64_t lens[kFmtRounds];   // the values' lengths, 4 bits each
   int32_t cur[STRIDE];   // the records of the round being printed (round 0 kept from here)
 #pragma unroll
   for (int r = 0; r < kFmtRounds; ++r) {
     const int64_t i = first + r * kFmtBlock + t;
     uint32_t len = 0;
+    lens[r] = 0;
 #pragma unroll
     for (int k = 0; k < STRIDE; ++k) {
       const int32_t x = i < O ? octree[i * STRIDE + k] : 0;
       if (r == 0) cur[k] = x;
-      len += (uint32_t)dec_len(x) + 1u;
+      const int n = dec_len(x);
+      lens[r] |= (uint64_t)n << (4 * k);
+      len += (uint32_t)n + 1u;
     }
     packed |= (uint64_t)(i < O ? len : 0u) << (16 * r);
   }
@@ -131,7 +146,7 @@ __global__ __launch_bounds__(kFmtBlock) void format_text_kernel(
   }
 #pragma unroll
   for (int r = 0; r < kFmtRounds; ++r) {
-    const uint32_t rtotal = (uint32_t)(tot_packed >> (16 * r)) & 0xffffu;
+    const int rtotal = (int)((uint32_t)(tot_packed >> (16 * r)) & 0xffffu);
     const int64_t i = first + r * kFmtBlock + t;
     // the next round's records load while this round prints
     int32_t nxt[STRIDE];
@@ -139,27 +154,26 @@ __global__ __launch_bounds__(kFmtBlock) void format_text_kernel(
 #pragma unroll
     for (int k = 0; k < STRIDE; ++k)
       nxt[k] = (r + 1 < kFmtRounds && in < O) ? octree[in * STRIDE + k] : 0;
+    const int lead = (int)((uintptr_t)(text + g0) & 15);
     if (r > 0) __syncthreads();   // the previous round's copy has read s_txt
     if (i < O) {
-      int at = (int)((ex >> (16 * r)) & 0xffffu);
+      int at = lead + (int)((ex >> (16 * r)) & 0xffffu);
 #pragma unroll
-      for (int k = 0; k < STRIDE; ++k) at = put_dec(s_txt, at, cur[k]);
+      for (int k = 0; k < STRIDE; ++k)
+        at = put_dec(s_txt, at, cur[k], (int)(lens[r] >> (4 * k)) & 15, s_pairs);
     }
     __syncthreads();
-    // the round's run: bytes up to the first 4-byte boundary, whole words, tail
-    uint8_t *dst = text + g0;
-    int head = (int)((4 - ((uintptr_t)dst & 3)) & 3);
-    if (head > (int)rtotal) head = (int)rtotal;
-    if (t < head) dst[t] = s_txt[t];
-    const int nw = ((int)rtotal - head) >> 2;
-    uint32_t *dw = reinterpret_cast<uint32_t *>(dst + head);
-    for (int w = t; w < nw; w += kFmtBlock) {
-      const int b = head + 4 * w;
-      dw[w] = (uint32_t)s_txt[b] | ((uint32_t)s_txt[b + 1] << 8) |
-              ((uint32_t)s_txt[b + 2] << 16) | ((uint32_t)s_txt[b + 3] << 24);
+    // s_txt[lead, end) is the run; line w is its bytes 16 w .. 16 w + 15
+    uint8_t *dst = text + g0 - lead;
+    const int end = lead + rtotal;
+    const int w0 = lead ? 1 : 0, w1 = end >> 4;
+    for (int w = w0 + t; w < w1; w += kFmtBlock)
+      reinterpret_cast<uint4 *>(dst)[w] = reinterpret_cast<const uint4 *>(s_txt)[w];
+    if (t < 16) {
+      if (lead && t >= lead && t < end) dst[t] = s_txt[t];
+      const int b = 16 * w1 + t;
+      if (w1 >= w0 && b < end) dst[b] = s_txt[b];
     }
-    const int tail0 = head + 4 * nw;
-    if (t < (int)rtotal - tail0) dst[tail0 + t] = s_txt[tail0 + t];
     g0 += rtotal;
 #pragma unroll
     for (int k = 0; k < STRIDE; ++k) cur[k] = nxt[k];
@@ -169,6 +183,47 @@ __global__ __launch_bounds__(kFmtBlock) void format_text_kernel(
 // ' ', '\t', '\n', '\v', '\f', '\r' (codes 32 and 9..13) as one mask test
 __device__ inline bool is_space(uint8_t c) {
   return c <= 32 && ((0x100003E00ull >> c) & 1ull);
+}
+
+// Bits 0..3: which of w's four bytes are spaces.
+__device__ inline uint32_t space_bits(uint32_t w) {
+  const uint32_t lo = w & 0x7f7f7f7fu;                       // no sum below carries
+  const uint32_t from9 = lo + 0x77777777u, from14 = lo + 0x72727272u;
+  const uint32_t not32 = (lo ^ 0x20202020u) + 0x7f7f7f7fu;
+  const uint32_t m = ((from9 & ~from14) | ~not32) & ~w & 0x80808080u;
+  return ((m >> 7) * 0x01020408u) >> 24;                     // bits 0, 8, 16, 24 -> 24..27
+}
+
+// Four decimal digits, the first in the lowest byte.
+__device__ inline uint32_t digits4(uint32_t d) {
+  return __builtin_amdgcn_udot4(d, 0x010Au, 0u, false) * 100u +
+         __builtin_amdgcn_udot4(d, 0x010A0000u, 0u, false);
+}
+
+// The common token at byte p of s, which has 12 bytes after p: an optional
+// minus, 1 to 8 digits and a space.  The digits are found and added up four
+// to a word; false where the token has another form (parse_staged decides).
+__device__ inline bool parse_short(const uint8_t *s, int p, int32_t *out) {
+  const uint32_t *q = reinterpret_cast<const uint32_t *>(s) + (p >> 2);
+  const uint32_t q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3], sh = (uint32_t)p & 3u;
+  uint32_t w0 = __builtin_amdgcn_alignbyte(q1, q0, sh), w1 = __builtin_amdgcn_alignbyte(q2, q1, sh),
+           w2 = __builtin_amdgcn_alignbyte(q3, q2, sh);
+  const uint32_t neg = (w0 & 0xffu) == '-' ? 1u : 0u;
+  w0 = __builtin_amdgcn_alignbyte(w1, w0, neg);
+  w1 = __builtin_amdgcn_alignbyte(w2, w1, neg);
+  w2 = __builtin_amdgcn_alignbyte(0u, w2, neg);
+  // bit 7 of each byte: no digit (right up to the first such byte)
+  const uint32_t x0 = w0 ^ 0x30303030u, x1 = w1 ^ 0x30303030u;
+  const uint32_t m0 = ((x0 + 0x76767676u) | x0) & 0x80808080u;
+  const uint32_t m1 = ((x1 + 0x76767676u) | x1) & 0x80808080u;
+  const uint32_t n = m0 ? (uint32_t)__builtin_ctz(m0) >> 3
+                        : (m1 ? 4u + ((uint32_t)__builtin_ctz(m1) >> 3) : 8u);
+  const uint32_t endw = n < 4 ? w0 : (n < 8 ? w1 : w2);
+  if (n == 0 || !is_space((uint8_t)(endw >> (8 * (n & 3u))))) return false;
+  const uint64_t d = ((uint64_t)x1 << 32 | x0) << (8 * (8 - n));   // right-aligned, zeros before
+  const uint32_t v = digits4((uint32_t)d) * 10000u + digits4((uint32_t)(d >> 32));
+  *out = neg ? -(int32_t)v : (int32_t)v;
+  return true;
 }
 
 // Token parse from the staged bytes: an optional sign and digits, at most
@@ -213,16 +268,21 @@ __device__ inline bool parse_staged(const uint8_t *s, int p, int staged, const u
 // word (a round holds at most kParseTile / 2 starts), then each round's
 // bytes and the 16 after it are staged in LDS (a token starting in the round
 // without leading zeros is decided within 12 bytes: sign, 10 digits, one
-// more byte; a longer one reads on from global memory), its tokens
-// parsed into LDS in token order and written out as one run of records.
+// more byte; a longer one reads on from global memory), the starts listed in
+// token order, and the tokens parsed one to a lane, each lane writing its
+// value where it belongs, next to its neighbours'.  What bounds it is the
+// VALU: tokens differ in number per 16 bytes and in length, so neither the
+// bytes' owners (which held a wave for its most crowded 16 bytes) nor a loop
+// over digits divides them evenly.  The text of an octree of 2^22 uniform 3D
+// points: 259 us by owners and digit by digit, 79 us so.
 template <int DIM>
 __global__ __launch_bounds__(kParseBlock) void parse_text_kernel(
     const uint8_t *__restrict__ text, int64_t len, int64_t N, int32_t *__restrict__ octree,
     uint64_t *__restrict__ ws, int ntiles) {
-  constexpr int STRIDE = (1 << DIM) + 1;
+  constexpr uint32_t STRIDE = (1 << DIM) + 1;
   constexpr int kHalo = 16;
   __shared__ __align__(16) uint8_t s_txt[kParseTile + kHalo];
-  __shared__ int32_t s_val[kParseTile / 2];
+  __shared__ uint16_t s_pos[kParseTile / 2];
   __shared__ uint64_t s_w[kParseBlock / 64];
   __shared__ int s_tile;
   const int t = threadIdx.x;
@@ -232,8 +292,6 @@ __global__ __launch_bounds__(kParseBlock) void parse_text_kernel(
   const int64_t tb = (int64_t)tile * kParseTile * kParseRounds;
   uint4 qs[kParseRounds];          // this thread's bytes of every round
   uint32_t smask[kParseRounds];    // and where tokens start in them
-  uint8_t halo[kParseRounds];      // threads below kHalo: byte t after each round
-  uint64_t packed = 0;
 #pragma unroll
   for (int r = 0; r < kParseRounds; ++r) {
     const int64_t p0 = tb + (int64_t)r * kParseTile + (int64_t)t * kParseBytes;
@@ -246,19 +304,20 @@ __global__ __launch_bounds__(kParseBlock) void parse_text_kernel(
         wv[k >> 2] |= (uint32_t)(p0 + k < len ? text[p0 + k] : (uint8_t)' ') << (8 * (k & 3));
       qs[r] = make_uint4(wv[0], wv[1], wv[2], wv[3]);
     }
-    bool prev_space = p0 == 0 || p0 > len || is_space(text[p0 - 1]);
-    const uint32_t qw[4] = {qs[r].x, qs[r].y, qs[r].z, qs[r].w};
-    uint32_t m = 0;
+  }
+  // threads below kHalo: byte t after the tile
+  const int64_t ph = tb + (int64_t)kParseRounds * kParseTile + t;
+  const uint8_t halo = (t < kHalo && ph < len) ? text[ph] : (uint8_t)' ';
+  uint64_t packed = 0;
 #pragma unroll
-    for (int k = 0; k < kParseBytes; ++k) {
-      const bool sp = is_space((uint8_t)(qw[k >> 2] >> (8 * (k & 3))));
-      if (!sp && prev_space) m |= 1u << k;
-      prev_space = sp;
-    }
-    smask[r] = m;
-    packed |= (uint64_t)__popc(m) << (16 * r);
-    const int64_t ph = tb + (int64_t)(r + 1) * kParseTile + t;
-    halo[r] = (t < kHalo && ph < len) ? text[ph] : (uint8_t)' ';
+  for (int r = 0; r < kParseRounds; ++r) {
+    const int64_t p0 = tb + (int64_t)r * kParseTile + (int64_t)t * kParseBytes;
+    const uint32_t sp = space_bits(qs[r].x) | space_bits(qs[r].y) << 4 |
+                        space_bits(qs[r].z) << 8 | space_bits(qs[r].w) << 12;
+    uint32_t prev = __shfl_up(sp >> 15, 1, 64);   // is the byte before this thread's a space?
+    if ((t & 63) == 0) prev = p0 == 0 || p0 > len || is_space(text[p0 - 1]);
+    smask[r] = ~sp & (sp << 1 | prev) & 0xffffu;
+    packed |= (uint64_t)__popc(smask[r]) << (16 * r);
   }
   uint64_t tot_packed;
   const uint64_t ex = block_excl_sum<uint64_t, kParseBlock / 64>(packed, s_w, &tot_packed);
@@ -272,33 +331,30 @@ __global__ __launch_bounds__(kParseBlock) void parse_text_kernel(
 #pragma unroll
   for (int r = 0; r < kParseRounds; ++r) {
     const uint32_t rtotal = (uint32_t)(tot_packed >> (16 * r)) & 0xffffu;
-    if (r > 0) __syncthreads();   // the previous round is done with s_txt and s_val
+    if (r > 0) __syncthreads();   // the previous round is done with s_txt and s_pos
     *reinterpret_cast<uint4 *>(s_txt + t * kParseBytes) = qs[r];
-    if (t < kHalo) s_txt[kParseTile + t] = halo[r];
-    __syncthreads();
-    uint32_t starts = smask[r];
-    uint32_t li = (uint32_t)(ex >> (16 * r)) & 0xffffu;
-    while (starts) {
-      const int j = __ffs(starts) - 1;
-      starts &= starts - 1;
-      const uint64_t k = base + li;
-      if (k >= 1 && k <= last) {
-        int32_t val = 0;
-        if (!parse_staged(s_txt, t * kParseBytes + j, kParseTile + kHalo, text,
-                          tb + (int64_t)r * kParseTile, len, &val))
-          atomicMin(reinterpret_cast<unsigned long long *>(ws + kWsBad), (unsigned long long)k + 1);
-        s_val[li] = val;
-      }
-      ++li;
+    if (r + 1 < kParseRounds) {
+      if (t == 0) *reinterpret_cast<uint4 *>(s_txt + kParseTile) = qs[r + 1 < kParseRounds ? r + 1 : r];
+    } else if (t < kHalo) {
+      s_txt[kParseTile + t] = halo;
     }
+    uint32_t li = (uint32_t)(ex >> (16 * r)) & 0xffffu;
+    for (uint32_t starts = smask[r]; starts; starts &= starts - 1)
+      s_pos[li++] = (uint16_t)(t * kParseBytes + __ffs(starts) - 1);
     __syncthreads();
+    // token base + i is value k - 1 of the records: its column by 32-bit steps
+    const uint32_t col0 = (uint32_t)((base + STRIDE - 1) % STRIDE);
     for (uint32_t i = t; i < rtotal; i += kParseBlock) {
       const uint64_t k = base + i;
-      if (k >= 1 && k <= last) {
-        const uint64_t rr = k - 1;
-        const int32_t v = s_val[i];
-        octree[rr] = (rr % STRIDE == STRIDE - 1) ? (int32_t)(uint8_t)v : v;
+      if (k < 1 || k > last) continue;
+      int32_t v = 0;
+      const int p = s_pos[i];
+      if (!parse_short(s_txt, p, &v) &&
+          !parse_staged(s_txt, p, kParseTile + kHalo, text, tb + (int64_t)r * kParseTile, len, &v)) {
+        v = 0;
+        atomicMin(reinterpret_cast<unsigned long long *>(ws + kWsBad), (unsigned long long)k + 1);
       }
+      octree[k - 1] = (col0 + i) % STRIDE == STRIDE - 1 ? (int32_t)(uint8_t)v : v;
     }
     base += rtotal;
   }

@@ -118,6 +118,45 @@ def test_parse_misaligned_text(dev):
         out.free()
 
 
+@pytest.mark.parametrize("O,dim", [(1, 2), (300, 3), (40000, 2)])
+def test_text_at_every_line_offset(dev, O, dim):
+    """The text written and read at each place in a 16-byte line, and tokens of
+    every length after each kind of space: the copy's first and last lines, and
+    the tokens that cross the lines, rounds and tiles of the parse."""
+    rec = _records(O, dim, seed=3 * O)
+    text = oracle.octree_format_text(rec, dim)
+    want = oracle.octree_parse_text(text, dim)
+    toks = text.split()
+    spaces = [b" ", b"\t", b"\n", b"\v", b"\f", b"\r", b"  ", b" \n\r "]
+    mixed = b"".join(tok + spaces[i % len(spaces)] for i, tok in enumerate(toks)).rstrip()
+    d, out = dev.upload(rec), dev.alloc(rec.nbytes)
+    buf = dev.alloc(max(len(text), len(mixed)) + 64)
+    total = C.c_int64()
+
+    def put(a):
+        dev._check(P.lib().pgvd_memcpy_htod(dev.ctx, buf.ptr, a.ctypes.data, a.nbytes, None))
+
+    try:
+        for lead in range(16) if O < 1000 else (1, 7, 15):
+            put(np.full(len(text) + 64, 7, np.uint8))
+            rc = P.lib().pgvd_octree_format_text(dev.ctx, d.ptr, O, dim, buf.ptr + lead, len(text),
+                                                 C.byref(total), None)
+            assert rc == 0 and total.value == len(text)
+            got = dev.download(buf, np.uint8, len(text) + 64)
+            assert got[lead:lead + len(text)].tobytes() == text
+            assert (got[:lead] == 7).all() and (got[lead + len(text):] == 7).all()
+            for body in (text, mixed):
+                put(np.frombuffer(b"9" * lead + body, np.uint8))
+                rc = P.lib().pgvd_octree_parse_text(dev.ctx, buf.ptr + lead, len(body), dim,
+                                                    out.ptr, O, C.byref(total), None)
+                assert rc == 0 and total.value == O
+                assert np.array_equal(dev.download(out, np.int32, rec.size).reshape(rec.shape), want)
+    finally:
+        d.free()
+        out.free()
+        buf.free()
+
+
 @pytest.mark.parametrize("bad", [b"2 1 -1 -1 -1 14 -1 -1 -1 -1", b"1 1 x -1 -1 14",
                                  b"1 2147483648 0 0 0 0", b"1 - 0 0 0 0", b"-1 ", b"   ",
                                  b"1 0 0 0 0 99999999999"])
