@@ -10,7 +10,8 @@
 // first of equal ones stays).  The reference folds the visits one by one;
 // here every visit is a record at its position g in walk order (polygon by
 // polygon, segment by segment, cell by cell) and the fold is three
-// order-independent reductions per (node, octant):
+// order-independent reductions per (node, octant), the first of them taken
+// where the visits are made:
 //   first  = min g of the visits that keep a part      -> label 0
 //   second = min g of those whose label differs         -> label 1
 //   best   = max (length^2 bits << 32 | ~g) per label   -> the kept part
@@ -18,8 +19,8 @@
 //
 // FitBoxes.  One lane per pair of segments runs the reference's loop with
 // the same float and double operations (no contraction, correctly rounded
-// division and square root): a counting pass, a scan of the counts, and a
-// writing pass.  The reference's loop has no bound; here a pair stops with
+// division and square root): a counting pass that keeps what it finds, a scan
+// of the counts, and a pass that moves it into place.  The reference's loop has no bound; here a pair stops with
 // an error after kFitMaxRounds rounds.
 #include "kernels.hpp"
 #include "tilescan.hpp"
@@ -209,12 +210,16 @@ __device__ void closest_segs(seg2 a, seg2 b, v2 &ca, v2 &cb, bool &ca_end, bool 
 constexpr int kFitMaxRounds = 4096;
 constexpr int kFitOffsetFactor = 4;
 
-// Where FitBoxes puts what it finds: counts always, values while WRITE.
+// Where FitBoxes puts what it finds.  The counting pass (WRITE false) counts,
+// and keeps the first kFitKept boxes with the one or two samples before each
+// as two float4: (sample, sample), (origin, length, 0).
 template <bool WRITE>
 struct FitSink {
   float *samples, *origins, *lengths;
   int32_t *extra;
+  float4 *keep;            // nullable
   int64_t ns = 0, nb = 0;  // running positions (start at the item's offsets)
+  v2 s0 = {0, 0}, s1 = {0, 0};
   __device__ void sample(v2 p) {
     if (WRITE) {
       samples[2 * ns] = p.x;
@@ -223,6 +228,9 @@ struct FitSink {
         extra[2 * ns] = (int32_t)p.x;      // convert_intn (truncation)
         extra[2 * ns + 1] = (int32_t)p.y;
       }
+    } else {
+      s0 = s1;
+      s1 = p;
     }
     ++ns;
   }
@@ -231,6 +239,9 @@ struct FitSink {
       origins[2 * nb] = o.x;
       origins[2 * nb + 1] = o.y;
       lengths[nb] = d;
+    } else if (keep && nb < kFitKept) {
+      keep[2 * nb] = make_float4(s0.x, s0.y, s1.x, s1.y);
+      keep[2 * nb + 1] = make_float4(o.x, o.y, d, 0);
     }
     ++nb;
   }
@@ -402,39 +413,83 @@ __device__ inline bool fit_item(const float *__restrict__ src, int64_t i, seg2 &
   return !multi_isect(A.a, A.b, B.a, B.b);
 }
 
+// Clears what the counting pass and its scans count in.
+__global__ __launch_bounds__(kBlock) void fit_init_kernel(uint64_t *__restrict__ ws, int64_t words,
+                                                          FitResult *__restrict__ res) {
+  const int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  for (int64_t i = i0; i < words; i += (int64_t)gridDim.x * kBlock) ws[i] = 0;
+  if (i0 == 0) {
+    res->samples = res->boxes = 0;
+    res->err = ~0ull;
+    res->kept = res->rest = 0;
+  }
+}
+
 // Counting pass: per item the number of samples and boxes; the first
-// failing item and its error go to *err as (item << 8 | code) (min).
+// failing item and its error go to res->err as (item << 8 | code) (min).  The
+// longest chain of rounds bounds it (up to 18 of about 2 us in a scene of
+// 2,500 loops, 4.7 on average), so it runs once: what it finds is kept (45 us
+// and 4 to move it; 40 and 40 where the writing pass worked it out again).
 template <bool FROM_CI>
 __global__ __launch_bounds__(kBlock) void fit_count_kernel(const float *__restrict__ src,
                                                            int64_t n, float min_d,
                                                            uint32_t *__restrict__ ns,
                                                            uint32_t *__restrict__ nb,
                                                            int32_t *__restrict__ status,
-                                                           unsigned long long *__restrict__ err) {
+                                                           FitKeep keep,
+                                                           FitResult *__restrict__ res) {
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * kBlock) {
     seg2 A, B;
-    FitSink<false> o{nullptr, nullptr, nullptr, nullptr};
+    FitSink<false> o{nullptr, nullptr, nullptr, nullptr, nullptr};
     int rc = 0;
-    if (fit_item<FROM_CI>(src, i, A, B)) rc = fit_boxes(A, B, min_d, o);
+    if (fit_item<FROM_CI>(src, i, A, B)) {
+      const uint32_t chunk = atomicAdd(&res->kept, 1u);
+      if (chunk < keep.chunks) o.keep = keep.rec + (int64_t)chunk * (2 * kFitKept);
+      rc = fit_boxes(A, B, min_d, o);
+      const bool kept = o.keep && o.nb <= kFitKept;
+      if (chunk < keep.chunks) keep.owner[chunk] = kept ? (uint32_t)i : ~0u;
+      if (!kept) keep.rest[atomicAdd(&res->rest, 1u)] = (uint32_t)i;
+    }
     ns[i] = (uint32_t)o.ns;
     nb[i] = (uint32_t)o.nb;
     if (status) status[i] = rc;
-    if (rc) atomicMin(err, ((unsigned long long)i << 8) | (unsigned long long)rc);
+    if (rc) atomicMin(&res->err, ((unsigned long long)i << 8) | (unsigned long long)rc);
   }
 }
 
-template <bool FROM_CI>
-__global__ __launch_bounds__(kBlock) void fit_write_kernel(
-    const float *__restrict__ src, int64_t n, float min_d, const int64_t *__restrict__ soff,
-    const int64_t *__restrict__ boff, const uint32_t *__restrict__ ns, float *__restrict__ samples,
+// One thread per kept record.  Every box comes after two samples, but the
+// first of an item whose segments meet after one (an odd number of samples).
+__global__ __launch_bounds__(kBlock) void fit_move_kernel(
+    FitKeep keep, uint32_t kept, const int64_t *__restrict__ soff, const int64_t *__restrict__ boff,
+    const uint32_t *__restrict__ ns, const uint32_t *__restrict__ nb, float *__restrict__ samples,
     float *__restrict__ origins, float *__restrict__ lengths, int32_t *__restrict__ extra) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kBlock) {
-    if (ns[i] == 0) continue;
+  const uint32_t id = blockIdx.x * kBlock + threadIdx.x;
+  const uint32_t chunk = id / kFitKept, k = id % kFitKept;
+  if (chunk >= kept) return;
+  const uint32_t i = keep.owner[chunk];
+  if (i == ~0u || k >= nb[i]) return;
+  const float4 p = keep.rec[2 * id], q = keep.rec[2 * id + 1];
+  const bool one = ns[i] & 1;
+  FitSink<true> o{samples, origins, lengths, extra, nullptr};
+  o.ns = soff[i] + 2 * k - (one && k > 0);
+  o.nb = boff[i] + k;
+  if (k > 0 || !one) o.sample(mk(p.x, p.y));
+  o.sample(mk(p.z, p.w));
+  o.box(mk(q.x, q.y), q.z);
+}
+
+// The items that were not kept, from the beginning.
+template <bool FROM_CI>
+__global__ __launch_bounds__(kBlock) void fit_rest_kernel(
+    const float *__restrict__ src, const uint32_t *__restrict__ rest, uint32_t n, float min_d,
+    const int64_t *__restrict__ soff, const int64_t *__restrict__ boff, float *__restrict__ samples,
+    float *__restrict__ origins, float *__restrict__ lengths, int32_t *__restrict__ extra) {
+  for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < n; k += gridDim.x * kBlock) {
+    const int64_t i = rest[k];
     seg2 A, B;
     if (!fit_item<FROM_CI>(src, i, A, B)) continue;
-    FitSink<true> o{samples, origins, lengths, extra};
+    FitSink<true> o{samples, origins, lengths, extra, nullptr};
     o.ns = soff[i];
     o.nb = boff[i];
     (void)fit_boxes(A, B, min_d, o);
@@ -487,70 +542,94 @@ __global__ __launch_bounds__(kBlock) void poly_segments_kernel(
   }
 }
 
+__device__ inline int64_t slot_of(const int32_t *c) { return (int64_t)c[3] * 4 + c[4]; }
+
+// The arrays' empty states, and the flag's.
+__global__ __launch_bounds__(kBlock) void mc_init_kernel(int64_t slots, uint32_t *__restrict__ first,
+                                                         uint32_t *__restrict__ second,
+                                                         ulonglong2 *__restrict__ best,
+                                                         uint32_t *__restrict__ walk_bad) {
+  const int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  for (int64_t i = i0; i < slots; i += (int64_t)gridDim.x * kBlock) {
+    first[i] = second[i] = 0xFFFFFFFFu;
+    best[i] = make_ulonglong2(0, 0);
+  }
+  if (i0 == 0 && walk_bad) *walk_bad = 0;
+}
+
 // MCCallback for every visited cell: the part kept (float4) and the label,
-// or -1 where nothing is kept.  One lane per segment, over its cells.
+// or -1 where nothing is kept, and first[slot] = min g of the visits that keep
+// a part.  One lane per visit (a lane per segment took as long as the longest
+// walk: 48 us for the walks of 20,000 segments and 5 for the first visits,
+// against 11 for both so): a workgroup finds its 256 visits' range of
+// segments, each lane its own in that.
 __global__ __launch_bounds__(kBlock) void mc_visit_kernel(
     const float *__restrict__ segs, const int32_t *__restrict__ labels, int64_t n,
-    const int64_t *__restrict__ offsets, const int32_t *__restrict__ cells,
-    float4 *__restrict__ parts, int32_t *__restrict__ vlabel) {
-  for (int64_t s = (int64_t)blockIdx.x * kBlock + threadIdx.x; s < n;
-       s += (int64_t)gridDim.x * kBlock) {
+    const int64_t *__restrict__ offsets, const int32_t *__restrict__ cells, int64_t total,
+    float4 *__restrict__ parts, int32_t *__restrict__ vlabel, uint32_t *__restrict__ first) {
+  __shared__ int64_t s_seg[2];
+  for (int64_t g0 = (int64_t)blockIdx.x * kBlock; g0 < total; g0 += (int64_t)gridDim.x * kBlock) {
+    // the segment of visit x: the last s with offsets[s] <= x
+    auto seg_of = [&](int64_t x, int64_t lo, int64_t hi) {
+      while (lo < hi) {
+        const int64_t mid = (lo + hi + 1) >> 1;
+        if (offsets[mid] <= x) lo = mid;
+        else hi = mid - 1;
+      }
+      return lo;
+    };
+    __syncthreads();   // the previous round is done with s_seg
+    if ((threadIdx.x & 63) == 0 && threadIdx.x < 128) {
+      const int64_t x = threadIdx.x ? g0 + kBlock - 1 : g0;
+      s_seg[threadIdx.x >> 6] = seg_of(x < total ? x : total - 1, 0, n - 1);
+    }
+    __syncthreads();
+    const int64_t g = g0 + threadIdx.x;
+    if (g >= total) continue;
+    const int64_t s = seg_of(g, s_seg[0], s_seg[1]);
     const float ax = segs[4 * s], ay = segs[4 * s + 1], bx = segs[4 * s + 2], by = segs[4 * s + 3];
     const int32_t ai0 = (int32_t)ax, ai1 = (int32_t)ay, bi0 = (int32_t)bx, bi1 = (int32_t)by;
     const int32_t lab = labels[s];
-    for (int64_t g = offsets[s]; g < offsets[s + 1]; ++g) {
-      const int32_t *c = cells + 5 * g;
-      const int32_t ox = c[0], oy = c[1], w = c[2];
-      float ts[4], px[4], py[4];
-      float vx, vy, len;
-      walk_dir(ax, ay, bx, by, vx, vy, len);
-      const uint32_t keep = walk_isects(ax, ay, vx, vy, len, ox, oy, w, ts, px, py);
-      const int nk = __popc(keep);
-      float4 part = make_float4(0, 0, 0, 0);
-      int32_t l = -1;
-      if (nk >= 1) {
-        const int f0 = __ffs(keep) - 1;
-        float x0 = 0, y0 = 0, x1 = 0, y1 = 0;
+    const int32_t *c = cells + 5 * g;
+    const int32_t ox = c[0], oy = c[1], w = c[2];
+    float ts[4], px[4], py[4];
+    float vx, vy, len;
+    walk_dir(ax, ay, bx, by, vx, vy, len);
+    const uint32_t keep = walk_isects(ax, ay, vx, vy, len, ox, oy, w, ts, px, py);
+    const int nk = __popc(keep);
+    float4 part = make_float4(0, 0, 0, 0);
+    int32_t l = -1;
+    if (nk >= 1) {
+      const int f0 = __ffs(keep) - 1;
+      float x0 = 0, y0 = 0, x1 = 0, y1 = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i == f0) { x0 = px[i]; y0 = py[i]; }
+      if (nk == 2) {
+        const int f1 = 31 - __clz(keep);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (i == f0) { x0 = px[i]; y0 = py[i]; }
-        if (nk == 2) {
-          const int f1 = 31 - __clz(keep);
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (i == f1) { x1 = px[i]; y1 = py[i]; }
-          part = make_float4(x0, y0, x1, y1);
+          if (i == f1) { x1 = px[i]; y1 = py[i]; }
+        part = make_float4(x0, y0, x1, y1);
+        l = lab;
+      } else if (nk == 1) {
+        // the endpoint whose truncated coordinates lie in the cell's
+        // half-open box (BoundingBox.h:97-103)
+        const bool ain = ai0 >= ox && ai0 < ox + w && ai1 >= oy && ai1 < oy + w;
+        const bool bin = bi0 >= ox && bi0 < ox + w && bi1 >= oy && bi1 < oy + w;
+        if (ain) {
+          part = make_float4(x0, y0, ax, ay);
           l = lab;
-        } else if (nk == 1) {
-          // the endpoint whose truncated coordinates lie in the cell's
-          // half-open box (BoundingBox.h:97-103)
-          const bool ain = ai0 >= ox && ai0 < ox + w && ai1 >= oy && ai1 < oy + w;
-          const bool bin = bi0 >= ox && bi0 < ox + w && bi1 >= oy && bi1 < oy + w;
-          if (ain) {
-            part = make_float4(x0, y0, ax, ay);
-            l = lab;
-          } else if (bin) {
-            part = make_float4(x0, y0, bx, by);
-            l = lab;
-          }
+        } else if (bin) {
+          part = make_float4(x0, y0, bx, by);
+          l = lab;
         }
       }
-      parts[g] = part;
-      vlabel[g] = l;
     }
+    parts[g] = part;
+    vlabel[g] = l;
+    if (l >= 0) atomicMin(first + slot_of(c), (uint32_t)g);
   }
-}
-
-__device__ inline int64_t slot_of(const int32_t *c) { return (int64_t)c[3] * 4 + c[4]; }
-
-// first[slot] = min g of the visits that keep a part.
-__global__ __launch_bounds__(kBlock) void mc_first_kernel(const int32_t *__restrict__ cells,
-                                                          const int32_t *__restrict__ vlabel,
-                                                          int64_t total,
-                                                          uint32_t *__restrict__ first) {
-  for (int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x; g < total;
-       g += (int64_t)gridDim.x * kBlock)
-    if (vlabel[g] >= 0) atomicMin(first + slot_of(cells + 5 * g), (uint32_t)g);
 }
 
 // second[slot] = min g of the kept visits whose label is not first's.
@@ -602,7 +681,17 @@ __global__ __launch_bounds__(kBlock) void mc_write_kernel(int64_t slots,
                                                           const uint32_t *__restrict__ first,
                                                           const uint32_t *__restrict__ second,
                                                           const unsigned long long *__restrict__ best,
-                                                          int32_t *__restrict__ ci) {
+                                                          int32_t *__restrict__ ci,
+                                                          const int32_t *__restrict__ walk_status,
+                                                          int64_t n,
+                                                          uint32_t *__restrict__ walk_bad) {
+  if (walk_bad) {
+    bool any = false;
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * kBlock)
+      any |= walk_status[i] != 0;
+    if (__any(any) && (threadIdx.x & 63) == 0) atomicOr(walk_bad, 1u);
+  }
   for (int64_t slot = (int64_t)blockIdx.x * kBlock + threadIdx.x; slot < slots;
        slot += (int64_t)gridDim.x * kBlock) {
     const int64_t node = slot >> 2;
@@ -623,18 +712,6 @@ __global__ __launch_bounds__(kBlock) void mc_write_kernel(int64_t slots,
       seg[2 * oc + j] = p;
     }
   }
-}
-
-__global__ void fill_u32_kernel(uint32_t *p, int64_t n, uint32_t v) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kBlock)
-    p[i] = v;
-}
-
-__global__ void fill_u64_kernel(unsigned long long *p, int64_t n, unsigned long long v) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kBlock)
-    p[i] = v;
 }
 
 inline unsigned grid_for(int64_t n, int64_t cap = 16384) {
@@ -660,42 +737,53 @@ void launch_poly_segments(const float *verts, int64_t nv, const int64_t *voff, c
 void launch_multi_cells(const float *segs, const int32_t *labels, int64_t n,
                         const int64_t *offsets, const int32_t *cells, int64_t total, int64_t O,
                         float4 *parts, int32_t *vlabel, uint32_t *first, uint32_t *second,
-                        unsigned long long *best, int32_t *ci, hipStream_t s) {
+                        unsigned long long *best, int32_t *ci, const int32_t *walk_status,
+                        uint32_t *walk_bad, hipStream_t s) {
   const int64_t slots = 4 * O;
-  fill_u32_kernel<<<grid_for(slots), kBlock, 0, s>>>(first, slots, 0xFFFFFFFFu);
-  fill_u32_kernel<<<grid_for(slots), kBlock, 0, s>>>(second, slots, 0xFFFFFFFFu);
-  fill_u64_kernel<<<grid_for(2 * slots), kBlock, 0, s>>>(best, 2 * slots, 0ull);
+  mc_init_kernel<<<grid_for(slots), kBlock, 0, s>>>(slots, first, second,
+                                                    reinterpret_cast<ulonglong2 *>(best), walk_bad);
   if (n > 0 && total > 0) {
-    mc_visit_kernel<<<grid_for(n), kBlock, 0, s>>>(segs, labels, n, offsets, cells, parts, vlabel);
-    mc_first_kernel<<<grid_for(total), kBlock, 0, s>>>(cells, vlabel, total, first);
+    mc_visit_kernel<<<grid_for(total), kBlock, 0, s>>>(segs, labels, n, offsets, cells, total,
+                                                       parts, vlabel, first);
     mc_second_kernel<<<grid_for(total), kBlock, 0, s>>>(cells, vlabel, total, first, second);
     mc_best_kernel<<<grid_for(total), kBlock, 0, s>>>(cells, vlabel, parts, total, first, second,
                                                        best);
   }
-  mc_write_kernel<<<grid_for(slots), kBlock, 0, s>>>(slots, vlabel, parts, first, second, best, ci);
+  mc_write_kernel<<<grid_for(slots), kBlock, 0, s>>>(slots, vlabel, parts, first, second, best, ci,
+                                                     walk_status, n, walk_bad);
 }
 
 void launch_fit_count(const float *src, bool from_ci, int64_t items, float min_d, uint32_t *ns,
-                      uint32_t *nb, int32_t *status, unsigned long long *err, hipStream_t s) {
-  fill_u64_kernel<<<1, kBlock, 0, s>>>(err, 1, ~0ull);
+                      uint32_t *nb, int64_t *so, int64_t *bo, uint64_t *ws, int32_t *status,
+                      const FitKeep &keep, FitResult *res, hipStream_t s) {
   if (items == 0) return;
+  const int64_t words = walk_scan_ws_words(items);
+  fit_init_kernel<<<grid_for(2 * words, 64), kBlock, 0, s>>>(ws, 2 * words, res);
   if (from_ci)
-    fit_count_kernel<true><<<grid_for(items), kBlock, 0, s>>>(src, items, min_d, ns, nb, status, err);
+    fit_count_kernel<true><<<grid_for(items), kBlock, 0, s>>>(src, items, min_d, ns, nb, status,
+                                                              keep, res);
   else
     fit_count_kernel<false><<<grid_for(items), kBlock, 0, s>>>(src, items, min_d, ns, nb, status,
-                                                                err);
+                                                               keep, res);
+  launch_offsets_scan(ScanJob{ns, so, ws, &res->samples}, ScanJob{nb, bo, ws + words, &res->boxes},
+                      2, items, s);
 }
 
-void launch_fit_write(const float *src, bool from_ci, int64_t items, float min_d,
-                      const int64_t *soff, const int64_t *boff, const uint32_t *ns, float *samples,
+void launch_fit_write(const float *src, bool from_ci, float min_d, const int64_t *soff,
+                      const int64_t *boff, const uint32_t *ns, const uint32_t *nb,
+                      const FitKeep &keep, uint32_t kept, uint32_t rest, float *samples,
                       float *origins, float *lengths, int32_t *extra, hipStream_t s) {
-  if (items == 0) return;
+  kept = std::min(kept, keep.chunks);
+  if (kept)
+    fit_move_kernel<<<(kept * kFitKept + kBlock - 1) / kBlock, kBlock, 0, s>>>(
+        keep, kept, soff, boff, ns, nb, samples, origins, lengths, extra);
+  if (!rest) return;
   if (from_ci)
-    fit_write_kernel<true><<<grid_for(items), kBlock, 0, s>>>(src, items, min_d, soff, boff, ns,
-                                                              samples, origins, lengths, extra);
+    fit_rest_kernel<true><<<grid_for(rest), kBlock, 0, s>>>(src, keep.rest, rest, min_d, soff, boff,
+                                                            samples, origins, lengths, extra);
   else
-    fit_write_kernel<false><<<grid_for(items), kBlock, 0, s>>>(src, items, min_d, soff, boff, ns,
-                                                               samples, origins, lengths, extra);
+    fit_rest_kernel<false><<<grid_for(rest), kBlock, 0, s>>>(src, keep.rest, rest, min_d, soff,
+                                                             boff, samples, origins, lengths, extra);
 }
 
 }  // namespace pgvd
@@ -711,22 +799,5 @@ __global__ void narrow_i64_kernel(const int64_t *__restrict__ in, int64_t n, int
 
 void launch_narrow_i64(const int64_t *in, int64_t n, int32_t *out, hipStream_t s) {
   if (n > 0) narrow_i64_kernel<<<grid_for(n), kBlock, 0, s>>>(in, n, out);
-}
-}  // namespace pgvd
-
-namespace pgvd {
-namespace {
-__global__ void any_nonzero_kernel(const int32_t *__restrict__ v, int64_t n, uint32_t *flag) {
-  bool any = false;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kBlock)
-    any |= v[i] != 0;
-  if (__any(any) && (threadIdx.x & 63) == 0) atomicOr(flag, 1u);
-}
-}  // namespace
-
-void launch_any_nonzero(const int32_t *v, int64_t n, uint32_t *flag, hipStream_t s) {
-  fill_u32_kernel<<<1, kBlock, 0, s>>>(flag, 1, 0u);
-  if (n > 0) any_nonzero_kernel<<<grid_for(n, 2048), kBlock, 0, s>>>(v, n, flag);
 }
 }  // namespace pgvd

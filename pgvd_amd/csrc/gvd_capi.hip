@@ -69,7 +69,7 @@ int walk_pooled(pgvd_ctx *ctx, const float *segs, int64_t n, int bits, const int
 
 int multi_cells_impl(pgvd_ctx *ctx, const float *segs, const int32_t *labels, int64_t n, int bits,
                      const int32_t *octree, int64_t O, int32_t *ci, int32_t *walk_status,
-                     hipStream_t st) {
+                     uint32_t *walk_bad, hipStream_t st) {
   int64_t *offsets = nullptr;
   int32_t *cells = nullptr;
   int64_t total = 0;
@@ -85,7 +85,7 @@ int multi_cells_impl(pgvd_ctx *ctx, const float *segs, const int32_t *labels, in
     launch_multi_cells(segs, labels, n, offsets, cells, total, O, static_cast<float4 *>(parts),
                        static_cast<int32_t *>(vlabel), static_cast<uint32_t *>(first),
                        static_cast<uint32_t *>(second), static_cast<unsigned long long *>(best),
-                       ci, st);
+                       ci, walk_status, walk_bad, st);
   }
   HIPCHK(hipGetLastError());
   return PGVD_OK;
@@ -93,41 +93,54 @@ int multi_cells_impl(pgvd_ctx *ctx, const float *segs, const int32_t *labels, in
 
 // FitBoxes over items (pairs or CellIntersections slots) in three steps:
 // fit_count enqueues the counting pass and the scans of the counts;
-// fit_totals reads the totals, the first error (~0, or item << 8 | code)
-// and, optionally, one more device word back and waits; fit_write enqueues
-// the writing pass into buffers that hold the totals.
+// fit_totals reads the result words back and waits; fit_write enqueues the
+// writing pass into buffers that hold the totals.
 struct FitWork {
   uint32_t *ns = nullptr, *nb = nullptr;
   int64_t *so = nullptr, *bo = nullptr;
-  unsigned long long *err = nullptr;
+  FitResult *res = nullptr;
+  FitKeep keep = {};
+  FitResult host = {};
   int64_t items = 0;
 };
+
+// At most 64 MB of records; more items than chunks are worked out twice.
+constexpr int64_t kFitChunks = 1 << 16;
+
+int fit_result(pgvd_ctx *ctx, FitWork *w) {
+  void *res = nullptr;
+  CHK(pool_get(ctx, "fit_res", sizeof(FitResult), &res));
+  w->res = static_cast<FitResult *>(res);
+  return PGVD_OK;
+}
 
 int fit_count(pgvd_ctx *ctx, const float *src, bool from_ci, int64_t items, float min_d,
               int64_t *sample_offsets, int64_t *box_offsets, int32_t *status, FitWork *w,
               hipStream_t st) {
-  void *ns = nullptr, *nb = nullptr, *soff = nullptr, *boff = nullptr, *ws = nullptr, *err = nullptr;
+  void *ns = nullptr, *nb = nullptr, *soff = nullptr, *boff = nullptr, *ws = nullptr;
+  void *rec = nullptr, *owner = nullptr, *rest = nullptr;
   const size_t m = static_cast<size_t>(std::max<int64_t>(items, 1));
+  const size_t chunks = static_cast<size_t>(std::min<int64_t>(m, kFitChunks));
+  CHK(fit_result(ctx, w));
   CHK(pool_get(ctx, "fit_ns", 4 * m, &ns));
   CHK(pool_get(ctx, "fit_nb", 4 * m, &nb));
   if (!sample_offsets) CHK(pool_get(ctx, "fit_soff", 8 * (m + 1), &soff));
   if (!box_offsets) CHK(pool_get(ctx, "fit_boff", 8 * (m + 1), &boff));
-  CHK(pool_get(ctx, "fit_ws", 8 * static_cast<size_t>(walk_scan_ws_words(items)), &ws));
-  CHK(pool_get(ctx, "fit_err", 8, &err));
+  CHK(pool_get(ctx, "fit_ws", 16 * static_cast<size_t>(walk_scan_ws_words(items)), &ws));
+  CHK(pool_get(ctx, "fit_rec", 32 * kFitKept * chunks, &rec));
+  CHK(pool_get(ctx, "fit_owner", 4 * chunks, &owner));
+  CHK(pool_get(ctx, "fit_rest", 4 * m, &rest));
   w->ns = static_cast<uint32_t *>(ns);
   w->nb = static_cast<uint32_t *>(nb);
   w->so = sample_offsets ? sample_offsets : static_cast<int64_t *>(soff);
   w->bo = box_offsets ? box_offsets : static_cast<int64_t *>(boff);
-  w->err = static_cast<unsigned long long *>(err);
+  w->keep = FitKeep{static_cast<float4 *>(rec), static_cast<uint32_t *>(owner),
+                    static_cast<uint32_t *>(rest), static_cast<uint32_t>(chunks)};
   w->items = items;
-  {
-    Stage t(ctx, "gvd_fit_count", st);
-    launch_fit_count(src, from_ci, items, min_d, w->ns, w->nb, status, w->err, st);
-  }
-  HIPCHK(hipGetLastError());
   if (items > 0) {
-    launch_offsets_scan(w->ns, items, w->so, static_cast<uint64_t *>(ws), st);
-    launch_offsets_scan(w->nb, items, w->bo, static_cast<uint64_t *>(ws), st);
+    Stage t(ctx, "gvd_fit_count", st);
+    launch_fit_count(src, from_ci, items, min_d, w->ns, w->nb, w->so, w->bo,
+                     static_cast<uint64_t *>(ws), status, w->keep, w->res, st);
   } else {
     const int64_t zero = 0;
     HIPCHK(hipMemcpyAsync(w->so, &zero, 8, hipMemcpyHostToDevice, st));
@@ -138,21 +151,16 @@ int fit_count(pgvd_ctx *ctx, const float *src, bool from_ci, int64_t items, floa
   return PGVD_OK;
 }
 
-int fit_totals(const FitWork &w, int64_t *samples_out, int64_t *boxes_out,
-               unsigned long long *first_err, const uint32_t *extra_word, uint32_t *extra_out,
+int fit_totals(FitWork *w, int64_t *samples_out, int64_t *boxes_out, unsigned long long *first_err,
                hipStream_t st) {
-  int64_t totals[2] = {0, 0};
-  unsigned long long e = ~0ull;
-  uint32_t x = 0;
-  HIPCHK(hipMemcpyAsync(&totals[0], w.so + w.items, 8, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(&totals[1], w.bo + w.items, 8, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(&e, w.err, 8, hipMemcpyDeviceToHost, st));
-  if (extra_word) HIPCHK(hipMemcpyAsync(&x, extra_word, 4, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  *samples_out = totals[0];
-  *boxes_out = totals[1];
-  *first_err = e;
-  if (extra_out) *extra_out = x;
+  w->host.err = ~0ull;
+  if (w->items > 0) {
+    HIPCHK(hipMemcpyAsync(&w->host, w->res, sizeof w->host, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+  }
+  *samples_out = static_cast<int64_t>(w->host.samples);
+  *boxes_out = static_cast<int64_t>(w->host.boxes);
+  *first_err = w->host.err;
   return PGVD_OK;
 }
 
@@ -160,8 +168,8 @@ int fit_write(pgvd_ctx *ctx, const FitWork &w, const float *src, bool from_ci, f
               int32_t *extra, float *samples, float *origins, float *lengths, hipStream_t st) {
   if (w.items == 0) return PGVD_OK;
   Stage t(ctx, "gvd_fit_write", st);
-  launch_fit_write(src, from_ci, w.items, min_d, w.so, w.bo, w.ns, samples, origins, lengths,
-                   extra, st);
+  launch_fit_write(src, from_ci, min_d, w.so, w.bo, w.ns, w.nb, w.keep, w.host.kept, w.host.rest,
+                   samples, origins, lengths, extra, st);
   HIPCHK(hipGetLastError());
   return PGVD_OK;
 }
@@ -174,7 +182,7 @@ int fit_impl(pgvd_ctx *ctx, const float *src, bool from_ci, int64_t items, float
              hipStream_t st) {
   FitWork w;
   CHK(fit_count(ctx, src, from_ci, items, min_d, sample_offsets, box_offsets, status, &w, st));
-  CHK(fit_totals(w, samples_out, boxes_out, first_err, nullptr, nullptr, st));
+  CHK(fit_totals(&w, samples_out, boxes_out, first_err, st));
   if (*samples_out > capacity || *boxes_out > capacity)
     return fail(PGVD_ERR_CAPACITY, "FitBoxes output exceeds the capacity (*samples_out, *boxes_out)");
   if (*samples_out > 0 || *boxes_out > 0)
@@ -262,7 +270,7 @@ int pgvd_multi_cells(pgvd_ctx *ctx, const float *segs, const int32_t *labels, in
     return fail(PGVD_ERR_INVALID, "octree_size must be in [1, 2^29)");
   CHK(use_device(ctx));
   return multi_cells_impl(ctx, segs, labels, n, bits, octree, octree_size,
-                          reinterpret_cast<int32_t *>(ci), walk_status, pick(ctx, s));
+                          reinterpret_cast<int32_t *>(ci), walk_status, nullptr, pick(ctx, s));
 }
 
 int pgvd_fit_boxes(pgvd_ctx *ctx, const float *pairs, int64_t n, float min_d, float *samples,
@@ -345,34 +353,23 @@ int pgvd_gvd_refine(pgvd_ctx *ctx, const float *verts, const int64_t *counts, in
   HIPCHK(hipGetLastError());
   if (nq == 1) HIPCHK(hipMemsetAsync(q, 0, 8, st));     // Karras.cpp:84-88: one point {0,0}
 
-  void *segs = nullptr, *labels = nullptr, *wstat = nullptr, *flag = nullptr;
+  void *segs = nullptr, *labels = nullptr, *wstat = nullptr;
   CHK(pool_get(ctx, "gvd_segs", 16 * static_cast<size_t>(std::max<int64_t>(nseg, 1)), &segs));
   CHK(pool_get(ctx, "gvd_labels", 4 * static_cast<size_t>(std::max<int64_t>(nseg, 1)), &labels));
   CHK(pool_get(ctx, "gvd_wstat", 4 * static_cast<size_t>(std::max<int64_t>(nseg, 1)), &wstat));
-  CHK(pool_get(ctx, "gvd_flag", 4, &flag));
   CHK(segments_impl(ctx, verts, counts, P, bb, bbw, bits, static_cast<float *>(segs),
                     static_cast<int32_t *>(labels), nv, st));
 
   int it = 0;
   int64_t n_extra = 0, n_boxes = 0, O = 0;
   const int32_t *octree = nullptr;
-  void *ci = nullptr, *extra = nullptr, *samples = nullptr, *origins = nullptr, *lengths = nullptr;
+  void *ci = nullptr, *samples = nullptr, *origins = nullptr, *lengths = nullptr;
+  int32_t *extra = nullptr;
   int64_t ecap = 0;
   for (;;) {
-    // Octree2.cpp:178-181: the extra points join the points
-    if (n_extra > 0) {
-      if (nq + n_extra > qcap) {
-        qcap = 2 * (nq + n_extra);
-        void *nqbuf = nullptr;
-        CHK(pool_get(ctx, qkey[1 - qcur], 8 * static_cast<size_t>(qcap), &nqbuf));
-        HIPCHK(hipMemcpyAsync(nqbuf, q, 8 * static_cast<size_t>(nq), hipMemcpyDeviceToDevice, st));
-        q = nqbuf;
-        qcur = 1 - qcur;
-      }
-      HIPCHK(hipMemcpyAsync(static_cast<int32_t *>(q) + 2 * nq, extra,
-                            8 * static_cast<size_t>(n_extra), hipMemcpyDeviceToDevice, st));
-      nq += n_extra;
-    }
+    // Octree2.cpp:178-181: the extra points join the points (they were written
+    // behind them)
+    nq += n_extra;
     n_extra = 0;
     n_boxes = 0;
     O = 0;
@@ -389,27 +386,34 @@ int pgvd_gvd_refine(pgvd_ctx *ctx, const float *verts, const int64_t *counts, in
       octree = r.octree;
       // :186, FindMultiCells
       CHK(pool_get(ctx, "gvd_ci", 160 * static_cast<size_t>(O), &ci));
+      FitWork w;
+      CHK(fit_result(ctx, &w));
       CHK(multi_cells_impl(ctx, static_cast<float *>(segs), static_cast<int32_t *>(labels), nseg,
                            bits, octree, O, static_cast<int32_t *>(ci),
-                           static_cast<int32_t *>(wstat), st));
-      launch_any_nonzero(static_cast<int32_t *>(wstat), nseg, static_cast<uint32_t *>(flag), st);
-      HIPCHK(hipGetLastError());
+                           static_cast<int32_t *>(wstat), &w.res->walk_bad, st));
       // the sampling: counts, then the points into buffers that hold them
-      FitWork w;
       CHK(fit_count(ctx, static_cast<float *>(ci), true, 4 * O, min_d, nullptr, nullptr, nullptr,
                     &w, st));
       unsigned long long e = ~0ull;
-      uint32_t walk_bad = 0;
-      CHK(fit_totals(w, &n_extra, &n_boxes, &e, static_cast<uint32_t *>(flag), &walk_bad, st));
-      if (walk_bad) return fail(PGVD_ERR_GEOMETRY, "a cell walk passed 10000 cells (Infinite loop)");
+      CHK(fit_totals(&w, &n_extra, &n_boxes, &e, st));
+      if (w.host.walk_bad)
+        return fail(PGVD_ERR_GEOMETRY, "a cell walk passed 10000 cells (Infinite loop)");
       CHK(fit_error(e, "node*4+octant"));
       ecap = std::max<int64_t>(std::max(n_extra, n_boxes), 1);
-      CHK(pool_get(ctx, "gvd_extra", 8 * static_cast<size_t>(ecap), &extra));
+      if (nq + ecap > qcap) {
+        qcap = 2 * (nq + ecap);
+        void *nqbuf = nullptr;
+        CHK(pool_get(ctx, qkey[1 - qcur], 8 * static_cast<size_t>(qcap), &nqbuf));
+        HIPCHK(hipMemcpyAsync(nqbuf, q, 8 * static_cast<size_t>(nq), hipMemcpyDeviceToDevice, st));
+        q = nqbuf;
+        qcur = 1 - qcur;
+      }
+      extra = static_cast<int32_t *>(q) + 2 * nq;
       CHK(pool_get(ctx, "gvd_samples", 8 * static_cast<size_t>(ecap), &samples));
       CHK(pool_get(ctx, "gvd_origins", 8 * static_cast<size_t>(ecap), &origins));
       CHK(pool_get(ctx, "gvd_lengths", 4 * static_cast<size_t>(ecap), &lengths));
       if (n_extra > 0 || n_boxes > 0)
-        CHK(fit_write(ctx, w, static_cast<float *>(ci), true, min_d, static_cast<int32_t *>(extra),
+        CHK(fit_write(ctx, w, static_cast<float *>(ci), true, min_d, extra,
                       static_cast<float *>(samples), static_cast<float *>(origins),
                       static_cast<float *>(lengths), st));
     }
@@ -427,7 +431,7 @@ int pgvd_gvd_refine(pgvd_ctx *ctx, const float *verts, const int64_t *counts, in
   out->qpoints = static_cast<const int32_t *>(q);
   out->octree = octree;
   out->ci = static_cast<const pgvd_cell_intersections *>(ci);
-  out->extra = static_cast<const int32_t *>(extra);
+  out->extra = extra;
   out->samples = static_cast<const float *>(samples);
   out->origins = static_cast<const float *>(origins);
   out->lengths = static_cast<const float *>(lengths);

@@ -208,9 +208,16 @@ void launch_cell_walk_write(const float *segs, int64_t n, int bits, const int32_
                             int64_t size, const int64_t *offsets, int32_t *cells,
                             const void *scratch, uint32_t *counts, int log2k, hipStream_t s);
 // offsets[0] = 0, offsets[i + 1] = counts[0] + ... + counts[i] (n + 1
-// entries); ws holds walk_scan_ws_words(n) words.
-void launch_offsets_scan(const uint32_t *counts, int64_t n, int64_t *offsets, uint64_t *ws,
-                         hipStream_t s);
+// entries), *total (nullable) the last of them; ws holds
+// walk_scan_ws_words(n) words, all zero.  One or two such scans (jobs) of n > 0
+// counts each in one launch.
+struct ScanJob {
+  const uint32_t *counts;
+  int64_t *offsets;
+  uint64_t *ws;
+  uint64_t *total;
+};
+void launch_offsets_scan(const ScanJob &a, const ScanJob &b, int jobs, int64_t n, hipStream_t s);
 
 // ---- gvd.hip ----
 // obj2Oct of every vertex and the segments of every polygon (vertices
@@ -221,23 +228,42 @@ void launch_poly_segments(const float *verts, int64_t nv, const int64_t *voff, c
                           int32_t *labels, uint32_t *bad, hipStream_t s);
 // MCCallback over a finished walk (offsets, cells; `total` cells) into the
 // CellIntersections records ci (40 words per node).  parts/vlabel: total
-// entries; first/second: 4*O; best: 8*O.
+// entries; first/second: 4*O; best: 8*O.  With walk_bad (nullable), it
+// receives whether some walk_status[i] (n) is not 0.
 void launch_multi_cells(const float *segs, const int32_t *labels, int64_t n,
                         const int64_t *offsets, const int32_t *cells, int64_t total, int64_t O,
                         float4 *parts, int32_t *vlabel, uint32_t *first, uint32_t *second,
-                        unsigned long long *best, int32_t *ci, hipStream_t s);
+                        unsigned long long *best, int32_t *ci, const int32_t *walk_status,
+                        uint32_t *walk_bad, hipStream_t s);
 // FitBoxes over items: pairs (8 floats each) or CellIntersections slots
-// (from_ci, items = 4*O).  Count pass: ns/nb per item, status (nullable),
-// *err = min(item << 8 | code) over failing items (~0 if none).
+// (from_ci, items = 4*O).  The count pass leaves ns/nb per item, their scans
+// in so/bo, status (nullable), and in res the totals, the first error
+// (item << 8 | code, ~0 if none), and how many items were kept and not: an
+// item's boxes and samples, up to kFitKept boxes, are kept in a chunk of
+// records while there are chunks; the others are listed in rest.  The write
+// pass moves the kept ones and works the others out again.
+constexpr int kFitKept = 32;
+struct FitResult {
+  uint64_t samples, boxes;
+  unsigned long long err;
+  uint32_t kept, rest;         // chunks asked for (maybe more than there are), items in rest
+  uint32_t walk_bad, pad;      // launch_multi_cells' flag, where it is given it
+};
+struct FitKeep {
+  float4 *rec;                 // chunks x kFitKept x 2
+  uint32_t *owner;             // chunks: the item, or ~0
+  uint32_t *rest;              // items
+  uint32_t chunks;
+};
 void launch_fit_count(const float *src, bool from_ci, int64_t items, float min_d, uint32_t *ns,
-                      uint32_t *nb, int32_t *status, unsigned long long *err, hipStream_t s);
-void launch_fit_write(const float *src, bool from_ci, int64_t items, float min_d,
-                      const int64_t *soff, const int64_t *boff, const uint32_t *ns, float *samples,
+                      uint32_t *nb, int64_t *so, int64_t *bo, uint64_t *ws, int32_t *status,
+                      const FitKeep &keep, FitResult *res, hipStream_t s);
+void launch_fit_write(const float *src, bool from_ci, float min_d, const int64_t *soff,
+                      const int64_t *boff, const uint32_t *ns, const uint32_t *nb,
+                      const FitKeep &keep, uint32_t kept, uint32_t rest, float *samples,
                       float *origins, float *lengths, int32_t *extra, hipStream_t s);
 // out[i] = (int32_t)in[i]
 void launch_narrow_i64(const int64_t *in, int64_t n, int32_t *out, hipStream_t s);
-// *flag = 1 if some v[i] != 0, else 0
-void launch_any_nonzero(const int32_t *v, int64_t n, uint32_t *flag, hipStream_t s);
 
 // ---- textio.hip ----
 // The octree's text form (operator<< / operator>>, C/OctNode.h:58-98).  ws

@@ -118,7 +118,13 @@ __global__ __launch_bounds__(kBlock) void cell_walk_kernel(
     const float *__restrict__ segs, int64_t n, int64_t per, int bits,
     const int32_t *__restrict__ octree, int64_t size, uint32_t *__restrict__ counts,
     int32_t *__restrict__ status, const int64_t *__restrict__ offsets,
-    int32_t *__restrict__ cells, int4 *__restrict__ scratch, int K) {
+    int32_t *__restrict__ cells, int4 *__restrict__ scratch, int K, uint64_t *__restrict__ zero,
+    int64_t words) {
+  // the scan that follows finds its workspace clear
+  if (MODE == kWalkCount || MODE == kWalkSpec)
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < words;
+         i += (int64_t)gridDim.x * kBlock)
+      zero[i] = 0;
   // each lane's last descent, node per depth (depth 0 is the root)
   __shared__ int32_t s_path[(kMaxBits + 1) * kBlock];
   int32_t *path = s_path + threadIdx.x;
@@ -231,40 +237,34 @@ __global__ __launch_bounds__(kBlock) void walk_compact_kernel(
   }
 }
 
-// offsets[0] = 0, offsets[i + 1] = counts[0] + ... + counts[i]; 1024 counts
-// per tile; ws: word 0 tile counter, status array from word 4.
-__global__ __launch_bounds__(kBlock) void walk_scan_kernel(const uint32_t *__restrict__ counts,
-                                                           int64_t n,
-                                                           int64_t *__restrict__ offsets,
-                                                           uint64_t *__restrict__ ws) {
+// offsets[0] = 0, offsets[i + 1] = counts[0] + ... + counts[i], of one array
+// of counts to each row of the grid; 1024 counts per tile; ws: word 0 tile
+// counter, status array from word 4.
+__global__ __launch_bounds__(kBlock) void walk_scan_kernel(ScanJob a, ScanJob b, int64_t n) {
   __shared__ uint32_t s_w[kBlock / 64];
   __shared__ int s_tile;
+  const ScanJob j = blockIdx.y ? b : a;
   const int t = threadIdx.x;
-  if (t == 0) s_tile = (int)atomicAdd(reinterpret_cast<unsigned int *>(ws), 1u);
+  if (t == 0) s_tile = (int)atomicAdd(reinterpret_cast<unsigned int *>(j.ws), 1u);
   __syncthreads();
   const int tile = s_tile;
   const int64_t i0 = ((int64_t)tile * kBlock + t) * 4;
   uint32_t c[4], sum = 0;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    c[k] = i0 + k < n ? counts[i0 + k] : 0u;
+    c[k] = i0 + k < n ? j.counts[i0 + k] : 0u;
     sum += c[k];
   }
   uint32_t total;
   const uint32_t ex = block_excl_sum<uint32_t>(sum, s_w, &total);
-  uint64_t run = tile_prefix<kBlock>(ws + 4, tile, total) + ex;
-  if (tile == 0 && t == 0) offsets[0] = 0;
+  uint64_t run = tile_prefix<kBlock>(j.ws + 4, tile, total) + ex;
+  if (tile == 0 && t == 0) j.offsets[0] = 0;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     run += c[k];
-    if (i0 + k < n) offsets[i0 + k + 1] = (int64_t)run;
+    if (i0 + k < n) j.offsets[i0 + k + 1] = (int64_t)run;
+    if (j.total && i0 + k == n - 1) *j.total = run;
   }
-}
-
-__global__ void walk_ws_zero_kernel(uint64_t *ws, int64_t words) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < words;
-       i += (int64_t)gridDim.x * kBlock)
-    ws[i] = 0;
 }
 
 }  // namespace
@@ -291,23 +291,23 @@ void launch_cell_walk_count(const float *segs, int64_t n, int bits, const int32_
                             uint64_t *ws, void *scratch, int log2k, hipStream_t s) {
   int64_t per;
   const unsigned grid = walk_grid(n, &per);
+  const int64_t words = walk_scan_ws_words(n);
   if (scratch)
     cell_walk_kernel<kWalkSpec><<<grid, kBlock, 0, s>>>(segs, n, per, bits, octree, size, counts,
                                                         status, nullptr, nullptr,
-                                                        static_cast<int4 *>(scratch), 1 << log2k);
+                                                        static_cast<int4 *>(scratch), 1 << log2k,
+                                                        ws, words);
   else
     cell_walk_kernel<kWalkCount><<<grid, kBlock, 0, s>>>(segs, n, per, bits, octree, size, counts,
-                                                         status, nullptr, nullptr, nullptr, 0);
-  launch_offsets_scan(counts, n, offsets, ws, s);
+                                                         status, nullptr, nullptr, nullptr, 0, ws,
+                                                         words);
+  const ScanJob j{counts, offsets, ws, nullptr};
+  launch_offsets_scan(j, j, 1, n, s);
 }
 
-void launch_offsets_scan(const uint32_t *counts, int64_t n, int64_t *offsets, uint64_t *ws,
-                         hipStream_t s) {
-  const int64_t words = walk_scan_ws_words(n);
-  walk_ws_zero_kernel<<<(unsigned)std::min<int64_t>((words + kBlock - 1) / kBlock, 1024), kBlock,
-                        0, s>>>(ws, words);
+void launch_offsets_scan(const ScanJob &a, const ScanJob &b, int jobs, int64_t n, hipStream_t s) {
   const int64_t tiles = (n + 4 * kBlock - 1) / (4 * kBlock);
-  if (tiles > 0) walk_scan_kernel<<<(unsigned)tiles, kBlock, 0, s>>>(counts, n, offsets, ws);
+  if (tiles > 0) walk_scan_kernel<<<dim3((unsigned)tiles, jobs), kBlock, 0, s>>>(a, b, n);
 }
 
 void launch_cell_walk_write(const float *segs, int64_t n, int bits, const int32_t *octree,
@@ -317,7 +317,8 @@ void launch_cell_walk_write(const float *segs, int64_t n, int bits, const int32_
   const unsigned grid = walk_grid(n, &per);
   if (!scratch) {
     cell_walk_kernel<kWalkWrite><<<grid, kBlock, 0, s>>>(segs, n, per, bits, octree, size, nullptr,
-                                                         nullptr, offsets, cells, nullptr, 0);
+                                                         nullptr, offsets, cells, nullptr, 0,
+                                                         nullptr, 0);
     return;
   }
   int64_t cgrid = ((n << log2k) + kBlock - 1) / kBlock;
@@ -326,7 +327,7 @@ void launch_cell_walk_write(const float *segs, int64_t n, int bits, const int32_
                                                          offsets, n, log2k, bits, cells);
   cell_walk_kernel<kWalkRest><<<grid, kBlock, 0, s>>>(segs, n, per, bits, octree, size, counts,
                                                       nullptr, offsets, cells, nullptr,
-                                                      1 << log2k);
+                                                      1 << log2k, nullptr, 0);
 }
 
 }  // namespace pgvd

@@ -55,6 +55,24 @@ def test_fit_boxes_pairs_match_oracle(dev, kind):
         assert _bits_equal(got["lengths"][bo[i]:bo[i + 1]], want["lengths"]), (i, p)
 
 
+@pytest.mark.parametrize("n", [1, 255, 66000])
+def test_fit_boxes_kept_and_rest(dev, n):
+    """Pairs of up to 32 boxes, whose records are kept, pairs of more, and more
+    pairs than there is room for (65,536): each as the oracle's."""
+    base = np.concatenate([_pairs(k, 60, seed=5).reshape(-1, 8) for k in KINDS])
+    want = [oracle.fit_boxes(p[:4], p[4:]) for p in base]
+    boxes = np.array([len(w["lengths"]) for w in want])
+    use = np.flatnonzero(boxes <= 200)
+    assert (boxes[use] > 32).any() or n == 1
+    assert any(len(want[u]["samples"]) % 2 for u in use)       # segments that meet
+    pick = use[np.random.default_rng(n).integers(0, use.size, n)]
+    got = dev.fit_boxes(base[pick])
+    assert np.array_equal(got["status"], [want[u]["status"] for u in pick])
+    assert np.array_equal(np.diff(got["box_offsets"]), boxes[pick])
+    for k in ("samples", "origins", "lengths"):
+        assert _bits_equal(got[k], np.concatenate([want[u][k] for u in pick])), k
+
+
 @pytest.mark.parametrize("bits", [8, 11, 12, 16, 24])
 def test_polyline_segments_match_oracle(dev, bits):
     """obj2Oct and the per-polygon segments, including the far side of the
