@@ -12,7 +12,7 @@ One step = the whole path (bounding box, FP32 quantize, 63-bit Morton keys,
 radix sort, unique, Karras BRT with local splits, octree fill) over 2^24
 float3 points that are already in HBM.  Prints one JSON line: sorted Morton
 keys/s (whole job), the per-launch roofline of the dominant kernel (the
-octree gather when the bucket sort ran, else an onesweep sort pass), the
+octree gather, or an onesweep sort pass where the LSD passes sorted), the
 whole-path roofline against the path's algorithmic byte model, and the
 serial CPU path (the oracle, one core) timed on a bounded sample.
 """
@@ -478,7 +478,7 @@ def bench_cellwalk(args) -> int:
     8; a uniform in the grid, b within 1/256 of the grid's width of a) walked
     through the quadtree of 2^22 uniform 2D points at 20 bits/axis; segments
     and quadtree already in HBM.  One step = one pgvd_cell_walk call with a
-    cell buffer (a walk keeping each segment's first 32 cells, the offset
+    cell buffer (a walk keeping each segment's first cells, the offset
     scan, the copy to the offsets, a re-walk of longer segments).  Algorithmic bytes:
     16 B in and 8 B of offset out per segment, 20 B out per visited cell."""
     import pgvd_amd as P
@@ -554,7 +554,7 @@ def bench_cellwalk(args) -> int:
         },
         "roofline": {
             "kernel": "cell_walk_kernel (one lane per segment: FindLeaf descents and edge "
-                      "intersections per visited cell, the first 32 cells kept) + offset scan + "
+                      "intersections per visited cell, the first cells kept) + offset scan + "
                       "walk_compact_kernel + re-walk of longer segments, timed together",
             "bound": "hbm",
             "achieved": gbps,
@@ -627,8 +627,8 @@ def bench_gvd(args) -> int:
         got = dev.gvd_refine(v, c, bits, iters)
     dev.close()
     walk = stages.get("gvd_walk", {"avg_ms": float("nan"), "launches_per_step": 0})
-    # the walk that keeps each segment's first 32 cells: 16 B in, 8 B of
-    # offset and (up to 32) 20 B cells out per segment; the visited cells are
+    # the walk that keeps each segment's first cells: 16 B in, 8 B of
+    # offset and a 16 B record per kept cell out per segment; the visited cells are
     # not counted here (they are known only per build)
     wbytes = nseg * 24
     gbps = wbytes / (walk["avg_ms"] * 1e-3) / 1e9
@@ -923,7 +923,9 @@ def measure_build(P, workload: str, n: int, steps: int, warmup: int, cpu: bool,
     for _ in range(max(warmup, 1)):
         dev.build_octree_async(dpts, n, dim, bits, dlab)
         res = dev.build_octree_finish()
-    bucket = bool(res.bucket_sort)
+    # (clustered keys: the sample sort takes up to 2^20 of them, the LSD passes more)
+    sampled = not res.bucket_sort and n <= 1 << 20
+    bucket = bool(res.bucket_sort) or sampled
 
     # Timed region.  HIP events cost ~10 us of queue time each, so the only
     # events inside it are one pair per step around the dominant kernel: the
@@ -1003,7 +1005,8 @@ def measure_build(P, workload: str, n: int, steps: int, warmup: int, cpu: bool,
                         "points-in-HBM to octree-in-HBM",
             "n_points": n, "dim": dim, "bits": bits, "distribution": workload,
             "unique_keys": m, "octree_nodes": O, "malformed_brt": int(res.malformed),
-            "sort": "bucket sort (2 scatters + in-LDS buckets)" if bucket else "LSD onesweep",
+            "sort": "sample sort" if sampled else
+                    "bucket sort (2 scatters + in-LDS buckets)" if bucket else "LSD onesweep",
             **({"labels": "uint32 loop id per point", "flags": flagged} if conflict else {}),
         },
         "roofline": {

@@ -331,8 +331,7 @@ __global__ __launch_bounds__(BS) void ss_sort_kernel(const K *kin, const uint32_
 
 // Buckets above CAP, one workgroup each: stable LSD passes through global
 // memory (the bucket's range of both buffers) over the bits that vary in it;
-// equal keys are copied.  Rare, and slow beside the LDS sort (~10 us per
-// 1024 keys).  Always reports duplicates: telling equal neighbours apart is
+// equal keys are copied.  Rare, and slow beside the LDS sort.  Always reports duplicates: telling equal neighbours apart is
 // left to unique.
 template <typename K, bool LAB>
 __global__ __launch_bounds__(kSsBlock) void ss_big_kernel(K *kmid, uint32_t *vmid, K *kA,
