@@ -919,17 +919,18 @@ def measure_build(P, workload: str, n: int, steps: int, warmup: int, cpu: bool,
     dpts = dev.upload(pts)
     dlab = dev.upload(labels) if conflict else None
 
+    # (the LSD passes record a span; the bucket and sample sorts do not)
+    dev.timing(True, sort_span_only=True)
+    dev.timing_reset()
     res = None
     for _ in range(max(warmup, 1)):
         dev.build_octree_async(dpts, n, dim, bits, dlab)
         res = dev.build_octree_finish()
-    # (clustered keys: the sample sort takes up to 2^20 of them, the LSD passes more)
-    sampled = not res.bucket_sort and n <= 1 << 20
-    bucket = bool(res.bucket_sort) or sampled
+    bucket = dev.timing_read("sort")[1] == 0
 
     # Timed region.  HIP events cost ~10 us of queue time each, so the only
     # events inside it are one pair per step around the dominant kernel: the
-    # octree gather when the bucket sort ran, else the radix-sort passes
+    # octree gather, or the radix-sort passes where they sorted
     # (launched back to back).
     passes = (dim * bits + 7) // 8
     dev.timing(True, sort_span_only=not bucket, gather_only=bucket)
@@ -1005,8 +1006,8 @@ def measure_build(P, workload: str, n: int, steps: int, warmup: int, cpu: bool,
                         "points-in-HBM to octree-in-HBM",
             "n_points": n, "dim": dim, "bits": bits, "distribution": workload,
             "unique_keys": m, "octree_nodes": O, "malformed_brt": int(res.malformed),
-            "sort": "sample sort" if sampled else
-                    "bucket sort (2 scatters + in-LDS buckets)" if bucket else "LSD onesweep",
+            "sort": ("bucket sort (2 scatters + in-LDS buckets)" if res.bucket_sort else
+                     "sample sort" if bucket else "LSD onesweep"),
             **({"labels": "uint32 loop id per point", "flags": flagged} if conflict else {}),
         },
         "roofline": {
