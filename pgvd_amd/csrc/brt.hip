@@ -250,8 +250,8 @@ __global__ __launch_bounds__(kBlock) void brt_ls_defer_kernel(const K *__restric
                                                               RunState *st) {
   const int m = (int)st->m;
   const uint32_t nwords = m > 1 ? (uint32_t)(m - 1 + 63) / 64u : 0u;
-  for_each_masked(miss_words, nwords, [&](uint32_t cu) {
-    const int c = (int)cu;
+  for_each_masked(miss_words, nwords, [&](uint32_t word, uint32_t bit) {
+    const int c = (int)(word * 64u + bit);
     const K cur = keys[c];
     const BrtOut<K> o = brt_eval_wide(cur, [&](int x) { return keys[x]; }, mbits, m, c);
     brt_flags(o, st);
@@ -298,11 +298,11 @@ __global__ __launch_bounds__(kBlock) void brt_seg_defer_kernel(
     BrtNodeT<K> *__restrict__ brt, int32_t *__restrict__ parent, uint32_t *__restrict__ lsx,
     uint32_t *__restrict__ chunk_tot, const uint64_t *__restrict__ miss_words, RunState *st) {
   constexpr uint32_t SEG = R * kBlock;
-  for_each_masked(miss_words, ntiles * (SEG / 64), [&](uint32_t q) {
-    const uint32_t tile = q / SEG;
-    const uint32_t s = tt.seg[tile];
+  for_each_masked(miss_words, ntiles * (SEG / 64), [&](uint32_t word, uint32_t bit) {
+    const TileSlot at = tile_slot(word, bit, SEG / 64);
+    const uint32_t s = tt.seg[at.tile];
     const uint32_t kofs = seg[s].kofs;
-    const int c = (int)((tile - tt.first[s]) * SEG + q % SEG);
+    const int c = (int)((at.tile - tt.first[s]) * SEG + at.slot);
     const int m = (int)ss[s].m;
     const K *kk = keys + kofs;
     const K cur = kk[c];

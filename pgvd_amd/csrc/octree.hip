@@ -771,7 +771,8 @@ __global__ __launch_bounds__(kBlock) void gather_defer_kernel(
     }
     return true;
   };
-  for_each_masked(miss_words, nwords, [&](uint32_t q) {
+  for_each_masked(miss_words, nwords, [&](uint32_t word, uint32_t bit) {
+    const uint32_t q = word * 64u + bit;
     const uint32_t excl = q ? ps[q - 1] : 0u;
     (void)gather_one_bfs<K, DIM, CONF>(q, load_links(brt + q), brt, excl, ps[q] - excl, fetch,
                                        keys, conflict_bits, mbits,
@@ -787,11 +788,12 @@ __global__ __launch_bounds__(kBlock) void gather_seg_defer_kernel(
     int64_t capacity, const uint64_t *__restrict__ miss_words, RunState *st) {
   constexpr int STRIDE = (1 << DIM) + 1;
   if ((int64_t)st->octree_size > capacity) return;
-  for_each_masked(miss_words, ntiles * (uint32_t)(kGatherTile / 64), [&](uint32_t w) {
-    const uint32_t tile = w / kGatherTile;
-    const uint32_t s = tt.seg[tile];
+  constexpr uint32_t W = kGatherTile / 64;
+  for_each_masked(miss_words, ntiles * W, [&](uint32_t word, uint32_t bit) {
+    const TileSlot at = tile_slot(word, bit, W);
+    const uint32_t s = tt.seg[at.tile];
     const uint32_t kofs = seg[s].kofs;
-    const uint32_t q = (tile - tt.first[s]) * kGatherTile + w % kGatherTile;
+    const uint32_t q = (at.tile - tt.first[s]) * kGatherTile + at.slot;
     const BrtNodeT<K> *b = brt + kofs;
     const uint32_t *p = ps + kofs;
     const uint32_t *lx = lsx + kofs;

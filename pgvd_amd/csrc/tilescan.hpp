@@ -102,11 +102,12 @@ __device__ inline T block_excl_sum(T x, T *s_w, T *total) {
   return before + incl - x;
 }
 
-// Calls f(index) for every bit set in words[0..nwords), index = word * 64 +
-// bit.  A workgroup takes 256 words at a time and spreads their set bits
-// over its threads (entry e goes to thread e % 256), so a word with many
-// bits does not hold one lane for all of them.  Uniform over the workgroup;
-// all 256 threads call it.
+// Calls f(word, bit) for every bit set in words[0..nwords).  A workgroup takes
+// 256 words at a time and spreads their set bits over its threads (entry e
+// goes to thread e % 256), so a word with many bits does not hold one lane for
+// all of them.  Uniform over the workgroup; all 256 threads call it.  (Word and
+// bit apart: a batch pads every instance to whole tiles, so its bits may
+// number more than 2^32.)
 template <typename F>
 __device__ inline void for_each_masked(const uint64_t *__restrict__ words, uint32_t nwords, F f) {
   __shared__ uint64_t s_word[kBlock];
@@ -131,11 +132,23 @@ __device__ inline void for_each_masked(const uint64_t *__restrict__ words, uint3
       }
       uint64_t x = s_word[lo];
       for (uint32_t k = e - s_ofs[lo]; k; --k) x &= x - 1;   // drop the lower set bits
-      f((base + lo) * 64u + (uint32_t)(__ffsll((unsigned long long)x) - 1));
+      f(base + lo, (uint32_t)(__ffsll((unsigned long long)x) - 1));
     }
     __syncthreads();   // s_word, s_ofs and s_w4 are refilled next round
   }
 }
+
+// The tile and the slot within it of one bit of the batched form's miss words,
+// `words` words to a tile.
+struct TileSlot {
+  uint32_t tile, slot;
+};
+__host__ __device__ constexpr TileSlot tile_slot(uint32_t word, uint32_t bit, uint32_t words) {
+  return {word / words, word % words * 64u + bit};
+}
+// (8.5 M tiles of 1024 slots: past 2^32 slots in all)
+static_assert(tile_slot(136000015u, 63u, 16u).tile == 8500000u &&
+              tile_slot(136000015u, 63u, 16u).slot == 1023u, "word and bit, not their index");
 
 // R consecutive elements starting at p (valid of them in range): 16-byte
 // vector loads when the run is whole and aligned, else element loads.

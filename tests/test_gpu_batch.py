@@ -246,3 +246,39 @@ def test_digest_matches_definition(dev):
     z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
     z = z ^ (z >> np.uint64(31))
     assert got == int(z.sum(dtype=np.uint64))
+
+
+@pytest.mark.gpu
+def test_batch_of_more_slots_than_32_bits(dev):
+    """An instance behind 2^23 one-point ones: every instance is padded to
+    whole tiles, so the overflow passes' slots number more than 2^32 (1024 a
+    BRT tile, 512 a gather tile), and the last instance's nodes that a window
+    does not resolve have to be found in its own tiles all the same."""
+    bits, tiny, n = 8, (1 << 23) + 1000, 30000
+    rng = np.random.default_rng(3)
+    last = rng.integers(0, 1 << bits, (n, 2)).astype(np.int32)
+    pts = np.concatenate([rng.integers(1, 1 << bits, (tiny, 2)).astype(np.int32), last])
+    sizes = np.ones(tiny + 1, np.int64)
+    sizes[-1] = n
+    d = dev.upload(pts)
+    try:
+        with pgvd_amd.Batch(dev, sizes, 2, bits, quantized=True, use_graph=False,
+                            sort_waves=3) as b:
+            b.run(d)
+            r = b.finish()
+            c = pgvd_amd.Batch.counts(r)
+            assert (c["m"][:-1] == 2).all()
+            k0, m = int(c["key_offset"][-1]), int(c["m"][-1])
+            o0, O = int(c["octree_offset"][-1]), int(c["octree_size"][-1])
+            item = pgvd_amd.BRT_DTYPES[4].itemsize
+            one = dict(m=[m], octree_size=[O], key_offset=[0], octree_offset=[0],
+                       words=dev.download(r.keys + 4 * k0, np.uint32, m),
+                       brt=dev.download(r.brt + item * k0, np.uint8,
+                                        m * item).view(pgvd_amd.BRT_DTYPES[4]),
+                       parent=dev.download(r.parent + 4 * k0, np.int32, m),
+                       ps=dev.download(r.prefix_sums + 4 * k0, np.uint32, m),
+                       octree=dev.download(r.octree + 20 * o0, np.int32, 5 * O).reshape(-1, 5))
+            assert_tree_equal(pgvd_amd.Batch.instance(one, 0, 4, 2), dev.build_octree(last, bits),
+                              BATCH_FIELDS)
+    finally:
+        d.free()
