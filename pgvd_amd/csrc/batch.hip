@@ -28,6 +28,7 @@ struct pgvd_batch {
   int digit_bits = 8, sort_waves = 3;
   bool sample_ok = false;           // every instance fits the sample sort
   bool use_sample = false;          // it sorts (else the radix passes)
+  std::vector<uint32_t> h_bucket_first, h_multi;   // its buckets; its segments of two or more
   SsPlan ss_plan;
   char *ss_ws = nullptr;
   std::vector<SegInfo> h_seg;
@@ -104,16 +105,32 @@ int ss_tile_for(int kb) {
   return kb == 4 ? ss_tile<uint32_t>() : (kb == 8 ? ss_tile<uint64_t>() : ss_tile<Key128>());
 }
 
-// The sample sort's workspace (its size does not depend on the settings).
-int ss_alloc(pgvd_batch *b, int64_t buckets) {
-  const size_t bytes = b->kb == 4   ? ss_ws_bytes<uint32_t>(buckets, b->B, b->total_slots)
-                       : b->kb == 8 ? ss_ws_bytes<uint64_t>(buckets, b->B, b->total_slots)
-                                    : ss_ws_bytes<Key128>(buckets, b->B, b->total_slots);
-  CHK(dalloc(&b->ss_ws, bytes));
-  if (b->kb == 4) ss_carve<uint32_t>(b->ss_ws, buckets, b->B, b->total_slots, b->ss_plan);
-  else if (b->kb == 8) ss_carve<uint64_t>(b->ss_ws, buckets, b->B, b->total_slots, b->ss_plan);
-  else ss_carve<Key128>(b->ss_ws, buckets, b->B, b->total_slots, b->ss_plan);
+// The sample sort's workspace, which only a plan that sorts with it (or is
+// tuned) holds; its size does not depend on the settings.  A plan that cannot
+// have it takes the radix passes.
+template <typename K>
+int ss_alloc(pgvd_batch *b) {
+  const int64_t buckets = b->h_bucket_first.back(), multi = (int64_t)b->h_multi.size();
+  CHK(dalloc(&b->ss_ws, ss_ws_bytes<K>(buckets, multi, b->total_slots)));
+  ss_carve<K>(b->ss_ws, buckets, multi, b->total_slots, b->ss_plan);
+  std::vector<BkItem> items(buckets, BkItem{0, 0, 0, 0});
+  for (size_t i = 0; i < b->h_seg.size(); ++i)
+    if (b->h_bucket_first[i + 1] - b->h_bucket_first[i] == 1)
+      items[b->h_bucket_first[i]] = ss_single_item(b->h_seg[i], (uint32_t)i);
+  HIPCHK(hipMemcpy(b->ss_plan.items, items.data(), items.size() * sizeof(BkItem),
+                   hipMemcpyHostToDevice));
   return PGVD_OK;
+}
+int ss_prepare(pgvd_batch *b) {
+  if (!b->sample_ok || b->ss_ws) return PGVD_OK;
+  const int rc = b->kb == 4   ? ss_alloc<uint32_t>(b)
+                 : b->kb == 8 ? ss_alloc<uint64_t>(b)
+                              : ss_alloc<Key128>(b);
+  if (rc == PGVD_ERR_ALLOC) {
+    b->sample_ok = b->use_sample = false;
+    return PGVD_OK;
+  }
+  return rc;
 }
 
 void release_graph(pgvd_batch *b) {
@@ -145,20 +162,25 @@ int build_tables(pgvd_batch *b) {
   }
   // the sample sort's tiles and buckets
   HostTable sst;
-  std::vector<uint32_t> bucket_first(si.size() + 1, 0);
-  if (b->sample_ok) {
-    sst = make_table(si, ss_tile_for(b->kb), [](const SegInfo &x) { return (int64_t)x.n; });
-    for (size_t i = 0; i < si.size(); ++i) {
-      const uint32_t nb = (uint32_t)ss_buckets_for(b->kb, si[i].n);
-      bucket_first[i + 1] = bucket_first[i] + nb;
-      b->ss_plan.max_nb = std::max(b->ss_plan.max_nb, nb);
-    }
+  const std::vector<uint32_t> &bf = b->h_bucket_first;
+  std::vector<uint32_t> multi_of;
+  if (b->ss_ws) {
+    const SegInfo *s0 = si.data();
+    sst = make_table(si, ss_tile_for(b->kb), [&](const SegInfo &x) {
+      return bf[&x - s0 + 1] - bf[&x - s0] > 1 ? (int64_t)x.n : 0;
+    });
+    multi_of.resize(si.size(), 0);
+    for (size_t j = 0; j < b->h_multi.size(); ++j) multi_of[b->h_multi[j]] = (uint32_t)j;
   }
   const size_t off_sst = all.size();
   all.insert(all.end(), sst.seg.begin(), sst.seg.end());
   all.insert(all.end(), sst.first.begin(), sst.first.end());
   const size_t off_bf = all.size();
-  all.insert(all.end(), bucket_first.begin(), bucket_first.end());
+  if (b->ss_ws) all.insert(all.end(), bf.begin(), bf.end());
+  const size_t off_multi = all.size();
+  if (b->ss_ws) all.insert(all.end(), b->h_multi.begin(), b->h_multi.end());
+  const size_t off_multi_of = all.size();
+  all.insert(all.end(), multi_of.begin(), multi_of.end());
   const size_t off_row = all.size();
   all.insert(all.end(), row.first.begin(), row.first.end());
   dfree(b->tables);
@@ -179,14 +201,15 @@ int build_tables(pgvd_batch *b) {
   d.digit_bits = b->digit_bits;
   d.sort_waves = b->sort_waves;
   b->passes = (b->mbits + b->digit_bits - 1) / b->digit_bits;
-  if (b->sample_ok) {
+  if (b->ss_ws) {
     b->ss_plan.seg = b->seg;
     b->ss_plan.ss = b->ss;
     b->ss_plan.tiles.seg = b->tables + off_sst;
     b->ss_plan.tiles.first = b->tables + off_sst + sst.seg.size();
     b->ss_plan.bucket_first = b->tables + off_bf;
+    b->ss_plan.multi = b->tables + off_multi;
+    b->ss_plan.multi_of = b->tables + off_multi_of;
     b->ss_plan.n_tiles = (int64_t)sst.seg.size();
-    if (!b->ss_ws) CHK(ss_alloc(b, bucket_first.back()));
   }
   // zero-initialised workspace: unique look-back and, for the radix passes,
   // digit histograms and their look-back (all passes)
@@ -421,10 +444,20 @@ int pgvd_batch_create(pgvd_ctx *ctx, const int64_t *sizes, int64_t count, int di
     return bail(fail(PGVD_ERR_ALLOC, "hipHostMalloc failed"));
   if (hipMemcpy(b->seg, b->h_seg.data(), count * sizeof(SegInfo), hipMemcpyHostToDevice) != hipSuccess)
     return bail(fail(PGVD_ERR_HIP, "batch table upload failed"));
-  // the sample sort unless an instance is too large for it or the caller
-  // chose how the radix passes run
+  // the sample sort unless an instance is too large for it, they are too many,
+  // or the caller chose how the radix passes run
   b->sample_ok = true;
-  for (int64_t i = 0; i < count; ++i) b->sample_ok &= ss_buckets_for(b->kb, sizes[i]) > 0;
+  int64_t buckets = 0;
+  b->h_bucket_first.assign(count + 1, 0);
+  for (int64_t i = 0; i < count; ++i) {
+    const int nb = ss_buckets_for(b->kb, sizes[i]);
+    b->sample_ok &= nb > 0;
+    buckets += nb;
+    b->h_bucket_first[i + 1] = (uint32_t)buckets;
+    b->ss_plan.max_nb = std::max(b->ss_plan.max_nb, (uint32_t)nb);
+    if (nb > 1) b->h_multi.push_back((uint32_t)i);
+  }
+  b->sample_ok &= buckets <= kSsMaxPlanBuckets;
   b->use_sample = b->sample_ok && !(opts && (opts->sort_ipt || opts->digit_bits || opts->sort_waves));
   const size_t kbytes = (size_t)slots * b->kb;
   if ((rc = dalloc(&b->keys_a, kbytes))) return bail(rc);
@@ -440,6 +473,7 @@ int pgvd_batch_create(pgvd_ctx *ctx, const int64_t *sizes, int64_t count, int di
   b->dev.seg = b->seg;
   b->dev.ss = b->ss;
   b->dev.B = count;
+  if (b->use_sample && (rc = ss_prepare(b))) return bail(rc);
   if ((rc = build_tables(b))) return bail(rc);
   if ((rc = ensure_octree(b, std::max<int64_t>(slots, 1024)))) return bail(rc);
   if (hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess)
@@ -514,6 +548,7 @@ int pgvd_batch_tune(pgvd_batch *b, const void *pts, int *sort_ipt, int *brt_rows
                     int *digit_bits, int *sort_waves) {
   if (!b || !pts) return fail(PGVD_ERR_INVALID, "null argument");
   CHK(use_device(b->ctx));
+  CHK(ss_prepare(b));
   const bool graph = b->use_graph;
   b->use_graph = false;
   // the fastest of three runs (after one that warms up) of the current setting
@@ -575,9 +610,13 @@ int pgvd_batch_tune(pgvd_batch *b, const void *pts, int *sort_ipt, int *brt_rows
     if ((rc = time_it(&t))) break;
     if (t < best) { best = t; bw = waves[k]; }
   }
+  // (where the device has no room for the radix passes beside it, too)
+  if (rc == PGVD_ERR_ALLOC && sbest < 1e30f) rc = PGVD_OK;
   if (b->sample_ok && sbest <= best) {
     b->use_sample = true;
     br = sr;
+  } else {
+    dfree(b->ss_ws);
   }
   b->use_graph = graph;
   b->sort_ipt = bi;

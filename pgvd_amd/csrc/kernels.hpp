@@ -313,14 +313,20 @@ struct BkItem {
 constexpr int kSsMaxBuckets = 512;    // per segment
 constexpr int kSsLutWords = 2049;     // a segment's splitter table
 // A plan: the segments (tables as a batch's, or seg null and one segment of n
-// keys in nb buckets) and the workspace ss_carve lays out.
+// keys in nb buckets) and the workspace ss_carve lays out.  n_segs counts the
+// segments of two buckets or more: only those have tiles, a splitter table and
+// workgroups of the steps before the LDS sort.  A segment of one bucket is an
+// LDS sort's item that the plan's owner writes once (ss_single_item).
 struct SsPlan {
   const SegInfo *seg = nullptr;
   SegState *ss = nullptr;                  // with seg: where duplicates are reported
   TileTable tiles{};                       // of ss_tile<K>() keys
   const uint32_t *bucket_first = nullptr;  // B + 1 entries
-  // for segments the device listed (ss_segments_from_buckets): the tiles and
-  // buckets in use, at most n_tiles and n_buckets; null: all of them
+  // the n_segs segments, and each one's place among them; null: segment i is
+  // the i-th
+  const uint32_t *multi = nullptr, *multi_of = nullptr;
+  // for segments that the device listed (launch_sample_sort_buckets): the
+  // tiles and buckets in use, at most n_tiles and n_buckets; null: all of them
   const uint32_t *limits = nullptr;
   uint32_t n = 0, nb = 0;
   uint32_t max_nb = 0;                     // buckets of the largest segment
@@ -330,6 +336,10 @@ struct SsPlan {
   BkItem *items = nullptr, *big = nullptr;
   uint16_t *ids = nullptr;                 // every key's bucket
 };
+inline BkItem ss_single_item(const SegInfo &x, uint32_t s) { return {x.kofs, x.n, 0u, s}; }
+// Most buckets of a plan (the LDS sort's grid is a workgroup of up to 512
+// threads for each, and a grid holds fewer than 2^32 threads).
+constexpr int64_t kSsMaxPlanBuckets = int64_t(1) << 22;
 // Buckets of a segment of n keys; 0: too many keys for this sort.
 template <typename K> int ss_buckets(int64_t n);
 template <typename K> int64_t ss_max_keys();   // the most that gives buckets

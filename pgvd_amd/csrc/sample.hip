@@ -83,9 +83,8 @@ __global__ __launch_bounds__(kSsBlock) void ss_splitters_kernel(const K *__restr
   __shared__ K s_keys[kSsBlock * IPT];
   __shared__ __align__(16) uint32_t s_tmp[bin_words<K, kSsBlock>()];
   __shared__ K s_sp[kSsMaxBuckets];
-  const uint32_t s = blockIdx.x;
+  const uint32_t s = p.multi ? p.multi[blockIdx.x] : blockIdx.x;
   const SsSeg sg = ss_segment(p, s);
-  if (sg.nb < 2) return;
   const int t = threadIdx.x;
   const uint32_t S = sg.nb * 16;   // <= kSsBlock * IPT, and S <= n (a bucket averages above 16)
   // stratum i: keys [i n / S, (i + 1) n / S) in 16-bit fixed point; the key
@@ -115,7 +114,7 @@ __global__ __launch_bounds__(kSsBlock) void ss_splitters_kernel(const K *__restr
   }
   __syncthreads();
   const int shift = mbits > kSsLutBits ? mbits - kSsLutBits : 0;
-  uint16_t *lut = reinterpret_cast<uint16_t *>(p.lut + (size_t)s * kSsLutWords);
+  uint16_t *lut = reinterpret_cast<uint16_t *>(p.lut + (size_t)blockIdx.x * kSsLutWords);
   for (uint32_t x = t; x < (uint32_t)kSsLut; x += kSsBlock) {
     // splitters j in [1, nb) whose window is below x
     uint32_t lo = 0, hi = sg.nb - 1;
@@ -140,7 +139,6 @@ __global__ __launch_bounds__(kBlock) void ss_count_kernel(const K *__restrict__ 
   if (p.limits && tile >= p.limits[0]) return;
   const uint32_t s = p.seg ? p.tiles.seg[tile] : 0u;
   const SsSeg sg = ss_segment(p, s);
-  if (sg.nb < 2) return;
   const int t = threadIdx.x;
   const uint32_t lo0 = (tile - (p.seg ? p.tiles.first[s] : 0u)) * (uint32_t)TILE;
   const uint32_t hi0 = min(lo0 + (uint32_t)TILE, sg.n);
@@ -155,7 +153,7 @@ __global__ __launch_bounds__(kBlock) void ss_count_kernel(const K *__restrict__ 
     s_cnt[j] = 0;
     s_sp[j] = sp[j];
   }
-  const uint32_t *lut = p.lut + (size_t)s * kSsLutWords;
+  const uint32_t *lut = p.lut + (size_t)(p.multi_of ? p.multi_of[s] : s) * kSsLutWords;
   for (uint32_t j = t; j < (uint32_t)kSsLutWords; j += kBlock) s_lut[j] = lut[j];
   __syncthreads();
   const uint16_t *s_l = reinterpret_cast<const uint16_t *>(s_lut);
@@ -180,20 +178,20 @@ __global__ __launch_bounds__(kBlock) void ss_count_kernel(const K *__restrict__ 
 }
 
 // One workgroup per segment: bucket starts from the counts, as the scatter's
-// cursors and the LDS sort's items (a single bucket is sorted from where it
-// is); buckets above CAP are listed for ss_big_kernel.
+// cursors and the LDS sort's items; buckets above CAP are listed for
+// ss_big_kernel.
 __global__ __launch_bounds__(kSsMaxBuckets) void ss_plan_kernel(SsPlan p, uint32_t cap,
                                                                 RunState *st) {
   __shared__ uint32_t s_w[kSsMaxBuckets / 64];
-  const uint32_t s = blockIdx.x;
+  const uint32_t s = p.multi ? p.multi[blockIdx.x] : blockIdx.x;
   const SsSeg sg = ss_segment(p, s);
   const uint32_t b = threadIdx.x;
-  const uint32_t c = sg.nb < 2 ? (b == 0 ? sg.n : 0u) : (b < sg.nb ? p.counts[sg.bucket + b] : 0u);
+  const uint32_t c = b < sg.nb ? p.counts[sg.bucket + b] : 0u;
   uint32_t total;
   const uint32_t at = sg.kofs + block_excl_sum<uint32_t, kSsMaxBuckets / 64>(c, s_w, &total);
-  if (b < max(sg.nb, 1u)) {
+  if (b < sg.nb) {
     p.cursors[sg.bucket + b] = at;
-    BkItem it{at, c, sg.nb < 2 ? 0u : 1u, s};   // (sbits: the segment)
+    BkItem it{at, c, 1u, s};   // (sbits: the segment)
     if (c > cap) {
       p.big[atomicAdd(p.n_big, 1u)] = it;
       it.count = 0;
@@ -226,7 +224,6 @@ __global__ __launch_bounds__(kBlock) void ss_scatter_kernel(const K *__restrict_
   if (p.limits && tile >= p.limits[0]) return;
   const uint32_t s = p.seg ? p.tiles.seg[tile] : 0u;
   const SsSeg sg = ss_segment(p, s);
-  if (sg.nb < 2) return;
   const uint32_t t = threadIdx.x;
   const uint32_t lo = (tile - (p.seg ? p.tiles.first[s] : 0u)) * (uint32_t)TILE;
   const uint32_t hi = min(lo + (uint32_t)TILE, sg.n);
@@ -590,19 +587,21 @@ void launch_sample_sort(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, 
   uint32_t *vmid = kin == kA ? vB : vA;
   const unsigned segs = (unsigned)p.n_segs, tiles = (unsigned)p.n_tiles;
   const unsigned zgrid = (unsigned)std::min<int64_t>((p.n_buckets + kBlock - 1) / kBlock, 1024);
-  ss_zero_kernel<<<zgrid, kBlock, 0, s>>>(p.counts, (uint32_t)p.n_buckets, p.n_big);
-  if (p.max_nb <= kSsMaxBuckets / 4)
-    ss_splitters_kernel<K, kSsIpt / 4><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
-  else if (p.max_nb <= kSsMaxBuckets / 2)
-    ss_splitters_kernel<K, kSsIpt / 2><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
-  else
-    ss_splitters_kernel<K, kSsIpt><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
-  ss_count_kernel<K><<<tiles, kBlock, 0, s>>>(kin, p, mbits);
-  ss_plan_kernel<<<segs, kSsMaxBuckets, 0, s>>>(p, (uint32_t)SsItem<K>::CAP, st);
-  if (vin)
-    ss_scatter_kernel<K, true><<<tiles, kBlock, 0, s>>>(kin, vin, kmid, vmid, p);
-  else
-    ss_scatter_kernel<K, false><<<tiles, kBlock, 0, s>>>(kin, nullptr, kmid, nullptr, p);
+  if (segs) {
+    ss_zero_kernel<<<zgrid, kBlock, 0, s>>>(p.counts, (uint32_t)p.n_buckets, p.n_big);
+    if (p.max_nb <= kSsMaxBuckets / 4)
+      ss_splitters_kernel<K, kSsIpt / 4><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
+    else if (p.max_nb <= kSsMaxBuckets / 2)
+      ss_splitters_kernel<K, kSsIpt / 2><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
+    else
+      ss_splitters_kernel<K, kSsIpt><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
+    ss_count_kernel<K><<<tiles, kBlock, 0, s>>>(kin, p, mbits);
+    ss_plan_kernel<<<segs, kSsMaxBuckets, 0, s>>>(p, (uint32_t)SsItem<K>::CAP, st);
+    if (vin)
+      ss_scatter_kernel<K, true><<<tiles, kBlock, 0, s>>>(kin, vin, kmid, vmid, p);
+    else
+      ss_scatter_kernel<K, false><<<tiles, kBlock, 0, s>>>(kin, nullptr, kmid, nullptr, p);
+  }
   // Few buckets leave the chip to one workgroup per CU or less: then twice
   // the threads on each (300,000 keys: 170 against 181 us a build); with many,
   // two workgroups of half of them on each CU (55 M keys: 3.03 against 3.35 ms
@@ -612,6 +611,7 @@ void launch_sample_sort(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, 
     ss_sort<K, CAP, 1024>(kin, vin, kmid, vmid, kA, vA, p, prepend, st, s);
   else
     ss_sort<K, CAP, 512>(kin, vin, kmid, vmid, kA, vA, p, prepend, st, s);
+  if (!segs) return;
   if (vin)
     ss_big_kernel<K, true><<<64, kSsBlock, 0, s>>>(kmid, vmid, kA, vA, kB, vB, p, st);
   else

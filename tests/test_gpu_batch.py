@@ -4,6 +4,8 @@ reference digests pin (test_gpu_parity.py); a sample of instances is also
 checked against the oracle directly."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -249,11 +251,13 @@ def test_digest_matches_definition(dev):
 
 
 @pytest.mark.gpu
-def test_batch_of_more_slots_than_32_bits(dev):
+@pytest.mark.parametrize("kw", [{}, {"sort_waves": 3}])
+def test_batch_of_more_slots_than_32_bits(dev, kw):
     """An instance behind 2^23 one-point ones: every instance is padded to
     whole tiles, so the overflow passes' slots number more than 2^32 (1024 a
     BRT tile, 512 a gather tile), and the last instance's nodes that a window
-    does not resolve have to be found in its own tiles all the same."""
+    does not resolve have to be found in its own tiles all the same.  (By
+    default too: a grid of the sample sort's would hold 2^32 threads.)"""
     bits, tiny, n = 8, (1 << 23) + 1000, 30000
     rng = np.random.default_rng(3)
     last = rng.integers(0, 1 << bits, (n, 2)).astype(np.int32)
@@ -262,8 +266,7 @@ def test_batch_of_more_slots_than_32_bits(dev):
     sizes[-1] = n
     d = dev.upload(pts)
     try:
-        with pgvd_amd.Batch(dev, sizes, 2, bits, quantized=True, use_graph=False,
-                            sort_waves=3) as b:
+        with pgvd_amd.Batch(dev, sizes, 2, bits, quantized=True, use_graph=False, **kw) as b:
             b.run(d)
             r = b.finish()
             c = pgvd_amd.Batch.counts(r)
@@ -280,5 +283,36 @@ def test_batch_of_more_slots_than_32_bits(dev):
                        octree=dev.download(r.octree + 20 * o0, np.int32, 5 * O).reshape(-1, 5))
             assert_tree_equal(pgvd_amd.Batch.instance(one, 0, 4, 2), dev.build_octree(last, bits),
                               BATCH_FIELDS)
+    finally:
+        d.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("large", [(), (6000, 40000)])
+def test_batch_of_tiny_instances_stays_small(dev, large):
+    """A million instances of ten points hold some 1.7 GB of keys, trees and
+    tables; none of them has a splitter table (8 KB each) of the sample sort.
+    Larger instances among them sort by it."""
+    hip = C.CDLL("libamdhip64.so")
+    free0, free1, total = C.c_size_t(), C.c_size_t(), C.c_size_t()
+    sizes = np.full(1_000_000, 10, np.int64)
+    for j, n in enumerate(large):
+        sizes[300_000 * (j + 1)] = n
+    pts = np.random.default_rng(2).random((int(sizes.sum()), 3), dtype=np.float32) * 2 - 1
+    d = dev.upload(pts)
+    try:
+        assert hip.hipMemGetInfo(C.byref(free0), C.byref(total)) == 0
+        with pgvd_amd.Batch(dev, sizes, 3, 21) as b:
+            assert hip.hipMemGetInfo(C.byref(free1), C.byref(total)) == 0
+            assert free0.value - free1.value < 3 << 30
+            for _ in range(2):
+                b.run(d)
+                r = b.finish()
+            all_ = b.fetch_all(r)
+        first = np.concatenate([[0], np.cumsum(sizes)])
+        for i in [0, 299_999, 300_000, 300_001, 600_000, 999_999]:
+            assert_tree_equal(pgvd_amd.Batch.instance(all_, i, 8, 3),
+                              dev.build_octree(pts[first[i]:first[i + 1]], 21), BATCH_FIELDS,
+                              where=f"instance {i}")
     finally:
         d.free()
