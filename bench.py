@@ -173,8 +173,11 @@ def bench_batch(args) -> int:
     offs = np.concatenate([[0], np.cumsum(sizes)])
     b = P.Batch(dev, sizes, dim, bits)
     ipt, rows, dbits, waves = b.tune(dpts)
-    print(f"batch: tuned sort_ipt={ipt} brt_rows={rows} digit_bits={dbits} sort_waves={waves}",
-          file=sys.stderr, flush=True)
+    sample = b.sample_sort()
+    tuned = {"sort": "sample sort", "brt_rows": rows} if sample else {
+        "sort": "LSD onesweep", "sort_ipt": ipt, "brt_rows": rows, "digit_bits": dbits,
+        "sort_waves": waves}
+    print(f"batch: tuned {tuned}", file=sys.stderr, flush=True)
     for _ in range(args.warmup):
         b.run(dpts)
         b.finish()
@@ -251,8 +254,7 @@ def bench_batch(args) -> int:
                         f"clusters; {bits} bits/axis, 63-bit keys; one segmented pipeline "
                         f"replayed as a HIP graph",
             "instances": int(sizes.size), "total_points": total,
-            "tuned": {"sort_ipt": ipt, "brt_rows": rows, "digit_bits": dbits,
-                      "sort_waves": waves},
+            "tuned": tuned,
         },
         "roofline": _batch_roofline(sizes, counts, dim, float(np.median(gpu_ms))),
         "batched_gpu_ms": float(np.median(gpu_ms)),

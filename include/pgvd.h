@@ -577,6 +577,10 @@ typedef struct pgvd_batch_opts {
                            128-bit keys); 0: 8                                */
   int sort_waves;       /* waves per SIMD the sort kernel is compiled for: 2, 3
                            or 4; 0: 3                                         */
+  /* With sort_ipt, digit_bits and sort_waves 0, a sample sort orders the keys
+   * where every instance is small enough for it (1,677,312, 1,048,576 or
+   * 628,736 points by key width) and the device has room for its workspace;
+   * otherwise, and where one of the three is given, the radix passes do. */
 } pgvd_batch_opts;
 
 typedef struct pgvd_batch_result {
@@ -609,13 +613,19 @@ int pgvd_batch_run(pgvd_batch *b, const void *pts);
 /* Waits for the last run, grows the octree buffer and refills it if it was
  * too small, and fills *out. */
 int pgvd_batch_finish(pgvd_batch *b, pgvd_batch_result *out);
-/* Picks the plan's sort tile (sort_ipt), BRT window (brt_rows), radix digit
- * width (digit_bits) and the sort kernel's waves per SIMD (sort_waves) by
- * timing runs on pts: every (sort_ipt, brt_rows) pair, then each digit
- * width, then each wave count, keeping the fastest at each step.  Every
- * setting gives bit-identical results.  Any output may be NULL. */
+/* Picks the plan's sort, and the radix passes' sort tile (sort_ipt), digit
+ * width (digit_bits) and waves per SIMD (sort_waves), with the BRT window
+ * (brt_rows), by timing runs on pts: the sample sort with each window, every
+ * (sort_ipt, brt_rows) pair, then each digit width, then each wave count,
+ * keeping the fastest at each step.  Every setting gives bit-identical
+ * results.  Any output may be NULL.  sort_ipt, digit_bits and sort_waves are
+ * what the radix passes ran fastest with, whichever sort is kept: a later plan
+ * like the tuned one is given them only where pgvd_batch_sort says that the
+ * radix passes were kept, and brt_rows alone otherwise. */
 int pgvd_batch_tune(pgvd_batch *b, const void *pts, int *sort_ipt, int *brt_rows,
                     int *digit_bits, int *sort_waves);
+/* Which sort the plan's runs take: 1 the sample sort, 0 the radix passes. */
+int pgvd_batch_sort(const pgvd_batch *b, int *sample_sort);
 /* Milliseconds of the last pgvd_batch_run, from events around it. */
 int pgvd_batch_last_ms(pgvd_batch *b, float *ms);
 

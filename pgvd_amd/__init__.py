@@ -176,6 +176,7 @@ def lib():
             "pgvd_batch_tune": ([vp, vp, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32),
                                  C.POINTER(i32)], i32),
             "pgvd_batch_last_ms": ([vp, C.POINTER(C.c_float)], i32),
+            "pgvd_batch_sort": ([vp, C.POINTER(i32)], i32),
             "pgvd_server_create": ([i32, i32, C.c_size_t, C.POINTER(vp)], i32),
             "pgvd_server_destroy": ([vp], i32),
             "pgvd_server_run": ([vp, C.POINTER(Request), i64, C.POINTER(ServerStats)], i32),
@@ -931,8 +932,16 @@ class Batch:
         self.dev._check(lib().pgvd_batch_last_ms(self.h, C.byref(ms)))
         return ms.value
 
+    def sample_sort(self) -> bool:
+        """The plan's runs take the sample sort (else the radix passes)."""
+        v = C.c_int()
+        self.dev._check(lib().pgvd_batch_sort(self.h, C.byref(v)))
+        return bool(v.value)
+
     def tune(self, pts) -> tuple[int, int, int, int]:
-        """(sort_ipt, brt_rows, digit_bits, sort_waves) the tuner kept."""
+        """(sort_ipt, brt_rows, digit_bits, sort_waves) the tuner kept; all but
+        brt_rows are for the radix passes (given to a later plan, they choose
+        them: see sample_sort)."""
         p = pts.ptr if isinstance(pts, DeviceBuffer) else int(pts)
         a, b, d, w = C.c_int(), C.c_int(), C.c_int(), C.c_int()
         self.dev._check(lib().pgvd_batch_tune(self.h, p, C.byref(a), C.byref(b), C.byref(d),

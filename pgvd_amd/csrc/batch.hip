@@ -536,6 +536,12 @@ int pgvd_batch_finish(pgvd_batch *b, pgvd_batch_result *out) {
   return PGVD_OK;
 }
 
+int pgvd_batch_sort(const pgvd_batch *b, int *sample_sort) {
+  if (!b || !sample_sort) return fail(PGVD_ERR_INVALID, "null argument");
+  *sample_sort = b->use_sample ? 1 : 0;
+  return PGVD_OK;
+}
+
 int pgvd_batch_last_ms(pgvd_batch *b, float *ms) {
   if (!b || !ms) return fail(PGVD_ERR_INVALID, "null argument");
   if (!b->ran) return fail(PGVD_ERR_INVALID, "no run yet");

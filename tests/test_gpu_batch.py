@@ -163,6 +163,29 @@ def test_batch_tuner_keeps_results(dev):
 
 
 @pytest.mark.gpu
+def test_batch_tells_its_sort(dev):
+    """The sample sort by default, the radix passes where an option chooses
+    how they run or an instance is too large; a plan made like a tuned one, as
+    the header says, takes the tuned one's sort."""
+    d = dev.upload(make_batch([3000, 70000, 12], 3, seed=1)[0])
+    sizes = [3000]
+    try:
+        for s, kw, want in [([3000, 70000], {}, True), ([3000, (1 << 20) + 1], {}, False),
+                            ([3000], {"brt_rows": 2}, True), ([3000], {"sort_waves": 2}, False),
+                            ([3000], {"sort_ipt": 8}, False), ([3000], {"digit_bits": 7}, False)]:
+            with pgvd_amd.Batch(dev, s, 3, 21, **kw) as b:
+                assert b.sample_sort() == want, (s, kw)
+        with pgvd_amd.Batch(dev, sizes, 3, 21) as b:
+            ipt, rows, dbits, waves = b.tune(d)
+            kept = b.sample_sort()
+        kw = {} if kept else dict(sort_ipt=ipt, digit_bits=dbits, sort_waves=waves)
+        with pgvd_amd.Batch(dev, sizes, 3, 21, brt_rows=rows, **kw) as b:
+            assert b.sample_sort() == kept
+    finally:
+        d.free()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("ipt,rows", [(8, 2), (12, 4), (15, 4), (16, 2)])
 def test_batch_every_config(dev, ipt, rows):
     dim, bits = 3, 21
