@@ -292,7 +292,8 @@ __device__ inline void lds_split_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t 
 // less the smallest); where some bin holds more than kBinRank of them, every
 // bin is cut into as many bins as it holds keys (rounded down to a power of
 // two) and the keys are counted again; then each key is ranked within its bin.
-// Keys too close together even for that (and repeated ones) go to
+// A bin of more than kBinRank2 keys that are all the same (many points at one
+// place) needs no ranking; keys too close together even for that go to
 // lds_split_sort, whose splitters cost four times the counting.  s_tmp:
 // bin_words<K, BS>() words, aligned as K.
 constexpr int kBins = 4096;
@@ -412,10 +413,6 @@ __device__ inline void lds_bin_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cn
     most = max(most, c2[i]);
   }
   most = block_max<BS>(most, s_mx);
-  if (most > kBinRank2) {
-    lds_split_sort<K, LAB, BS, IPT>(k, v, cnt, pick, s_keys, s_vals, s_tmp);
-    return;
-  }
   uint32_t ex = block_excl_sum<uint32_t, NW>(run, s_w, &total);
 #pragma unroll
   for (int i = 0; i < IPT; ++i) {
@@ -435,6 +432,20 @@ __device__ inline void lds_bin_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cn
   for (int j = 0; j < IPT; ++j)
     if ((uint32_t)j * BS + t < cnt) s_keys[at[j]] = k[j];
   __syncthreads();
+  if (most > kBinRank2) {   // uniform
+    // a crowded bin of one key's copies is in order as it is
+    uint32_t mixed = 0;
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+      if ((uint32_t)j * BS + t < cnt && b1[j] - b0[j] > kBinRank2) {
+        mixed |= keq(k[j], s_keys[b0[j]]) ? 0u : 1u;
+        b0[j] = b1[j] = at[j];
+      }
+    if (block_max<BS>(mixed, s_mx)) {
+      lds_split_sort<K, LAB, BS, IPT>(k, v, cnt, pick, s_keys, s_vals, s_tmp);
+      return;
+    }
+  }
   lds_rank<K, LAB, BS, IPT>(k, v, cnt, at, b0, b1, s_keys, s_vals);
 }
 

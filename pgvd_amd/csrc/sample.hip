@@ -177,10 +177,25 @@ __global__ __launch_bounds__(kBlock) void ss_count_kernel(const K *__restrict__ 
     if (s_cnt[j]) atomicAdd(&p.counts[sg.bucket + j], s_cnt[j]);
 }
 
+constexpr unsigned kSsBigGrid = 256;
+// How ss_big_kernel treats an item: as keys to sort, or as a run of one key.
+constexpr uint32_t kSsBigSort = 1, kSsBigRun = 2;
+
+// Bucket b holds copies of its splitter alone: the next splitter is its
+// successor (ss_splitters_kernel closes a repeated key's bucket so), or it is
+// the largest key there is.
+template <typename K>
+__device__ inline bool ss_one_key(const K *sp, uint32_t b, uint32_t nb, int mbits) {
+  const K x = sp[b];
+  if (b + 1 < nb) return keq(sp[b + 1], ksucc(x));
+  return keq(x, kshr(kones<K>(), (int)sizeof(K) * 8 - mbits));
+}
+
 // One workgroup per segment: bucket starts from the counts, as the scatter's
 // cursors and the LDS sort's items; buckets above CAP are listed for
-// ss_big_kernel.
-__global__ __launch_bounds__(kSsMaxBuckets) void ss_plan_kernel(SsPlan p, uint32_t cap,
+// ss_big_kernel, one key's copies in runs of up to CAP.
+template <typename K>
+__global__ __launch_bounds__(kSsMaxBuckets) void ss_plan_kernel(SsPlan p, uint32_t cap, int mbits,
                                                                 RunState *st) {
   __shared__ uint32_t s_w[kSsMaxBuckets / 64];
   const uint32_t s = p.multi ? p.multi[blockIdx.x] : blockIdx.x;
@@ -193,7 +208,14 @@ __global__ __launch_bounds__(kSsMaxBuckets) void ss_plan_kernel(SsPlan p, uint32
     p.cursors[sg.bucket + b] = at;
     BkItem it{at, c, 1u, s};   // (sbits: the segment)
     if (c > cap) {
-      p.big[atomicAdd(p.n_big, 1u)] = it;
+      if (ss_one_key(static_cast<const K *>(p.splitters) + sg.bucket, b, sg.nb, mbits)) {
+        constexpr uint32_t RUN = (uint32_t)SsItem<K>::CAP;
+        const uint32_t runs = (c + RUN - 1) / RUN, first = atomicAdd(p.n_big, runs);
+        for (uint32_t r = 0; r < runs; ++r)
+          p.big[first + r] = {at + r * RUN, min(RUN, c - r * RUN), kSsBigRun, s};
+      } else {
+        p.big[atomicAdd(p.n_big, 1u)] = {at, c, kSsBigSort, s};
+      }
       it.count = 0;
     }
     p.items[sg.bucket + b] = it;
@@ -326,10 +348,15 @@ __global__ __launch_bounds__(BS) void ss_sort_kernel(const K *kin, const uint32_
   if (__any(dup) && (t & 63) == 0) raise_flag(o.dups);
 }
 
-// Buckets above CAP, one workgroup each: stable LSD passes through global
-// memory (the bucket's range of both buffers) over the bits that vary in it;
-// equal keys are copied.  Rare, and slow beside the LDS sort.  Always reports duplicates: telling equal neighbours apart is
-// left to unique.
+// Buckets above CAP, one workgroup to an item.  One key's copies are runs of up
+// to CAP, each written from the first key of it (and its labels moved): many
+// points at one place, as a scanner's missing returns leave them, spread over
+// the chip like any others (one workgroup for all of them took a build of 2^24
+// points, 5% of them at one place, from 875 to 1384 us).  Other buckets
+// are a sample that misjudged them, a few in 10^6: stable LSD passes through
+// global memory (the bucket's range of both buffers) over the bits that vary in
+// it, slow beside the LDS sort.  Always reports duplicates: telling equal
+// neighbours apart is left to unique.
 template <typename K, bool LAB>
 __global__ __launch_bounds__(kSsBlock) void ss_big_kernel(K *kmid, uint32_t *vmid, K *kA,
                                                           uint32_t *vA, K *kB, uint32_t *vB,
@@ -343,6 +370,15 @@ __global__ __launch_bounds__(kSsBlock) void ss_big_kernel(K *kmid, uint32_t *vmi
     const BkItem it = p.big[e];
     const SsOut o = ss_out(p, it.sbits, 0u, st);
     if (t == 0) raise_flag(o.dups);
+    if (it.parity == kSsBigRun) {   // uniform
+      if (kmid == kA) continue;     // where they go already (no shift then)
+      const K x = kmid[it.start];
+      for (uint32_t i = t; i < it.count; i += kSsBlock) {
+        kA[it.start + o.shift + i] = x;
+        if (LAB) vA[it.start + o.shift + i] = vmid[it.start + i];
+      }
+      continue;
+    }
     // from kmid (a big bucket was scattered: a segment of one bucket fits)
     // and the other buffer in turn, to end in A (shifted only where kmid is B)
     K *const outk = kA + o.shift;
@@ -457,7 +493,8 @@ template <typename K>
 size_t ss_ws_bytes(int64_t buckets, int64_t segs, int64_t slots) {
   return align256_dev((size_t)buckets * sizeof(K)) +
          align256_dev((size_t)segs * kSsLutWords * 4) +
-         2 * align256_dev((size_t)buckets * 4) + 2 * align256_dev((size_t)buckets * sizeof(BkItem)) +
+         2 * align256_dev((size_t)buckets * 4) + align256_dev((size_t)buckets * sizeof(BkItem)) +
+         align256_dev((size_t)buckets * 2 * sizeof(BkItem)) +
          align256_dev((size_t)slots * 2) + 256;
 }
 
@@ -470,7 +507,9 @@ void ss_carve(void *ws, int64_t buckets, int64_t segs, int64_t slots, SsPlan &p)
   p.counts = reinterpret_cast<uint32_t *>(take((size_t)buckets * 4));
   p.cursors = reinterpret_cast<uint32_t *>(take((size_t)buckets * 4));
   p.items = reinterpret_cast<BkItem *>(take((size_t)buckets * sizeof(BkItem)));
-  p.big = reinterpret_cast<BkItem *>(take((size_t)buckets * sizeof(BkItem)));
+  // (a bucket of c keys gives at most max(1, 2 c / CAP) items, and a bucket
+  // averages 0.4 CAP keys)
+  p.big = reinterpret_cast<BkItem *>(take((size_t)buckets * 2 * sizeof(BkItem)));
   p.ids = reinterpret_cast<uint16_t *>(take((size_t)slots * 2));
   p.n_big = reinterpret_cast<uint32_t *>(take(4));
   p.n_buckets = buckets;
@@ -596,7 +635,7 @@ void launch_sample_sort(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, 
     else
       ss_splitters_kernel<K, kSsIpt><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
     ss_count_kernel<K><<<tiles, kBlock, 0, s>>>(kin, p, mbits);
-    ss_plan_kernel<<<segs, kSsMaxBuckets, 0, s>>>(p, (uint32_t)SsItem<K>::CAP, st);
+    ss_plan_kernel<K><<<segs, kSsMaxBuckets, 0, s>>>(p, (uint32_t)SsItem<K>::CAP, mbits, st);
     if (vin)
       ss_scatter_kernel<K, true><<<tiles, kBlock, 0, s>>>(kin, vin, kmid, vmid, p);
     else
@@ -613,9 +652,9 @@ void launch_sample_sort(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, 
     ss_sort<K, CAP, 512>(kin, vin, kmid, vmid, kA, vA, p, prepend, st, s);
   if (!segs) return;
   if (vin)
-    ss_big_kernel<K, true><<<64, kSsBlock, 0, s>>>(kmid, vmid, kA, vA, kB, vB, p, st);
+    ss_big_kernel<K, true><<<kSsBigGrid, kSsBlock, 0, s>>>(kmid, vmid, kA, vA, kB, vB, p, st);
   else
-    ss_big_kernel<K, false><<<64, kSsBlock, 0, s>>>(kmid, nullptr, kA, nullptr, kB, nullptr, p, st);
+    ss_big_kernel<K, false><<<kSsBigGrid, kSsBlock, 0, s>>>(kmid, nullptr, kA, nullptr, kB, nullptr, p, st);
 }
 
 template <typename K>
