@@ -61,7 +61,7 @@ constexpr int kPlanBlock = 1024;
 #endif
 __global__ __launch_bounds__(kPlanBlock) void bk_plan_kernel(
     const uint32_t *__restrict__ hist, uint32_t n, int nb, int nb2, int tile2, uint32_t cap,
-    int wide, int lsd_ok, uint32_t seg_max, uint32_t *__restrict__ start,
+    int wide, int lsd_ok, uint32_t whole_max, uint32_t seg_max, uint32_t *__restrict__ start,
     uint32_t *__restrict__ cursor,
     BkSeg *__restrict__ segs, uint32_t *__restrict__ hrows, RunState *st, RunState *host) {
   __shared__ uint32_t s_w[kPlanBlock / 64];
@@ -105,14 +105,14 @@ __global__ __launch_bounds__(kPlanBlock) void bk_plan_kernel(
   for (uint32_t i = t; i < nseg * 256u; i += kPlanBlock) hrows[i] = 0u;
   if (t == 0) {
     // Crowded buckets go to the sample sort.  Where they hold more than a
-    // quarter of the keys (of at most 64 bits), an array small enough for it
-    // is left to it whole (no scatter first), and past a bucket too large for
-    // it the LSD passes take the array.  Either way the scatters and bucket
-    // sorts then do nothing and the host launches the other sort over the
-    // keys as encoded.
+    // quarter of the keys (of at most 64 bits), an array of at most whole_max
+    // keys is left to it whole (no scatter first), and past a bucket of more
+    // than seg_max the LSD passes take the array (any of 32-bit keys, whose
+    // seg_max is 0 here).  Either way the scatters and bucket sorts then do
+    // nothing and the host launches the other sort over the keys as encoded.
     const bool crowded = PGVD_BK_LSD_SHARE > 0 &&
                          (uint64_t)s_bigkeys * PGVD_BK_LSD_SHARE > (uint64_t)n;
-    const bool lsd = crowded && lsd_ok && (n <= seg_max || s_max > seg_max);
+    const bool lsd = crowded && lsd_ok && (n <= whole_max || s_max > seg_max);
     st->bk_lsd = lsd ? 1u : 0u;
     st->bk_segs = lsd ? 0u : nseg;
     st->bk_keys = lsd ? 0u : s_bigkeys;
@@ -317,103 +317,6 @@ __global__ __launch_bounds__(kBlock) void bk_split2_kernel(TileIO<K, LAB> io, ui
   const uint32_t hi = min(lo + (uint32_t)TILE, ghi);
   scatter_tile<K, LAB, Bk<K>::TIPT, false>(io, n, lo, hi, shift, nb2, cursor + g * nb2, 1,
                                            sm.keys, sm.vals);
-}
-
-// ---- merge sort of one item in LDS -----------------------------------------------
-// (key, position) pairs in a strict total order: equal keys by position, so
-// the sort is stable and slots past the item (all-ones keys, positions >=
-// cnt) stay behind every real key.
-template <typename K>
-__device__ inline bool pair_lt(const K &a, uint32_t ia, const K &b, uint32_t ib) {
-  return kless(a, b) || (keq(a, b) && ia < ib);
-}
-
-// The item's cnt keys (and labels) from in[s0 ..] sorted by merging: each
-// thread sorts IPT consecutive keys in registers, then log2(BS) rounds merge
-// runs pairwise, every thread producing IPT outputs of its run pair from a
-// merge-path split found by binary search.  The cost does not depend on how
-// the keys are spread, which suits wide keys that no few digits separate
-// (sparse 128-bit keys on curves).  Positions travel in s_idx (16 bits);
-// labels, staged in s_vals in input order, are gathered by position at the
-// end.  On return s_keys[0 .. cnt) (and s_vals) hold the item in order.
-template <typename K, bool LAB, int BS, int IPT>
-__device__ inline void lds_merge_sort(const K *__restrict__ in, const uint32_t *__restrict__ vin,
-                                      uint32_t s0, uint32_t cnt, K *s_keys, uint32_t *s_vals,
-                                      uint16_t *s_idx) {
-  constexpr uint32_t CAP = (uint32_t)BS * IPT;
-  static_assert(CAP <= 65536, "positions fit 16 bits");
-  const uint32_t t = threadIdx.x;
-  const uint32_t p0 = t * IPT;
-  K k[IPT];
-  uint32_t x[IPT];
-#pragma unroll
-  for (int j = 0; j < IPT; ++j) {
-    const uint32_t p = p0 + j;
-    k[j] = p < cnt ? in[s0 + p] : kones<K>();
-    x[j] = p;
-    if (LAB && p < cnt) s_vals[p] = vin[s0 + p];
-  }
-  // odd-even transposition sort of the thread's IPT pairs
-#pragma unroll
-  for (int r = 0; r < IPT; ++r) {
-#pragma unroll
-    for (int j = r & 1; j + 1 < IPT; j += 2) {
-      if (pair_lt(k[j + 1], x[j + 1], k[j], x[j])) {
-        const K tk = k[j]; k[j] = k[j + 1]; k[j + 1] = tk;
-        const uint32_t tx = x[j]; x[j] = x[j + 1]; x[j + 1] = tx;
-      }
-    }
-  }
-  for (uint32_t w = IPT; w < CAP; w *= 2) {
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      s_keys[p0 + j] = k[j];
-      s_idx[p0 + j] = (uint16_t)x[j];
-    }
-    __syncthreads();
-    const uint32_t base = p0 / (2 * w) * (2 * w);
-    const uint32_t d = p0 - base;   // this thread's first output in the merged pair
-    const uint32_t A = base, B = base + w;
-    // i keys from run A and d - i from run B come first
-    uint32_t lo = d > w ? d - w : 0u, hi = d < w ? d : w;
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi) >> 1;
-      const uint32_t bj = B + d - 1 - mid;
-      if (pair_lt(s_keys[bj], (uint32_t)s_idx[bj], s_keys[A + mid], (uint32_t)s_idx[A + mid]))
-        hi = mid;
-      else
-        lo = mid + 1;
-    }
-    uint32_t ai = A + lo, bi = B + (d - lo);
-    const uint32_t ae = A + w, be = B + w;
-    K ka = ai < ae ? s_keys[ai] : kones<K>(), kb = bi < be ? s_keys[bi] : kones<K>();
-    uint32_t xa = ai < ae ? s_idx[ai] : 0xffffffffu, xb = bi < be ? s_idx[bi] : 0xffffffffu;
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      const bool take_a = pair_lt(ka, xa, kb, xb);   // an exhausted run compares last
-      k[j] = take_a ? ka : kb;
-      x[j] = take_a ? xa : xb;
-      if (take_a) {
-        ++ai;
-        ka = ai < ae ? s_keys[ai] : kones<K>();
-        xa = ai < ae ? s_idx[ai] : 0xffffffffu;
-      } else {
-        ++bi;
-        kb = bi < be ? s_keys[bi] : kones<K>();
-        xb = bi < be ? s_idx[bi] : 0xffffffffu;
-      }
-    }
-    __syncthreads();   // every read of this round is done before the next writes
-  }
-  uint32_t lab[IPT];
-#pragma unroll
-  for (int j = 0; j < IPT; ++j) lab[j] = (LAB && x[j] < cnt) ? s_vals[x[j]] : 0u;
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < IPT; ++j) {
-    s_keys[p0 + j] = k[j];
-    if (LAB) s_vals[p0 + j] = lab[j];
-  }
 }
 
 constexpr int kSubBits = 12;                 // sub-buckets of the counting pass
@@ -649,7 +552,8 @@ bk_sort_kernel(SortArgs<K, LAB> a, int list, int sbits0, RunState *st) {
   } else if constexpr (WPE <= 4) {
     // many varying bits and crowded sub-buckets: merge sort (the counters
     // are no longer needed; their space holds the positions)
-    lds_merge_sort<K, LAB, BS, IPT>(in, vin, s0, cnt, s_keys, s_vals,
+    lds_merge_sort<K, LAB, BS, IPT>([&](uint32_t i) { return in[s0 + i]; },
+                                    [&](uint32_t i) { return vin[s0 + i]; }, cnt, s_keys, s_vals,
                                     reinterpret_cast<uint16_t *>(s_sub));
   }
   __syncthreads();
@@ -1000,7 +904,9 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host,
   constexpr int wide = sizeof(K) > 8 ? 1 : 0;
   bk_plan_kernel<<<1, kPlanBlock, 0, s>>>(a.hist, (uint32_t)n, nb, nb2, TILE, (uint32_t)C::CAP,
                                           wide, sizeof(K) <= 8 ? 1 : 0,
-                                          (uint32_t)ss_max_keys<K>(), m.start, m.cursor,
+                                          (uint32_t)ss_max_whole<K>(a.mbits),
+                                          sizeof(K) == 4 ? 0u : (uint32_t)ss_max_keys<K>(), m.start,
+                                          m.cursor,
                                           m.segs[0], m.hrows[0], st, st_host);
   if (hipGetLastError() != hipSuccess) return 1;
   // the host learns the level-1 segment count (written by the plan into its
@@ -1053,7 +959,7 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host,
   if (hipGetLastError() != hipSuccess) return 1;
   if (!spin_wait(ev)) return 1;
   if (st_host->bk_lsd) {
-    if (n > ss_max_keys<K>()) return 3;   // the LSD passes sort instead
+    if (n > ss_max_whole<K>(a.mbits)) return 3;   // the LSD passes sort instead
     launch_sample_sort<K>(kA, a.labels, kA, vA, kB, vB, m.ss.whole, a.mbits, a.prepend, st, s);
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }

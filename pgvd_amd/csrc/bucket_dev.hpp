@@ -119,6 +119,102 @@ __device__ inline void lds_radix(K (&k)[IPT], uint32_t (&v)[IPT], int passes, in
   }
 }
 
+// ---- merge sort of one item in LDS -----------------------------------------------
+// (key, position) pairs in a strict total order: equal keys by position, so
+// the sort is stable and slots past the item (all-ones keys, positions >=
+// cnt) stay behind every real key.
+template <typename K>
+__device__ inline bool pair_lt(const K &a, uint32_t ia, const K &b, uint32_t ib) {
+  return kless(a, b) || (keq(a, b) && ia < ib);
+}
+
+// The cnt keys pick(i) (and labels vpick(i)) sorted by merging: each
+// thread sorts IPT consecutive keys in registers, then log2(BS) rounds merge
+// runs pairwise, every thread producing IPT outputs of its run pair from a
+// merge-path split found by binary search.  The cost does not depend on how
+// the keys are spread, which suits wide keys that no few digits separate
+// (sparse 128-bit keys on curves).  Positions travel in s_idx (16 bits);
+// labels, staged in s_vals in input order, are gathered by position at the
+// end.  On return s_keys[0 .. cnt) (and s_vals) hold the item in order.
+template <typename K, bool LAB, int BS, int IPT, typename Pick, typename VPick>
+__device__ inline void lds_merge_sort(Pick pick, VPick vpick, uint32_t cnt, K *s_keys,
+                                      uint32_t *s_vals, uint16_t *s_idx) {
+  constexpr uint32_t CAP = (uint32_t)BS * IPT;
+  static_assert(CAP <= 65536, "positions fit 16 bits");
+  const uint32_t t = threadIdx.x;
+  const uint32_t p0 = t * IPT;
+  K k[IPT];
+  uint32_t x[IPT];
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const uint32_t p = p0 + j;
+    k[j] = p < cnt ? pick(p) : kones<K>();
+    x[j] = p;
+    if (LAB && p < cnt) s_vals[p] = vpick(p);
+  }
+  // odd-even transposition sort of the thread's IPT pairs
+#pragma unroll
+  for (int r = 0; r < IPT; ++r) {
+#pragma unroll
+    for (int j = r & 1; j + 1 < IPT; j += 2) {
+      if (pair_lt(k[j + 1], x[j + 1], k[j], x[j])) {
+        const K tk = k[j]; k[j] = k[j + 1]; k[j + 1] = tk;
+        const uint32_t tx = x[j]; x[j] = x[j + 1]; x[j + 1] = tx;
+      }
+    }
+  }
+  for (uint32_t w = IPT; w < CAP && w < cnt; w *= 2) {   // (past cnt: nothing but the slots after it)
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      s_keys[p0 + j] = k[j];
+      s_idx[p0 + j] = (uint16_t)x[j];
+    }
+    __syncthreads();
+    const uint32_t base = p0 / (2 * w) * (2 * w);
+    const uint32_t d = p0 - base;   // this thread's first output in the merged pair
+    const uint32_t A = base, B = base + w;
+    // i keys from run A and d - i from run B come first
+    uint32_t lo = d > w ? d - w : 0u, hi = d < w ? d : w;
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      const uint32_t bj = B + d - 1 - mid;
+      if (pair_lt(s_keys[bj], (uint32_t)s_idx[bj], s_keys[A + mid], (uint32_t)s_idx[A + mid]))
+        hi = mid;
+      else
+        lo = mid + 1;
+    }
+    uint32_t ai = A + lo, bi = B + (d - lo);
+    const uint32_t ae = A + w, be = B + w;
+    K ka = ai < ae ? s_keys[ai] : kones<K>(), kb = bi < be ? s_keys[bi] : kones<K>();
+    uint32_t xa = ai < ae ? s_idx[ai] : 0xffffffffu, xb = bi < be ? s_idx[bi] : 0xffffffffu;
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      const bool take_a = pair_lt(ka, xa, kb, xb);   // an exhausted run compares last
+      k[j] = take_a ? ka : kb;
+      x[j] = take_a ? xa : xb;
+      if (take_a) {
+        ++ai;
+        ka = ai < ae ? s_keys[ai] : kones<K>();
+        xa = ai < ae ? s_idx[ai] : 0xffffffffu;
+      } else {
+        ++bi;
+        kb = bi < be ? s_keys[bi] : kones<K>();
+        xb = bi < be ? s_idx[bi] : 0xffffffffu;
+      }
+    }
+    __syncthreads();   // every read of this round is done before the next writes
+  }
+  uint32_t lab[IPT];
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) lab[j] = (LAB && x[j] < cnt) ? s_vals[x[j]] : 0u;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    s_keys[p0 + j] = k[j];
+    if (LAB) s_vals[p0 + j] = lab[j];
+  }
+}
+
 // ---- minimum and maximum, differences of keys -------------------------------------
 __device__ inline uint32_t ksub(uint32_t a, uint32_t b) { return a - b; }
 __device__ inline uint64_t ksub(uint64_t a, uint64_t b) { return a - b; }
@@ -198,111 +294,28 @@ __device__ inline void lds_rank(const K (&k)[IPT], const uint32_t (&v)[IPT], uin
     }
 }
 
-// ---- LDS sort by splitters -------------------------------------------------------
-// Sorts the cnt <= BS IPT pairs (k[j], v[j]) at index i = j BS + threadIdx.x in
-// LDS, whatever their distribution: 255 splitters, evenly spaced positions of
-// the input ranked against each other, bound 256 buckets; every key finds its
-// bucket (8 LDS reads), and its rank within the bucket by reading the others
-// in it (cnt / 256 on average).  Keys compare together with their index, so
-// equal keys spread over buckets like distinct ones.  pick(i) reads key i.  On
-// return (no barrier passed since) s_keys / s_vals hold the pairs in order;
-// s_tmp: split_words<K>() words, aligned as K.
-constexpr int kSplits = 256;
-template <typename K>
-constexpr int split_words() { return kSplits * ((int)sizeof(K) / 4 + 3) + 1 + 16; }
-
-template <typename K, bool LAB, int BS, int IPT, typename Pick>
-__device__ inline void lds_split_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cnt, Pick pick,
-                                      K *s_keys, uint32_t *s_vals, uint32_t *s_tmp) {
-  constexpr int NW = BS / 64, PARTS = BS / kSplits, PER = kSplits / PARTS;
-  static_assert(BS % kSplits == 0 && NW <= 16, "every thread ranks against a part");
-  K *s_sp = reinterpret_cast<K *>(s_tmp);              // splitters as picked, then in order
-  uint32_t *s_pos = s_tmp + kSplits * (int)sizeof(K) / 4;   // their indexes, in order
-  uint32_t *s_cnt = s_pos + kSplits;                   // their ranks, then the buckets' counts
-  uint32_t *s_start = s_cnt + kSplits;                 // kSplits + 1
-  uint32_t *s_w = s_start + kSplits + 1;
-  const uint32_t t = threadIdx.x;
-  const uint32_t pos = (t & (kSplits - 1)) * cnt / kSplits;
-  K mine = kzero_value<K>();
-  if (t < kSplits) {
-    mine = pick(pos);
-    s_sp[t] = mine;
-    s_cnt[t] = 0;
-  }
-  __syncthreads();
-  {
-    const uint32_t j = t & (kSplits - 1), i0 = t / kSplits * PER;
-    const K x = s_sp[j];
-    uint32_t r = 0;
-#pragma unroll 8
-    for (uint32_t i = i0; i < i0 + PER; ++i) {
-      const K y = s_sp[i];
-      r += (kless(y, x) || (keq(y, x) && i < j)) ? 1u : 0u;
-    }
-    atomicAdd(&s_cnt[j], r);
-  }
-  __syncthreads();
-  if (t < kSplits) {
-    const uint32_t r = s_cnt[t];
-    s_sp[r] = mine;
-    s_pos[r] = pos;
-    s_cnt[t] = 0;
-  }
-  __syncthreads();
-  uint32_t lo[IPT], rs[IPT];
-#pragma unroll
-  for (int j = 0; j < IPT; ++j) lo[j] = 0;
-  // (every key's search at once: their reads are independent)
-#pragma unroll
-  for (uint32_t step = kSplits / 2; step >= 1; step >>= 1) {
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      if ((uint32_t)j * BS >= cnt) break;   // uniform
-      const uint32_t at = lo[j] + step;
-      const K y = s_sp[at];
-      const bool le = kless(y, k[j]) || (keq(y, k[j]) && s_pos[at] <= (uint32_t)j * BS + t);
-      lo[j] = le ? at : lo[j];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < IPT; ++j)
-    rs[j] = (uint32_t)j * BS + t < cnt ? atomicAdd(&s_cnt[lo[j]], 1u) : 0u;
-  __syncthreads();
-  uint32_t total;
-  const uint32_t ex = block_excl_sum<uint32_t, NW>(t < kSplits ? s_cnt[t] : 0u, s_w, &total);
-  if (t < kSplits) s_start[t] = ex;
-  if (t == 0) s_start[kSplits] = total;
-  __syncthreads();
-  uint32_t b1[IPT];
-#pragma unroll
-  for (int j = 0; j < IPT; ++j)
-    if ((uint32_t)j * BS + t < cnt) {
-      b1[j] = s_start[lo[j] + 1];
-      lo[j] = s_start[lo[j]];
-      rs[j] += lo[j];
-      s_keys[rs[j]] = k[j];
-    }
-  __syncthreads();
-  lds_rank<K, LAB, BS, IPT>(k, v, cnt, rs, lo, b1, s_keys, s_vals);
-}
-
 // ---- LDS sort by bins -------------------------------------------------------------
-// Sorts cnt <= BS IPT pairs as lds_split_sort does, for keys that are spread
-// smoothly for the most part: counted in 4096 bins of their range (the keys
-// less the smallest); where some bin holds more than kBinRank of them, every
-// bin is cut into as many bins as it holds keys (rounded down to a power of
-// two) and the keys are counted again; then each key is ranked within its bin.
-// A bin of more than kBinRank2 keys that are all the same (many points at one
-// place) needs no ranking; keys too close together even for that go to
-// lds_split_sort, whose splitters cost four times the counting.  s_tmp:
-// bin_words<K, BS>() words, aligned as K.
+// Sorts in LDS the cnt <= BS IPT pairs (k[j], v[j]) at index i = j BS +
+// threadIdx.x, for keys that are spread smoothly for the most part: counted in
+// 4096 bins of their range (the keys less the smallest); where some bin holds
+// more than kBinRank of them, every bin is cut into as many bins as it holds
+// keys (rounded down to a power of two) and the keys are counted again; then
+// each key is ranked within its bin.  A bin of more than kBinRank2 keys that are
+// all the same (many points at one place) needs no ranking; keys too close
+// together even for that (a range that spans two tight clusters) go to the
+// merge sort, which took 60 us for 8192 64-bit keys where ranking against 256
+// splitters took 117.  pick(i) and vpick(i) read pair i again.  On return (no
+// barrier passed since) s_keys / s_vals hold the pairs in order, equal keys in
+// any order; s_tmp: bin_words<K, BS>() words, aligned as K.
+// kBinRank 12, 24 and 48 time alike.  kBinRank2 128 against 64: 300,000 2D
+// points at 20 bits/axis in clusters of sigma 0.003 166 against 179 us, others
+// alike; at 256 the same points in 3D take 10% longer.
 constexpr int kBins = 4096;
 constexpr uint32_t kBinRank = 24;
-constexpr uint32_t kBinRank2 = 64;
+constexpr uint32_t kBinRank2 = 128;
 template <typename K, int BS>
 constexpr int bin_words() {
-  return (kBins + 4 > split_words<K>() ? kBins + 4 : split_words<K>() + 3) / 4 * 4 +
-         2 * (BS / 64) * ((int)sizeof(K) / 4) + 2 * (BS / 64);
+  return kBins + 4 + 2 * (BS / 64) * ((int)sizeof(K) / 4) + 2 * (BS / 64);
 }
 
 // Largest v over the workgroup (two barriers); s_mx holds BS / 64 words.
@@ -317,11 +330,12 @@ __device__ inline uint32_t block_max(uint32_t v, uint32_t *s_mx) {
   return v;
 }
 
-template <typename K, bool LAB, int BS, int IPT, typename Pick>
+template <typename K, bool LAB, int BS, int IPT, typename Pick, typename VPick>
 __device__ inline void lds_bin_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cnt, Pick pick,
-                                    K *s_keys, uint32_t *s_vals, uint32_t *s_tmp) {
+                                    VPick vpick, K *s_keys, uint32_t *s_vals, uint32_t *s_tmp) {
   constexpr int NW = BS / 64, PER = kBins / BS;
-  constexpr int kMid = (kBins + 4 > split_words<K>() ? kBins + 4 : split_words<K>() + 3) / 4 * 4;
+  constexpr int kMid = kBins + 4;
+  static_assert(2 * BS * IPT <= 4 * kMid, "the merge sort's positions fit");
   uint32_t *s_bin = s_tmp;
   K *s_mm = reinterpret_cast<K *>(s_tmp + kMid);
   uint32_t *s_w = s_tmp + kMid + 2 * NW * ((int)sizeof(K) / 4), *s_mx = s_w + NW;
@@ -442,7 +456,8 @@ __device__ inline void lds_bin_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cn
         b0[j] = b1[j] = at[j];
       }
     if (block_max<BS>(mixed, s_mx)) {
-      lds_split_sort<K, LAB, BS, IPT>(k, v, cnt, pick, s_keys, s_vals, s_tmp);
+      lds_merge_sort<K, LAB, BS, IPT>(pick, vpick, cnt, s_keys, s_vals,
+                                      reinterpret_cast<uint16_t *>(s_tmp));
       return;
     }
   }

@@ -343,6 +343,17 @@ constexpr int64_t kSsMaxPlanBuckets = int64_t(1) << 22;
 // Buckets of a segment of n keys; 0: too many keys for this sort.
 template <typename K> int ss_buckets(int64_t n);
 template <typename K> int64_t ss_max_keys();   // the most that gives buckets
+// Largest crowded array that a build sorts whole by it.  Past it, its crowded
+// buckets are the segments, each with a sample of its own range: 10^6 points in
+// 8 clusters of sigma 1e-4 took 350 us a build whole and 242 so (3D, 63-bit
+// keys; 234 and 244 at sigma 0.1), 500,000 2D points (40 bits) 227 and 159 (167
+// and 162).  Arrays of 32-bit keys past it take the LSD passes, which are four:
+// 300,000 3D points at 10 bits/axis 153 us whole and 130 so (148 and 153), 10^6
+// 253 and 159 (207 and 202).
+template <typename K> int64_t ss_max_whole(int mbits) {
+  if (sizeof(K) == 4) return int64_t(1) << 16;
+  return mbits > 48 ? int64_t(1) << 19 : int64_t(1) << 18;
+}
 template <typename K> int ss_tile();
 template <typename K> size_t ss_ws_bytes(int64_t buckets, int64_t segs, int64_t slots);
 template <typename K>

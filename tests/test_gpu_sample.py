@@ -43,7 +43,13 @@ def clustered(n, dim, seed, sigma=0.02, repeats=()):
     (3, 21, 100003, 1e-6, (0.3,)), (2, 30, 70001, 0.001, (0.6,)),
     (2, 16, 200003, 0.01, ()), (3, 10, 150001, 0.02, (0.5,)),
     (3, 21, LIMIT[8], 0.01, ()), (3, 21, LIMIT[8] + 1, 0.01, ()),
-    (2, 16, LIMIT[4], 0.01, ())])
+    (2, 16, LIMIT[4], 0.01, ()),
+    # either side of the largest array that is one segment, by key width
+    (2, 16, 1 << 16, 0.01, ()), (2, 16, (1 << 16) + 1, 0.01, ()),
+    (2, 20, 1 << 18, 1e-4, ()), (2, 20, (1 << 18) + 1, 1e-4, (0.3,)),
+    (3, 21, 1 << 19, 1e-4, (0.3,)), (3, 21, (1 << 19) + 1, 1e-4, ()),
+    # keys that repeat some tens of times each: bins of several keys' copies
+    (3, 10, 60000, 0.005, ()), (2, 17, 250000, 2e-4, ())])
 def test_clustered_builds_match_radix(dev, dim, bits, n, sigma, repeats):
     pts = clustered(n, dim, n + bits, sigma, repeats)
     got = dev.build_octree(pts, bits)
