@@ -83,6 +83,18 @@ int pgvd_debug_fail_launch(const char *stage);
  * on the current device.  Results do not change, only where they are
  * computed. */
 int pgvd_debug_gather_queue(int entries);
+/* Test hooks, no counterpart in the reference: builds and batch runs that this
+ * thread launches from now on take an array or bucket of more than
+ * segment_keys keys as too large for the sample sort, and sort a bucket of
+ * more than item_keys of its keys outside LDS (0 restores the sort's own
+ * limit; no limit is raised), so that tests reach the forms that take over
+ * there at small sizes.  Results do not change.  pgvd_debug_last_sort: which
+ * sort the context's last pgvd_build_octree took: 0 the LSD passes, 1 the
+ * bucket sort, 2 the bucket sort with further levels for crowded buckets, 3
+ * the sample sort, 4 the bucket sort with the sample sort for crowded
+ * buckets. */
+int pgvd_debug_sort_limits(int64_t segment_keys, int item_keys);
+int pgvd_debug_last_sort(const pgvd_ctx *ctx, int *kind);
 int pgvd_synchronize(pgvd_ctx *ctx, pgvd_stream s);
 int pgvd_alloc(pgvd_ctx *ctx, size_t bytes, void **dptr);
 int pgvd_free(pgvd_ctx *ctx, void *dptr);

@@ -21,6 +21,7 @@ one.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 from dataclasses import dataclass
@@ -138,6 +139,8 @@ def lib():
             "pgvd_ctx_pool_bytes": ([vp, C.POINTER(C.c_size_t)], i32),
             "pgvd_debug_fail_launch": ([C.c_char_p], i32),
             "pgvd_debug_gather_queue": ([i32], i32),
+            "pgvd_debug_sort_limits": ([i64, i32], i32),
+            "pgvd_debug_last_sort": ([vp, C.POINTER(i32)], i32),
             "pgvd_synchronize": ([vp, vp], i32),
             "pgvd_alloc": ([vp, C.c_size_t, C.POINTER(vp)], i32),
             "pgvd_free": ([vp, vp], i32),
@@ -309,6 +312,18 @@ def debug_gather_queue(entries: int) -> None:
         raise PgvdError(rc, lib().pgvd_last_error().decode())
 
 
+@contextlib.contextmanager
+def debug_sort_limits(segment_keys: int = 0, item_keys: int = 0):
+    """Test hook: lower limits of the sorts launched from this thread (0: their
+    own); results must not change."""
+    if lib().pgvd_debug_sort_limits(int(segment_keys), int(item_keys)) != 0:
+        raise PgvdError(-1, lib().pgvd_last_error().decode())
+    try:
+        yield
+    finally:
+        lib().pgvd_debug_sort_limits(0, 0)
+
+
 def debug_fail_launch(stage) -> None:
     """Test hook: the next launch check of `stage` on this thread reports
     PGVD_ERR_HIP (None clears it)."""
@@ -358,6 +373,14 @@ class Device:
 
     def __exit__(self, *a):
         self.close()
+
+    SORTS = ("lsd", "buckets", "levels", "sample", "sample buckets")
+
+    def last_sort(self) -> str:
+        """Which sort the last build took (test hook pgvd_debug_last_sort)."""
+        v = C.c_int()
+        self._check(lib().pgvd_debug_last_sort(self.ctx, C.byref(v)))
+        return self.SORTS[v.value]
 
     def set_pool_limit(self, nbytes: int) -> None:
         """Most device bytes this context's pool may hold (0: no limit);

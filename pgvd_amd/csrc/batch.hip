@@ -255,6 +255,7 @@ void enqueue_typed(pgvd_batch *b, const void *pts) {
                        b->use_sample ? 0 : b->passes, b->st, s);
   if (b->use_sample) {
     // (sorted in place for unique: keys in A, B free)
+    b->ss_plan.item_keys = g_sort_limits.item_keys;
     launch_sample_sort<K>(kA, nullptr, kA, nullptr, kB, nullptr, b->ss_plan, b->mbits, 0, b->st,
                           s);
     b->parity = 1;

@@ -884,9 +884,13 @@ void bucket_carve(void *ws, int64_t n, BucketMem &m) {
 }
 
 template <typename K>
-int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host,
+int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, SortKind *kind,
                        hipEvent_t ev, hipStream_t s) {
   using C = Bk<K>;
+  const int64_t seg_max = a.limits.segment_keys > 0
+                              ? std::min(a.limits.segment_keys, ss_max_keys<K>())
+                              : ss_max_keys<K>();
+  const int64_t whole_max = std::min(ss_max_whole<K>(a.mbits), seg_max);
   const int64_t n = a.n;
   const int b = a.b;
   const int nb = 1 << b;
@@ -904,9 +908,8 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host,
   constexpr int wide = sizeof(K) > 8 ? 1 : 0;
   bk_plan_kernel<<<1, kPlanBlock, 0, s>>>(a.hist, (uint32_t)n, nb, nb2, TILE, (uint32_t)C::CAP,
                                           wide, sizeof(K) <= 8 ? 1 : 0,
-                                          (uint32_t)ss_max_whole<K>(a.mbits),
-                                          sizeof(K) == 4 ? 0u : (uint32_t)ss_max_keys<K>(), m.start,
-                                          m.cursor,
+                                          (uint32_t)whole_max,
+                                          sizeof(K) == 4 ? 0u : (uint32_t)seg_max, m.start, m.cursor,
                                           m.segs[0], m.hrows[0], st, st_host);
   if (hipGetLastError() != hipSuccess) return 1;
   // the host learns the level-1 segment count (written by the plan into its
@@ -959,16 +962,22 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host,
   if (hipGetLastError() != hipSuccess) return 1;
   if (!spin_wait(ev)) return 1;
   if (st_host->bk_lsd) {
-    if (n > ss_max_whole<K>(a.mbits)) return 3;   // the LSD passes sort instead
-    launch_sample_sort<K>(kA, a.labels, kA, vA, kB, vB, m.ss.whole, a.mbits, a.prepend, st, s);
+    if (n > whole_max) return 3;   // the LSD passes sort instead
+    *kind = kSortSample;
+    SsPlan p = m.ss.whole;
+    p.item_keys = a.limits.item_keys;
+    launch_sample_sort<K>(kA, a.labels, kA, vA, kB, vB, p, a.mbits, a.prepend, st, s);
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }
   uint32_t nseg = st_host->bk_segs;
   uint64_t nkeys = st_host->bk_keys;
-  if (nseg > 0 && st_host->bk_max <= ss_max_keys<K>()) {
+  *kind = nseg > 0 ? kSortLevels : kSortBuckets;
+  if (nseg > 0 && st_host->bk_max <= seg_max) {
+    *kind = kSortSampleBuckets;
     // (the segments' keys are where the level-0 scatters left them)
     launch_sample_sort_buckets<K>(p0 ? kB : kA, lab ? v0 : nullptr, kA, vA, kB, vB, m.ss, m.segs[0],
-                                  nseg, nkeys, st_host->bk_max, n, a.mbits, a.prepend, st, s);
+                                  nseg, nkeys, st_host->bk_max, n, a.mbits, a.prepend,
+                                  a.limits.item_keys, st, s);
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }
   int levels = 0;
@@ -1034,7 +1043,7 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host,
   template size_t bucket_ws_bytes<K>(int64_t);                                            \
   template void bucket_carve<K>(void *, int64_t, BucketMem &);                            \
   template int launch_bucket_sort<K>(const BucketArgs<K> &, RunState *, RunState *,       \
-                                     hipEvent_t, hipStream_t);
+                                     SortKind *, hipEvent_t, hipStream_t);
 PGVD_BK_INST(uint32_t)
 PGVD_BK_INST(uint64_t)
 PGVD_BK_INST(Key128)

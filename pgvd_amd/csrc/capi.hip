@@ -193,6 +193,7 @@ struct BuildOut {
   K *uniq = nullptr;
   uint32_t *lsx = nullptr;
   uint32_t *cbits = nullptr;
+  SortKind sort = kSortLsd;
 };
 
 // Takes every buffer of one build from get(key, bytes, &ptr): the
@@ -329,13 +330,14 @@ int build_launch(pgvd_ctx *ctx, const BuildBufs<K> &b, RunState *st, int32_t *oc
   if (bucket) {
     // the bucket sort leaves keys and labels in (kA, vA)
     Stage t(ctx, "msd", s);
-    BucketArgs<K> ba{kA, kB, b.vA, b.vB, labels, msd_hist, n, mbits, bk_b, prepend, b.bk};
-    const int rc = launch_bucket_sort<K>(ba, st, ctx->st_host, ctx->sync_ev, s);
+    BucketArgs<K> ba{kA, kB, b.vA, b.vB, labels, msd_hist, n, mbits, bk_b, prepend, b.bk,
+                     g_sort_limits};
+    const int rc = launch_bucket_sort<K>(ba, st, ctx->st_host, &out.sort, ctx->sync_ev, s);
     if (rc == 2) return fail(PGVD_ERR_INTERNAL, "bucket sort: a segment outlived its levels");
     if (rc == 1) return launch_status("bucket sort") != PGVD_OK ? PGVD_ERR_HIP
                                                                   : fail(PGVD_ERR_HIP, "bucket sort");
     bucket_sorted = rc == 0;
-    // rc 3: clustered keys of at most 64 bits; the encoded keys are untouched
+    // rc 3: the encoded keys are untouched
     if (!bucket_sorted)
       launch_histogram<K>(kA, n, hist, passes, s, nullptr, sort_lb, (z.total - z.sort_lb) / 4);
   }
@@ -439,6 +441,7 @@ int build_impl(pgvd_ctx *ctx, const void *pts, int64_t n, int dim, int bits,
   L.conflict_bits = o.cbits;
   L.lb_splits = reinterpret_cast<uint64_t *>(b.zb + b.z.lb_splits);
   L.exact_deferred = true;
+  L.sort = o.sort;
   L.stream = s;
   return PGVD_OK;
 }
@@ -739,6 +742,18 @@ int pgvd_debug_gather_queue(int entries) {
   if (entries < 0) return fail(PGVD_ERR_INVALID, "entries must be >= 0");
   if (pgvd::set_gather_queue_cap((uint32_t)entries) != 0)
     return fail(PGVD_ERR_HIP, "hipMemcpyToSymbol failed for the gather queue cap");
+  return PGVD_OK;
+}
+
+int pgvd_debug_sort_limits(int64_t segment_keys, int item_keys) {
+  if (segment_keys < 0 || item_keys < 0) return fail(PGVD_ERR_INVALID, "limits must be >= 0");
+  g_sort_limits = SortLimits{segment_keys, (uint32_t)item_keys};
+  return PGVD_OK;
+}
+
+int pgvd_debug_last_sort(const pgvd_ctx *ctx, int *kind) {
+  if (!ctx || !kind) return fail(PGVD_ERR_INVALID, "null argument");
+  *kind = (int)ctx->last.sort;
   return PGVD_OK;
 }
 

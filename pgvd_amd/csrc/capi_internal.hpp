@@ -19,6 +19,8 @@ inline thread_local std::string g_err;
 // Stage whose next launch check on this thread reports a failure
 // (pgvd_debug_fail_launch); empty: none.
 inline thread_local std::string g_fail_launch;
+// Limits of the sorts that this thread launches (pgvd_debug_sort_limits).
+inline thread_local pgvd::SortLimits g_sort_limits;
 
 inline int fail(int code, const std::string &msg) {
   g_err = msg;
@@ -79,6 +81,7 @@ struct LastBuild {
   uint32_t *defer = nullptr;
   uint32_t *conflict_bits = nullptr;
   uint64_t *lb_splits = nullptr;   // look-back words of the order-exact scan (zero)
+  pgvd::SortKind sort = pgvd::kSortLsd;
   bool exact_deferred = false;     // the order-exact path waits for finish
   hipStream_t stream = nullptr;
 };

@@ -329,6 +329,7 @@ struct SsPlan {
   // tiles and buckets in use, at most n_tiles and n_buckets; null: all of them
   const uint32_t *limits = nullptr;
   uint32_t n = 0, nb = 0;
+  uint32_t item_keys = 0;                  // most keys of an LDS sort's item; 0: what it holds
   uint32_t max_nb = 0;                     // buckets of the largest segment
   int64_t n_segs = 0, n_tiles = 0, n_buckets = 0;
   void *splitters = nullptr;
@@ -381,7 +382,7 @@ template <typename K>
 void launch_sample_sort_buckets(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, K *kB,
                                 uint32_t *vB, const SsTree &t, const BkSeg *segs, uint32_t nseg,
                                 uint64_t nkeys, uint32_t max_keys, int64_t n, int mbits,
-                                int prepend, RunState *st, hipStream_t s);
+                                int prepend, uint32_t item_keys, RunState *st, hipStream_t s);
 
 struct BucketMem {
   uint32_t *start = nullptr, *cursor = nullptr;
@@ -392,6 +393,16 @@ struct BucketMem {
   uint32_t max_segs = 0, max_items = 0;
   SsTree ss;               // the sample sort's workspace
 };
+// Which sort ordered a build's keys: the LSD passes, the bucket sort alone or
+// with its levels for the crowded buckets, the sample sort (of the whole array)
+// or the bucket sort with the sample sort for the crowded buckets.
+enum SortKind { kSortLsd = 0, kSortBuckets, kSortLevels, kSortSample, kSortSampleBuckets };
+// Lower limits for tests (0: the sort's own): a larger bucket or array is too
+// large for the sample sort; a larger bucket of its own is not sorted in LDS.
+struct SortLimits {
+  int64_t segment_keys = 0;
+  uint32_t item_keys = 0;
+};
 template <typename K>
 struct BucketArgs {
   K *kA, *kB;                 // keys in kA (encode's output); kB the other buffer
@@ -401,6 +412,7 @@ struct BucketArgs {
   int64_t n;
   int mbits, b, prepend;
   BucketMem mem;
+  SortLimits limits;
 };
 inline constexpr size_t align256_dev(size_t x) { return (x + 255) & ~(size_t)255; }
 template <typename K> int bucket_cap();
@@ -408,12 +420,15 @@ template <typename K> int bucket_bits_for(int64_t n);
 template <typename K> size_t bucket_ws_bytes(int64_t n);
 template <typename K> void bucket_carve(void *ws, int64_t n, BucketMem &m);
 // Enqueues the sort on s.  Waits on the host (ev, st_host: pinned) for the
-// level-0 plan and each level's scan while the device works on.  0: sorted;
-// 3: keys of at most 64 bits too clustered (a quarter of them in buckets
-// above CAP): nothing moved, the caller sorts by the LSD passes; else a
-// launch failed (1) or a segment outlived the levels (2).
+// level-0 plan and each level's scan while the device works on.  0: sorted
+// (*kind: how); 3: the keys, of at most 64 bits, are ones that the LSD passes
+// sort faster (more than a quarter of them in buckets above CAP, and one of
+// those too large for the sample sort, or 32-bit keys past ss_max_whole):
+// nothing moved, the caller launches the passes; else a launch failed (1) or a
+// segment outlived the levels (2).
 template <typename K>
-int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, hipEvent_t ev,
+int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, SortKind *kind,
+                       hipEvent_t ev,
                        hipStream_t s);
 
 // Bucket histogram bins the vectorised encode kernel holds in LDS beside

@@ -636,7 +636,9 @@ void launch_sample_sort(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, 
     else
       ss_splitters_kernel<K, kSsIpt><<<segs, kSsBlock, 0, s>>>(kin, p, mbits);
     ss_count_kernel<K><<<tiles, kBlock, 0, s>>>(kin, p, mbits);
-    ss_plan_kernel<K><<<segs, kSsMaxBuckets, 0, s>>>(p, (uint32_t)SsItem<K>::CAP, mbits, st);
+    const uint32_t cap = (uint32_t)SsItem<K>::CAP;
+    ss_plan_kernel<K><<<segs, kSsMaxBuckets, 0, s>>>(
+        p, p.item_keys ? std::min(p.item_keys, cap) : cap, mbits, st);
     if (vin)
       ss_scatter_kernel<K, true><<<tiles, kBlock, 0, s>>>(kin, vin, kmid, vmid, p);
     else
@@ -662,12 +664,13 @@ template <typename K>
 void launch_sample_sort_buckets(const K *kin, const uint32_t *vin, K *kA, uint32_t *vA, K *kB,
                                 uint32_t *vB, const SsTree &t, const BkSeg *segs, uint32_t nseg,
                                 uint64_t nkeys, uint32_t max_keys, int64_t n, int mbits,
-                                int prepend, RunState *st, hipStream_t s) {
+                                int prepend, uint32_t item_keys, RunState *st, hipStream_t s) {
   const SsTables o = ss_tables(t.tables, ss_crowded_segs<K>(n));
   const uint32_t T = (uint32_t)ss_bucket_keys<K>();
   ss_tables_kernel<<<1, kSsBlock, 0, s>>>(segs, nseg, T, (uint32_t)ss_tile<K>(), (uint32_t)n,
                                           sizeof(K) <= 8 ? 1 : 0, o, st);
   SsPlan p = t.crowded;
+  p.item_keys = item_keys;
   p.seg = o.seg;
   p.tiles.seg = o.tile_seg;
   p.tiles.first = o.tile_first;
@@ -694,7 +697,7 @@ void launch_sample_sort_buckets(const K *kin, const uint32_t *vin, K *kA, uint32
   template void launch_sample_sort_buckets<K>(const K *, const uint32_t *, K *, uint32_t *,   \
                                               K *, uint32_t *, const SsTree &, const BkSeg *, \
                                               uint32_t, uint64_t, uint32_t, int64_t, int,     \
-                                              int, RunState *, hipStream_t);
+                                              int, uint32_t, RunState *, hipStream_t);
 PGVD_SS_INST(uint32_t)
 PGVD_SS_INST(uint64_t)
 PGVD_SS_INST(Key128)

@@ -1,8 +1,9 @@
 """The whole path's bucket sort (bucket.hip) through pgvd_build_octree,
 against the oracle: every key width (32-, 64- and 128-bit keys), with and
 without labels, at sizes that take each level-0 shape (one LDS item, one
-scatter, two scatters), on clustered keys that need further levels, and on
-runs of equal keys (copied rather than split)."""
+scatter, two scatters), on clustered keys, whose crowded buckets go to the
+sample sort or, past its limits, to further levels or the LSD passes, and on
+runs of equal keys."""
 from __future__ import annotations
 
 import numpy as np
@@ -11,6 +12,7 @@ import pytest
 from conftest import assert_tree_equal
 
 import oracle
+import pgvd_amd
 from pgvd_amd import workloads
 
 pytestmark = pytest.mark.gpu
@@ -58,7 +60,8 @@ def test_bucket_uniform_sizes(dev, dim, bits, n):
 @pytest.mark.parametrize("n", [50_000, 1 << 20])
 def test_bucket_clustered_levels(dev, dim, bits, n):
     """A sixth of the points in tight clusters: their top-level buckets
-    exceed one LDS item and go through the levels."""
+    exceed one LDS item and go to the sample sort (through the levels:
+    test_bucket_past_the_sample_sort)."""
     pts = _uniform(n, dim, seed=n % 991 + dim)
     k = n // 6
     pts[:k] = _clusters(k, dim, seed=7 + dim)
@@ -67,9 +70,9 @@ def test_bucket_clustered_levels(dev, dim, bits, n):
 
 @pytest.mark.parametrize("dim,bits", [(2, 16), (3, 21), (3, 42)])
 def test_bucket_heavy_clusters(dev, dim, bits):
-    """Every point in a tight cluster.  128-bit keys go through the levels;
-    keys of at most 64 bits, with more than a quarter of them left to the
-    levels, are sorted by the LSD passes instead."""
+    """Every point in a tight cluster.  Each crowded bucket of 128-bit keys is
+    a segment of the sample sort; keys of at most 64 bits, more than a quarter
+    of them crowded, are its segments too or go to the LSD passes (32 bits)."""
     pts = _clusters(1 << 20, dim, seed=17 + dim)
     got = _check(dev, pts, bits, where="heavy clusters", bucket=bits * dim > 64)
     assert got["m"] < pts.shape[0] or bits == 42     # duplicates at the coarser grids
@@ -88,7 +91,7 @@ def test_bucket_equal_runs(dev):
         pts = _uniform(300_000, dim, seed=3)
         pts[1000:200_000] = pts[5]
         pts[250_000:260_000] = pts[7]
-        # two thirds of the keys equal: narrower keys take the LSD passes
+        # two thirds of the keys equal: narrower keys take another sort whole
         _check(dev, pts, bits, where="equal runs", bucket=bits * dim > 64)
 
 
@@ -102,7 +105,7 @@ def test_bucket_labels(dev):
     dst = rng.integers(0, pts.shape[0], 20_000)
     pts[dst] = pts[src]
     for bits, dim in ((42, 3), (21, 3)):
-        # (63-bit keys on loops: bucket sort or LSD passes, by how clustered)
+        # (63-bit keys on loops: the bucket sort or another, by how clustered)
         _check(dev, pts, bits, labels=lab, where=f"labels {bits}", bucket=True if bits == 42 else None)
     p2 = _clusters(200_000, 2, seed=14, k=4, sigma=1e-3)
     l2 = np.random.default_rng(15).integers(0, 5, p2.shape[0]).astype(np.uint32)
@@ -131,4 +134,67 @@ def test_int32_grid_points_match_radix(dev, dim, bits, n, spread):
     want = dev.build_octree(q, bits, no_host_wait=True)
     assert want["bucket_sort"] == 0
     assert got["bucket_sort"] == (spread == 1 << bits)      # else crowded
+    assert_tree_equal(got, want)
+
+
+@pytest.mark.parametrize("dim,bits", [(2, 16), (3, 21), (3, 42)])
+@pytest.mark.parametrize("labels", [False, True])
+@pytest.mark.parametrize("kind", ["clusters", "runs", "heavy"])
+def test_bucket_past_the_sample_sort(dev, dim, bits, labels, kind):
+    """The sorts that take over where a bucket is too large for the sample
+    sort, at sizes that reach them by a lower limit: the levels (clusters and
+    runs of one point, up to a quarter of the keys; 128-bit keys always) and
+    the LSD passes (more of them)."""
+    n = 300_007
+    pts = _uniform(n, dim, seed=31)
+    if kind == "clusters":
+        pts[:n // 8] = _clusters(n // 8, dim, seed=5, k=4)
+    elif kind == "runs":
+        pts[1000:40_000] = pts[5]
+        pts[250_000:270_000] = pts[7]
+    else:
+        pts = _clusters(n, dim, seed=6)
+        pts[1000:40_000] = pts[5]
+    lab = np.random.default_rng(4).integers(0, 3, n).astype(np.uint32) if labels else None
+    lsd = kind == "heavy" and bits != 42
+    with pgvd_amd.debug_sort_limits(segment_keys=1):
+        _check(dev, pts, bits, labels=lab, where=kind, bucket=not lsd)
+        assert dev.last_sort() == ("lsd" if lsd else "levels")
+
+
+@pytest.mark.parametrize("dim,bits,n,crowd,labels,sort", [
+    (3, 21, 4_600_001, 1_100_000, False, "levels"), (3, 21, 3_000_001, 1_100_000, True, "lsd"),
+    (3, 21, 4_600_001, 1_000_000, False, "sample buckets"),
+    (3, 42, 700_001, 640_000, True, "levels"), (3, 42, 700_001, 600_000, True, "sample buckets"),
+    (2, 16, 7_000_001, 1_700_000, False, "levels"), (2, 16, 300_001, 200_000, False, "lsd")])
+def test_bucket_at_the_sample_sort_limits(dev, dim, bits, n, crowd, labels, sort):
+    """One bucket just below and just above the most keys that the sample sort
+    takes (1,048,576 of 64 bits, 628,736 of 128, 1,677,312 of 32), in one cluster
+    inside a top-level bucket, a tenth of it one repeated point."""
+    pts = _uniform(n, dim, seed=41)
+    rng = np.random.default_rng(42)
+    pts[:crowd] = 0.4 + rng.standard_normal((crowd, dim)).astype(np.float32) * 2e-4
+    pts[:crowd // 10] = pts[0]
+    pts[-2], pts[-1] = -1.0, 1.0
+    lab = rng.integers(0, 3, n).astype(np.uint32) if labels else None
+    got = dev.build_octree(pts, bits, labels=lab)
+    assert dev.last_sort() == sort
+    want = dev.build_octree(pts, bits, labels=lab, no_host_wait=True)
+    assert dev.last_sort() == "lsd"
+    assert_tree_equal(got, want)
+    if labels:
+        for f in ("key_conflict", "node_conflict"):
+            assert np.array_equal(got[f], want[f]), f
+
+
+def test_int32_grid_points_take_the_lsd_passes(dev):
+    """Clustered int32 grid points whose largest bucket the sample sort does
+    not take."""
+    rng = np.random.default_rng(8)
+    q = (_clusters(200_003, 2, seed=9, sigma=1e-3) * 0.5 + 0.5) * ((1 << 20) - 1)
+    q = np.concatenate([q.astype(np.int32), rng.integers(0, 1 << 20, (1000, 2)).astype(np.int32)])
+    want = dev.build_octree(q, 20, no_host_wait=True)
+    with pgvd_amd.debug_sort_limits(segment_keys=1):
+        got = dev.build_octree(q, 20)
+    assert dev.last_sort() == "lsd" and got["bucket_sort"] == 0
     assert_tree_equal(got, want)

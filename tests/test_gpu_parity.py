@@ -179,9 +179,7 @@ def test_full_size_3d_digests(dev, golden_digests, name):
 def test_bucket_sort_large_and_clustered(dev):
     """A build of 2^23 + 4097 64-bit keys: the keys scatter by their top bits
     into buckets that each sort inside one workgroup; buckets that are too
-    full (points near the centre) are split further below their highest
-    varying bit, or, when they hold more than a quarter of the keys, the LSD
-    passes sort.  Against the oracle at a size that is not a power of two."""
+    full (points near the centre) go to the sample sort.  Against the oracle at a size that is not a power of two."""
     n = (1 << 23) + 4097
     pts = _pts(n, 3, seed=23)
     got = dev.build_octree(pts, 21)
@@ -202,8 +200,7 @@ def test_bucket_sort_large_and_clustered(dev):
     got = dev.build_octree(corner, 21)
     assert got["bucket_sort"] == 1 and got["keys_lo"][0] == 0
     assert_tree_equal(got, oracle.build(oracle.quantize(corner, 1 << 21), 21), where="zero key")
-    # an eighth of the points near the centre: their buckets go through the
-    # levels; half of them: the LSD passes sort instead
+    # an eighth of the points near the centre, and half of them
     for frac, bucket in ((8, 1), (2, 0)):
         clustered = pts.copy()
         clustered[: n // frac] *= np.float32(1e-3)

@@ -123,3 +123,49 @@ def test_crowded_buckets_match_radix(dev, dim, bits, n, labels, share, sigma):
     if labels:
         for f in ("key_conflict", "node_conflict"):
             assert np.array_equal(got[f], want[f]), f
+
+
+@pytest.mark.parametrize("dim,bits", [(2, 16), (3, 21), (3, 42), (2, 20)])
+@pytest.mark.parametrize("labels", [False, True])
+@pytest.mark.parametrize("n,crowd", [(60000, 60000), (290000, 290000), (700001, 120000)])
+def test_oversize_buckets(dev, dim, bits, labels, n, crowd):
+    """Buckets that outgrow an LDS sort, which a sample seldom leaves of
+    distinct keys: made of ordinary ones by a lower limit, with runs of
+    repeated keys among them, of whole arrays and of crowded buckets in either
+    buffer."""
+    pts = np.random.default_rng(6).random((n, dim), dtype=np.float32) * 2 - 1
+    pts[:crowd] = clustered(crowd, dim, 11, 0.002, (0.2, 0.05))
+    lab = np.random.default_rng(5).integers(0, 3, n).astype(np.uint32) if labels else None
+    with pgvd_amd.debug_sort_limits(item_keys=700):
+        got = dev.build_octree(pts, bits, labels=lab)
+    sort = dev.last_sort()
+    want = dev.build_octree(pts, bits, labels=lab, no_host_wait=True)
+    assert "sample" in sort or (dim, bits) == (2, 16) and n == 290000, sort
+    assert_tree_equal(got, want, FIELDS)
+    if labels:
+        for f in ("key_conflict", "node_conflict"):
+            assert np.array_equal(got[f], want[f]), f
+
+
+@pytest.mark.parametrize("dim,bits", [(2, 16), (3, 21), (3, 42)])
+def test_batch_oversize_buckets(dev, dim, bits):
+    """The same in a batch, of instances with a prepended zero key and without
+    (16384 and 32768 points), one of them on the grid's corner."""
+    sizes = [16384, 20000, 32768, 40001, 9, 30000]
+    parts = [clustered(n, dim, i, 0.003, (0.3, 0.1)) for i, n in enumerate(sizes)]
+    parts[5][:10000] = -1.0
+    d = dev.upload(np.concatenate(parts))
+    try:
+        with pgvd_amd.Batch(dev, sizes, dim, bits) as b, \
+                pgvd_amd.debug_sort_limits(item_keys=700):
+            assert b.sample_sort()
+            for _ in range(2):
+                b.run(d)
+                r = b.finish()
+            all_ = b.fetch_all(r)
+        for i, p in enumerate(parts):
+            assert_tree_equal(pgvd_amd.Batch.instance(all_, i, r.key_bytes, dim),
+                              dev.build_octree(p, bits, no_host_wait=True), FIELDS,
+                              where=f"instance {i}")
+    finally:
+        d.free()
