@@ -92,7 +92,7 @@ int pgvd_debug_gather_queue(int entries);
  * sort the context's last pgvd_build_octree took: 0 the LSD passes, 1 the
  * bucket sort, 2 the bucket sort with further levels for crowded buckets, 3
  * the sample sort, 4 the bucket sort with the sample sort for crowded
- * buckets. */
+ * buckets, 5 the bucket sort or the LSD passes as the device chose. */
 int pgvd_debug_sort_limits(int64_t segment_keys, int item_keys);
 int pgvd_debug_last_sort(const pgvd_ctx *ctx, int *kind);
 int pgvd_synchronize(pgvd_ctx *ctx, pgvd_stream s);
@@ -403,10 +403,15 @@ typedef struct pgvd_octree_result {
  * (device, n u32, nullable) are object ids carried through the sort for the
  * conflict-cell pass.  Enqueues the whole path on the stream and returns;
  * pgvd_build_octree_finish waits and reports the sizes.  With float points
- * the sort is a bucket sort whose levels the host decides from small counts
- * the device reports mid-build: the call then returns once the device has
- * reached the sort's last level (the work queued behind keeps it busy), not
- * at once, unless opts->no_host_wait. */
+ * the sort is a bucket sort after whose first step the host chooses what sorts
+ * crowded buckets, from counts the device reports mid-build: the call then
+ * returns once the device has reached that step (the work queued behind keeps
+ * it busy; a crowded bucket too large for the sample sort makes it wait for
+ * each further level), not at once, unless opts->no_host_wait.  With int32
+ * points it polls for those counts as long as an idle device takes to reach
+ * them (50 us and 1 us more per 100,000 points at most); where other work comes
+ * first, or under stream capture, the device chooses between the bucket sort
+ * and the radix passes. */
 int pgvd_build_octree(pgvd_ctx *ctx, const void *pts, int64_t n, int dim, int bits,
                       const uint32_t *labels, const pgvd_build_opts *opts, pgvd_stream s);
 

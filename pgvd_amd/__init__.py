@@ -374,7 +374,7 @@ class Device:
     def __exit__(self, *a):
         self.close()
 
-    SORTS = ("lsd", "buckets", "levels", "sample", "sample buckets")
+    SORTS = ("lsd", "buckets", "levels", "sample", "sample buckets", "device")
 
     def last_sort(self) -> str:
         """Which sort the last build took (test hook pgvd_debug_last_sort)."""

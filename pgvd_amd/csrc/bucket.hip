@@ -21,6 +21,8 @@
 // (OR == AND) is copied, not split.  The host reads the segment count after
 // the level-0 plan and after each level's scan while the device keeps
 // working, and stops launching levels when none is left.
+#include <chrono>
+
 #include "bucket_dev.hpp"
 
 namespace pgvd {
@@ -59,9 +61,16 @@ constexpr int kPlanBlock = 1024;
 #ifndef PGVD_BK_LSD_SHARE
 #define PGVD_BK_LSD_SHARE 4
 #endif
+__device__ inline bool bk_crowded(uint64_t keys, uint64_t n) {
+  return PGVD_BK_LSD_SHARE > 0 && keys * PGVD_BK_LSD_SHARE > n;
+}
+// Where another sort takes the array: never (128-bit keys); by that share; the
+// same, with msd_ok left clear while crowded buckets remain; or wherever a
+// bucket is crowded.
+enum { kPlanKeep = 0, kPlanShare, kPlanShareOpen, kPlanAny };
 __global__ __launch_bounds__(kPlanBlock) void bk_plan_kernel(
     const uint32_t *__restrict__ hist, uint32_t n, int nb, int nb2, int tile2, uint32_t cap,
-    int wide, int lsd_ok, uint32_t whole_max, uint32_t seg_max, uint32_t *__restrict__ start,
+    int wide, int rule, uint32_t whole_max, uint32_t seg_max, uint32_t *__restrict__ start,
     uint32_t *__restrict__ cursor,
     BkSeg *__restrict__ segs, uint32_t *__restrict__ hrows, RunState *st, RunState *host) {
   __shared__ uint32_t s_w[kPlanBlock / 64];
@@ -110,23 +119,24 @@ __global__ __launch_bounds__(kPlanBlock) void bk_plan_kernel(
     // than seg_max the LSD passes take the array (any of 32-bit keys, whose
     // seg_max is 0 here).  Either way the scatters and bucket sorts then do
     // nothing and the host launches the other sort over the keys as encoded.
-    const bool crowded = PGVD_BK_LSD_SHARE > 0 &&
-                         (uint64_t)s_bigkeys * PGVD_BK_LSD_SHARE > (uint64_t)n;
-    const bool lsd = crowded && lsd_ok && (n <= whole_max || s_max > seg_max);
+    const bool lsd = rule == kPlanAny
+                         ? nseg > 0
+                         : rule != kPlanKeep && bk_crowded(s_bigkeys, n) &&
+                               (n <= whole_max || s_max > seg_max);
     st->bk_lsd = lsd ? 1u : 0u;
     st->bk_segs = lsd ? 0u : nseg;
     st->bk_keys = lsd ? 0u : s_bigkeys;
-    // the same three words straight into the host's pinned mirror, which
-    // reads them once the plan's completion event has fired (no copy
-    // launch between the plan and the first scatter)
+    // what the host decides by, straight into its pinned mirror, which it
+    // reads once the plan's completion event has fired (no copy launch
+    // between the plan and the first scatter)
     host->bk_lsd = lsd ? 1u : 0u;
-    host->bk_segs = lsd ? 0u : nseg;
-    host->bk_keys = lsd ? 0u : s_bigkeys;
+    host->bk_segs = nseg;
+    host->bk_keys = s_bigkeys;
     host->bk_max = s_max;
     __threadfence_system();
     // (a histogram that does not count every key leaves the keys unsorted:
     // then the status says so and nothing downstream trusts the order)
-    st->msd_ok = (total == n && !lsd) ? 1u : 0u;
+    st->msd_ok = (total == n && !lsd && (rule != kPlanShareOpen || nseg == 0)) ? 1u : 0u;
     if (total != n) atomicOr(&st->status, (uint32_t)ST_TOO_LARGE);
     st->msd_dups = 0;
   }
@@ -828,6 +838,22 @@ static bool spin_wait(hipEvent_t ev) {
   }
 }
 
+// The same for at most us microseconds: 1 when ev has fired, 0 when not, -1
+// on an error.
+static int poll_event(hipEvent_t ev, int64_t us) {
+  if (us <= 0) return 0;
+  const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(us);
+  for (;;) {
+    const hipError_t e = hipEventQuery(ev);
+    if (e == hipSuccess) return 1;
+    if (e != hipErrorNotReady) return -1;
+    if (std::chrono::steady_clock::now() >= end) {
+      (void)hipGetLastError();   // (not ready: not left for the next launch check)
+      return 0;
+    }
+  }
+}
+
 template <typename K>
 int bucket_cap() { return Bk<K>::CAP; }
 
@@ -890,7 +916,13 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, 
   const int64_t seg_max = a.limits.segment_keys > 0
                               ? std::min(a.limits.segment_keys, ss_max_keys<K>())
                               : ss_max_keys<K>();
-  const int64_t whole_max = std::min(ss_max_whole<K>(a.mbits), seg_max);
+  const bool bounded = a.poll_us >= 0;
+  // (bounded: past it, and after one scatter, the LSD passes follow an encode
+  // that did not count their digits: 300,000 2D points of 40 bits in clusters
+  // take 146 us whole and 163 so)
+  const int64_t whole_max = std::min(ss_max_whole<K>(bounded ? 64 : a.mbits), seg_max);
+  // the largest bucket with which crowded keys stay with the bucket sort
+  const uint32_t crowd_max = sizeof(K) == 4 ? 0u : (uint32_t)seg_max;
   const int64_t n = a.n;
   const int b = a.b;
   const int nb = 1 << b;
@@ -906,21 +938,30 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, 
   }
   constexpr int TILE = kBlock * C::TIPT;
   constexpr int wide = sizeof(K) > 8 ? 1 : 0;
-  bk_plan_kernel<<<1, kPlanBlock, 0, s>>>(a.hist, (uint32_t)n, nb, nb2, TILE, (uint32_t)C::CAP,
-                                          wide, sizeof(K) <= 8 ? 1 : 0,
-                                          (uint32_t)whole_max,
-                                          sizeof(K) == 4 ? 0u : (uint32_t)seg_max, m.start, m.cursor,
-                                          m.segs[0], m.hrows[0], st, st_host);
-  if (hipGetLastError() != hipSuccess) return 1;
-  // the host learns the level-1 segment count (written by the plan into its
-  // pinned mirror) while the scatters run
-  if (hipEventRecord(ev, s) != hipSuccess) return 1;
   K *kA = a.kA, *kB = a.kB;
   uint32_t *vA = a.vA, *vB = a.vB;
+  K *const kO = a.out_b ? kB : kA, *const kP = a.out_b ? kA : kB;   // the result's buffer, the other
+  uint32_t *const vO = a.out_b ? vB : vA, *const vP = a.out_b ? vA : vB;
   const unsigned tiles1 = (unsigned)((n + TILE - 1) / TILE);
-  int p0 = 0;   // buffer holding the level-0 buckets
-  const K *k0 = kA;
-  const uint32_t *v0 = lab ? a.labels : nullptr;
+  const int p0 = splits == 1 ? 1 : 0;   // buffer holding the level-0 buckets
+  const K *k0 = p0 ? kB : kA;
+  const uint32_t *v0 = lab ? (p0 ? vB : (splits ? vA : a.labels)) : nullptr;
+  SortArgs<K, true> sa{{kA, kB}, {vA, vB}, k0, v0, kO, vO, m.start, m.items, (uint32_t)a.prepend};
+  SortArgs<K, false> san{{kA, kB}, {nullptr, nullptr}, k0, nullptr, kO, nullptr, m.start, m.items,
+                         (uint32_t)a.prepend};
+  // With a bounded wait the LSD passes may have to take over from whatever the
+  // device has done by itself: after two scatters without labels every key is
+  // in kA again, in some order; otherwise a crowded bucket stops the scatters.
+  const bool again = splits == 2 && !lab;
+  const int rule = !bounded ? (sizeof(K) <= 8 ? kPlanShare : kPlanKeep)
+                            : (again ? kPlanShareOpen : kPlanAny);
+  bk_plan_kernel<<<1, kPlanBlock, 0, s>>>(a.hist, (uint32_t)n, nb, nb2, TILE, (uint32_t)C::CAP,
+                                          wide, rule, (uint32_t)whole_max, crowd_max, m.start,
+                                          m.cursor, m.segs[0], m.hrows[0], st, st_host);
+  if (hipGetLastError() != hipSuccess) return 1;
+  // the host learns the crowded buckets (written by the plan into its pinned
+  // mirror) while the scatters run
+  if ((!bounded || a.poll_us > 0) && hipEventRecord(ev, s) != hipSuccess) return 1;
   if (splits >= 1) {
     TileIO<K, true> io1{kA, a.labels, kB, vB};
     TileIO<K, false> io1n{kA, nullptr, kB, nullptr};
@@ -932,9 +973,6 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, 
     else
       bk_split1_kernel<K, false><<<tiles1, kBlock, 0, s>>>(io1n, (uint32_t)n, a.mbits - b1, nb1,
                                                            cur1, cstride, st);
-    p0 = 1;
-    k0 = kB;
-    v0 = vB;
   }
   if (splits == 2) {
     TileIO<K, true> io2{kB, vB, kA, vA};
@@ -946,13 +984,7 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, 
     else
       bk_split2_kernel<K, false><<<grid2, kBlock, 0, s>>>(io2n, (uint32_t)n, a.mbits - b, nb2, nb1,
                                                           m.start, m.cursor, st);
-    p0 = 0;
-    k0 = kA;
-    v0 = vA;
   }
-  SortArgs<K, true> sa{{kA, kB}, {vA, vB}, k0, v0, kA, vA, m.start, m.items, (uint32_t)a.prepend};
-  SortArgs<K, false> san{{kA, kB}, {nullptr, nullptr}, k0, nullptr, kA, nullptr, m.start, m.items,
-                         (uint32_t)a.prepend};
   if (lab)
     bk_sort_kernel<K, true, C::BS, C::IPT, sort_wpe<K, true, false>(), false>
         <<<(unsigned)nb, C::BS, 0, s>>>(sa, 0, a.mbits - b, st);
@@ -960,26 +992,31 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, 
     bk_sort_kernel<K, false, C::BS, C::IPT, sort_wpe<K, false, false>(), false>
         <<<(unsigned)nb, C::BS, 0, s>>>(san, 0, a.mbits - b, st);
   if (hipGetLastError() != hipSuccess) return 1;
-  if (!spin_wait(ev)) return 1;
+  *kind = kSortBuckets;
+  if (bounded && n <= C::CAP) return 0;   // (none can be crowded)
+  const int w = bounded ? poll_event(ev, a.poll_us) : (spin_wait(ev) ? 1 : -1);
+  if (w < 0) return 1;
+  if (w == 0) return 4;
   if (st_host->bk_lsd) {
     if (n > whole_max) return 3;   // the LSD passes sort instead
     *kind = kSortSample;
     SsPlan p = m.ss.whole;
     p.item_keys = a.limits.item_keys;
-    launch_sample_sort<K>(kA, a.labels, kA, vA, kB, vB, p, a.mbits, a.prepend, st, s);
+    launch_sample_sort<K>(kA, a.labels, kO, vO, kP, vP, p, a.mbits, a.prepend, st, s);
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }
   uint32_t nseg = st_host->bk_segs;
   uint64_t nkeys = st_host->bk_keys;
-  *kind = nseg > 0 ? kSortLevels : kSortBuckets;
+  if (nseg > 0) *kind = kSortLevels;
   if (nseg > 0 && st_host->bk_max <= seg_max) {
     *kind = kSortSampleBuckets;
     // (the segments' keys are where the level-0 scatters left them)
-    launch_sample_sort_buckets<K>(p0 ? kB : kA, lab ? v0 : nullptr, kA, vA, kB, vB, m.ss, m.segs[0],
-                                  nseg, nkeys, st_host->bk_max, n, a.mbits, a.prepend,
-                                  a.limits.item_keys, st, s);
+    launch_sample_sort_buckets<K>(k0, v0, kO, vO, kP, vP, m.ss, m.segs[0], nseg, nkeys,
+                                  st_host->bk_max, n, a.mbits, a.prepend, a.limits.item_keys, st,
+                                  s);
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }
+  if (bounded && nseg > 0) return 3;   // (the levels' counts would be waited for)
   int levels = 0;
   int parity = p0;
   int cur = 0;

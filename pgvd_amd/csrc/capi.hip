@@ -234,9 +234,9 @@ int carve_build(Get &&get, const void *pts, int64_t n, int dim, int bits, bool l
   const bool custom = opts && opts->use_custom_bb;
   // aligned points (vectorised encode, which builds the bucket histogram) on
   // a context (the sort's levels are decided on the host): bucket sort;
-  // otherwise the LSD passes
+  // otherwise, and for int32 points with 128-bit keys, the LSD passes
   b.bk_b = -1;
-  if (bucket_ok && encode_vectorised(pts, b.kA))
+  if (bucket_ok && encode_vectorised(pts, b.kA) && !(quantized && kb == 16))
     b.bk_b = std::min(bucket_bits_for<K>(n), std::min(mbits, kBkMaxBits));
   // the LSD passes' look-back words stay for keys of at most 64 bits (the
   // bucket sort hands clustered keys to the passes)
@@ -327,25 +327,42 @@ int build_launch(pgvd_ctx *ctx, const BuildBufs<K> &b, RunState *st, int32_t *oc
   CHK(launch_status("encode"));
   int parity = 0;
   bool bucket_sorted = false;
+  const RunState *decides = nullptr;   // the device decides whether the LSD passes run
   if (bucket) {
     // the bucket sort leaves keys and labels in (kA, vA)
     Stage t(ctx, "msd", s);
     BucketArgs<K> ba{kA, kB, b.vA, b.vB, labels, msd_hist, n, mbits, bk_b, prepend, b.bk,
                      g_sort_limits};
+    if (quantized) {
+      // int32 builds return without waiting for work queued before them: they
+      // poll about as long as an idle device takes to reach the plan (2^24
+      // points: some 110 us of 650), and under capture not at all; both sorts
+      // leave the keys where the LSD passes would
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      HIPCHK(hipStreamIsCapturing(s, &cs));
+      ba.poll_us = cs == hipStreamCaptureStatusNone ? 50 + n / 100000 : 0;
+      ba.out_b = n > 1 && (passes & 1);
+    }
     const int rc = launch_bucket_sort<K>(ba, st, ctx->st_host, &out.sort, ctx->sync_ev, s);
     if (rc == 2) return fail(PGVD_ERR_INTERNAL, "bucket sort: a segment outlived its levels");
     if (rc == 1) return launch_status("bucket sort") != PGVD_OK ? PGVD_ERR_HIP
                                                                   : fail(PGVD_ERR_HIP, "bucket sort");
     bucket_sorted = rc == 0;
-    // rc 3: the encoded keys are untouched
+    parity = ba.out_b;
+    if (rc == 3) out.sort = kSortLsd;
+    if (rc == 4) {
+      out.sort = kSortDevice;
+      decides = st;
+    }
+    // (where they are not sorted, the encoded keys are all in kA)
     if (!bucket_sorted)
-      launch_histogram<K>(kA, n, hist, passes, s, nullptr, sort_lb, (z.total - z.sort_lb) / 4);
+      launch_histogram<K>(kA, n, hist, passes, s, decides, sort_lb, (z.total - z.sort_lb) / 4);
   }
   if (!bucket_sorted) {
     Stage span(ctx, "sort", s, 2);
     PassTimer pt(ctx, n > 1 ? passes : 0);
     parity = launch_onesweep<K>(kA, kB, labels, b.vA, b.vB, n, passes, hist, sort_lb, st, s,
-                                pt.events(), nullptr);
+                                pt.events(), decides);
   }
   CHK(launch_status("sort"));
   K *sorted = parity ? kB : kA;
@@ -353,11 +370,11 @@ int build_launch(pgvd_ctx *ctx, const BuildBufs<K> &b, RunState *st, int32_t *oc
   // packed local splits go to the sort's other buffer, free after the sort
   uint32_t *lsx = reinterpret_cast<uint32_t *>(parity ? kA : kB);
   const uint32_t *sortedv =
-      lab ? (bucket_sorted ? b.vA : (n <= 1 ? labels : (parity ? b.vB : b.vA))) : nullptr;
+      lab ? (!bucket_sorted && n <= 1 ? labels : (parity ? b.vB : b.vA)) : nullptr;
   {
     Stage t(ctx, "unique", s);
     launch_unique<K>(sorted, sortedv, n, prepend, uniq, cbits, lb_u, st, s,
-                     bucket_sorted ? st : nullptr);
+                     bucket_sorted ? st : decides);
   }
   CHK(launch_status("unique"));
   {

@@ -394,9 +394,11 @@ struct BucketMem {
   SsTree ss;               // the sample sort's workspace
 };
 // Which sort ordered a build's keys: the LSD passes, the bucket sort alone or
-// with its levels for the crowded buckets, the sample sort (of the whole array)
-// or the bucket sort with the sample sort for the crowded buckets.
-enum SortKind { kSortLsd = 0, kSortBuckets, kSortLevels, kSortSample, kSortSampleBuckets };
+// with its levels for the crowded buckets, the sample sort (of the whole array),
+// the bucket sort with the sample sort for the crowded buckets, or the bucket
+// sort or the LSD passes as the device decided.
+enum SortKind { kSortLsd = 0, kSortBuckets, kSortLevels, kSortSample, kSortSampleBuckets,
+                kSortDevice };
 // Lower limits for tests (0: the sort's own): a larger bucket or array is too
 // large for the sample sort; a larger bucket of its own is not sorted in LDS.
 struct SortLimits {
@@ -413,6 +415,9 @@ struct BucketArgs {
   int mbits, b, prepend;
   BucketMem mem;
   SortLimits limits;
+  // >= 0: the host waits for the plan this many microseconds at most
+  int64_t poll_us = -1;
+  bool out_b = false;         // the result goes to (kB, vB), not (kA, vA)
 };
 inline constexpr size_t align256_dev(size_t x) { return (x + 255) & ~(size_t)255; }
 template <typename K> int bucket_cap();
@@ -424,8 +429,12 @@ template <typename K> void bucket_carve(void *ws, int64_t n, BucketMem &m);
 // (*kind: how); 3: the keys, of at most 64 bits, are ones that the LSD passes
 // sort faster (more than a quarter of them in buckets above CAP, and one of
 // those too large for the sample sort, or 32-bit keys past ss_max_whole):
-// nothing moved, the caller launches the passes; else a launch failed (1) or a
-// segment outlived the levels (2).
+// nothing moved, or kA holds them in another order (no labels, and a bounded
+// wait), and the caller launches the passes; 4: the wait was bounded and
+// ran out, and the device decides: the keys are sorted, and st->msd_ok set, or
+// they are all in kA (with labels, as they were), so the caller launches the
+// passes for that case (they skip themselves when msd_ok is set); else a launch failed (1) or a segment outlived
+// the levels (2).
 template <typename K>
 int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, SortKind *kind,
                        hipEvent_t ev,

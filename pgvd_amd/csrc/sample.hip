@@ -603,6 +603,7 @@ __global__ __launch_bounds__(kSsBlock) void ss_tables_kernel(const BkSeg *__rest
     o.bucket_first[nseg] = buckets;
     o.limits[0] = tiles;
     o.limits[1] = buckets;
+    st->msd_ok = 1u;   // (sorted from here on)
     if (mostly && (uint64_t)st->bk_keys * 4 > n) st->ss_ok = 1u;
   }
 }

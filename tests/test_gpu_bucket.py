@@ -6,6 +6,9 @@ sample sort or, past its limits, to further levels or the LSD passes, and on
 runs of equal keys."""
 from __future__ import annotations
 
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
@@ -191,10 +194,107 @@ def test_int32_grid_points_take_the_lsd_passes(dev):
     """Clustered int32 grid points whose largest bucket the sample sort does
     not take."""
     rng = np.random.default_rng(8)
-    q = (_clusters(200_003, 2, seed=9, sigma=1e-3) * 0.5 + 0.5) * ((1 << 20) - 1)
-    q = np.concatenate([q.astype(np.int32), rng.integers(0, 1 << 20, (1000, 2)).astype(np.int32)])
-    want = dev.build_octree(q, 20, no_host_wait=True)
-    with pgvd_amd.debug_sort_limits(segment_keys=1):
-        got = dev.build_octree(q, 20)
-    assert dev.last_sort() == "lsd" and got["bucket_sort"] == 0
-    assert_tree_equal(got, want)
+    c = (_clusters(200_003, 2, seed=9, sigma=1e-3) * 0.5 + 0.5) * ((1 << 20) - 1)
+    for more in (1000, 1_000_000):       # most of the points crowded, and a few of them
+        q = np.concatenate([c.astype(np.int32),
+                            rng.integers(0, 1 << 20, (more, 2)).astype(np.int32)])
+        want = dev.build_octree(q, 20, no_host_wait=True)
+        with pgvd_amd.debug_sort_limits(segment_keys=1):
+            got = dev.build_octree(q, 20)
+        assert dev.last_sort() in ("lsd", "device") and got["bucket_sort"] == 0
+        assert_tree_equal(got, want)
+
+
+def _grid(n, dim, bits, crowded, seed):
+    """int32 grid points, spread evenly or half of them in 8 tight clusters."""
+    rng = np.random.default_rng(seed)
+    q = rng.integers(0, 1 << bits, (n, dim)).astype(np.int32)
+    if crowded:
+        c = _clusters(n // 2, dim, seed, sigma=1e-3)
+        q[:n // 2] = ((c * 0.5 + 0.5) * ((1 << bits) - 1)).astype(np.int32)
+    return q
+
+
+INT32_CASES = [(2, 16, 4000), (2, 16, 100_003), (2, 20, 300_001), (3, 21, 200_003),
+               (3, 10, 1 << 17), (3, 30, 50_001), (2, 20, 800_001), (3, 21, 800_001),
+               (2, 16, 1_200_001)]
+
+
+@pytest.mark.parametrize("dim,bits,n", INT32_CASES)
+@pytest.mark.parametrize("labels", [False, True])
+def test_int32_build_does_not_wait_for_earlier_work(dev, dim, bits, n, labels):
+    """An int32 build returns while the stream still waits for work enqueued
+    before it (here a host function that this thread lets go afterwards), and
+    the device then chooses its sort."""
+    hip = C.CDLL("libamdhip64.so")
+    gate, late = threading.Event(), []
+    fn = C.CFUNCTYPE(None, C.c_void_p)(lambda _: late.append(1) if not gate.wait(20) else None)
+    stream = C.c_void_p()
+    dev._check(pgvd_amd.lib().pgvd_ctx_stream(dev.ctx, C.byref(stream)))
+    for crowded in (False, True):
+        q = _grid(n, dim, bits, crowded, seed=n)
+        lab = np.random.default_rng(1).integers(0, 3, n).astype(np.uint32) if labels else None
+        want = dev.build_octree(q, bits, labels=lab, no_host_wait=True)
+        dev.build_octree(q, bits, labels=lab)          # (allocates)
+        d, dl = dev.upload(q), dev.upload(lab) if labels else None
+        try:
+            gate.clear()
+            assert hip.hipLaunchHostFunc(stream, fn, None) == 0
+            dev.build_octree_async(d, n, dim, bits, dl, quantized_input=True)
+            assert not late
+            gate.set()
+            r = dev.build_octree_finish()
+            got = dev.fetch(r)
+            assert dev.last_sort() == ("lsd" if bits == 30 else "buckets" if n == 4000 else "device")
+            assert_tree_equal(got, want)
+            if labels:
+                for f in ("key_conflict", "node_conflict"):
+                    assert np.array_equal(got[f], want[f]), f
+        finally:
+            gate.set()
+            dev.synchronize()
+            d.free()
+            if labels:
+                dl.free()
+
+
+@pytest.mark.parametrize("dim,bits,n", INT32_CASES)
+def test_int32_build_under_capture(dev, dim, bits, n):
+    """An int32 build captured into a graph (its buffers allocated before) and
+    replayed on evenly spread and on clustered points, with eager work between:
+    every replay leaves the octree of the points that were there."""
+    hip = C.CDLL("libamdhip64.so")
+    stream, graph, run = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    dev._check(pgvd_amd.lib().pgvd_ctx_stream(dev.ctx, C.byref(stream)))
+    sets = [_grid(n, dim, bits, c, seed=n) for c in (False, True)]
+    want = [dev.build_octree(q, bits, no_host_wait=True) for q in sets]
+    assert not any(w["malformed"] for w in want)   # (finished on the host)
+    d = dev.upload(sets[0])
+    try:
+        for _ in range(2):
+            dev.build_octree_async(d, n, dim, bits, quantized_input=True)
+            r = dev.build_octree_finish()
+        oct_ptr, stride = r.octree, (1 << dim) + 1
+        assert hip.hipStreamBeginCapture(stream, 2) == 0      # relaxed mode
+        try:
+            dev.build_octree_async(d, n, dim, bits, quantized_input=True)
+        finally:
+            assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+        for which in (0, 1, 1, 0, 1):
+            dev._check(pgvd_amd.lib().pgvd_memcpy_htod(dev.ctx, d.ptr, sets[which].ctypes.data,
+                                                       sets[which].nbytes, None))
+            dev.synchronize()
+            assert hip.hipGraphLaunch(run, stream) == 0
+            dev.synchronize()
+            O = want[which]["octree_size"]
+            rec = dev.download(oct_ptr, np.int32, O * stride).reshape(O, stride)
+            assert np.array_equal(rec[:, :-1], want[which]["children"])
+            assert np.array_equal(rec[:, -1], want[which]["leaf"])
+    finally:
+        if run:
+            hip.hipGraphExecDestroy(run)
+        if graph:
+            hip.hipGraphDestroy(graph)
+        d.free()
+    assert_tree_equal(dev.build_octree(sets[1], bits), want[1])
