@@ -294,25 +294,114 @@ __device__ inline void lds_rank(const K (&k)[IPT], const uint32_t (&v)[IPT], uin
     }
 }
 
+// ---- LDS sort by splitters -------------------------------------------------------
+// Sorts the cnt <= BS IPT pairs (k[j], v[j]) at index i = j BS + threadIdx.x in
+// LDS, whatever their distribution: 255 splitters, evenly spaced positions of
+// the input ranked against each other, bound 256 buckets; every key finds its
+// bucket (8 LDS reads), and its rank within the bucket by reading the others
+// in it (cnt / 256 on average).  Keys compare together with their index, so
+// equal keys spread over buckets like distinct ones.  pick(i) reads key i.  On
+// return (no barrier passed since) s_keys / s_vals hold the pairs in order;
+// s_tmp: split_words<K>() words, aligned as K.
+constexpr int kSplits = 256;
+template <typename K>
+constexpr int split_words() { return kSplits * ((int)sizeof(K) / 4 + 3) + 1 + 16; }
+
+template <typename K, bool LAB, int BS, int IPT, typename Pick>
+__device__ inline void lds_split_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cnt, Pick pick,
+                                      K *s_keys, uint32_t *s_vals, uint32_t *s_tmp) {
+  constexpr int NW = BS / 64, PARTS = BS / kSplits, PER = kSplits / PARTS;
+  static_assert(BS % kSplits == 0 && NW <= 16, "every thread ranks against a part");
+  K *s_sp = reinterpret_cast<K *>(s_tmp);              // splitters as picked, then in order
+  uint32_t *s_pos = s_tmp + kSplits * (int)sizeof(K) / 4;   // their indexes, in order
+  uint32_t *s_cnt = s_pos + kSplits;                   // their ranks, then the buckets' counts
+  uint32_t *s_start = s_cnt + kSplits;                 // kSplits + 1
+  uint32_t *s_w = s_start + kSplits + 1;
+  const uint32_t t = threadIdx.x;
+  const uint32_t pos = (t & (kSplits - 1)) * cnt / kSplits;
+  K mine = kzero_value<K>();
+  if (t < kSplits) {
+    mine = pick(pos);
+    s_sp[t] = mine;
+    s_cnt[t] = 0;
+  }
+  __syncthreads();
+  {
+    const uint32_t j = t & (kSplits - 1), i0 = t / kSplits * PER;
+    const K x = s_sp[j];
+    uint32_t r = 0;
+#pragma unroll 8
+    for (uint32_t i = i0; i < i0 + PER; ++i) {
+      const K y = s_sp[i];
+      r += (kless(y, x) || (keq(y, x) && i < j)) ? 1u : 0u;
+    }
+    atomicAdd(&s_cnt[j], r);
+  }
+  __syncthreads();
+  if (t < kSplits) {
+    const uint32_t r = s_cnt[t];
+    s_sp[r] = mine;
+    s_pos[r] = pos;
+    s_cnt[t] = 0;
+  }
+  __syncthreads();
+  uint32_t lo[IPT], rs[IPT];
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) lo[j] = 0;
+  // (every key's search at once: their reads are independent)
+#pragma unroll
+  for (uint32_t step = kSplits / 2; step >= 1; step >>= 1) {
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      if ((uint32_t)j * BS >= cnt) break;   // uniform
+      const uint32_t at = lo[j] + step;
+      const K y = s_sp[at];
+      const bool le = kless(y, k[j]) || (keq(y, k[j]) && s_pos[at] <= (uint32_t)j * BS + t);
+      lo[j] = le ? at : lo[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < IPT; ++j)
+    rs[j] = (uint32_t)j * BS + t < cnt ? atomicAdd(&s_cnt[lo[j]], 1u) : 0u;
+  __syncthreads();
+  uint32_t total;
+  const uint32_t ex = block_excl_sum<uint32_t, NW>(t < kSplits ? s_cnt[t] : 0u, s_w, &total);
+  if (t < kSplits) s_start[t] = ex;
+  if (t == 0) s_start[kSplits] = total;
+  __syncthreads();
+  uint32_t b1[IPT];
+#pragma unroll
+  for (int j = 0; j < IPT; ++j)
+    if ((uint32_t)j * BS + t < cnt) {
+      b1[j] = s_start[lo[j] + 1];
+      lo[j] = s_start[lo[j]];
+      rs[j] += lo[j];
+      s_keys[rs[j]] = k[j];
+    }
+  __syncthreads();
+  lds_rank<K, LAB, BS, IPT>(k, v, cnt, rs, lo, b1, s_keys, s_vals);
+}
+
 // ---- LDS sort by bins -------------------------------------------------------------
 // Sorts in LDS the cnt <= BS IPT pairs (k[j], v[j]) at index i = j BS +
 // threadIdx.x, for keys that are spread smoothly for the most part: counted in
 // 4096 bins of their range (the keys less the smallest); where some bin holds
 // more than kBinRank of them, every bin is cut into as many bins as it holds
 // keys (rounded down to a power of two) and the keys are counted again; then
-// each key is ranked within its bin.  A bin of more than kBinRank2 keys that are
-// all the same (many points at one place) needs no ranking; keys too close
-// together even for that (a range that spans two tight clusters) go to the
-// merge sort, which took 60 us for 8192 64-bit keys where ranking against 256
-// splitters took 117.  pick(i) and vpick(i) read pair i again.  On return (no
-// barrier passed since) s_keys / s_vals hold the pairs in order, equal keys in
-// any order; s_tmp: bin_words<K, BS>() words, aligned as K.
-// kBinRank 12, 24 and 48 time alike.  kBinRank2 128 against 64: 300,000 2D
-// points at 20 bits/axis in clusters of sigma 0.003 166 against 179 us, others
-// alike; at 256 the same points in 3D take 10% longer.
+// each key is ranked within its bin.  A bin of more than RANK2 keys that are all
+// the same (many points at one place) needs no ranking; keys too close together
+// even for that (a range that spans two tight clusters) go to the merge sort
+// (MERGE) or are ranked against splitters.  The merge sort is the better one for
+// many keys a thread (8192 64-bit keys of 1024 threads 60 us, by splitters 117;
+// the 512-thread sorts of a batch of 384 instances 487 and 507 us), the splitters
+// for few (300,007 clustered points, 1024 threads a bucket: 33.6 and 29.7 us)
+// and for 128-bit keys (2^22 labelled loop samples: 159 and 151 us), each with
+// the RANK2 that suited it of 64 and 128; kBinRank 12, 24 and 48 time alike.
+// pick(i) and vpick(i) read pair i again.  On return (no barrier passed since)
+// s_keys / s_vals hold the pairs in order, equal keys in any order; s_tmp:
+// bin_words<K, BS>() words, aligned as K.
 constexpr int kBins = 4096;
 constexpr uint32_t kBinRank = 24;
-constexpr uint32_t kBinRank2 = 128;
 template <typename K, int BS>
 constexpr int bin_words() {
   return kBins + 4 + 2 * (BS / 64) * ((int)sizeof(K) / 4) + 2 * (BS / 64);
@@ -330,12 +419,14 @@ __device__ inline uint32_t block_max(uint32_t v, uint32_t *s_mx) {
   return v;
 }
 
-template <typename K, bool LAB, int BS, int IPT, typename Pick, typename VPick>
+template <typename K, bool LAB, int BS, int IPT, bool MERGE, typename Pick, typename VPick>
 __device__ inline void lds_bin_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cnt, Pick pick,
                                     VPick vpick, K *s_keys, uint32_t *s_vals, uint32_t *s_tmp) {
   constexpr int NW = BS / 64, PER = kBins / BS;
+  constexpr uint32_t RANK2 = MERGE ? 128 : 64;
   constexpr int kMid = kBins + 4;
-  static_assert(2 * BS * IPT <= 4 * kMid, "the merge sort's positions fit");
+  static_assert(2 * BS * IPT <= 4 * kMid && split_words<K>() <= kMid,
+                "the other sorts' tables fit");
   uint32_t *s_bin = s_tmp;
   K *s_mm = reinterpret_cast<K *>(s_tmp + kMid);
   uint32_t *s_w = s_tmp + kMid + 2 * NW * ((int)sizeof(K) / 4), *s_mx = s_w + NW;
@@ -446,18 +537,21 @@ __device__ inline void lds_bin_sort(K (&k)[IPT], uint32_t (&v)[IPT], uint32_t cn
   for (int j = 0; j < IPT; ++j)
     if ((uint32_t)j * BS + t < cnt) s_keys[at[j]] = k[j];
   __syncthreads();
-  if (most > kBinRank2) {   // uniform
+  if (most > RANK2) {   // uniform
     // a crowded bin of one key's copies is in order as it is
     uint32_t mixed = 0;
 #pragma unroll
     for (int j = 0; j < IPT; ++j)
-      if ((uint32_t)j * BS + t < cnt && b1[j] - b0[j] > kBinRank2) {
+      if ((uint32_t)j * BS + t < cnt && b1[j] - b0[j] > RANK2) {
         mixed |= keq(k[j], s_keys[b0[j]]) ? 0u : 1u;
         b0[j] = b1[j] = at[j];
       }
     if (block_max<BS>(mixed, s_mx)) {
-      lds_merge_sort<K, LAB, BS, IPT>(pick, vpick, cnt, s_keys, s_vals,
-                                      reinterpret_cast<uint16_t *>(s_tmp));
+      if constexpr (!MERGE)
+        lds_split_sort<K, LAB, BS, IPT>(k, v, cnt, pick, s_keys, s_vals, s_tmp);
+      else
+        lds_merge_sort<K, LAB, BS, IPT>(pick, vpick, cnt, s_keys, s_vals,
+                                        reinterpret_cast<uint16_t *>(s_tmp));
       return;
     }
   }

@@ -102,8 +102,8 @@ __global__ __launch_bounds__(kSsBlock) void ss_splitters_kernel(const K *__restr
     k[j] = i < S ? sample(i) : kzero_value<K>();
     v[j] = 0;
   }
-  lds_bin_sort<K, false, kSsBlock, IPT>(k, v, S, sample, [](uint32_t) { return 0u; }, s_keys,
-                                        nullptr, s_tmp);
+  lds_bin_sort<K, false, kSsBlock, IPT, (IPT > 4)>(
+      k, v, S, sample, [](uint32_t) { return 0u; }, s_keys, nullptr, s_tmp);
   __syncthreads();
   // splitter j = sample 16 j; the second of a run of equal ones becomes the
   // run's successor, which closes the repeated key's own bucket
@@ -332,8 +332,9 @@ __global__ __launch_bounds__(BS) void ss_sort_kernel(const K *kin, const uint32_
     k[j] = i < cnt ? in[s0 + i] : kzero_value<K>();
     v[j] = (LAB && i < cnt) ? lin[s0 + i] : 0u;
   }
-  lds_bin_sort<K, LAB, BS, IPT>(k, v, cnt, [&](uint32_t i) { return in[s0 + i]; },
-                                [&](uint32_t i) { return lin[s0 + i]; }, s_keys, s_vals, s_tmp);
+  lds_bin_sort<K, LAB, BS, IPT, (BS == 512 && sizeof(K) <= 8)>(
+      k, v, cnt, [&](uint32_t i) { return in[s0 + i]; }, [&](uint32_t i) { return lin[s0 + i]; },
+      s_keys, s_vals, s_tmp);
   __syncthreads();   // (every read of a bucket sorted in place is done too)
   bool dup = false;
 #pragma unroll
