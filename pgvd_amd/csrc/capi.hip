@@ -108,9 +108,6 @@ size_t pgvd_capi::plain_footprint_bytes(int64_t n, int dim, int bits, bool label
   b += kBboxPartBytes;                                   // bbox_part
   b += kb == 4 ? bucket_ws_bytes<uint32_t>(n)            // the bucket sort's workspace
                 : (kb == 8 ? bucket_ws_bytes<uint64_t>(n) : bucket_ws_bytes<Key128>(n));
-  if (kb == 4 && n > bucket_cap<uint32_t>()) b += ss_tree_bytes<uint32_t>(n);   // and the
-  if (kb == 8 && n > bucket_cap<uint64_t>()) b += ss_tree_bytes<uint64_t>(n);   // sample sort's
-  if (kb == 16 && n > bucket_cap<Key128>()) b += ss_tree_bytes<Key128>(n);
   b += (size_t)((nk + kBlock - 1) / kBlock) * 4;         // chunks
   b += zero_layout(n, kb, (mbits + 7) / 8, labels).total;
   b += (size_t)oct_nodes * ((1u << dim) + 1) * 4;        // octree
@@ -251,8 +248,11 @@ int carve_build(Get &&get, const void *pts, int64_t n, int dim, int bits, bool l
     CHK(get("bucket_ws", bucket_ws_bytes<K>(n), &p));
     bucket_carve<K>(p, n, b.bk);
     if (n > bucket_cap<K>()) {   // else no bucket can be crowded
-      CHK(get("sample_ws", ss_tree_bytes<K>(n), &p));
-      ss_tree_carve<K>(p, n, b.bk.ss);
+      // the sample sort's workspace lies in the BRT's nodes, which are written
+      // after the sort (12, 16 or 24 bytes a key; the workspace takes 3 to 6)
+      if (ss_tree_bytes<K>(n) > (size_t)nk * brt_node_bytes<K>())
+        return fail(PGVD_ERR_INTERNAL, "the sample sort's workspace outgrew the BRT");
+      ss_tree_carve<K>(b.brt, n, b.bk.ss);
     }
   }
   return PGVD_OK;

@@ -94,3 +94,12 @@ def test_key_word_layout_roundtrip():
             assert np.array_equal(a, lo)
         else:
             assert np.array_equal(a, lo & np.uint64(0xFFFFFFFF))
+
+
+def test_footprint_holds_no_sort_workspace_beside_the_tree():
+    """A build's admission size: keys, BRT, prefix sums, octree, the bucket
+    sort's lists.  The sample sort's workspace lies in the BRT's nodes, so it
+    adds nothing: 145, 91 and 182 bytes a key as without it."""
+    foot = P.lib().pgvd_build_footprint
+    for n, dim, bits, per_key in ((1 << 24, 3, 21, 145), (1_000_000, 2, 16, 91), (1 << 22, 3, 42, 182)):
+        assert foot(n, dim, bits) <= per_key * n

@@ -120,3 +120,26 @@ def test_injected_failure_of_a_stage_entry(dev):
     want = oracle.find_leaf(q, 21, t["children"], t["leaf"])
     for k in ("parent", "octant", "data", "level", "status"):
         assert np.array_equal(np.asarray(got[k]).astype(np.int64), np.asarray(want[k]).astype(np.int64)), k
+
+
+@pytest.mark.parametrize("dim,bits", [(2, 16), (3, 21), (3, 42)])
+def test_clustered_builds_fit_the_pool_of_spread_ones(dev, dim, bits):
+    """Whatever sorts a build's keys, its pool is the same: with the limit at
+    what a build of spread points holds, builds of clustered ones, whole and in
+    part, succeed and are right."""
+    n = 300000
+    rng = np.random.default_rng(3)
+    pts = rng.random((n, dim), dtype=np.float32) * 2 - 1
+    with P.Device(0) as d:
+        d.build_octree(pts, bits)
+        held = d.pool_bytes()
+        # (each buffer is rounded up to 256 bytes)
+        assert held <= P.Server.footprint(n, dim, bits) - n * dim * 4 + 8192
+        d.set_pool_limit(held)
+        for k in (n // 8, n):
+            q = pts.copy()
+            q[2:k] = 0.3 + rng.standard_normal((max(k - 2, 0), dim)).astype(np.float32) * 1e-3
+            got = d.build_octree(q, bits)
+            assert "sample" in d.last_sort() or (bits, k) == (16, n)
+            assert_tree_equal(got, dev.build_octree(q, bits, no_host_wait=True))
+            assert d.pool_bytes() == held
