@@ -164,9 +164,12 @@ int pgvd_points_to_morton(pgvd_ctx *ctx, const void *pts, int coord_bytes, int64
  *           throws); 2 when a child index leaves the octree (not one the
  *           build wrote).
  * 1 <= bits <= 31.  A batch of at least 2^22 queries in 3D or 2^21 in 2D
- * (fewer when bits is small) first tabulates the octree's cells at depth 7
- * (3D) or 10 (2D) in a 16 MB (8 MB) buffer the context owns: such calls on
- * one context on different streams must not overlap. */
+ * (fewer when bits is small) first tabulates the octree's cells, at depth 7
+ * (3D) or 10 (2D) or less in a small octree, in a 16 MB (8 MB) buffer the
+ * context owns: such calls on one context on different streams must not
+ * overlap.  On the context's own stream (outside stream capture, and without a
+ * pool limit) batches from 2^18 queries on do, in a buffer that no other call
+ * uses. */
 int pgvd_find_leaf(pgvd_ctx *ctx, const int32_t *pts, int64_t q, int dim, int bits,
                    const int32_t *octree, int64_t octree_size, int32_t *parent, int32_t *octant,
                    int32_t *data, int32_t *level, uint32_t *status, pgvd_stream s);

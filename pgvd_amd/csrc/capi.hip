@@ -969,9 +969,21 @@ int pgvd_find_leaf(pgvd_ctx *ctx, const int32_t *pts, int64_t q, int dim, int bi
   if (q == 0) return PGVD_OK;
   CHK(use_device(ctx));
   hipStream_t st = pick(ctx, s);
-  const int D = find_leaf_table_depth(q, dim, bits, octree_size);
+  int D = find_leaf_table_depth(q, dim, bits, octree_size);
   void *table = nullptr;
-  if (D > 0) CHK(pool_get(ctx, "find_leaf_table", size_t(8) << (D * dim), &table));
+  const int full = std::min(kFindLeafTableBits / dim, bits) * dim;   // the largest table's bits
+  if (D > 0 && q >= (int64_t(2) << full)) {
+    CHK(pool_get(ctx, "find_leaf_table", size_t(8) << full, &table));
+  } else if (D > 0) {
+    // Smaller batches may run on several streams at once, be captured with
+    // nothing allocated before, and need nothing of the pool.  They share a
+    // table only where none of that can be: on the context's own stream.
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (st != ctx->stream || ctx->pool_limit) D = 0;
+    else HIPCHK(hipStreamIsCapturing(st, &cs));
+    if (cs != hipStreamCaptureStatusNone) D = 0;
+    if (D > 0 && pool_get(ctx, "find_leaf_own", size_t(8) << kFindLeafTableBits, &table)) D = 0;
+  }
   Stage t(ctx, "find_leaf", st);
   launch_find_leaf(pts, q, dim, bits, octree, octree_size, table, D, parent, octant, data, level,
                    status, st);

@@ -187,7 +187,8 @@ int launch_onesweep(K *keys, K *keys_alt, const uint32_t *vals_in, uint32_t *val
 // ---- query.hip ----
 // OctreeUtils::FindLeaf for q int32 grid points (see pgvd_find_leaf).  With
 // D > 0 the launch first fills `table` (at most 8 << (D * dim) bytes) with the
-// octree's cells at depth D; find_leaf_table_depth picks D (0: no table).
+// octree's cells at depth D; find_leaf_table_depth picks D (0: no table), at
+// most kFindLeafTableBits / dim.
 constexpr int kFindLeafTableBits = 21;
 int find_leaf_table_depth(int64_t q, int dim, int bits, int64_t octree_size);
 void launch_find_leaf(const int32_t *pts, int64_t q, int dim, int bits, const int32_t *octree,

@@ -461,12 +461,10 @@ def test_find_leaf_matches_oracle(dev, dim, bits, n):
     """OctreeUtils::FindLeaf batched on the GPU against the oracle's
     restatement (pinned by brute force), on the octree the GPU built: the
     build's own points and random grid points, every output field.  Batches
-    of at least twice the cell count at the table depth (2^21 cells in 3D,
-    2^20 in 2D, fewer when bits is small) start from the depth table: here
-    3D 21 bits at 2^22 points, 2D 16 bits at 2^21 points, and 3D 5 bits and
-    2D 2 bits, where the table covers every level; 3D 23 bits (69-bit keys:
-    the table index straddles the two key words) and 31 bits (93-bit keys:
-    the index in the high word)."""
+    of 2^18 queries and more start from a depth table (2^21 cells in 3D, 2^20
+    in 2D at most, and four per node): here at 2^20 points and more; 3D 23
+    bits (69-bit keys: the table index straddles the two key words) and 31
+    bits (93-bit keys: the index in the high word)."""
     rng = np.random.default_rng(dim * 31 + bits)
     pts = _pts(n, dim, seed=dim * 7 + bits)
     tree = dev.build_octree(pts, bits)
@@ -479,10 +477,10 @@ def test_find_leaf_matches_oracle(dev, dim, bits, n):
     assert (want["status"] == 0).all() and (want["level"] > 1).any()
 
 
-@pytest.mark.parametrize("reps", [1, 4])
+@pytest.mark.parametrize("reps", [1, 4, 100000])
 def test_find_leaf_rejects_foreign_child_index(dev, reps):
     """A child index outside the octree stops the descent with status 2 (the
-    oracle agrees) instead of reading past the nodes; with 12 queries the
+    oracle agrees) instead of reading past the nodes; with 300,000 queries the
     descent starts from the depth table, which records the stop."""
     children = np.array([[3, -1, -1, -1], [-1, -1, -1, -1]], np.int32)   # node 0 -> node 3 of 2
     leaf = np.array([0b1110, 0b1111], np.int32)
@@ -528,6 +526,70 @@ def test_find_leaf_table_of_any_octree(dev, dim, nodes):
         assert np.array_equal(got[k].astype(np.int64), want[k].astype(np.int64)), k
     assert set(np.unique(want["status"])) >= {0, 2}
     assert (want["data"][want["status"] == 0] >= 0).any()
+
+
+@pytest.mark.parametrize("dim,bits", [(2, 12), (3, 10)])
+def test_find_leaf_on_several_streams(dev, dim, bits):
+    """Batches of 2^19 queries, each in its own octree, on two streams at once:
+    below the sizes whose table the context shares they have none to share,
+    take nothing of the pool, and run in a captured graph with nothing
+    allocated before.  (On the context's own stream they have a table.)"""
+    hip = C.CDLL("libamdhip64.so")
+    q = 1 << 19
+    names = ("parent", "octant", "data", "level", "status")
+    with P.Device(0) as d:
+        jobs = []
+        for j, n in enumerate((300, 60000)):
+            tree = dev.build_octree(_pts(n, dim, seed=j), bits)
+            pts = np.random.default_rng(j).integers(0, 1 << bits, (q, dim)).astype(np.int32)
+            oct_ = np.concatenate([tree["children"], tree["leaf"][:, None]], axis=1).astype(np.int32)
+            stream = C.c_void_p()
+            assert hip.hipStreamCreate(C.byref(stream)) == 0
+            jobs.append(dict(stream=stream, pts=d.upload(pts), oct=d.upload(oct_), size=len(oct_),
+                             outs={k: d.alloc(4 * q) for k in names},
+                             want=oracle.find_leaf(pts, bits, tree["children"], tree["leaf"])))
+
+        def call(job, stream):
+            o = job["outs"]
+            d._check(P.lib().pgvd_find_leaf(
+                d.ctx, job["pts"].ptr, q, dim, bits, job["oct"].ptr, job["size"], o["parent"].ptr,
+                o["octant"].ptr, o["data"].ptr, o["level"].ptr, o["status"].ptr, stream))
+
+        def check(job):
+            for k in names:
+                got = d.download(job["outs"][k], np.int32, q)
+                assert np.array_equal(got.astype(np.int64), job["want"][k].astype(np.int64)), k
+
+        held = d.pool_bytes()
+        graph, run = C.c_void_p(), C.c_void_p()
+        s0 = jobs[0]["stream"]
+        assert hip.hipStreamBeginCapture(s0, 0) == 0          # global mode: no allocation
+        call(jobs[0], s0)
+        assert hip.hipStreamEndCapture(s0, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+        for _ in range(6):
+            assert hip.hipGraphLaunch(run, s0) == 0
+            call(jobs[1], jobs[1]["stream"])
+        assert hip.hipDeviceSynchronize() == 0
+        for job in jobs:
+            check(job)
+        assert d.pool_bytes() == held
+        for job in jobs:
+            call(job, None)
+        assert d.pool_bytes() > held
+        d.synchronize()
+        for job in jobs:
+            check(job)
+        d.set_pool_limit(held)
+        call(jobs[0], None)
+        d.synchronize()
+        check(jobs[0])
+        hip.hipGraphExecDestroy(run)
+        hip.hipGraphDestroy(graph)
+        for job in jobs:
+            hip.hipStreamDestroy(job["stream"])
+            for b in (job["pts"], job["oct"], *job["outs"].values()):
+                b.free()
 
 
 # ----------------------------------------------------- reference data ----
