@@ -189,8 +189,8 @@ int pgvd_find_leaf(pgvd_ctx *ctx, const int32_t *pts, int64_t q, int dim, int bi
  *            (the reference throws; the first 10000 are kept).
  * *total_out (host) receives the number of cells; PGVD_ERR_CAPACITY when
  * it exceeds capacity (offsets and status are then valid).  With a cell
- * buffer, one walk counts and keeps each segment's first cells (32; up to
- * 1024 for few segments) in a scratch buffer the context owns (up to 2 GB;
+ * buffer, one walk counts and keeps each segment's first cells (32; without
+ * a pool limit up to 1024 for few segments) in a scratch buffer the context owns (up to 2 GB;
  * past that, a count walk and a write walk), and only segments with more
  * cells walk again.  Returns
  * after the count is read back; the rest is asynchronous on the stream.

@@ -1016,12 +1016,10 @@ int pgvd_cell_walk(pgvd_ctx *ctx, const float *segs, int64_t n, int bits, const 
   // or more for few segments; up to 2 GB of scratch, or PGVD_WALK_SCRATCH_BYTES from the
   // environment), so that only longer walks run twice; past that, a count
   // walk and a write walk.
-  const int log2k = walk_log2_kept(n);
-  const size_t spec_bytes = (static_cast<size_t>(n) << log2k) * 16;
+  int log2k = 5;
   size_t spec_limit = size_t(2) << 30;
   if (const char *e = std::getenv("PGVD_WALK_SCRATCH_BYTES")) spec_limit = std::strtoull(e, nullptr, 10);
-  if (cells && spec_bytes <= spec_limit)
-    CHK(pool_get(ctx, "walk_scratch", spec_bytes, &scratch));
+  if (cells) CHK(walk_scratch(ctx, n, spec_limit, &log2k, &scratch));
   int64_t total = 0;
   {
     Stage t(ctx, "cell_walk_count", st);

@@ -155,6 +155,23 @@ inline int pool_get(pgvd_ctx *ctx, const char *key, size_t bytes, void **out) {
   return PGVD_OK;
 }
 
+// The scratch a walk of n segments keeps its first cells in, 16 bytes each, of
+// at most `limit` bytes (*scratch null: none): 32 cells a segment, or more for
+// few segments (walk_log2_kept) where the pool has no limit and the device room.
+inline int walk_scratch(pgvd_ctx *ctx, int64_t n, size_t limit, int *log2k, void **scratch) {
+  *scratch = nullptr;
+  const int more = ctx->pool_limit ? 5 : pgvd::walk_log2_kept(n);
+  for (*log2k = more;; *log2k = 5) {
+    const size_t bytes = (static_cast<size_t>(n) << *log2k) * 16;
+    if (bytes <= limit) {
+      const int rc = pool_get(ctx, "walk_scratch", bytes, scratch);
+      if (rc == PGVD_OK || *log2k == 5) return rc;
+    } else if (*log2k == 5) {
+      return PGVD_OK;
+    }
+  }
+}
+
 inline hipEvent_t take_event(pgvd_ctx *ctx) {
   if (!ctx->spare.empty()) {
     hipEvent_t e = ctx->spare.back();

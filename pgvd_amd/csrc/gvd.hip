@@ -444,12 +444,12 @@ __global__ __launch_bounds__(kBlock) void fit_count_kernel(const float *__restri
     FitSink<false> o{nullptr, nullptr, nullptr, nullptr, nullptr};
     int rc = 0;
     if (fit_item<FROM_CI>(src, i, A, B)) {
-      const uint32_t chunk = atomicAdd(&res->kept, 1u);
+      const uint32_t chunk = keep.chunks ? atomicAdd(&res->kept, 1u) : 0u;
       if (chunk < keep.chunks) o.keep = keep.rec + (int64_t)chunk * (2 * kFitKept);
       rc = fit_boxes(A, B, min_d, o);
       const bool kept = o.keep && o.nb <= kFitKept;
       if (chunk < keep.chunks) keep.owner[chunk] = kept ? (uint32_t)i : ~0u;
-      if (!kept) keep.rest[atomicAdd(&res->rest, 1u)] = (uint32_t)i;
+      if (!kept && keep.rest) keep.rest[atomicAdd(&res->rest, 1u)] = (uint32_t)i;
     }
     ns[i] = (uint32_t)o.ns;
     nb[i] = (uint32_t)o.nb;
@@ -479,14 +479,17 @@ __global__ __launch_bounds__(kBlock) void fit_move_kernel(
   o.box(mk(q.x, q.y), q.z);
 }
 
-// The items that were not kept, from the beginning.
+// The items that were not kept (rest, or all n of them that found something),
+// from the beginning.
 template <bool FROM_CI>
 __global__ __launch_bounds__(kBlock) void fit_rest_kernel(
     const float *__restrict__ src, const uint32_t *__restrict__ rest, uint32_t n, float min_d,
-    const int64_t *__restrict__ soff, const int64_t *__restrict__ boff, float *__restrict__ samples,
+    const int64_t *__restrict__ soff, const int64_t *__restrict__ boff,
+    const uint32_t *__restrict__ ns, float *__restrict__ samples,
     float *__restrict__ origins, float *__restrict__ lengths, int32_t *__restrict__ extra) {
   for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < n; k += gridDim.x * kBlock) {
-    const int64_t i = rest[k];
+    const int64_t i = rest ? rest[k] : k;
+    if (ns[i] == 0) continue;
     seg2 A, B;
     if (!fit_item<FROM_CI>(src, i, A, B)) continue;
     FitSink<true> o{samples, origins, lengths, extra, nullptr};
@@ -779,11 +782,11 @@ void launch_fit_write(const float *src, bool from_ci, float min_d, const int64_t
         keep, kept, soff, boff, ns, nb, samples, origins, lengths, extra);
   if (!rest) return;
   if (from_ci)
-    fit_rest_kernel<true><<<grid_for(rest), kBlock, 0, s>>>(src, keep.rest, rest, min_d, soff, boff,
+    fit_rest_kernel<true><<<grid_for(rest), kBlock, 0, s>>>(src, keep.rest, rest, min_d, soff, boff, ns,
                                                             samples, origins, lengths, extra);
   else
-    fit_rest_kernel<false><<<grid_for(rest), kBlock, 0, s>>>(src, keep.rest, rest, min_d, soff,
-                                                             boff, samples, origins, lengths, extra);
+    fit_rest_kernel<false><<<grid_for(rest), kBlock, 0, s>>>(src, keep.rest, rest, min_d, soff, boff, ns,
+                                                             samples, origins, lengths, extra);
 }
 
 }  // namespace pgvd

@@ -39,9 +39,8 @@ int walk_pooled(pgvd_ctx *ctx, const float *segs, int64_t n, int bits, const int
   CHK(pool_get(ctx, "mc_offsets", 8 * static_cast<size_t>(n + 1), &offsets));
   CHK(pool_get(ctx, "walk_counts", 4 * static_cast<size_t>(n), &counts));
   CHK(pool_get(ctx, "walk_ws", 8 * static_cast<size_t>(walk_scan_ws_words(n)), &ws));
-  const int log2k = walk_log2_kept(n);
-  const size_t spec_bytes = (static_cast<size_t>(n) << log2k) * 16;
-  if (spec_bytes <= (size_t(2) << 30)) CHK(pool_get(ctx, "walk_scratch", spec_bytes, &scratch));
+  int log2k = 5;
+  CHK(walk_scratch(ctx, n, size_t(2) << 30, &log2k, &scratch));
   {
     Stage t(ctx, "gvd_walk", st);
     launch_cell_walk_count(segs, n, bits, octree, O, static_cast<uint32_t *>(counts), status,
@@ -104,7 +103,8 @@ struct FitWork {
   int64_t items = 0;
 };
 
-// At most 64 MB of records; more items than chunks are worked out twice.
+// At most 64 MB of records; more items than chunks are worked out twice, and
+// all of them under a pool limit or where the device has no room for records.
 constexpr int64_t kFitChunks = 1 << 16;
 
 int fit_result(pgvd_ctx *ctx, FitWork *w) {
@@ -127,15 +127,16 @@ int fit_count(pgvd_ctx *ctx, const float *src, bool from_ci, int64_t items, floa
   if (!sample_offsets) CHK(pool_get(ctx, "fit_soff", 8 * (m + 1), &soff));
   if (!box_offsets) CHK(pool_get(ctx, "fit_boff", 8 * (m + 1), &boff));
   CHK(pool_get(ctx, "fit_ws", 16 * static_cast<size_t>(walk_scan_ws_words(items)), &ws));
-  CHK(pool_get(ctx, "fit_rec", 32 * kFitKept * chunks, &rec));
-  CHK(pool_get(ctx, "fit_owner", 4 * chunks, &owner));
-  CHK(pool_get(ctx, "fit_rest", 4 * m, &rest));
+  const bool keep = !ctx->pool_limit && !pool_get(ctx, "fit_rec", 32 * kFitKept * chunks, &rec) &&
+                    !pool_get(ctx, "fit_owner", 4 * chunks, &owner) &&
+                    !pool_get(ctx, "fit_rest", 4 * m, &rest);
   w->ns = static_cast<uint32_t *>(ns);
   w->nb = static_cast<uint32_t *>(nb);
   w->so = sample_offsets ? sample_offsets : static_cast<int64_t *>(soff);
   w->bo = box_offsets ? box_offsets : static_cast<int64_t *>(boff);
-  w->keep = FitKeep{static_cast<float4 *>(rec), static_cast<uint32_t *>(owner),
-                    static_cast<uint32_t *>(rest), static_cast<uint32_t>(chunks)};
+  if (keep)
+    w->keep = FitKeep{static_cast<float4 *>(rec), static_cast<uint32_t *>(owner),
+                      static_cast<uint32_t *>(rest), static_cast<uint32_t>(chunks)};
   w->items = items;
   if (items > 0) {
     Stage t(ctx, "gvd_fit_count", st);
@@ -168,8 +169,8 @@ int fit_write(pgvd_ctx *ctx, const FitWork &w, const float *src, bool from_ci, f
               int32_t *extra, float *samples, float *origins, float *lengths, hipStream_t st) {
   if (w.items == 0) return PGVD_OK;
   Stage t(ctx, "gvd_fit_write", st);
-  launch_fit_write(src, from_ci, min_d, w.so, w.bo, w.ns, w.nb, w.keep, w.host.kept, w.host.rest,
-                   samples, origins, lengths, extra, st);
+  launch_fit_write(src, from_ci, min_d, w.so, w.bo, w.ns, w.nb, w.keep, w.host.kept,
+                   w.keep.rest ? w.host.rest : static_cast<uint32_t>(w.items), samples, origins, lengths, extra, st);
   HIPCHK(hipGetLastError());
   return PGVD_OK;
 }

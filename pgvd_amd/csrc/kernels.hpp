@@ -257,7 +257,7 @@ struct FitResult {
 struct FitKeep {
   float4 *rec;                 // chunks x kFitKept x 2
   uint32_t *owner;             // chunks: the item, or ~0
-  uint32_t *rest;              // items
+  uint32_t *rest;              // items (null: nothing is kept, the write pass takes them all)
   uint32_t chunks;
 };
 void launch_fit_count(const float *src, bool from_ci, int64_t items, float min_d, uint32_t *ns,

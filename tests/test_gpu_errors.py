@@ -11,6 +11,7 @@ import pytest
 import oracle
 import pgvd_amd as P
 from conftest import assert_tree_equal
+from pgvd_amd import workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -143,3 +144,51 @@ def test_clustered_builds_fit_the_pool_of_spread_ones(dev, dim, bits):
             assert "sample" in d.last_sort() or (bits, k) == (16, n)
             assert_tree_equal(got, dev.build_octree(q, bits, no_host_wait=True))
             assert d.pool_bytes() == held
+
+
+def test_walks_and_refinement_keep_no_more_than_they_must_under_a_limit(dev):
+    """Under a pool limit a walk keeps 32 cells a segment and FitBoxes keeps no
+    results: the pool of a few long walks stays below 1 MB (8 MB of kept cells
+    without a limit), a refinement's below its unlimited one by the records'
+    megabytes; the results are the same, also with the limit at what they
+    hold."""
+    bits, n = 12, 500
+    rng = np.random.default_rng(4)
+    tree = dev.build_octree(_pts(20000, 2, 5), bits)
+    W = 1 << bits
+    a = rng.random((n, 2)) * (W - 1e-3)
+    b = np.clip(a + (rng.random((n, 2)) * 2 - 1) * 0.5 * W, 0, W - 1e-3)
+    segs = np.concatenate([a, b], axis=1).astype(np.float32)
+    want = dev.cell_walk(segs, bits, tree["children"], tree["leaf"])
+    verts, counts = workloads.polyline_scene(60, 2, 3, 0.01)
+    ref = dev.gvd_refine(verts, counts, 14, 6)
+    assert ref["extra"].size or sum(ref["extra_per_iteration"])
+    with P.Device(0) as d:
+        d.set_pool_limit(1 << 20)
+        got = d.cell_walk(segs, bits, tree["children"], tree["leaf"])
+        for k in want:
+            assert np.array_equal(got[k], want[k]), k
+    held = []
+    for limit in (0, 1 << 40, None):
+        with P.Device(0) as d:
+            d.set_pool_limit(held[-1] if limit is None else limit)
+            got = d.gvd_refine(verts, counts, 14, 6)
+            held.append(d.pool_bytes())
+        for k in ref:
+            assert np.array_equal(got[k], ref[k]), k
+    assert held[1] < held[0] - (1 << 20) and held[2] == held[1]
+
+
+@pytest.mark.parametrize("n", [1, 300, 70000])
+def test_fit_boxes_under_a_limit(dev, n):
+    """FitBoxes without kept results: the write pass works every pair out again
+    and skips those that found nothing."""
+    rng = np.random.default_rng(n)
+    pairs = rng.random((n, 8)).astype(np.float32) * 64
+    pairs[1::3, 4:] = pairs[1::3, :4]                      # (some fail, some meet)
+    want = dev.fit_boxes(pairs)
+    with P.Device(0) as d:
+        d.set_pool_limit(1 << 40)
+        got = d.fit_boxes(pairs)
+    for k in want:
+        assert np.asarray(got[k]).tobytes() == np.asarray(want[k]).tobytes(), k
