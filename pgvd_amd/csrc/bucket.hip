@@ -10,17 +10,21 @@
 // Level 0 splits the keys by their top b bits (b chosen so that a bucket
 // averages well under CAP keys) in one or two LDS-staged scatters; every
 // bucket of at most CAP keys is then sorted inside one workgroup's LDS.
-// Buckets above CAP (clustered keys) go to further levels: a level first ORs
-// and ANDs each segment's keys, so it knows the segment's highest varying
-// bit hb (of OR ^ AND) and splits it on the 8 bits below hb -- never on bits
-// all its keys share.  Each level is that pass, a histogram, a per-segment
-// scan and a scatter; sub-buckets of at most CAP keys become
-// LDS sort items (consecutive small ones merged up to CAP), larger ones the
-// next level's segments.  A level consumes at least 8 varying bits, so a
-// 128-bit key needs at most 16 levels; a segment whose keys are all equal
-// (OR == AND) is copied, not split.  The host reads the segment count after
-// the level-0 plan and after each level's scan while the device keeps
-// working, and stops launching levels when none is left.
+// Buckets above CAP (clustered keys) are segments of the sample sort
+// (sample.hip); where they hold more than a quarter of the keys, the whole
+// array is left to that sort or to the LSD passes (bk_plan_kernel).  Only a
+// bucket too large for the sample sort that leaves the others most of the keys
+// (or has 128-bit keys) goes to further levels: a level first ORs and ANDs each
+// segment's keys, so it knows the segment's highest varying bit hb (of OR ^ AND)
+// and splits it on the 8 bits below hb -- never on bits all its keys share.
+// Each level is that pass, a histogram, a per-segment scan and a scatter;
+// sub-buckets of at most CAP keys become LDS sort items (consecutive small ones
+// merged up to CAP), larger ones the next level's segments.  A level consumes at
+// least 8 varying bits, so a 128-bit key needs at most 16 levels; a segment
+// whose keys are all equal (OR == AND) is copied, not split.  The host reads
+// the crowded buckets' counts after the level-0 plan and the segment count
+// after each level's scan while the device keeps working, and stops launching
+// levels when none is left.
 #include <chrono>
 
 #include "bucket_dev.hpp"

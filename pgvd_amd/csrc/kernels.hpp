@@ -106,7 +106,7 @@ constexpr size_t kBboxPartBytes = (size_t)kBboxParts * 8 * sizeof(float);
 // where the points allow.  fold: where the points leave at most 64 records
 // (one to a lane), they are left to launch_encode, whose vectorised form then
 // takes the box from them and puts it into st; returns how many records are
-// left so, else 0 (the box is in st): up to 524,283 3D points, a launch of
+// left so, else 0 (the box is in st): up to 524,287 3D points, a launch of
 // 1.9 us and its gap less, for a load in each wave of the encode.
 int launch_bbox(const float *pts, int64_t n, int dim, float *partials, RunState *st,
                 hipStream_t s, uint32_t *zero_words = nullptr, size_t nzero = 0,
@@ -286,9 +286,10 @@ void launch_parse_text(const uint8_t *text, int64_t len, int dim, int64_t N, int
 // ---- bucket.hip ----
 // The whole path's sort for 32/64/128-bit keys with optional u32 labels:
 // level 0 splits by the top b bits (b <= kBkMaxBits) and sorts every bucket
-// of at most bucket_cap<K>() keys in LDS; larger buckets go through levels
-// that split them below their highest varying bit.  The result (keys, and
-// labels in the same order) is in (kA, vA); not stable among equal keys.
+// of at most bucket_cap<K>() keys in LDS; larger buckets are segments of the
+// sample sort or, too large for it, go through levels that split them below
+// their highest varying bit.  The result (keys, and labels in the same order)
+// is in (kA, vA), or (kB, vB) where asked; not stable among equal keys.
 constexpr int kBkMaxBits = 14;
 constexpr int kBkMaxBuckets = 1 << kBkMaxBits;
 constexpr int kBkCursor1 = kBkMaxBuckets;                       // first scatter's cursors

@@ -10,8 +10,8 @@
 // written twice, where eight radix passes read and write them eight times.
 // A key that the sample holds twice gets a bucket of its own (its successor
 // is a splitter too), so repeated keys do not swell a bucket of distinct
-// ones.  A bucket above CAP (a rare sample, or a repeated key) goes to a
-// kernel that sorts it in global memory.
+// ones.  A bucket above CAP is written from its one key by many workgroups
+// (a repeated key) or sorted in global memory by one (a rare sample).
 //
 // Equal keys may come out in any order (their labels too), as from the bucket
 // sort.  No count comes back to the host: the launches depend only on the
@@ -64,7 +64,9 @@ __device__ inline SsOut ss_out(const SsPlan &p, uint32_t s, uint32_t prepend, Ru
   return {p.seg[s].kofs, pre, pre, &p.ss[s].dups};
 }
 
-// Deterministic 32-bit mix (the sample's position within its stratum).
+// Deterministic 32-bit mix (the sample's position within its stratum):
+// "lowbias32", a published xor-shift-multiply hash whose constants a search by
+// C. Wellons (hash-prospector) found.
 __device__ inline uint32_t mix32(uint32_t x) {
   x ^= x >> 16;
   x *= 0x7feb352du;
@@ -475,6 +477,9 @@ __global__ __launch_bounds__(kBlock) void ss_zero_kernel(uint32_t *counts, uint3
 
 }  // namespace
 
+// Keys that a bucket averages: with 16 samples to a bucket and room for 2.5 times
+// the average, one outgrows CAP where 40 expected samples drew 15 or fewer, some
+// 5 buckets in 10^6.
 template <typename K>
 int64_t ss_bucket_keys() { return (int64_t)SsItem<K>::CAP * 40 / 100; }
 

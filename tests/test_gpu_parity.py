@@ -45,11 +45,11 @@ def test_build_octree_matches_oracle(dev, n, dim, bits):
     assert_tree_equal(got, want, where=f"n={n} dim={dim} bits={bits}")
 
 
-@pytest.mark.parametrize("n,dim", [((1 << 18) - 1, 2), (1 << 18, 3), (524280, 3), (524300, 3)])
+@pytest.mark.parametrize("n,dim", [((1 << 18) - 1, 2), (1 << 18, 3), (524287, 3), (524288, 3)])
 def test_build_octree_at_the_small_forms_edges(dev, n, dim):
     """Either side of the sizes up to which the gather adds up its own chunks
     (2^18 - 1 points) and the encode takes the box from the 64 records of its
-    pass (524,283 3D points), the box reached by the last points alone."""
+    pass (524,287 3D points), the box reached by the last points alone."""
     pts = _pts(n, dim, seed=n) * np.float32(0.75)
     pts[-2:] = [[-1] * dim, [1] * dim]
     assert_tree_equal(dev.build_octree(pts, 16), oracle.build(oracle.quantize(pts, 1 << 16), 16),
