@@ -924,7 +924,8 @@ int launch_bucket_sort(const BucketArgs<K> &a, RunState *st, RunState *st_host, 
   // (bounded: past it, and after one scatter, the LSD passes follow an encode
   // that did not count their digits: 300,000 2D points of 40 bits in clusters
   // take 146 us whole and 163 so)
-  const int64_t whole_max = std::min(ss_max_whole<K>(bounded ? 64 : a.mbits), seg_max);
+  const int64_t whole_max = std::min(
+      bounded && sizeof(K) == 8 ? int64_t(1) << 19 : ss_max_whole<K>(a.mbits), seg_max);
   // the largest bucket with which crowded keys stay with the bucket sort
   const uint32_t crowd_max = sizeof(K) == 4 ? 0u : (uint32_t)seg_max;
   const int64_t n = a.n;

@@ -347,15 +347,17 @@ constexpr int64_t kSsMaxPlanBuckets = int64_t(1) << 22;
 template <typename K> int ss_buckets(int64_t n);
 template <typename K> int64_t ss_max_keys();   // the most that gives buckets
 // Largest crowded array that a build sorts whole by it.  Past it, its crowded
-// buckets are the segments, each with a sample of its own range: 10^6 points in
-// 8 clusters of sigma 1e-4 took 350 us a build whole and 242 so (3D, 63-bit
-// keys; 234 and 244 at sigma 0.1), 500,000 2D points (40 bits) 227 and 159 (167
-// and 162).  Arrays of 32-bit keys past it take the LSD passes, which are four:
-// 300,000 3D points at 10 bits/axis 153 us whole and 130 so (148 and 153), 10^6
-// 253 and 159 (207 and 202).
+// buckets are the segments, each with a sample of its own range: of 40-bit keys
+// (whose five LSD passes are the mark), 500,000 2D points in 8 clusters of sigma
+// 1e-4 took 210 us a build whole and 159 so (165 and 161 at sigma 0.1), 300,000
+// 191 and 184 (146 and 148).  10^6 3D points (63-bit keys) take 281 us whole and
+// 242 so in those tight clusters, but 224 and 250 in clusters of sigma 0.01 to
+// 0.1: they stay whole (278 by the LSD passes).  Arrays of 32-bit keys past it
+// take the LSD passes, which are four: 300,000 3D points at 10 bits/axis 153 us
+// whole and 130 so (148 and 153), 10^6 253 and 159 (207 and 202).
 template <typename K> int64_t ss_max_whole(int mbits) {
   if (sizeof(K) == 4) return int64_t(1) << 16;
-  return mbits > 48 ? int64_t(1) << 19 : int64_t(1) << 18;
+  return mbits > 48 ? ss_max_keys<K>() : int64_t(3) << 17;
 }
 template <typename K> int ss_tile();
 template <typename K> size_t ss_ws_bytes(int64_t buckets, int64_t segs, int64_t slots);
