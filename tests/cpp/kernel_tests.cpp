@@ -17,6 +17,16 @@
 
 using namespace pgvd;
 
+#ifdef __has_feature
+#if __has_feature(address_sanitizer)
+// The sanitizer keeps freed blocks, device buffers among them, in a quarantine
+// and gives the oldest back when it is full.  Filled by the runtime's own frees
+// after it has unloaded the device, it fails its check that the device is there;
+// it holds all that these scenarios free instead.
+extern "C" const char *__asan_default_options() { return "quarantine_size_mb=16384"; }
+#endif
+#endif
+
 static int failures = 0;
 #define CHECK(cond, what)                                                   \
   do {                                                                      \
